@@ -697,7 +697,10 @@ extern "C" int pmpm_context_create(pmpm_context **ctx) {
   const char *hint_min = getenv("PMPM_PARTITION_HINT_MIN");
   if (hint_min && hint_min[0]) c->hint_min_particles = (int32_t)strtol(hint_min, nullptr, 10);
   if (!hip_ok(hipMalloc(&c->counters, 4 * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
-  if (!hip_ok(hipMemset(c->counters, 0, 4 * sizeof(uint32_t)), "hipMemset")) {
+  // (waited for: the context's first call may be on a stream that is not
+  // ordered after the null stream)
+  if (!hip_ok(hipMemset(c->counters, 0, 4 * sizeof(uint32_t)), "hipMemset") ||
+      !hip_ok(hipStreamSynchronize(nullptr), "hipStreamSynchronize")) {
     (void)hipFree(c->counters);
     delete c;
     return PMPM_ERR_HIP;

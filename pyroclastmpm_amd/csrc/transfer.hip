@@ -2728,7 +2728,10 @@ static size_t wrap_node_list_words(const pmpm_params &prm, const pmpm_grid &g) {
   const size_t cap = (size_t)(prm.dim == 3 ? wrap_target_count<3>(g) : (prm.dim == 2 ? wrap_target_count<2>(g) : 0));
   return (size_t)kWrapListShards * (1 + cap);
 }
-static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g) {
+// (new flags and counts are cleared on s, the stream that uses them first: a
+// hipMemset on the null stream returns before the fill is done and is not
+// ordered before work on a non-blocking stream, such as a batch's lanes)
+static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, hipStream_t s) {
   size_t floats = 0, tiles = 0;
   partial_sizes(prm, g, &floats, &tiles);
   int rc = ensure_partials(ctx, floats, tiles);
@@ -2745,7 +2748,7 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   const size_t words = ((size_t)g.num_cells_total + 3) / 4;
   if (words > ctx->wrap_touch_cap) {
     if ((rc = ensure_buffer(ctx->wrap_touch, ctx->wrap_touch_cap, words)) != PMPM_OK) return rc;
-    PMPM_HIP_CHECK(hipMemset(ctx->wrap_touch, 0, words * sizeof(float)));
+    if ((rc = zero_fill(ctx->wrap_touch, (int64_t)words, s)) != PMPM_OK) return rc;
   }
   // the gather's list: kWrapListShards counts, then as many parts of room
   // for every node the wrap-around can reach
@@ -2756,7 +2759,7 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
     if ((rc = ensure_buffer(lb, cap, lwords)) != PMPM_OK) return rc;
     ctx->wrap_list = reinterpret_cast<int32_t *>(lb);
     ctx->wrap_list_cap = cap;
-    PMPM_HIP_CHECK(hipMemset(ctx->wrap_list, 0, kWrapListShards * sizeof(int32_t)));
+    if ((rc = zero_fill(ctx->wrap_list, kWrapListShards, s)) != PMPM_OK) return rc;
   }
   return PMPM_OK;
 }
@@ -2835,7 +2838,7 @@ static int launch_wrap_gather(pmpm_context *ctx, const pmpm_params &prm, const p
 // (zeroed: the caller has already cleared mass, mom and mom_nt)
 int do_p2g(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &p,
            const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s, bool zeroed = false) {
-  int rc = reserve_tiles(ctx, prm, g);
+  int rc = reserve_tiles(ctx, prm, g, s);
   if (rc != PMPM_OK) return rc;
   if (!zeroed && (rc = do_zero_nodes(prm, g, nodes, s)) != PMPM_OK) return rc;
   PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags,
@@ -2880,7 +2883,7 @@ int do_g2p(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
 int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
                 const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s,
                 bool zeroed = false) {
-  int rc = reserve_tiles(ctx, prm, g);
+  int rc = reserve_tiles(ctx, prm, g, s);
   if (rc != PMPM_OK) return rc;
   // the fused pass reads the node velocity records, never mom_nt: clear it
   // for the re-map's wrap-around atomics first
@@ -3734,7 +3737,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
     if ((rc = pmpm_partition(ctx, D, grid, state->x, n, part, stream)) != PMPM_OK) return rc;
     if ((rc = do_p2g(ctx, *prm, g, *state, *part, *nodes, s)) != PMPM_OK) return rc;
     if ((rc = launch_grid(ctx, *prm, g, *nodes, 1, 0, prm->num_bcs, 0, 1, s)) != PMPM_OK) return rc;
-  } else if ((rc = reserve_tiles(ctx, *prm, g)) != PMPM_OK) {
+  } else if ((rc = reserve_tiles(ctx, *prm, g, s)) != PMPM_OK) {
     return rc;
   }
   if ((rc = ensure_buffer(ctx->adj_rec, ctx->adj_rec_cap, (size_t)15 * n)) != PMPM_OK) return rc;
