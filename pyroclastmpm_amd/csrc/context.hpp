@@ -180,10 +180,12 @@ bool params_ok(const pmpm_params *prm);
 bool step_args_ok(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *a, const pmpm_particles *b,
                   const pmpm_spatial *part, const pmpm_nodes *nodes);
 // Workspace the P2G passes of one step use on grid g: tile partials (floats)
-// and tile flags, wrap-around records (floats) and wrap cells.
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, size_t *partial_floats, size_t *tiles,
-                   size_t *wrap_floats, size_t *wrap_cells, size_t *wrap_touch_words, size_t *wrap_list_words,
-                   size_t *clamp_words);
+// and tile flags, the 2D typed-cubic wrap-around's records (floats), node
+// flags and node list (words), the clamp record (words).
+struct P2GWorkspace {
+  size_t partial_floats, tiles, wrap_floats, touch_words, list_words, clamp_words;
+};
+void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w);
 // pmpm_partition whose first kernel also clears the buffers of `extra`.
 int partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, const float *x, int n, pmpm_spatial *part,
                        hipStream_t s, const ZeroLists &extra);

@@ -15,7 +15,7 @@ int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
                 const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s,
                 bool zeroed);
 int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, int finalize,
-                int b0, int b1, int remap, int gather, hipStream_t s, int clear_mom_nt);
+                int b0, int b1, int remap, int gather, hipStream_t s, int n, int clear_mom_nt);
 }  // namespace pmpm
 
 using namespace pmpm;
@@ -38,10 +38,10 @@ int pmpm::step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *gr
   int rc = partition_clearing(ctx, prm->dim, grid, a->x, a->n, part, s, z);
   if (rc != PMPM_OK) return rc;
   if ((rc = do_p2g(ctx, *prm, *grid, *a, *part, *nodes, s, true)) != PMPM_OK) return rc;
-  if ((rc = launch_grid(ctx, *prm, *grid, *nodes, 1, 0, prm->num_bcs, 0, 1, s, musl ? 1 : 0)) != PMPM_OK) return rc;
+  if ((rc = launch_grid(ctx, *prm, *grid, *nodes, 1, 0, prm->num_bcs, 0, 1, s, a->n, musl ? 1 : 0)) != PMPM_OK) return rc;
   if (!musl) return do_g2p(*prm, *grid, *a, *b, *part, *nodes, 0, s);
   if ((rc = do_musl_map(ctx, *prm, *grid, *a, *b, *part, *nodes, s, true)) != PMPM_OK) return rc;
-  if ((rc = launch_grid(ctx, *prm, *grid, *nodes, 0, 0, prm->num_bcs, 1, 2, s, 0)) != PMPM_OK) return rc;
+  if ((rc = launch_grid(ctx, *prm, *grid, *nodes, 0, 0, prm->num_bcs, 1, 2, s, a->n, 0)) != PMPM_OK) return rc;
   return do_g2p(*prm, *grid, *a, *b, *part, *nodes, 2, s);
 }
 

@@ -326,6 +326,19 @@ __device__ inline void node_ids(const pmpm_grid &g, int64_t lin, int *ids) {
   ids[2] = (D > 2) ? (int)(lin / ((int64_t)g.num_cells[0] * g.num_cells[1])) : 0;
 }
 
+// node_ids in 32 bits (grids hold fewer than PMPM_MAX_GRID_NODES nodes).
+template <int D> __device__ inline void node_ids32(const pmpm_grid &g, int lin, int *ids) {
+  const uint32_t nx = (uint32_t)g.num_cells[0], row = (uint32_t)lin / nx;
+  ids[0] = (int)((uint32_t)lin - row * nx);
+  if (D > 1) {
+    const uint32_t ny = (uint32_t)g.num_cells[1], layer = D > 2 ? row / ny : 0u;
+    ids[1] = (int)(row - layer * ny);
+    ids[2] = D > 2 ? (int)layer : 0;
+  } else {
+    ids[1] = ids[2] = 0;
+  }
+}
+
 // Slow path of the scatter: every entry goes straight to global memory,
 // through the linear index (wrap-around reproduced when wrap_quirk is set).
 // Used for particles whose bin is not their cell's coordinates and for the
@@ -1103,72 +1116,146 @@ __global__ __launch_bounds__((P2GGeom<D, SF>::THREADS)) __attribute__((amdgpu_wa
   }
 }
 
-// P2G of one tile on the matrix cores (3D, cubic splines with node types):
-// the same tiles, slices and results as p2g_kernel MODE 0, with the per-cell
-// sums done by v_mfma_f32_16x16x4_f32. For one cell and its 4 x 4 x 4 node
-// window, with i, j, k the x, y, z node offsets and p the cell's particles,
-//   C1[(i, f)][(j, k)] = sum_p (Nx_i F_f)(p) (Ny_j Nz_k)(p),  F = (m, m v)
-//   C2[(i, a)][(j, k)] = sum_p (dNx_i A_ax)(Ny_j Nz_k) + (Nx_i A_ay)(dNy_j Nz_k)
-//                              + (Nx_i A_az)(Ny_j dNz_k),       A = -V sigma
-// which are the mass, momentum and force deposits (usl_inline.h:114-160) as
-// 16 x 16 products over K = particles, four particles per instruction. In the
-// instruction's layout lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16]
-// and receives D[4 (l / 16) + r][l % 16]: it evaluates x and y weights at
-// offset (l % 16) / 4 and the z weight at offset l % 4 for particle l / 16,
-// and owns node (i = l / 16, j = (l % 16) / 4, k = l % 4) of the result.
-// Wave w walks the 16 cells of z layer w one after another: it stages up to
-// 32 of a cell's particles in LDS (lane = particle, coalesced loads; the 24
-// span weights and derivatives and the products m v, -V sigma computed once
-// per particle), so an instruction's operands are a record read and one
-// multiply; it runs the products on four independent accumulators and adds
-// each lane's node into the wave's own LDS node block; the four blocks
-// overlap in z and are summed into the tile slice at the end.
-struct MfmaGeom {
-  // The tile: CELLS x 1 x 4 cells, one z layer per wave. Eight cells per
-  // wave keep a workgroup short enough that the chip's workgroup slots are
-  // refilled evenly (a tile is the unit of work, and a column whose x
-  // extent ends inside a tile leaves it partly empty).
-  static constexpr int CELLS = 8;                       // cells per wave (x)
-  static constexpr int BX = CELLS + 3, BY = 4, BZ = 4;  // a wave's node block
-  static constexpr int TZ = 4, NZ = TZ + 3;             // tile layers, slice node layers
-  static constexpr int NTN = BX * BY * NZ;              // nodes of one partial slice
-  // x pitch of the block in LDS: the 64 lanes of a flush, offsets
-  // pk + 12 s1 + 48 s2, fall into 64 distinct banks
-  static constexpr int BXP = BX + 1;
-  static constexpr int BN = BXP * BY * BZ;
-  static constexpr int CH = 32;  // particles staged per round
-  // a staged particle's record: per span offset s (7 s + 0..6) the weights
-  // Nx, dNx, Ny, dNy, Nz, dNz and mass / moment field s (m, m vx, m vy,
-  // m vz), then A = -V sigma (28..33: xx, yy, zz, xy, xz, yz) and a zero
-  // (34); the odd pitch puts the 16 records one read touches on distinct
-  // banks
-  static constexpr int RS = 35;
+// Per-axis weights of one fixed span offset as polynomials of the fraction
+// f = t - bin, for lanes that own one offset per axis: the coefficients are
+// set once per cell (or wave) and a weight costs a few multiply-adds.
+//
+// Cubic: N = a0 + a1 f + a2 f^2 + a3 f^3 of node type 0-3 at span offset s
+// (the piece 3 - s of the boundary-modified spline, cubic.cuh:28-197, in
+// powers of f instead of r = f + 1 - s: smaller coefficients, so less
+// cancellation near the spline's end than the r form).
+__device__ __constant__ static const float kSpanCubic[4][4][4] = {
+    {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+    {{1.f / 6.f, -0.5f, 0.5f, -1.f / 6.f}, {1.f, -1.f, 0.f, 1.f / 6.f}, {1.f / 6.f, 0.5f, 0.5f, -1.f / 6.f}, {0.f, 0.f, 0.f, 1.f / 6.f}},
+    {{1.f / 6.f, -0.5f, 0.5f, -1.f / 6.f}, {2.f / 3.f, 0.f, -1.f, 0.5f}, {0.f, 1.f, 0.f, -1.f / 3.f}, {0.f, 0.f, 0.f, 0.f}},
+    {{1.f / 6.f, -0.5f, 0.5f, -1.f / 6.f}, {2.f / 3.f, 0.f, -1.f, 0.5f}, {1.f / 6.f, 0.5f, 0.5f, -0.5f}, {0.f, 0.f, 0.f, 1.f / 6.f}}};
+
+template <int SF> struct SpanPoly;
+template <> struct SpanPoly<PMPM_SF_CUBIC> {
+  float a0, a1, a2, a3, d1, d2, d3;
+  // offset s, type of the node there; keep = 0 drops the offset
+  __device__ inline void set(int s, int type, float inv_h, float keep) {
+    const float4 c = *reinterpret_cast<const float4 *>(&kSpanCubic[type][s][0]);
+    a0 = keep * c.x; a1 = keep * c.y; a2 = keep * c.z; a3 = keep * c.w;
+    d1 = inv_h * a1; d2 = inv_h * (2.f * a2); d3 = inv_h * (3.f * a3);
+  }
+  __device__ inline float N(float f) const { return ((a3 * f + a2) * f + a1) * f + a0; }
+  __device__ inline float dN(float f) const { return (d3 * f + d2) * f + d1; }
+};
+// Quadratic: N = c0 + c1 b^2, dN = d1 b with b = f - e; one set for f < 1/2,
+// one above. Offset s is 0 where the particle's window does not reach it.
+template <> struct SpanPoly<PMPM_SF_QUADRATIC> {
+  float e[2], c0[2], c1[2], d1[2];
+  __device__ inline void set(int s, int, float inv_h, float keep) {
+    // f < 1/2: 0.5 (f - 0.5)^2, 0.75 - f^2, 0.5 (f + 0.5)^2, 0
+    // else:    0, 0.5 (f - 1.5)^2, 0.75 - (f - 1)^2, 0.5 (f - 0.5)^2
+    e[0] = s == 0 ? 0.5f : (s == 2 ? -0.5f : 0.f);
+    e[1] = s == 1 ? 1.5f : (s == 2 ? 1.f : 0.5f);
+    const float lo = s == 3 ? 0.f : (s == 1 ? -1.f : 0.5f), hi = s == 0 ? 0.f : (s == 2 ? -1.f : 0.5f);
+    c0[0] = keep * (s == 1 ? 0.75f : 0.f);
+    c0[1] = keep * (s == 2 ? 0.75f : 0.f);
+    c1[0] = keep * lo;
+    c1[1] = keep * hi;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) d1[k] = inv_h * (2.f * c1[k]);
+  }
+  __device__ inline float N(float f) const {
+    const bool h = f >= 0.5f;
+    const float b = f - (h ? e[1] : e[0]);
+    return (h ? c1[1] : c1[0]) * (b * b) + (h ? c0[1] : c0[0]);
+  }
+  __device__ inline float dN(float f) const {
+    const bool h = f >= 0.5f;
+    return (h ? d1[1] : d1[0]) * (f - (h ? e[1] : e[0]));
+  }
+};
+// Linear: N = c0 + c1 f; the derivative is 0 on a node (linear_eval).
+template <> struct SpanPoly<PMPM_SF_LINEAR> {
+  float c0, c1, d, d_at0;
+  __device__ inline void set(int s, int, float inv_h, float keep) {
+    const float k = s > 1 ? 0.f : keep;
+    c0 = s == 0 ? k : 0.f;
+    c1 = s == 0 ? -k : k;
+    d = inv_h * c1;
+    d_at0 = s == 0 ? 0.f : d;
+  }
+  __device__ inline float N(float f) const { return c1 * f + c0; }
+  __device__ inline float dN(float f) const { return f == 0.f ? d_at0 : d; }
+};
+
+// The matrix-core P2G of 3D scenes. Tile: CELLS x 1 x 4 cells, one wave per z
+// layer walking its CELLS cells along x.
+template <int SF, int CELLS, int NV> struct MfmaGeom {
+  static constexpr int SPAN = Spline<SF>::SPAN, NLO = Spline<SF>::NLO;
+  static constexpr int TZ = 4;                                      // waves (z layers) per tile
+  static constexpr int BX = CELLS + SPAN - 1, NZ = TZ + SPAN - 1;   // tile nodes along x and z (y: SPAN)
+  static constexpr int NTN = BX * SPAN * NZ;                        // nodes of one partial slice
+  // a wave's node columns in LDS, [field][x][4 y + z]: x pitch 17 and field
+  // pitch 16 mod 64, so that a flush (4 fields x 16 nodes) and the reads
+  // along x of the final sum fall into disjoint banks
+  static constexpr int XP = 17;
+  static constexpr int BN = (BX * XP - 16 + 63) / 64 * 64 + 16;
+  static_assert(BN >= BX * XP && BN % 64 == 16, "field pitch");
+  static_assert((BX - 1) / CELLS + 1 <= kCoverX && (NZ - 1) / TZ + 1 <= kCoverZ,
+                "the grid kernel's gather visits at most kCover tiles per axis");
+  static constexpr int CH = 64;  // particle rows staged per round, one per lane
 };
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// REMAP: the MUSL re-map instead (p2g_kernel MODE 1's deposit): m v' with v'
-// from slot j of `out` (written by the first map, g2p_kernel MODE 1) and the
-// weights of the old positions; the slice holds the 3 momentum fields.
-// FEXT: the step has planar-domain walls; each particle's wall force f
-// (planar_force) is staged too and w f joins the force product through its
-// A operand (Nx f_a next to dNx A_a.x, both against Ny Nz).
-template <int SF, bool REMAP = false, bool FEXT = false>
+// P2G of one tile on the matrix cores (3D, every spline).
+//   MODE 0: mass, momentum, force (FEXT: with planar-domain wall forces).
+//   MODE 1: the MUSL re-map of m v', v' from slot j of `out` (written by the
+//           first map, g2p_kernel MODE 1), weights of the old positions.
+//   MODE 2: adjoint scatter of the G2P record adjoints `rec` (cell order).
+// Per cell and its SPAN^3 node window, with i, j, k the x, y, z node offsets
+// and p the cell's particles, v_mfma_f32_16x16x4_f32 forms
+//   C1[(f, i)][(j, k)] = sum_p (Nx_i F_f)(p) (Ny_j Nz_k)(p),  F = (m, m v)
+//   C2[(a, i)][(j, k)] = sum_p (dNx_i A_ax [+ Nx_i fext_a])(Ny_j Nz_k)
+//                              + (Nx_i A_ay)(dNy_j Nz_k) + (Nx_i A_az)(Ny_j dNz_k),  A = -V sigma
+// (usl_inline.h:114-160), four particles per instruction; MODE 2 sums
+// (v_pic adjoint, dv adjoint) and the L adjoint's rows the same way. Lane l
+// supplies A[l % 16][l / 16] and B[l / 16][l % 16] and receives
+// D[4 (l / 16) + r][l % 16]: it evaluates the x and z weights at offset l % 4
+// and the y weight at offset (l % 16) / 4 for particle l / 16, and owns field
+// l / 16 of the nodes (r, j, k). The x offset being the register index, moving
+// on to the next cell is a register rotation: only the leftmost node column
+// leaves, and each column of the wave's row is written once, complete.
+//
+// What bounds it: instruction issue. Per four particles there are 4 (MODE 1:
+// 1) matrix instructions of 32 cycles and about 45 vector instructions, so
+// the weights are evaluated here from per-lane coefficients (about 20
+// multiply-adds) instead of being staged: a particle's LDS record is 20
+// floats written by one lane and read with two 16-byte broadcasts and one
+// word. The rows of a round are the wave's particles in sorted order, each
+// cell padded to a multiple of four, so a round fills its 64 lanes whatever
+// the particles per cell (at 8 per cell staging cell by cell left 3 of 4
+// lanes idle); the next round's fields load while a round is multiplied.
+//
+// Linear-index wrap-around (usl_inline.h:122-126; shapefunction.cpp:96-112):
+// a node offset outside the grid stays in the tile as a virtual node, with
+// the spline types of the node its linear index reaches (types matter to the
+// cubic spline only), and the grid kernel adds virtual nodes to the nodes
+// they reach. A carry out of x shifts the y index by one, so the x offsets
+// that leave the grid (cells next to an x face) are multiplied in a pass of
+// their own, with that carry's y and z types and the other x offsets' weights
+// zero; the carry out of y only changes the lane's own z type.
+template <int SF, int MODE, int CELLS, bool FEXT = false>
 __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles in,
                                                        pmpm_particles out, pmpm_spatial part, pmpm_nodes nodes,
                                                        int tiles_x, int tiles_y, float *__restrict__ partials,
-                                                       int32_t *__restrict__ flags) {
-  using G = P2GGeom<3, SF>;
-  using M = MfmaGeom;
-  static_assert(G::SPAN == 4 && G::NLO == -1, "cubic spans");
-  static_assert((M::BX - 1) / M::CELLS + 1 <= kCoverX && (M::NZ - 1) / M::TZ + 1 <= kCoverZ,
-                "the grid kernel's gather visits at most kCover tiles per axis");
-  constexpr int NV = REMAP ? 3 : 7, NTN = M::NTN, NLO = G::NLO;
-  static_assert(NV == p2g_nv<3, REMAP ? 1 : 0>(), "slice fields of the matching p2g_kernel mode");
-  static_assert(!(REMAP && FEXT), "the re-map carries no force");
-  constexpr int RS = M::RS + (FEXT ? 4 : 0);  // record pitch (35..37: wall force)
-  __shared__ float block[4][NV][M::BN];
-  __shared__ float stage[4][M::CH * RS];
-  __shared__ __attribute__((aligned(16))) float s_coef[5][4][4];
+                                                       int32_t *__restrict__ flags, const float *__restrict__ rec) {
+  constexpr int NV = p2g_nv<3, MODE>();
+  using M = MfmaGeom<SF, CELLS, NV>;
+  static_assert(MODE == 0 || !FEXT, "only the P2G carries the wall force");
+  static_assert(CELLS == 4 || CELLS == 8, "cells per wave");
+  constexpr int SPAN = M::SPAN, NLO = M::NLO, CH = M::CH, BN = M::BN;
+  constexpr bool TYPED = SF == PMPM_SF_CUBIC;
+  // floats of a staged record: the fractions, then MODE 0: (m, m v) and the
+  // rows of A with the wall force; MODE 1: m v'; MODE 2: per component
+  // (v_pic adjoint, L adjoint's column), dv.x, then (dv.y, dv.z)
+  constexpr int RS = MODE == 0 ? 20 : (MODE == 1 ? 8 : 24);
+  __shared__ float block[4][NV * BN];
+  __shared__ __attribute__((aligned(16))) float stage[4][CH * RS];
 
   const int n = in.n;
   const float inv_h = g.inv_cell_size;
@@ -1176,276 +1263,250 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
   const int bx = blockIdx.x % tiles_x;
   const int by = (blockIdx.x / tiles_x) % tiles_y;
   const int bz = blockIdx.x / (tiles_x * tiles_y);
-  const int cy = by, cz = bz * 4 + wave;  // this wave's cell row
-  // lanes 0..15 hold the ranges of the wave's 16 cells
+  const int cy = by, cz = bz * M::TZ + wave;  // this wave's cell row
+  // lanes 0..CELLS-1 hold the ranges of the wave's cells
   int cs = 0, ce = 0;
   {
-    const int cx = bx * M::CELLS + (lane & 15);
-    if (lane < 16 && cx < g.num_cells[0] && cy < g.num_cells[1] && cz < g.num_cells[2]) {
+    const int cx = bx * CELLS + lane;
+    if (lane < CELLS && cx < g.num_cells[0] && cz < g.num_cells[2]) {
       const int cell = cx + g.num_cells[0] * (cy + g.num_cells[1] * cz);
       ce = part.cell_end[cell];
       cs = part.cell_start[cell];
     }
   }
-  if (t < 80) (&s_coef[0][0][0])[t] = (&kCubic[0][0][0])[t];
-  if (!__syncthreads_or(ce > cs)) {
+  const bool none = TYPED && !prm.node_types_built;  // untyped cubic weights are zero
+  if (!__syncthreads_or(ce > cs) || none) {
     if (t == 0) flags[blockIdx.x] = 0;
     return;
   }
-  float *blk = &block[wave][0][0];
-  for (int i = lane; i < NV * M::BN; i += 64) blk[i] = 0.f;
+  float *blk = &block[wave][0];
   float *st = &stage[wave][0];
-
-  // lane roles in the products
-  const int s1 = (lane & 15) >> 2, s2 = lane & 3, pk = lane >> 4;
-  // staged entries this lane reads (a particle's record, RS floats): the
-  // weights of its offsets (x and y at s1, z at s2), mass / moment field s2,
-  // row a = s2 of A = -V sigma (row 3 of the product is padding and reads the
-  // record's zero) and, with walls, force component s2
-  const int ex = 7 * s1, ez = 7 * s2;
-  const int ax = s2 == 0 ? 28 : (s2 == 1 ? 31 : (s2 == 2 ? 32 : 34));
-  const int ay = s2 == 0 ? 31 : (s2 == 1 ? 29 : (s2 == 2 ? 33 : 34));
-  const int az = s2 == 0 ? 32 : (s2 == 1 ? 33 : (s2 == 2 ? 30 : 34));
-  const int af = s2 < 3 ? 35 + s2 : 34;
-  // span coefficients: piece 3 - s of the type of the node at offset s,
-  // read from the LDS copy of the table (the types: y and z fixed for the
-  // wave's row, x per cell; wave-uniform)
-  int tys[4], tzs[4], txs[4];
+  // rows of a cell: its particles, padded to a multiple of four
+  const int pad = (max(ce - cs, 0) + 3) & ~3;
+  int rend = pad;  // inclusive sum over the cells
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    tys[s] = cubic_node_type(cy + NLO + s, g.num_cells[1], prm.node_types_built);
-    tzs[s] = cubic_node_type(cz + NLO + s, g.num_cells[2], prm.node_types_built);
-    txs[s] = 0;
+  for (int o = 1; o < CELLS; o <<= 1) {
+    const int u = __shfl_up(rend, o, 64);
+    if (lane >= o) rend += u;
   }
-  auto coef = [&](int type, int s) { return reinterpret_cast<const float4 *>(&s_coef[type][3 - s][0])[0]; };
-  // cubic piece at r (offset s of the span), value and derivative; offset 0
-  // at frac = 1 - 2^-24 rounds to r = 2, where the spline is 0 (span_eval)
-  auto piece = [&](const float4 c, float r, bool first, float &N, float &dN) {
-    N = ((c.w * r + c.z) * r + c.y) * r + c.x;
-    dN = inv_h * ((3.f * c.w * r + 2.f * c.z) * r + c.y);
-    if (first && !(r < 2.f)) N = dN = 0.f;
-  };
+  int row_end[CELLS];
+#pragma unroll
+  for (int l = 0; l < CELLS; ++l) row_end[l] = __builtin_amdgcn_readlane(rend, l);
+  const int total = row_end[CELLS - 1];
+  const int shift = cs - (rend - pad);  // sorted index of a row, minus the row
 
-  // The wave walks its cells' particles in chunks of up to CH (lane =
-  // particle), cell by cell. Loads run ahead of the work: while a chunk's
-  // products run, the next chunk's particle fields and the slots of the one
-  // after are in flight, so the latency of the dependent slot -> field loads
-  // hides behind the products of the chunk before.
-  // a chunk: cell lx of the row, particles [w0, w0 + CH) of its range; the
-  // ranges are read from lanes 0..15 with scalar lane reads (the chunk walk
-  // stays in scalar registers)
-  auto cs_of = [&](int l) { return __builtin_amdgcn_readlane(cs, l); };
-  auto ce_of = [&](int l) { return __builtin_amdgcn_readlane(ce, l); };
-  auto first_chunk_from = [&](int l0, int &lx, int &w0) {  // wave-uniform
-    lx = M::CELLS;
-    for (int l = l0; l < M::CELLS; ++l) {
-      const int a = cs_of(l), b = ce_of(l);
-      if (b > a) { lx = l; w0 = a; return; }
-    }
-  };
-  auto next_chunk = [&](int lx, int w0, int &nlx, int &nw0) {
-    if (w0 + M::CH < ce_of(lx)) { nlx = lx; nw0 = w0 + M::CH; return; }
-    first_chunk_from(lx + 1, nlx, nw0);
-  };
-  // raw fields of one particle of a chunk, held in registers until staged.
-  // The loads are unconditional (lanes past the chunk read the chunk's last
-  // particle) so that no branch or select waits for them: they stay in
-  // flight while the chunk before is staged and multiplied.
+  // a particle's raw fields, held in registers until staged
   struct Raw {
-    int slot;
+    int slot, cx;
     bool valid;
     float x[3], v[3], m, vol;
     Sym sg;
+    float dv[3], Lb[9];
   };
-  // (lx == CELLS: no chunk; its loads read particle 0 and stage nothing, so
-  // that every step issues the same loads)
-  auto chunk_len = [&](int lx, int w0) { return lx < M::CELLS ? min(M::CH, ce_of(lx) - w0) : 0; };
-  // lanes l and l + CH hold the same particle (see stage_raw)
-  static_assert(M::CH == 32, "two lanes per staged particle");
-  const int prow = lane & (M::CH - 1);
-  auto chunk_j = [&](int lx, int w0) {  // this lane's sorted index, clamped to the chunk
-    return lx < M::CELLS ? w0 + min(prow, chunk_len(lx, w0) - 1) : 0;
-  };
-  auto chunk_slot = [&](int lx, int w0) { return part.sorted[chunk_j(lx, w0)]; };
-  auto load_raw = [&](int lx, int w0, int slot, Raw &r) {
+  auto load_raw = [&](int r0, Raw &r) {
+    const int row = r0 + lane;
+    int c = 0;
+#pragma unroll
+    for (int l = 0; l < CELLS - 1; ++l) c += row >= row_end[l] ? 1 : 0;
+    const int j = __shfl(shift, c) + row, je = __shfl(ce, c);
+    r.cx = bx * CELLS + c;
+    r.valid = row < total && j < je;
+    const int jj = r.valid ? j : 0;
+    const int slot = part.sorted[jj];
     r.slot = slot;
-    r.valid = prow < chunk_len(lx, w0);
-    const int j = chunk_j(lx, w0);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       r.x[a] = in.x[a * n + slot];
-      r.v[a] = REMAP ? out.v[a * n + j] : in.v[a * n + slot];
+      r.v[a] = MODE == 0 ? in.v[a * n + slot] : (MODE == 1 ? out.v[a * n + jj] : rec[a * n + jj]);
     }
-    r.m = in.mass[slot];
-    r.vol = REMAP ? 0.f : in.volume[slot];
-    r.sg = REMAP ? sym_zero() : load_sym(in.stress, n, slot);
-  };
-  // a chunk's particle records into the LDS stage: lanes l and l + 32 both
-  // hold particle l (row l) and each writes half of its record, half h =
-  // lane / 32 the weights of span offsets s = 2h, 2h + 1 with their fields,
-  // and half of A (the same instructions on both halves, so a record costs
-  // half the instructions of one lane per particle). The records past the
-  // chunk's particles are zero.
-  auto stage_raw = [&](int lx, const Raw &r) {
-    const int h = lane >> 5;
-    float *sp = st + prow * RS;
-    if (!r.valid) {
-      if (h == 0) {
+    r.m = MODE == 2 ? 1.f : in.mass[slot];
+    r.vol = MODE == 0 ? in.volume[slot] : 0.f;
+    r.sg = MODE == 0 ? load_sym(in.stress, n, slot) : sym_zero();
+    if (MODE == 2) {
 #pragma unroll
-        for (int e = 0; e < RS; ++e)
-          if (!REMAP || (e < 28 && (e % 7) % 2 == 0)) sp[e] = 0.f;  // (the entries the products read)
-      }
-      return;
+      for (int a = 0; a < 3; ++a) r.dv[a] = rec[(3 + a) * n + jj];
+#pragma unroll
+      for (int a = 0; a < 9; ++a) r.Lb[a] = rec[(6 + a) * n + jj];
     }
-    const int cx = bx * M::CELLS + lx;
+  };
+  // this lane's particle into its row of the stage (zero past the cell's
+  // particles, and for a particle that is not its own cell's)
+  auto stage_raw = [&](const Raw &r) {
     float fr[3];
-    bool own = true;
+    bool own = r.valid;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const float ta = cell_coord(r.x[a], g.origin[a], inv_h);
       const int ba = (int)ta;
-      own = own && ta >= 0.f && ba == (a == 0 ? cx : (a == 1 ? cy : cz));
+      own = own && ta >= 0.f && ba == (a == 0 ? r.cx : (a == 1 ? cy : cz));
       fr[a] = __fsub_rn(ta, (float)ba);
     }
+    float4 *sp = reinterpret_cast<float4 *>(st + lane * RS);
     Sym A = sym_zero();
     float fe[3] = {0.f, 0.f, 0.f};
-    if (!REMAP) {
+    if (MODE == 0) {
       const float mvol = -r.vol;
       A = Sym{mvol * r.sg.xx, mvol * r.sg.yy, mvol * r.sg.zz, mvol * r.sg.xy, mvol * r.sg.xz, mvol * r.sg.yz};
-      if (FEXT) planar_force<3>(prm, g, r.x, r.v, r.vol, r.m, fe);
+      if (FEXT && r.valid) planar_force<3>(prm, g, r.x, r.v, r.vol, r.m, fe);
     }
-    if (!own && h == 0) {
+    if (MODE != 2 && r.valid && !own) {
       // listed in this cell but binned elsewhere (a partition of other
-      // positions): deposited over its own window, no product terms here
+      // positions): deposited over its own window (MODE 2 runs on a
+      // partition of the same positions)
 #pragma unroll 1
       for (int sy = 0; sy < 4; ++sy)
-        p2g_stray<3, SF, REMAP ? 1 : 0>(prm, g, nodes, in.x, n, r.slot, sy, r.m, r.v, A, fe);
+        p2g_stray<3, SF, MODE == 1 ? 1 : 0>(prm, g, nodes, in.x, n, r.slot, sy, r.m, r.v, A, fe);
     }
-    const float keep = own ? 1.f : 0.f;
+    // (a row without an own particle is zero even if the fields it loaded
+    // are not finite)
+    sp[0] = own ? make_float4(fr[0], fr[1], fr[2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (MODE == 0) {
+      sp[1] = own ? make_float4(r.m, r.m * r.v[0], r.m * r.v[1], r.m * r.v[2]) : z4;
+      sp[2] = own ? make_float4(A.xx, A.xy, A.xz, fe[0]) : z4;
+      sp[3] = own ? make_float4(A.xy, A.yy, A.yz, fe[1]) : z4;
+      sp[4] = own ? make_float4(A.xz, A.yz, A.zz, fe[2]) : z4;
+    } else if (MODE == 1) {
+      sp[1] = own ? make_float4(r.m * r.v[0], r.m * r.v[1], r.m * r.v[2], 0.f) : z4;
+    } else {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int s = 2 * h + j;
-      const int tx = h ? txs[2 + j] : txs[j], ty = h ? tys[2 + j] : tys[j], tz = h ? tzs[2 + j] : tzs[j];
-      float N, dN;
-      // (the re-map's products use the weights only: no derivatives)
-      piece(coef(tx, s), __fsub_rn(fr[0], (float)(NLO + s)), s == 0, N, dN);
-      sp[7 * s + 0] = N;
-      if (!REMAP) sp[7 * s + 1] = dN;
-      piece(coef(ty, s), __fsub_rn(fr[1], (float)(NLO + s)), s == 0, N, dN);
-      sp[7 * s + 2] = N;
-      if (!REMAP) sp[7 * s + 3] = dN;
-      piece(coef(tz, s), __fsub_rn(fr[2], (float)(NLO + s)), s == 0, N, dN);
-      sp[7 * s + 4] = N;
-      if (!REMAP) sp[7 * s + 5] = dN;
-      // field s: the mass (the re-map's field 0 is padding), then m v_a
-      const float va = s == 1 ? r.v[0] : (s == 2 ? r.v[1] : r.v[2]);
-      sp[7 * s + 6] = s == 0 ? (REMAP ? 0.f : keep * r.m) : keep * r.m * va;
-    }
-    if (!REMAP) {  // half 0: xx, yy, zz; half 1: xy, xz, yz
-      sp[28 + 3 * h] = keep * (h ? A.xy : A.xx);
-      sp[29 + 3 * h] = keep * (h ? A.xz : A.yy);
-      sp[30 + 3 * h] = keep * (h ? A.yz : A.zz);
-    }
-    if (h == 0) {
-      sp[34] = 0.f;
-      if (FEXT) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) sp[35 + a] = keep * fe[a];
-      }
+      for (int a = 0; a < 3; ++a) sp[1 + a] = own ? make_float4(r.v[a], r.Lb[a], r.Lb[3 + a], r.Lb[6 + a]) : z4;
+      sp[4] = own ? make_float4(r.dv[0], 0.f, 0.f, 0.f) : z4;
+      sp[5] = own ? make_float4(r.dv[1], r.dv[2], 0.f, 0.f) : z4;
     }
   };
 
-  // The chunk walk: chunk k's fields in one register set while chunk k+1's
-  // load into the other and chunk k+2's slots load (the two sets alternate,
-  // so no register copy waits for a load in flight). Each step issues the
-  // slots before the fields, so the in-order load counter lets a wait for
-  // the slots leave the older fields in flight.
-  int lx, w0 = 0;
-  first_chunk_from(0, lx, w0);
-  int nlx = M::CELLS, nw0 = 0;
-  next_chunk(lx, w0, nlx, nw0);
-  Raw ra, rb;
-  int sa = chunk_slot(lx, w0), sb = chunk_slot(nlx, nw0);
-  load_raw(lx, w0, sa, ra);
-  int xc_cell = -1;
-  // four independent accumulation chains: mass and moments, and the three
-  // terms of the force (summed when the cell is done)
-  v4f C1 = {0.f, 0.f, 0.f, 0.f}, C2x = C1, C2y = C1, C2z = C1;
-  auto chunk = [&](Raw &cur, int &s_cur, Raw &nxt, int &s_nxt) {
-    int nnlx = M::CELLS, nnw0 = 0;
-    if (nlx < M::CELLS) next_chunk(nlx, nw0, nnlx, nnw0);
-    s_cur = chunk_slot(nnlx, nnw0);      // the slots of chunk k+2
-    load_raw(nlx, nw0, s_nxt, nxt);      // in flight during this chunk's products
-    if (xc_cell != lx) {  // x node types of the new cell's span
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        txs[s] = cubic_node_type(bx * M::CELLS + lx + NLO + s, g.num_cells[0], prm.node_types_built);
-      xc_cell = lx;
-    }
-    stage_raw(lx, cur);
-    wave_lds_sync();
-    const int wn = min(M::CH, ce_of(lx) - w0);
-#pragma unroll
-    for (int k0 = 0; k0 < M::CH; k0 += 4) {
-      if (k0 >= wn) break;  // wave-uniform
-      const float *sp = st + (k0 + pk) * RS;
-      const float Nx = sp[ex], dNx = sp[ex + 1], Ny = sp[ex + 2], dNy = sp[ex + 3];
-      const float Nz = sp[ez + 4], dNz = sp[ez + 5], Ff = sp[ez + 6];
-      const float b1 = Ny * Nz;
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * Ff, b1, C1, 0, 0, 0);
-      if (!REMAP) {
-        float a2x = dNx * sp[ax];
-        if (FEXT) a2x += Nx * sp[af];  // + w f_a
-        C2x = __builtin_amdgcn_mfma_f32_16x16x4f32(a2x, b1, C2x, 0, 0, 0);
-        C2y = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[ay], dNy * Nz, C2y, 0, 0, 0);
-        C2z = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[az], Ny * dNz, C2z, 0, 0, 0);
+  // lane roles in the products
+  const int s1 = (lane & 15) >> 2, s2 = lane & 3, pk = lane >> 4;
+  SpanPoly<SF> px, py, pz;
+  // y and z weights for x carry kx (see above)
+  auto set_yz = [&](int kx, SpanPoly<SF> &y, SpanPoly<SF> &z) {
+    int ty = 0, tz = 0;
+    if (TYPED) {
+      int yv = cy + NLO + s1 + kx, zv = cz + NLO + s2;
+      if (prm.wrap_quirk) {
+        while (yv < 0) { yv += g.num_cells[1]; --zv; }
+        while (yv >= g.num_cells[1]) { yv -= g.num_cells[1]; ++zv; }
       }
+      ty = cubic_node_type(yv, g.num_cells[1], 1);
+      tz = cubic_node_type(zv, g.num_cells[2], 1);
     }
-    wave_lds_sync();  // the stage is read; the next chunk may overwrite it
-    if (nlx != lx) {
-      // the cell is done: node (i, j, k) = (l / 16, (l % 16) / 4, l % 4) of
-      // its window
-      const int nb = (lx + pk) + M::BXP * (s1 + M::BY * s2);
-      if (REMAP) {  // rows 1..3: m v'
-#pragma unroll
-        for (int r = 1; r < 4; ++r) blk[(r - 1) * M::BN + nb] += C1[r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) blk[r * M::BN + nb] += C1[r];
-#pragma unroll
-        for (int r = 0; r < 3; ++r) blk[(4 + r) * M::BN + nb] += (C2x[r] + C2y[r]) + C2z[r];
-      }
-      C1 = v4f{0.f, 0.f, 0.f, 0.f};
-      C2x = C1;
-      C2y = C1;
-      C2z = C1;
-    }
-    lx = nlx;
-    w0 = nw0;
-    nlx = nnlx;
-    nw0 = nnw0;
+    y.set(s1, ty, inv_h, 1.f);
+    z.set(s2, tz, inv_h, 1.f);
   };
-  while (lx < M::CELLS) {  // wave-uniform
-    chunk(ra, sa, rb, sb);
-    if (lx >= M::CELLS) break;
-    chunk(rb, sb, ra, sa);
+  set_yz(0, py, pz);
+
+  v4f C1 = {0.f, 0.f, 0.f, 0.f}, C2 = C1;
+  auto product = [&](int row, const SpanPoly<SF> &x, const SpanPoly<SF> &y, const SpanPoly<SF> &z) {
+    const float *sp = st + (row + pk) * RS;
+    const float4 f = *reinterpret_cast<const float4 *>(sp);
+    const float Nx = x.N(f.x), Ny = y.N(f.y), Nz = z.N(f.z);
+    const float b1 = Ny * Nz;
+    if (MODE == 1) {
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[4 + s1], b1, C1, 0, 0, 0);
+      return;
+    }
+    const float dNx = x.dN(f.x), dNy = y.dN(f.y), dNz = z.dN(f.z);
+    const float b2 = dNy * Nz, b3 = Ny * dNz;
+    if (MODE == 0) {
+      // (field row 3 of the force is padding: it reads row 2)
+      const float4 A = *reinterpret_cast<const float4 *>(sp + 8 + 4 * min(s1, 2));
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[4 + s1], b1, C1, 0, 0, 0);
+      float a2 = dNx * A.x;
+      if (FEXT) a2 += Nx * A.w;
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, b1, C2, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.y, b2, C2, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.z, b3, C2, 0, 0, 0);
+    } else {
+      const float4 A = *reinterpret_cast<const float4 *>(sp + 4 + 4 * s1);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.x + dNx * A.y, b1, C1, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[20 + s1], b1, C2, 0, 0, 0);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.z, b2, C1, 0, 0, 0);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.w, b3, C1, 0, 0, 0);
+    }
+  };
+  // node column lx of the wave's row is complete: out of the accumulators
+  auto flush = [&](int lx) {
+    float *b = blk + lx * M::XP + (lane & 15);
+    if (MODE != 1 || pk < 3) b[pk * BN] = C1[0];
+    C1 = v4f{C1[1], C1[2], C1[3], 0.f};
+    if (MODE != 1) {
+      if (pk < (MODE == 0 ? 3 : 2)) b[(4 + pk) * BN] = C2[0];
+      C2 = v4f{C2[1], C2[2], C2[3], 0.f};
+    }
+  };
+
+  Raw raw;
+  int next = 0;  // first row not yet loaded
+  if (total > 0) {
+    load_raw(0, raw);
+    next = CH;
   }
+  int r0 = -CH, row = 0;  // first staged row, current row
+  int xt = -1;            // x cells [3, nx - 4] share their node types
+#pragma unroll 1
+  for (int l = 0; l < CELLS; ++l) {  // wave-uniform from here on
+    const int cx = bx * CELLS + l;
+    const int end = __builtin_amdgcn_readlane(rend, l);
+    if (row < end) {
+      const int nx = g.num_cells[0];
+      const bool inner = cx >= 3 && cx < nx - 3;
+      const int xv = cx + NLO + s2;  // this lane's x node
+      const bool out_x = xv < 0 || xv >= nx;
+      if (!TYPED) {
+        if (xt < 0) px.set(s2, 0, inv_h, 1.f);
+        xt = 0;
+      } else if (!inner || xt != 1) {
+        px.set(s2, cubic_node_type(xv, nx, 1), inv_h, out_x ? 0.f : 1.f);
+        xt = inner ? 1 : 0;
+      }
+      const bool leaves = TYPED && MODE != 2 && !inner && prm.wrap_quirk && __ballot(out_x) != 0ull;
+      while (row < end) {
+        if (row - r0 >= CH) {
+          wave_lds_sync();  // the rows staged before are read
+          stage_raw(raw);
+          r0 = row;
+          if (next < total) load_raw(next, raw);
+          next += CH;
+          wave_lds_sync();
+        }
+        const int stop = min(end, r0 + CH);
+        const int first = row;
+#pragma unroll 2
+        for (; row < stop; row += 4) product(row - r0, px, py, pz);
+        if (leaves) {
+#pragma unroll 1
+          for (int kx = -1; kx <= 2; ++kx) {  // (2: one-node grids only)
+            const bool mine = kx != 0 && xv - kx * nx >= 0 && xv - kx * nx < nx;
+            if (__ballot(mine) == 0ull) continue;
+            SpanPoly<SF> ox, oy, oz;
+            ox.set(s2, cubic_node_type(mine ? xv - kx * nx : 0, nx, 1), inv_h, mine ? 1.f : 0.f);
+            set_yz(kx, oy, oz);
+            for (int q = first; q < stop; q += 4) product(q - r0, ox, oy, oz);
+          }
+        }
+      }
+    }
+    flush(l);
+  }
+#pragma unroll
+  for (int l = 0; l < SPAN - 1; ++l) flush(CELLS + l);
   __syncthreads();
-  // slice node (ix, iy, iz): the blocks of waves iz - 3 .. iz
-  float *slice = partials + (int64_t)blockIdx.x * NV * NTN;
+  // slice node (ix, iy, iz): the columns of waves iz - SPAN + 1 .. iz
+  float *slice = partials + (int64_t)blockIdx.x * NV * M::NTN;
   if (t == 0) flags[blockIdx.x] = 1;
-  for (int i = t; i < NTN; i += 256) {
-    const int ix = i % M::BX, iy = (i / M::BX) % M::BY, iz = i / (M::BX * M::BY);
+  for (int i = t; i < M::NTN; i += 256) {
+    const int ix = i % M::BX, iy = (i / M::BX) % SPAN, iz = i / (M::BX * SPAN);
     float sum[NV] = {};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const int z = iz - w;
-      if (z < 0 || z >= M::BZ) continue;
+      if (z < 0 || z >= SPAN) continue;
 #pragma unroll
-      for (int f = 0; f < NV; ++f) sum[f] += block[w][f][ix + M::BXP * (iy + M::BY * z)];
+      for (int f = 0; f < NV; ++f) sum[f] += block[w][f * BN + ix * M::XP + 4 * iy + z];
     }
 #pragma unroll
-    for (int f = 0; f < NV; ++f) slice[f * NTN + i] = sum[f];
+    for (int f = 0; f < NV; ++f) slice[f * M::NTN + i] = sum[f];
   }
 }
 
@@ -1695,22 +1756,41 @@ struct TileGeom {
 // 0's first entries and adds zero), so a node waits for two loads in a row,
 // not one per tile. Returns whether any candidate tile was live (a node no
 // live tile covers skips the loads).
-template <int D, int NV>
+// TG: the tiling's constants (Tiles3) in 3D, where the divisions then become
+// shifts; the runtime values of tg in 1D and 2D.
+template <int SPAN_, int CELLS_> struct Tiles3 {
+  static constexpr int SPAN = SPAN_, NLO = SPAN_ == 2 ? 0 : -1, COVER_Y = SPAN_;
+  static constexpr int T[3] = {CELLS_, 1, 4}, N[3] = {CELLS_ + SPAN_ - 1, SPAN_, 3 + SPAN_};
+};
+struct TilesRuntime { static constexpr int COVER_Y = -1; };
+template <int D, int NV, class TG = TilesRuntime>
 __device__ inline bool gather_partials(const TileGeom &tg, const float *partials, const int32_t *flags,
                                        const int *ids, float *acc) {
-  constexpr int MX = kCoverX, MY = D > 1 ? kCoverY : 1, MZ = D > 2 ? kCoverZ : 1, MC = MX * MY * MZ;
+  constexpr bool FIXED = D == 3;
+  constexpr int MX = kCoverX, MY = TG::COVER_Y < 0 ? (D > 1 ? kCoverY : 1) : TG::COVER_Y, MZ = D > 2 ? kCoverZ : 1;
+  constexpr int MC = MX * MY * MZ;
+  int T[3], N[3], nlo;
+  if constexpr (FIXED) {
+    nlo = TG::NLO;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) { T[a] = TG::T[a]; N[a] = TG::N[a]; }
+  } else {
+    nlo = tg.nlo;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) { T[a] = tg.T[a]; N[a] = tg.N[a]; }
+  }
   int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
 #pragma unroll
   for (int a = 0; a < D; ++a) {
     // tile b covers nodes [b*T + nlo, b*T + nlo + N - 1]
-    const int r = ids[a] - tg.nlo;
-    int b_hi = r / tg.T[a];
-    int b_lo = (r - tg.N[a] + 1 + tg.T[a] - 1) >= 0 ? (r - tg.N[a] + tg.T[a]) / tg.T[a] : 0;
+    const int r = ids[a] - nlo;
+    int b_hi = r / T[a];
+    int b_lo = (r - N[a] + T[a]) >= 0 ? (r - N[a] + T[a]) / T[a] : 0;
     if (b_hi > tg.tiles[a] - 1) b_hi = tg.tiles[a] - 1;
     lo[a] = b_lo;
     hi[a] = b_hi;
   }
-  const int ntn = tg.N[0] * (D > 1 ? tg.N[1] : 1) * (D > 2 ? tg.N[2] : 1);
+  const int ntn = N[0] * (D > 1 ? N[1] : 1) * (D > 2 ? N[2] : 1);
   bool live[MC];
   int64_t off[MC];
 #pragma unroll
@@ -1724,9 +1804,9 @@ __device__ inline bool gather_partials(const TileGeom &tg, const float *partials
         const bool in = bx <= hi[0] && by <= hi[1] && bz <= hi[2];
         const int tile = in ? bx + tg.tiles[0] * (by + tg.tiles[1] * bz) : 0;
         live[c] = in && flags[tile] != 0;
-        int li = ids[0] - (bx * tg.T[0] + tg.nlo);
-        if (D > 1) li += tg.N[0] * (ids[1] - (by * tg.T[1] + tg.nlo));
-        if (D > 2) li += tg.N[0] * tg.N[1] * (ids[2] - (bz * tg.T[2] + tg.nlo));
+        int li = ids[0] - (bx * T[0] + nlo);
+        if (D > 1) li += N[0] * (ids[1] - (by * T[1] + nlo));
+        if (D > 2) li += N[0] * N[1] * (ids[2] - (bz * T[2] + nlo));
         off[c] = (int64_t)tile * NV * ntn + li;
       }
   bool any = false;
@@ -1987,28 +2067,94 @@ __global__ __launch_bounds__(256) void wrap_gather_list_kernel(pmpm_grid g, Tile
 // clamp (optional): per node, the components a NodeDomain condition set to
 // zero (bit a: moment, bit 3 + a: forward moment; a slip clamp counts when
 // its input was not on the kept side), for the adjoint. wlist (optional): the
-// typed-cubic wrap-around node list, emptied here for the next pass (its
+// typed-cubic wrap-around node list of 2D, emptied here for the next pass (its
 // gather ran before this pass).
-template <int D>
-__global__ void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int finalize, int bc_begin, int bc_end,
+// 3D (TG = Tiles3): the nodes the wrap-around can reach are left to the
+// launch's first nwrap workgroups, four lanes per node: the node itself and
+// the virtual nodes outside the grid that share its linear index (up to three
+// on grids of at least three nodes along x and y) are gathered by a lane each
+// and summed over the lanes in a fixed order. The workgroups after them take
+// the other nodes, one lane each.
+constexpr int kImageLanes = 4;
+template <int NV, class TG>
+__device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, const float *partials,
+                                     const int32_t *flags, const int *ids, int lane, float *acc) {
+  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = g.num_cells[2];
+  constexpr int lo = TG::NLO, hi = TG::NLO + TG::SPAN - 1;
+  const int kx_end = nx < 3 ? 2 : 1, ky_end = ny < 3 ? 2 : 1;
+  int count = 0;
+#pragma unroll 1
+  for (int round = 0; round == 0 || count > kImageLanes * round; ++round) {  // (one round but on tiny grids)
+    // this lane's image is picked first, so that the lanes gather together
+    int mine[3] = {0, 0, 0};
+    bool have = false;
+    count = 0;
+    for (int kx = -1; kx <= kx_end; ++kx) {
+      const int vx = ids[0] + kx * nx;
+      if (vx < lo || vx > nx - 1 + hi) continue;
+      int qy = ids[1] - kx, qz = ids[2];
+      while (qy < 0) { qy += ny; --qz; }
+      while (qy >= ny) { qy -= ny; ++qz; }
+      for (int ky = -1; ky <= ky_end; ++ky) {
+        const int vy = qy + ky * ny, vz = qz - ky;
+        if (vy < lo || vy > ny - 1 + hi || vz < lo || vz > nz - 1 + hi) continue;
+        if (count++ == kImageLanes * round + lane) {
+          mine[0] = vx;
+          mine[1] = vy;
+          mine[2] = vz;
+          have = true;
+        }
+      }
+    }
+    if (have) gather_partials<3, NV, TG>(tg, partials, flags, mine, acc);
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int o = 1; o < kImageLanes; o <<= 1) acc[k] += __shfl_xor(acc[k], o);
+}
+// GATHER as TileGeom::gather (fixed per instance: it sets the fields gathered).
+template <int D, int GATHER, class TG>
+__global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int finalize, int bc_begin, int bc_end,
                             int remap_pass, TileGeom tg, const float *__restrict__ partials,
                             const int32_t *__restrict__ flags, int clear_mom_nt, uint8_t *__restrict__ clamp,
-                            int32_t *__restrict__ wlist) {
+                            int32_t *__restrict__ wlist, int nwrap) {
   const int nn = g.num_cells_total;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  int i = ((int)blockIdx.x - nwrap) * blockDim.x + threadIdx.x;
   if (wlist && i == 0)  // the wrap-around list of this pass is consumed
     for (int p2 = 0; p2 < kWrapListShards; ++p2) wlist[p2] = 0;
-  if (i >= nn) return;
+  int ids0[3] = {0, 0, 0};
+  bool reached = false;  // a node the wrap-around can reach
+  if (D == 3 && (int)blockIdx.x < nwrap) {
+    const int t = (blockIdx.x * blockDim.x + threadIdx.x) / kImageLanes;
+    if (t >= wrap_target_count<D>(g) || !wrap_target<D>(g, t, ids0)) return;  // (a node's lanes together)
+    i = ids0[0] + g.num_cells[0] * (ids0[1] + g.num_cells[1] * ids0[2]);
+    reached = true;
+  } else {
+    if (i >= nn) return;
+    node_ids32<D>(g, i, ids0);
+    if (D == 3 && nwrap > 0 && (ids0[0] <= 1 || ids0[0] == g.num_cells[0] - 1 || ids0[1] <= 1 || ids0[1] == g.num_cells[1] - 1))
+      return;
+  }
   float m = nodes.mass[i];
   float P[3] = {0.f, 0.f, 0.f}, Q[3] = {0.f, 0.f, 0.f};
-  if (tg.gather) {
-    // node arrays hold the wrap-around deposits; add the tile partials
-    int ids0[3];
-    node_ids<D>(g, i, ids0);
-    float acc[1 + 2 * 3] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (tg.gather == 1) gather_partials<D, 1 + 2 * D>(tg, partials, flags, ids0, acc);
-    else gather_partials<D, D>(tg, partials, flags, ids0, acc);
-    if (tg.gather == 1) {
+  if constexpr (GATHER != 0) {
+    // node arrays hold the deposits of stray particles (and 2D's wrap-around
+    // sums); add the tile partials
+    constexpr int NV = GATHER == 1 ? 1 + 2 * D : D;
+    float acc[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[k] = 0.f;
+    if (reached) {
+      if constexpr (D == 3) {
+        const int lane = (int)threadIdx.x & (kImageLanes - 1);
+        gather_images<NV, TG>(g, tg, partials, flags, ids0, lane, acc);
+        if (lane != 0) return;
+      }
+    } else {
+      gather_partials<D, NV, TG>(tg, partials, flags, ids0, acc);
+    }
+    if constexpr (GATHER == 1) {
       m += acc[0];
 #pragma unroll
       for (int a = 0; a < D; ++a) {
@@ -2055,8 +2201,7 @@ __global__ void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int 
 #pragma unroll
     for (int a = 0; a < D; ++a) Q[a] = P[a] + Q[a] * prm.dt;
   }
-  int ids[3];
-  node_ids<D>(g, i, ids);
+  const int *ids = ids0;
   unsigned cbits = 0u;
   for (int k = bc_begin; k < bc_end; ++k) {
     const pmpm_bc &bc = prm.bcs[k];
@@ -2523,13 +2668,13 @@ __global__ void shape_function_kernel(pmpm_grid g, int types_built, const float 
     default: return PMPM_ERR_INVALID;                                             \
   }
 
-// How the wrap-around deposits of a P2G pass are summed (TileGeom::wrap).
+// How the wrap-around deposits of a P2G pass are summed (TileGeom::wrap): 1
+// from the virtual nodes of the tile partials (3D: in the grid kernel), 2 from
+// the records of p2g_wrap_kernel (2D, typed cubic).
 static int wrap_mode(const pmpm_params &prm, const pmpm_grid &g) {
   if (!prm.wrap_quirk || prm.dim < 2) return 0;
-  if (prm.shape_fn == PMPM_SF_CUBIC) {
-    if (!prm.node_types_built) return 0;  // untyped cubic weights are zero
-    return (prm.dim == 2 ? wrap_cell_count<2>(g) : wrap_cell_count<3>(g)) > 0 ? 2 : 0;
-  }
+  if (prm.shape_fn == PMPM_SF_CUBIC && !prm.node_types_built) return 0;  // untyped cubic weights are zero
+  if (prm.shape_fn == PMPM_SF_CUBIC && prm.dim == 2) return wrap_cell_count<2>(g) > 0 ? 2 : 0;
   return 1;
 }
 
@@ -2547,98 +2692,104 @@ template <int D, int SF> TileGeom tile_geom_of(const pmpm_grid &g, int gather) {
   tg.nv = gather == 2 ? D : (gather == 3 ? 2 * D : 1 + 2 * D);  // 3: adjoint scatter
   return tg;
 }
-TileGeom tile_geom(int dim, int sf, const pmpm_grid &g, int gather) {
-  switch (dim * 3 + sf) {
-    case 3: return tile_geom_of<1, PMPM_SF_LINEAR>(g, gather);
-    case 4: return tile_geom_of<1, PMPM_SF_QUADRATIC>(g, gather);
-    case 5: return tile_geom_of<1, PMPM_SF_CUBIC>(g, gather);
-    case 6: return tile_geom_of<2, PMPM_SF_LINEAR>(g, gather);
-    case 7: return tile_geom_of<2, PMPM_SF_QUADRATIC>(g, gather);
-    case 8: return tile_geom_of<2, PMPM_SF_CUBIC>(g, gather);
-    case 9: return tile_geom_of<3, PMPM_SF_LINEAR>(g, gather);
-    case 10: return tile_geom_of<3, PMPM_SF_QUADRATIC>(g, gather);
-    default: return tile_geom_of<3, PMPM_SF_CUBIC>(g, gather);
-  }
+// Cells per wave of the 3D P2G tiles (MfmaGeom): 8, or 4 on small grids, where
+// eight cells per wave leave most of the chip idle. A function of the grid and
+// the particle count only: every pass of a step, and pmpm_step_noalloc, must
+// agree on it.
+constexpr int kSmallGridNodes = 131072, kSmallParticles = 131072;
+static int mfma_cells(const pmpm_grid &g, int n) {
+  return g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles ? 4 : 8;
 }
-static size_t tile_count(const TileGeom &tg) { return (size_t)tg.tiles[0] * tg.tiles[1] * tg.tiles[2]; }
-// The forward P2G and MUSL re-map of 3D typed cubic run on the matrix cores
-// with their own tiles (MfmaGeom); every other pass uses p2g_kernel's.
-static bool mfma_tiles(const pmpm_params &prm, int gather) {
-  return prm.dim == 3 && prm.shape_fn == PMPM_SF_CUBIC && prm.node_types_built && (gather == 1 || gather == 2);
-}
-static TileGeom mfma_tile_geom(const pmpm_grid &g, int gather) {
-  using M = MfmaGeom;
+static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, int cells) {
   TileGeom tg{};
-  const int T[3] = {M::CELLS, 1, M::TZ}, N[3] = {M::BX, M::BY, M::NZ};
-  tg.nlo = -1;
+  const int span = sf == PMPM_SF_LINEAR ? 2 : 4;
+  const int T[3] = {cells, 1, 4}, N[3] = {cells + span - 1, span, 3 + span};
+  tg.nlo = sf == PMPM_SF_LINEAR ? 0 : -1;
   for (int a = 0; a < 3; ++a) {
     tg.T[a] = T[a];
     tg.N[a] = N[a];
     tg.tiles[a] = (int)ceil_div(g.num_cells[a], T[a]);
   }
   tg.gather = gather;
-  tg.nv = gather == 2 ? 3 : 7;
+  tg.nv = gather == 2 ? 3 : (gather == 3 ? 6 : 7);
   return tg;
 }
-static TileGeom tile_geom(const pmpm_params &prm, const pmpm_grid &g, int gather) {
-  return mfma_tiles(prm, gather) ? mfma_tile_geom(g, gather) : tile_geom(prm.dim, prm.shape_fn, g, gather);
+// The tiles of a P2G pass over n particles (gather: TileGeom::gather, or 3 for
+// the adjoint scatter).
+static TileGeom tile_geom(const pmpm_params &prm, const pmpm_grid &g, int gather, int n) {
+  switch (prm.dim * 3 + prm.shape_fn) {
+    case 3: return tile_geom_of<1, PMPM_SF_LINEAR>(g, gather);
+    case 4: return tile_geom_of<1, PMPM_SF_QUADRATIC>(g, gather);
+    case 5: return tile_geom_of<1, PMPM_SF_CUBIC>(g, gather);
+    case 6: return tile_geom_of<2, PMPM_SF_LINEAR>(g, gather);
+    case 7: return tile_geom_of<2, PMPM_SF_QUADRATIC>(g, gather);
+    case 8: return tile_geom_of<2, PMPM_SF_CUBIC>(g, gather);
+    default: return mfma_tile_geom(prm.shape_fn, g, gather, mfma_cells(g, n));
+  }
+}
+static size_t tile_count(const TileGeom &tg) { return (size_t)tg.tiles[0] * tg.tiles[1] * tg.tiles[2]; }
+
+template <int SF, int CELLS>
+static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
+                            const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, int mode,
+                            float *partials, int32_t *flags, hipStream_t s, const float *rec) {
+  const TileGeom mg = mfma_tile_geom(SF, g, mode + 1, CELLS);
+  const dim3 grid((unsigned)tile_count(mg)), block(256);
+  if (mode == 0 && has_planar(prm))
+    PMPM_LAUNCH((p2g_mfma_kernel<SF, 0, CELLS, true>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 0L, 1L})), grid,
+                block, 0, s, prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
+  else if (mode == 0)
+    PMPM_LAUNCH((p2g_mfma_kernel<SF, 0, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 0L})), grid, block, 0, s,
+                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
+  else if (mode == 1)
+    PMPM_LAUNCH((p2g_mfma_kernel<SF, 1, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 1L})), grid, block, 0, s,
+                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
+  else
+    PMPM_LAUNCH((p2g_mfma_kernel<SF, 2, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 2L})), grid, block, 0, s,
+                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
 }
 
 // mode 0: P2G, 1: MUSL first map + re-map, 2: adjoint scatter of the
-// records `rec`
+// records `rec` (never launched without them). 3D: the matrix-core tiles (the
+// re-map after a G2P-style first map); 1D and 2D: p2g_kernel.
 template <int D, int SF>
 void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in, const pmpm_particles &out,
                 const pmpm_spatial &part, const pmpm_nodes &nodes, int mode, float *partials, int32_t *flags,
                 float *wrec, uint8_t *wtouch, int32_t *wlist, hipStream_t s,
                 const float *rec = nullptr) {
-  const TileGeom tg = tile_geom_of<D, SF>(g, 1);
-  const dim3 grid((unsigned)tile_count(tg)), block(P2GGeom<D, SF>::THREADS);
-  // 3D typed cubic P2G and MUSL re-map on the matrix cores (the re-map after
-  // a G2P-style first map), on their own tiles; everything else on the VALU
-  // kernel
-  bool mfma = false;
-  if constexpr (D == 3 && SF == PMPM_SF_CUBIC) {
-    mfma = (mode == 0 || mode == 1) && prm.node_types_built;
-    const TileGeom mg = mfma_tile_geom(g, mode + 1);
-    const dim3 grid((unsigned)tile_count(mg));
-    if (mfma && mode == 0 && has_planar(prm)) {
-      PMPM_LAUNCH((p2g_mfma_kernel<SF, false, true>),
-                  (::pmpm::kname("p2g_mfma_kernel", {(long)(SF), (long)(false), (long)(true)})), grid, dim3(256), 0, s,
-                  prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags);
-    } else if (mfma && mode == 0) {
-      PMPM_LAUNCH((p2g_mfma_kernel<SF, false>), (::pmpm::kname("p2g_mfma_kernel", {(long)(SF), (long)(false)})), grid, dim3(256), 0, s, prm, g, in, out, part, nodes,
-                         mg.tiles[0], mg.tiles[1], partials, flags);
-    } else if (mfma && mode == 1) {
-      if (in.n > 0)
-        PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0,
-                           s, prm, g, in, out, part, nodes, 1);
-      PMPM_LAUNCH((p2g_mfma_kernel<SF, true>), (::pmpm::kname("p2g_mfma_kernel", {(long)(SF), (long)(true)})), grid, dim3(256), 0, s, prm, g, in, out, part, nodes,
-                         mg.tiles[0], mg.tiles[1], partials, flags);
-    }
-  }
-  // (each mode launches exactly one tile kernel; the adjoint scatter reads
-  // `rec` and is never launched without it)
-  if (mode == 0) {
-    if (!mfma)
+  if (mode == 2 && !rec) return;
+  if constexpr (D == 3) {
+    if (mode == 1 && in.n > 0)
+      PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0,
+                         s, prm, g, in, out, part, nodes, 1);
+    if (mfma_cells(g, in.n) == 4)
+      launch_p2g_mfma<SF, 4>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+    else
+      launch_p2g_mfma<SF, 8>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+  } else {
+    const TileGeom tg = tile_geom_of<D, SF>(g, 1);
+    const dim3 grid((unsigned)tile_count(tg)), block(P2GGeom<D, SF>::THREADS);
+    if (mode == 0)
       PMPM_LAUNCH((p2g_kernel<D, SF, 0>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(0)})), grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0],
                          tg.tiles[1], partials, flags, rec);
-  } else if (mode == 1) {
-    if (!mfma)
+    else if (mode == 1)
       PMPM_LAUNCH((p2g_kernel<D, SF, 1>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)tile_count(tg) + kMuslTailBlocks), block, 0, s, prm,
                          g, in, out, part, nodes, tg.tiles[0], tg.tiles[1], partials, flags, rec);
-  } else if (mode == 2 && rec) {
-    PMPM_LAUNCH((p2g_kernel<D, SF, 2>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(2)})), grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0],
-                       tg.tiles[1], partials, flags, rec);
-  }
-  const int wcells = wrap_cell_count<D>(g);
-  if (mode != 2 && wrap_mode(prm, g) == 2 && wcells > 0) {
-    const dim3 wgrid((unsigned)ceil_div(wcells, kWrapCellsPerBlock)), wblock(64 * kWrapCellsPerBlock);
-    if (mode == 0)
-      PMPM_LAUNCH((p2g_wrap_kernel<D, 0>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(0)})), wgrid, wblock,
-                  0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
     else
-      PMPM_LAUNCH((p2g_wrap_kernel<D, 1>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(1)})), wgrid, wblock,
-                  0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
+      PMPM_LAUNCH((p2g_kernel<D, SF, 2>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(2)})), grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0],
+                         tg.tiles[1], partials, flags, rec);
+  }
+  if constexpr (D == 2) {
+    const int wcells = wrap_cell_count<D>(g);
+    if (mode != 2 && wrap_mode(prm, g) == 2 && wcells > 0) {
+      const dim3 wgrid((unsigned)ceil_div(wcells, kWrapCellsPerBlock)), wblock(64 * kWrapCellsPerBlock);
+      if (mode == 0)
+        PMPM_LAUNCH((p2g_wrap_kernel<D, 0>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(0)})), wgrid, wblock,
+                    0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
+      else
+        PMPM_LAUNCH((p2g_wrap_kernel<D, 1>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(1)})), wgrid, wblock,
+                    0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
+    }
   }
 }
 template <int D, int SF>
@@ -2657,11 +2808,11 @@ void launch_shape(const pmpm_grid &g, int types_built, const float *x, int n, fl
 }
 
 // gather: 0 = node arrays only, 1 = add the P2G tile partials, 2 = add the
-// MUSL re-map tile partials (ctx holds them).
+// MUSL re-map tile partials (ctx holds them) of a pass over n particles.
 int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, int finalize,
-                int b0, int b1, int remap, int gather, hipStream_t s, int clear_mom_nt = 0) {
+                int b0, int b1, int remap, int gather, hipStream_t s, int n, int clear_mom_nt = 0) {
   const unsigned blocks = (unsigned)ceil_div(g.num_cells_total, 256);
-  TileGeom tg = tile_geom(prm, g, gather);
+  TileGeom tg = tile_geom(prm, g, gather, n);
   const float *partials = gather ? ctx->partials : nullptr;
   const int32_t *flags = gather ? ctx->tile_flags : nullptr;
   // the clamp record of a pass that applies node conditions (not the MUSL
@@ -2671,12 +2822,26 @@ int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
   if (!remap && b1 > b0)
     clamp = nodes.clamp ? nodes.clamp : (ctx ? reinterpret_cast<uint8_t *>(ctx->clamp_mask) : nullptr);
 
-  switch (prm.dim) {
-    case 1: PMPM_LAUNCH(grid_kernel<1>, (::pmpm::kname("grid_kernel", {(long)(1)}) + " gather " + std::to_string(gather)), dim3(blocks), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags, clear_mom_nt, clamp, wl); break;
-    case 2: PMPM_LAUNCH(grid_kernel<2>, (::pmpm::kname("grid_kernel", {(long)(2)}) + " gather " + std::to_string(gather)), dim3(blocks), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags, clear_mom_nt, clamp, wl); break;
-    case 3: PMPM_LAUNCH(grid_kernel<3>, (::pmpm::kname("grid_kernel", {(long)(3)}) + " gather " + std::to_string(gather)), dim3(blocks), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags, clear_mom_nt, clamp, wl); break;
-    default: return PMPM_ERR_INVALID;
-  }
+  // 3D with the wrap-around: the workgroups of the nodes it can reach
+  const int nwrap = prm.dim == 3 && gather && wrap_mode(prm, g) ? (int)ceil_div((int64_t)wrap_target_count<3>(g) * kImageLanes, 256) : 0;
+#define PMPM_GRID_LAUNCH(...)                                                                                          \
+  PMPM_LAUNCH((grid_kernel<__VA_ARGS__>), (::pmpm::kname("grid_kernel", {(long)prm.dim}) + " gather " + std::to_string(gather)), \
+              dim3(blocks + (unsigned)nwrap), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags,      \
+              clear_mom_nt, clamp, wl, nwrap)
+#define PMPM_GRID_GATHER(D, ...)                                 \
+  if (gather == 0) PMPM_GRID_LAUNCH(D, 0, TilesRuntime);         \
+  else if (gather == 1) PMPM_GRID_LAUNCH(D, 1, __VA_ARGS__);     \
+  else PMPM_GRID_LAUNCH(D, 2, __VA_ARGS__)
+  const bool lin = prm.shape_fn == PMPM_SF_LINEAR, small = tg.T[0] == 4;
+  if (prm.dim == 1) { PMPM_GRID_GATHER(1, TilesRuntime); }
+  else if (prm.dim == 2) { PMPM_GRID_GATHER(2, TilesRuntime); }
+  else if (prm.dim != 3) return PMPM_ERR_INVALID;
+  else if (lin && small) { PMPM_GRID_GATHER(3, Tiles3<2, 4>); }
+  else if (lin) { PMPM_GRID_GATHER(3, Tiles3<2, 8>); }
+  else if (small) { PMPM_GRID_GATHER(3, Tiles3<4, 4>); }
+  else { PMPM_GRID_GATHER(3, Tiles3<4, 8>); }
+#undef PMPM_GRID_GATHER
+#undef PMPM_GRID_LAUNCH
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -2709,24 +2874,20 @@ int do_zero_nodes(const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &
   return PMPM_OK;
 }
 
-// Partials and tile flags for the larger of the two tilings a step can use
-// (p2g_kernel's; the matrix-core passes' own).
+// Partials and tile flags of the P2G passes on grid g, for any particle count
+// (a small grid's passes use either tile width).
 static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, size_t *floats, size_t *tiles) {
-  const TileGeom tg = tile_geom(prm.dim, prm.shape_fn, g, 1);
-  *tiles = tile_count(tg);
-  *floats = *tiles * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2];
-  if (mfma_tiles(prm, 1)) {
-    const TileGeom mg = mfma_tile_geom(g, 1);
-    const size_t mt = tile_count(mg);
-    *tiles = std::max(*tiles, mt);
-    *floats = std::max(*floats, mt * mg.nv * (size_t)mg.N[0] * mg.N[1] * mg.N[2]);
+  *tiles = *floats = 0;
+  for (const int n : {0, kSmallParticles + 1}) {
+    const TileGeom tg = tile_geom(prm, g, 1, n);
+    *tiles = std::max(*tiles, tile_count(tg));
+    *floats = std::max(*floats, tile_count(tg) * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2]);
   }
 }
-// Words of the wrap-around node list: the part counts, then kWrapListShards
-// parts of wrap_target_count entries each.
-static size_t wrap_node_list_words(const pmpm_params &prm, const pmpm_grid &g) {
-  const size_t cap = (size_t)(prm.dim == 3 ? wrap_target_count<3>(g) : (prm.dim == 2 ? wrap_target_count<2>(g) : 0));
-  return (size_t)kWrapListShards * (1 + cap);
+// Words of the wrap-around node list (2D typed cubic): the part counts, then
+// kWrapListShards parts of wrap_target_count entries each.
+static size_t wrap_node_list_words(const pmpm_grid &g) {
+  return (size_t)kWrapListShards * (1 + (size_t)wrap_target_count<2>(g));
 }
 // (new flags and counts are cleared on s, the stream that uses them first: a
 // hipMemset on the null stream returns before the fill is done and is not
@@ -2740,7 +2901,7 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   if ((rc = ensure_buffer(ctx->clamp_mask, ctx->clamp_mask_cap, ((size_t)g.num_cells_total + 3) / 4)) != PMPM_OK)
     return rc;
   if (wrap_mode(prm, g) != 2) return rc;
-  const size_t wcells = (size_t)(prm.dim == 2 ? wrap_cell_count<2>(g) : wrap_cell_count<3>(g));
+  const size_t wcells = (size_t)wrap_cell_count<2>(g);
   if ((rc = ensure_buffer(ctx->wrap_rec, ctx->wrap_rec_cap, (size_t)wrap_rec_stride(1 + 2 * prm.dim) * wcells * 64)) != PMPM_OK)
     return rc;
   // node flags, one byte per node, cleared once here (the gather clears
@@ -2752,7 +2913,7 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   }
   // the gather's list: kWrapListShards counts, then as many parts of room
   // for every node the wrap-around can reach
-  const size_t lwords = wrap_node_list_words(prm, g);
+  const size_t lwords = wrap_node_list_words(g);
   if (lwords > ctx->wrap_list_cap) {
     float *lb = reinterpret_cast<float *>(ctx->wrap_list);
     size_t cap = ctx->wrap_list_cap;
@@ -2765,15 +2926,15 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
 }
 static uint8_t *wrap_touch(pmpm_context *ctx) { return reinterpret_cast<uint8_t *>(ctx->wrap_touch); }
 
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, size_t *partial_floats, size_t *tiles,
-                   size_t *wrap_floats, size_t *wrap_cells, size_t *wrap_touch_words, size_t *wrap_list_words,
-                   size_t *clamp_words) {
-  partial_sizes(prm, g, partial_floats, tiles);
-  *wrap_cells = (size_t)(prm.dim == 3 ? wrap_cell_count<3>(g) : (prm.dim == 2 ? wrap_cell_count<2>(g) : 0));
-  *wrap_floats = wrap_mode(prm, g) == 2 ? (size_t)wrap_rec_stride(1 + 2 * prm.dim) * *wrap_cells * 64 : 0;
-  *wrap_touch_words = wrap_mode(prm, g) == 2 ? ((size_t)g.num_cells_total + 3) / 4 : 0;
-  *wrap_list_words = wrap_mode(prm, g) == 2 ? wrap_node_list_words(prm, g) : 0;
-  *clamp_words = ((size_t)g.num_cells_total + 3) / 4;
+void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w) {
+  *w = P2GWorkspace{};
+  partial_sizes(prm, g, &w->partial_floats, &w->tiles);
+  if (wrap_mode(prm, g) == 2) {
+    w->wrap_floats = (size_t)wrap_rec_stride(1 + 2 * prm.dim) * (size_t)wrap_cell_count<2>(g) * 64;
+    w->touch_words = ((size_t)g.num_cells_total + 3) / 4;
+    w->list_words = wrap_node_list_words(g);
+  }
+  w->clamp_words = ((size_t)g.num_cells_total + 3) / 4;
 }
 
 // The wrap-around sums of a P2G pass (gather 1) or MUSL re-map (gather 2)
@@ -2781,53 +2942,35 @@ void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, size_t *partial_f
 static int launch_wrap_gather(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_spatial &part,
                               const pmpm_nodes &nodes, int gather, hipStream_t s) {
   const int mode = wrap_mode(prm, g);
-  if (mode == 0) return PMPM_OK;
-  TileGeom tg = tile_geom(prm, g, gather);
+  if (mode == 0 || prm.dim != 2) return PMPM_OK;  // (3D: the grid kernel adds them)
+  TileGeom tg = tile_geom(prm, g, gather, 0);
   tg.wrap = mode;
-  tg.wcells = prm.dim == 2 ? wrap_cell_count<2>(g) : wrap_cell_count<3>(g);
+  tg.wcells = wrap_cell_count<2>(g);
   tg.wrec = ctx->wrap_rec;
   tg.cstart = part.cell_start;
   tg.cend = part.cell_end;
-  const int targets = prm.dim == 2 ? wrap_target_count<2>(g) : wrap_target_count<3>(g);
+  const int targets = wrap_target_count<2>(g);
   if (targets <= 0) return PMPM_OK;
   if (mode == 2) {  // typed cubic: the nodes the wrap kernel listed
     const dim3 lgrid((unsigned)ceil_div(targets, 4)), block(256);  // a wave per possible entry
     uint8_t *touch = wrap_touch(ctx);
-    if (prm.dim == 2) {
-      if (gather == 1)
-        PMPM_LAUNCH((wrap_gather_list_kernel<2, 5>), (std::string("wrap_gather_list_kernel<2, 5>")), lgrid, block, 0,
-                    s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-      else
-        PMPM_LAUNCH((wrap_gather_list_kernel<2, 2>), (std::string("wrap_gather_list_kernel<2, 2>")), lgrid, block, 0,
-                    s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-    } else {
-      if (gather == 1)
-        PMPM_LAUNCH((wrap_gather_list_kernel<3, 7>), (std::string("wrap_gather_list_kernel<3, 7>")), lgrid, block, 0,
-                    s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-      else
-        PMPM_LAUNCH((wrap_gather_list_kernel<3, 3>), (std::string("wrap_gather_list_kernel<3, 3>")), lgrid, block, 0,
-                    s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-    }
+    if (gather == 1)
+      PMPM_LAUNCH((wrap_gather_list_kernel<2, 5>), (std::string("wrap_gather_list_kernel<2, 5>")), lgrid, block, 0,
+                  s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
+    else
+      PMPM_LAUNCH((wrap_gather_list_kernel<2, 2>), (std::string("wrap_gather_list_kernel<2, 2>")), lgrid, block, 0,
+                  s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
     PMPM_LAUNCH_CHECK();
     return PMPM_OK;
   }
   uint8_t *touch = nullptr;
   const dim3 grid((unsigned)ceil_div(targets, 4)), block(256);  // one wave per target node
-  if (prm.dim == 2) {
-    if (gather == 1)
-      PMPM_LAUNCH((wrap_gather_kernel<2, 5>), (std::string("wrap_gather_kernel<2, 5>")), grid, block, 0, s, g, tg,
-                  ctx->partials, ctx->tile_flags, nodes, touch);
-    else
-      PMPM_LAUNCH((wrap_gather_kernel<2, 2>), (std::string("wrap_gather_kernel<2, 2>")), grid, block, 0, s, g, tg,
-                  ctx->partials, ctx->tile_flags, nodes, touch);
-  } else {
-    if (gather == 1)
-      PMPM_LAUNCH((wrap_gather_kernel<3, 7>), (std::string("wrap_gather_kernel<3, 7>")), grid, block, 0, s, g, tg,
-                  ctx->partials, ctx->tile_flags, nodes, touch);
-    else
-      PMPM_LAUNCH((wrap_gather_kernel<3, 3>), (std::string("wrap_gather_kernel<3, 3>")), grid, block, 0, s, g, tg,
-                  ctx->partials, ctx->tile_flags, nodes, touch);
-  }
+  if (gather == 1)
+    PMPM_LAUNCH((wrap_gather_kernel<2, 5>), (std::string("wrap_gather_kernel<2, 5>")), grid, block, 0, s, g, tg,
+                ctx->partials, ctx->tile_flags, nodes, touch);
+  else
+    PMPM_LAUNCH((wrap_gather_kernel<2, 2>), (std::string("wrap_gather_kernel<2, 2>")), grid, block, 0, s, g, tg,
+                ctx->partials, ctx->tile_flags, nodes, touch);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -2915,14 +3058,14 @@ extern "C" int pmpm_p2g(pmpm_context *ctx, const pmpm_params *prm, const pmpm_gr
   int rc = do_p2g(ctx, *prm, *grid, *p, *part, *nodes, s);
   if (rc != PMPM_OK) return rc;
   // the reference's P2G ends with the cutoff and mom_nt = mom + f dt
-  return launch_grid(ctx, *prm, *grid, *nodes, 1, 0, 0, 0, 1, s);
+  return launch_grid(ctx, *prm, *grid, *nodes, 1, 0, 0, 0, 1, s, p->n);
 }
 
 extern "C" int pmpm_grid_bc(const pmpm_params *prm, const pmpm_grid *grid, pmpm_nodes *nodes, int32_t bc_begin,
                             int32_t bc_end, int32_t remap_pass, pmpm_stream_t stream) {
   if (!params_ok(prm) || !grid_ok(grid) || !nodes) return PMPM_ERR_INVALID;
   if (bc_begin < 0 || bc_end > prm->num_bcs || bc_begin > bc_end) return PMPM_ERR_INVALID;
-  return launch_grid(nullptr, *prm, *grid, *nodes, 0, bc_begin, bc_end, remap_pass ? 1 : 0, 0, (hipStream_t)stream);
+  return launch_grid(nullptr, *prm, *grid, *nodes, 0, bc_begin, bc_end, remap_pass ? 1 : 0, 0, (hipStream_t)stream, 0);
 }
 
 extern "C" int pmpm_g2p(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *in, pmpm_particles *out,
@@ -2942,7 +3085,7 @@ extern "C" int pmpm_musl_map(pmpm_context *ctx, const pmpm_params *prm, const pm
   int rc = do_musl_map(ctx, *prm, *grid, *in, *out, *part, *nodes, s);
   if (rc != PMPM_OK) return rc;
   // mom_nt := re-mapped momentum (mass cutoff as P2G), node velocities
-  return launch_grid(ctx, *prm, *grid, *nodes, 0, 0, 0, 1, 2, s);
+  return launch_grid(ctx, *prm, *grid, *nodes, 0, 0, 0, 1, 2, s, in->n);
 }
 
 extern "C" int pmpm_musl_g2p(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *in,
@@ -3239,17 +3382,17 @@ __device__ inline void store_node_adj(float *__restrict__ nbar, int node, float 
 // -> adjoints of mass, moment and force. Boundary conditions in reverse list
 // order with the forward's active sets, which the forward grid pass recorded
 // per node in `clamp` (components a NodeDomain condition set to zero).
-template <int D>
-__global__ void grid_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, TileGeom tg,
+template <int D, class TG = TilesRuntime>
+__global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, TileGeom tg,
                                     const float *__restrict__ partials, const int32_t *__restrict__ flags,
                                     const uint8_t *__restrict__ clamp, float *__restrict__ nbar) {
   const int nn = g.num_cells_total;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn) return;
   int ids[3];
-  node_ids<D>(g, i, ids);
+  node_ids32<D>(g, i, ids);
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  gather_partials<D, 2 * D>(tg, partials, flags, ids, acc);
+  gather_partials<D, 2 * D, TG>(tg, partials, flags, ids, acc);
   const float m = nodes.mass[i];
   float mb = 0.f, Pb[3] = {0.f, 0.f, 0.f}, Qb[3] = {0.f, 0.f, 0.f}, fb[3] = {0.f, 0.f, 0.f};
   if (m > prm.small_mass_cutoff) {
@@ -3736,7 +3879,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   if (recompute) {
     if ((rc = pmpm_partition(ctx, D, grid, state->x, n, part, stream)) != PMPM_OK) return rc;
     if ((rc = do_p2g(ctx, *prm, g, *state, *part, *nodes, s)) != PMPM_OK) return rc;
-    if ((rc = launch_grid(ctx, *prm, g, *nodes, 1, 0, prm->num_bcs, 0, 1, s)) != PMPM_OK) return rc;
+    if ((rc = launch_grid(ctx, *prm, g, *nodes, 1, 0, prm->num_bcs, 0, 1, s, n)) != PMPM_OK) return rc;
   } else if ((rc = reserve_tiles(ctx, *prm, g, s)) != PMPM_OK) {
     return rc;
   }
@@ -3761,13 +3904,23 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   PMPM_LAUNCH_CHECK();
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
-  const TileGeom tg = tile_geom(D, prm->shape_fn, g, 3);
+  const TileGeom tg = tile_geom(*prm, g, 3, n);
   const unsigned nblocks = (unsigned)ceil_div(g.num_cells_total, 256);
+#define PMPM_GRID_ADJOINT(...)                                                                                   \
+  PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
+              dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
+  const bool lin = prm->shape_fn == PMPM_SF_LINEAR, small = tg.T[0] == 4;
   switch (D) {
-    case 1: PMPM_LAUNCH(grid_adjoint_kernel<1>, (::pmpm::kname("grid_adjoint_kernel", {(long)(1)})), dim3(nblocks), dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes); break;
-    case 2: PMPM_LAUNCH(grid_adjoint_kernel<2>, (::pmpm::kname("grid_adjoint_kernel", {(long)(2)})), dim3(nblocks), dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes); break;
-    default: PMPM_LAUNCH(grid_adjoint_kernel<3>, (::pmpm::kname("grid_adjoint_kernel", {(long)(3)})), dim3(nblocks), dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes); break;
+    case 1: PMPM_GRID_ADJOINT(1, TilesRuntime); break;
+    case 2: PMPM_GRID_ADJOINT(2, TilesRuntime); break;
+    default:
+      if (lin && small) PMPM_GRID_ADJOINT(3, Tiles3<2, 4>);
+      else if (lin) PMPM_GRID_ADJOINT(3, Tiles3<2, 8>);
+      else if (small) PMPM_GRID_ADJOINT(3, Tiles3<4, 4>);
+      else PMPM_GRID_ADJOINT(3, Tiles3<4, 8>);
+      break;
   }
+#undef PMPM_GRID_ADJOINT
   PMPM_LAUNCH_CHECK();
   // P2G adjoint
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_adjoint_particles, *prm, g, *state, *out_bar, *in_bar, *part, *nodes,
