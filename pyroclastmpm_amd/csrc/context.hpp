@@ -19,6 +19,7 @@ struct pmpm_context {
   uint32_t *hist = nullptr;      // [radix][blocks] digit histograms
   size_t hist_len = 0;
   uint32_t *counters = nullptr;  // [4]: out-of-grid particles, hint unsorted flag, movers, -
+  bool counters_clear = false;   // cleared once, by the first call that uses them
   // P2G tile partials: per tile, the LDS node block of each accumulated field
   // (plain stores; the grid kernel sums the <= 2^D tiles covering a node)
   float *partials = nullptr;

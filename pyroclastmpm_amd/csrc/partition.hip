@@ -697,14 +697,6 @@ extern "C" int pmpm_context_create(pmpm_context **ctx) {
   const char *hint_min = getenv("PMPM_PARTITION_HINT_MIN");
   if (hint_min && hint_min[0]) c->hint_min_particles = (int32_t)strtol(hint_min, nullptr, 10);
   if (!hip_ok(hipMalloc(&c->counters, 4 * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
-  // (waited for: the context's first call may be on a stream that is not
-  // ordered after the null stream)
-  if (!hip_ok(hipMemset(c->counters, 0, 4 * sizeof(uint32_t)), "hipMemset") ||
-      !hip_ok(hipStreamSynchronize(nullptr), "hipStreamSynchronize")) {
-    (void)hipFree(c->counters);
-    delete c;
-    return PMPM_ERR_HIP;
-  }
   *ctx = c;
   return PMPM_OK;
 }
@@ -790,9 +782,20 @@ extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, in
   return PMPM_OK;
 }
 
+// A new context's counters, cleared on the stream that uses them first (a
+// hipMemset on the null stream is not ordered before a non-blocking stream).
+static int clear_counters(pmpm_context *ctx, hipStream_t s) {
+  if (ctx->counters_clear) return PMPM_OK;
+  int rc = zero_fill(ctx->counters, 4, s);
+  if (rc == PMPM_OK) ctx->counters_clear = true;
+  return rc;
+}
+
 extern "C" int pmpm_context_out_of_grid(pmpm_context *ctx, pmpm_stream_t stream, int32_t *count) {
   if (!ctx || !count) return PMPM_ERR_INVALID;
   uint32_t v = 0;
+  int rc = clear_counters(ctx, (hipStream_t)stream);
+  if (rc != PMPM_OK) return rc;
   PMPM_HIP_CHECK(hipMemcpyAsync(&v, ctx->counters, sizeof(uint32_t), hipMemcpyDeviceToHost, (hipStream_t)stream));
   PMPM_HIP_CHECK(hipStreamSynchronize((hipStream_t)stream));
   *count = (int32_t)v;
@@ -936,7 +939,8 @@ int pmpm::partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, 
   if (n > ctx->cap_particles) return PMPM_ERR_WORKSPACE;
   const pmpm_grid g = *grid;
   const uint32_t ncells = (uint32_t)g.num_cells_total;
-  int rc;
+  int rc = clear_counters(ctx, s);
+  if (rc != PMPM_OK) return rc;
   if (n == 0) {
     ZeroLists z = extra;
     z.add(ctx->counters, 1);

@@ -523,6 +523,10 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// A workgroup barrier that orders LDS accesses only: __syncthreads also waits
+// for the wave's global loads and stores in flight, which would drain a
+// kernel's prefetches.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ inline int wave_min(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
@@ -1116,6 +1120,14 @@ __global__ __launch_bounds__((P2GGeom<D, SF>::THREADS)) __attribute__((amdgpu_wa
   }
 }
 
+// Element i of a uniform base pointer through a 32-bit byte offset: the load
+// takes its base from scalar registers and one offset register serves every
+// array (a set of 2^30 particles would not fit the card, so 4 i stays below
+// 2^32).
+__device__ inline float ld32(const float *base, uint32_t i) {
+  return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + 4u * i);
+}
+
 // Per-axis weights of one fixed span offset as polynomials of the fraction
 // f = t - bin, for lanes that own one offset per axis: the coefficients are
 // set once per cell (or wave) and a weight costs a few multiply-adds.
@@ -1183,21 +1195,19 @@ template <> struct SpanPoly<PMPM_SF_LINEAR> {
   __device__ inline float dN(float f) const { return f == 0.f ? d_at0 : d; }
 };
 
-// The matrix-core P2G of 3D scenes. Tile: CELLS x 1 x 4 cells, one wave per z
-// layer walking its CELLS cells along x.
-template <int SF, int CELLS, int NV> struct MfmaGeom {
+// The matrix-core P2G of 3D scenes. Tile: CELLS x ROWS x 4 cells, one wave per
+// row of CELLS cells along x.
+template <int SF, int CELLS, int ROWS, int NV> struct MfmaGeom {
   static constexpr int SPAN = Spline<SF>::SPAN, NLO = Spline<SF>::NLO;
-  static constexpr int TZ = 4;                                      // waves (z layers) per tile
-  static constexpr int BX = CELLS + SPAN - 1, NZ = TZ + SPAN - 1;   // tile nodes along x and z (y: SPAN)
-  static constexpr int NTN = BX * SPAN * NZ;                        // nodes of one partial slice
-  // a wave's node columns in LDS, [field][x][4 y + z]: x pitch 17 and field
-  // pitch 16 mod 64, so that a flush (4 fields x 16 nodes) and the reads
-  // along x of the final sum fall into disjoint banks
-  static constexpr int XP = 17;
-  static constexpr int BN = (BX * XP - 16 + 63) / 64 * 64 + 16;
-  static_assert(BN >= BX * XP && BN % 64 == 16, "field pitch");
-  static_assert((BX - 1) / CELLS + 1 <= kCoverX && (NZ - 1) / TZ + 1 <= kCoverZ,
-                "the grid kernel's gather visits at most kCover tiles per axis");
+  static constexpr int TZ = 4, WAVES = TZ * ROWS, THREADS = 64 * WAVES;
+  static constexpr int BX = CELLS + SPAN - 1, NY = ROWS + SPAN - 1, NZ = TZ + SPAN - 1;  // tile nodes per axis
+  static constexpr int NTN = BX * NY * NZ;                                              // nodes of one partial slice
+  // a wave's node columns in LDS, [field][x][4 z + y]: the field pitch is 16
+  // mod 32, so the four fields x 16 nodes of a flush fall into disjoint banks,
+  // and a node's y window is one 16-byte read
+  static constexpr int XP = 16;
+  static constexpr int BN = BX * XP;
+  static_assert(BN % 32 == 16, "field pitch");
   static constexpr int CH = 64;  // particle rows staged per round, one per lane
 };
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1229,7 +1239,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // word. The rows of a round are the wave's particles in sorted order, each
 // cell padded to a multiple of four, so a round fills its 64 lanes whatever
 // the particles per cell (at 8 per cell staging cell by cell left 3 of 4
-// lanes idle); the next round's fields load while a round is multiplied.
+// lanes idle); the next round's fields load while a round is multiplied, the
+// slots of the round after with them.
 //
 // Linear-index wrap-around (usl_inline.h:122-126; shapefunction.cpp:96-112):
 // a node offset outside the grid stays in the tile as a virtual node, with
@@ -1239,23 +1250,23 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // that leave the grid (cells next to an x face) are multiplied in a pass of
 // their own, with that carry's y and z types and the other x offsets' weights
 // zero; the carry out of y only changes the lane's own z type.
-template <int SF, int MODE, int CELLS, bool FEXT = false>
-__global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles in,
+template <int SF, int MODE, int CELLS, int ROWS, bool FEXT = false>
+__global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles in,
                                                        pmpm_particles out, pmpm_spatial part, pmpm_nodes nodes,
                                                        int tiles_x, int tiles_y, float *__restrict__ partials,
                                                        int32_t *__restrict__ flags, const float *__restrict__ rec) {
   constexpr int NV = p2g_nv<3, MODE>();
-  using M = MfmaGeom<SF, CELLS, NV>;
+  using M = MfmaGeom<SF, CELLS, ROWS, NV>;
   static_assert(MODE == 0 || !FEXT, "only the P2G carries the wall force");
   static_assert(CELLS == 4 || CELLS == 8, "cells per wave");
   constexpr int SPAN = M::SPAN, NLO = M::NLO, CH = M::CH, BN = M::BN;
   constexpr bool TYPED = SF == PMPM_SF_CUBIC;
   // floats of a staged record: the fractions, then MODE 0: (m, m v) and the
-  // rows of A with the wall force; MODE 1: m v'; MODE 2: per component
-  // (v_pic adjoint, L adjoint's column), dv.x, then (dv.y, dv.z)
-  constexpr int RS = MODE == 0 ? 20 : (MODE == 1 ? 8 : 24);
-  __shared__ float block[4][NV * BN];
-  __shared__ __attribute__((aligned(16))) float stage[4][CH * RS];
+  // rows of A with the wall force; MODE 1: m v'; MODE 2: dv.x, per component
+  // (v_pic adjoint, L adjoint's column), then (dv.y, dv.z)
+  constexpr int RS = MODE == 1 ? 8 : 20;
+  __shared__ __attribute__((aligned(16))) float block[M::WAVES][NV * BN];
+  __shared__ __attribute__((aligned(16))) float stage[M::WAVES][CH * RS];
 
   const int n = in.n;
   const float inv_h = g.inv_cell_size;
@@ -1263,12 +1274,12 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
   const int bx = blockIdx.x % tiles_x;
   const int by = (blockIdx.x / tiles_x) % tiles_y;
   const int bz = blockIdx.x / (tiles_x * tiles_y);
-  const int cy = by, cz = bz * M::TZ + wave;  // this wave's cell row
+  const int cx0 = bx * CELLS, cy = by * ROWS + wave / M::TZ, cz = bz * M::TZ + wave % M::TZ;  // this wave's row
   // lanes 0..CELLS-1 hold the ranges of the wave's cells
   int cs = 0, ce = 0;
   {
-    const int cx = bx * CELLS + lane;
-    if (lane < CELLS && cx < g.num_cells[0] && cz < g.num_cells[2]) {
+    const int cx = cx0 + lane;
+    if (lane < CELLS && cx < g.num_cells[0] && cy < g.num_cells[1] && cz < g.num_cells[2]) {
       const int cell = cx + g.num_cells[0] * (cy + g.num_cells[1] * cz);
       ce = part.cell_end[cell];
       cs = part.cell_start[cell];
@@ -1289,10 +1300,7 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
     const int u = __shfl_up(rend, o, 64);
     if (lane >= o) rend += u;
   }
-  int row_end[CELLS];
-#pragma unroll
-  for (int l = 0; l < CELLS; ++l) row_end[l] = __builtin_amdgcn_readlane(rend, l);
-  const int total = row_end[CELLS - 1];
+  const int total = __builtin_amdgcn_readlane(rend, CELLS - 1);
   const int shift = cs - (rend - pad);  // sorted index of a row, minus the row
 
   // a particle's raw fields, held in registers until staged
@@ -1303,36 +1311,56 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
     Sym sg;
     float dv[3], Lb[9];
   };
-  auto load_raw = [&](int r0, Raw &r) {
+  // the particle of row r0 + lane: its sorted index, slot and cell (the slots
+  // are fetched a round before the fields that need them)
+  struct Where {
+    uint32_t j, slot;
+    int c;
+    bool valid;
+  };
+  auto find = [&](int r0) {
+    Where w;
     const int row = r0 + lane;
-    int c = 0;
+    int c = 0;  // the first cell whose rows end past this one
 #pragma unroll
-    for (int l = 0; l < CELLS - 1; ++l) c += row >= row_end[l] ? 1 : 0;
+    for (int l = 0; l < CELLS - 1; ++l) c += __builtin_amdgcn_readlane(rend, l) <= row ? 1 : 0;
     const int j = __shfl(shift, c) + row, je = __shfl(ce, c);
-    r.cx = bx * CELLS + c;
-    r.valid = row < total && j < je;
-    const int jj = r.valid ? j : 0;
-    const int slot = part.sorted[jj];
-    r.slot = slot;
+    w.c = c;
+    w.valid = row < total && j < je;
+    w.j = w.valid ? (uint32_t)j : 0u;
+    w.slot = __float_as_uint(ld32(reinterpret_cast<const float *>(part.sorted), w.j));
+    return w;
+  };
+  auto load_raw = [&](const Where &w, Raw &r) {
+    const uint32_t jj = w.j, slot = w.slot;
+    r.cx = cx0 + w.c;
+    r.valid = w.valid;
+    r.slot = (int)slot;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      r.x[a] = in.x[a * n + slot];
-      r.v[a] = MODE == 0 ? in.v[a * n + slot] : (MODE == 1 ? out.v[a * n + jj] : rec[a * n + jj]);
+      const int64_t row_a = (int64_t)a * n;
+      r.x[a] = ld32(in.x + row_a, slot);
+      r.v[a] = MODE == 0 ? ld32(in.v + row_a, slot) : (MODE == 1 ? ld32(out.v + row_a, jj) : ld32(rec + row_a, jj));
     }
-    r.m = MODE == 2 ? 1.f : in.mass[slot];
-    r.vol = MODE == 0 ? in.volume[slot] : 0.f;
-    r.sg = MODE == 0 ? load_sym(in.stress, n, slot) : sym_zero();
+    r.m = MODE == 2 ? 1.f : ld32(in.mass, slot);
+    r.vol = MODE == 0 ? ld32(in.volume, slot) : 0.f;
+    r.sg = sym_zero();
+    if (MODE == 0) {
+      const float *sg = in.stress;
+      r.sg = Sym{ld32(sg, slot), ld32(sg + (int64_t)n, slot), ld32(sg + 2 * (int64_t)n, slot),
+                 ld32(sg + 3 * (int64_t)n, slot), ld32(sg + 4 * (int64_t)n, slot), ld32(sg + 5 * (int64_t)n, slot)};
+    }
     if (MODE == 2) {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) r.dv[a] = rec[(3 + a) * n + jj];
+      for (int a = 0; a < 3; ++a) r.dv[a] = ld32(rec + (3 + a) * (int64_t)n, jj);
 #pragma unroll
-      for (int a = 0; a < 9; ++a) r.Lb[a] = rec[(6 + a) * n + jj];
+      for (int a = 0; a < 9; ++a) r.Lb[a] = ld32(rec + (6 + a) * (int64_t)n, jj);
     }
   };
   // this lane's particle into its row of the stage (zero past the cell's
   // particles, and for a particle that is not its own cell's)
-  auto stage_raw = [&](const Raw &r) {
-    float fr[3];
+  // is the particle in the cell it is listed in? fr: its fractions there
+  auto own_cell = [&](const Raw &r, float *fr) {
     bool own = r.valid;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -1341,38 +1369,43 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
       own = own && ta >= 0.f && ba == (a == 0 ? r.cx : (a == 1 ? cy : cz));
       fr[a] = __fsub_rn(ta, (float)ba);
     }
+    return own;
+  };
+  auto minus_v_sigma = [&](const Raw &r) {
+    const float mvol = -r.vol;
+    return Sym{mvol * r.sg.xx, mvol * r.sg.yy, mvol * r.sg.zz, mvol * r.sg.xy, mvol * r.sg.xz, mvol * r.sg.yz};
+  };
+  bool strays = false;  // wave-uniform: some particle is listed in another cell than its own
+  auto stage_raw = [&](const Raw &r) {
+    float fr[3];
+    const bool own = own_cell(r, fr);
+    strays = strays || __ballot(r.valid && !own) != 0ull;
     float4 *sp = reinterpret_cast<float4 *>(st + lane * RS);
     Sym A = sym_zero();
     float fe[3] = {0.f, 0.f, 0.f};
     if (MODE == 0) {
-      const float mvol = -r.vol;
-      A = Sym{mvol * r.sg.xx, mvol * r.sg.yy, mvol * r.sg.zz, mvol * r.sg.xy, mvol * r.sg.xz, mvol * r.sg.yz};
+      A = minus_v_sigma(r);
       if (FEXT && r.valid) planar_force<3>(prm, g, r.x, r.v, r.vol, r.m, fe);
     }
-    if (MODE != 2 && r.valid && !own) {
-      // listed in this cell but binned elsewhere (a partition of other
-      // positions): deposited over its own window (MODE 2 runs on a
-      // partition of the same positions)
-#pragma unroll 1
-      for (int sy = 0; sy < 4; ++sy)
-        p2g_stray<3, SF, MODE == 1 ? 1 : 0>(prm, g, nodes, in.x, n, r.slot, sy, r.m, r.v, A, fe);
-    }
-    // (a row without an own particle is zero even if the fields it loaded
-    // are not finite)
-    sp[0] = own ? make_float4(fr[0], fr[1], fr[2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (MODE == 0) {
-      sp[1] = own ? make_float4(r.m, r.m * r.v[0], r.m * r.v[1], r.m * r.v[2]) : z4;
-      sp[2] = own ? make_float4(A.xx, A.xy, A.xz, fe[0]) : z4;
-      sp[3] = own ? make_float4(A.xy, A.yy, A.yz, fe[1]) : z4;
-      sp[4] = own ? make_float4(A.xz, A.yz, A.zz, fe[2]) : z4;
-    } else if (MODE == 1) {
-      sp[1] = own ? make_float4(r.m * r.v[0], r.m * r.v[1], r.m * r.v[2], 0.f) : z4;
+    // (a row without an own particle is zero even if the fields it loaded are
+    // not finite)
+    if (own) {
+      sp[0] = make_float4(fr[0], fr[1], fr[2], MODE == 2 ? r.dv[0] : 0.f);
+      if (MODE == 0) {
+        sp[1] = make_float4(r.m, r.m * r.v[0], r.m * r.v[1], r.m * r.v[2]);
+        sp[2] = make_float4(A.xx, A.xy, A.xz, fe[0]);
+        sp[3] = make_float4(A.xy, A.yy, A.yz, fe[1]);
+        sp[4] = make_float4(A.xz, A.yz, A.zz, fe[2]);
+      } else if (MODE == 1) {
+        sp[1] = make_float4(r.m * r.v[0], r.m * r.v[1], r.m * r.v[2], 0.f);
+      } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) sp[1 + a] = make_float4(r.v[a], r.Lb[a], r.Lb[3 + a], r.Lb[6 + a]);
+        sp[4] = make_float4(r.dv[1], r.dv[2], 0.f, 0.f);
+      }
     } else {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) sp[1 + a] = own ? make_float4(r.v[a], r.Lb[a], r.Lb[3 + a], r.Lb[6 + a]) : z4;
-      sp[4] = own ? make_float4(r.dv[0], 0.f, 0.f, 0.f) : z4;
-      sp[5] = own ? make_float4(r.dv[1], r.dv[2], 0.f, 0.f) : z4;
+      for (int q = 0; q < RS / 4; ++q) sp[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
 
@@ -1380,7 +1413,7 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
   const int s1 = (lane & 15) >> 2, s2 = lane & 3, pk = lane >> 4;
   SpanPoly<SF> px, py, pz;
   // y and z weights for x carry kx (see above)
-  auto set_yz = [&](int kx, SpanPoly<SF> &y, SpanPoly<SF> &z) {
+  auto set_yz = [&](int kx) {
     int ty = 0, tz = 0;
     if (TYPED) {
       int yv = cy + NLO + s1 + kx, zv = cz + NLO + s2;
@@ -1391,43 +1424,58 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
       ty = cubic_node_type(yv, g.num_cells[1], 1);
       tz = cubic_node_type(zv, g.num_cells[2], 1);
     }
-    y.set(s1, ty, inv_h, 1.f);
-    z.set(s2, tz, inv_h, 1.f);
+    py.set(s1, ty, inv_h, 1.f);
+    pz.set(s2, tz, inv_h, 1.f);
   };
-  set_yz(0, py, pz);
+  set_yz(0);
 
   v4f C1 = {0.f, 0.f, 0.f, 0.f}, C2 = C1;
-  auto product = [&](int row, const SpanPoly<SF> &x, const SpanPoly<SF> &y, const SpanPoly<SF> &z) {
-    const float *sp = st + (row + pk) * RS;
-    const float4 f = *reinterpret_cast<const float4 *>(sp);
-    const float Nx = x.N(f.x), Ny = y.N(f.y), Nz = z.N(f.z);
+  // what a product step reads of the stage (rows row .. row + 3): read one
+  // step ahead, so that the reads' latency passes behind the step before
+  struct Step {
+    float4 f, A;
+    float F;
+  };
+  const float *st_f = st + pk * RS;
+  // (MODE 0: field row 3 of the force is padding and reads row 2; MODE 2: row
+  // 3 is dv.x, which the fractions' word 3 holds, and C2's rows 2 and 3 are
+  // padding)
+  const float *st_A = st_f + (MODE == 0 ? 8 : 4) + 4 * min(s1, 2);
+  const float *st_F = st_f + (MODE == 2 ? 16 : 4) + s1;
+  auto read_step = [&](int row) {
+    Step q;
+    q.f = *reinterpret_cast<const float4 *>(st_f + row * RS);
+    if (MODE != 1) q.A = *reinterpret_cast<const float4 *>(st_A + row * RS);
+    q.F = st_F[row * RS];
+    return q;
+  };
+  auto product = [&](const Step &q) {
+    const float Nx = px.N(q.f.x), Ny = py.N(q.f.y), Nz = pz.N(q.f.z);
     const float b1 = Ny * Nz;
     if (MODE == 1) {
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[4 + s1], b1, C1, 0, 0, 0);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * q.F, b1, C1, 0, 0, 0);
       return;
     }
-    const float dNx = x.dN(f.x), dNy = y.dN(f.y), dNz = z.dN(f.z);
+    const float dNx = px.dN(q.f.x), dNy = py.dN(q.f.y), dNz = pz.dN(q.f.z);
     const float b2 = dNy * Nz, b3 = Ny * dNz;
     if (MODE == 0) {
-      // (field row 3 of the force is padding: it reads row 2)
-      const float4 A = *reinterpret_cast<const float4 *>(sp + 8 + 4 * min(s1, 2));
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[4 + s1], b1, C1, 0, 0, 0);
-      float a2 = dNx * A.x;
-      if (FEXT) a2 += Nx * A.w;
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * q.F, b1, C1, 0, 0, 0);
+      float a2 = dNx * q.A.x;
+      if (FEXT) a2 += Nx * q.A.w;
       C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, b1, C2, 0, 0, 0);
-      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.y, b2, C2, 0, 0, 0);
-      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.z, b3, C2, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * q.A.y, b2, C2, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * q.A.z, b3, C2, 0, 0, 0);
     } else {
-      const float4 A = *reinterpret_cast<const float4 *>(sp + 4 + 4 * s1);
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.x + dNx * A.y, b1, C1, 0, 0, 0);
-      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * sp[20 + s1], b1, C2, 0, 0, 0);
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.z, b2, C1, 0, 0, 0);
-      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * A.w, b3, C1, 0, 0, 0);
+      const bool v = s1 < 3;
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(v ? Nx * q.A.x + dNx * q.A.y : Nx * q.f.w, b1, C1, 0, 0, 0);
+      C2 = __builtin_amdgcn_mfma_f32_16x16x4f32(Nx * q.F, b1, C2, 0, 0, 0);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(v ? Nx * q.A.z : 0.f, b2, C1, 0, 0, 0);
+      C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(v ? Nx * q.A.w : 0.f, b3, C1, 0, 0, 0);
     }
   };
   // node column lx of the wave's row is complete: out of the accumulators
   auto flush = [&](int lx) {
-    float *b = blk + lx * M::XP + (lane & 15);
+    float *b = blk + lx * M::XP + 4 * s2 + s1;
     if (MODE != 1 || pk < 3) b[pk * BN] = C1[0];
     C1 = v4f{C1[1], C1[2], C1[3], 0.f};
     if (MODE != 1) {
@@ -1436,54 +1484,70 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
     }
   };
 
+  // the fields of the round to be staged next, and the slots of the one after
   Raw raw;
-  int next = 0;  // first row not yet loaded
+  Where ahead_w{};
+  int next = 2 * CH;  // first row whose slots are not yet fetched
   if (total > 0) {
-    load_raw(0, raw);
-    next = CH;
+    load_raw(find(0), raw);
+    if (CH < total) ahead_w = find(CH);
   }
   int r0 = -CH, row = 0;  // first staged row, current row
-  int xt = -1;            // x cells [3, nx - 4] share their node types
+  Step cur{};
+  bool inner_x = false;  // px holds the weights of the x cells [3, nx - 4], which share their node types
+  const int nx = g.num_cells[0];
 #pragma unroll 1
-  for (int l = 0; l < CELLS; ++l) {  // wave-uniform from here on
-    const int cx = bx * CELLS + l;
+  for (int l = 0; l < CELLS; ++l) {  // wave-uniform
+    const int cx = cx0 + l;
     const int end = __builtin_amdgcn_readlane(rend, l);
     if (row < end) {
-      const int nx = g.num_cells[0];
-      const bool inner = cx >= 3 && cx < nx - 3;
+      const bool inx = !TYPED || (cx >= 3 && cx < nx - 3);
       const int xv = cx + NLO + s2;  // this lane's x node
       const bool out_x = xv < 0 || xv >= nx;
-      if (!TYPED) {
-        if (xt < 0) px.set(s2, 0, inv_h, 1.f);
-        xt = 0;
-      } else if (!inner || xt != 1) {
-        px.set(s2, cubic_node_type(xv, nx, 1), inv_h, out_x ? 0.f : 1.f);
-        xt = inner ? 1 : 0;
+      if (!inx || !inner_x) {
+        px.set(s2, TYPED ? cubic_node_type(xv, nx, 1) : 0, inv_h, TYPED && out_x ? 0.f : 1.f);
+        inner_x = inx;
       }
-      const bool leaves = TYPED && MODE != 2 && !inner && prm.wrap_quirk && __ballot(out_x) != 0ull;
+      const bool leaves = TYPED && MODE != 2 && !inx && prm.wrap_quirk && __ballot(out_x) != 0ull;
       while (row < end) {
         if (row - r0 >= CH) {
           wave_lds_sync();  // the rows staged before are read
           stage_raw(raw);
           r0 = row;
-          if (next < total) load_raw(next, raw);
+          if (r0 + CH < total) load_raw(ahead_w, raw);
+          if (next < total) ahead_w = find(next);
           next += CH;
           wave_lds_sync();
+          cur = read_step(0);
         }
         const int stop = min(end, r0 + CH);
         const int first = row;
-#pragma unroll 2
-        for (; row < stop; row += 4) product(row - r0, px, py, pz);
+        // (two steps per turn: no register copies between cur and ahead)
+        for (; row + 4 < stop; row += 8) {
+          const Step ahead = read_step(row + 4 - r0);
+          __builtin_amdgcn_sched_barrier(0);
+          product(cur);
+          cur = read_step((row + 8 - r0) & (CH - 1));
+          __builtin_amdgcn_sched_barrier(0);
+          product(ahead);
+        }
+        if (row < stop) {
+          const Step ahead = read_step((row + 4 - r0) & (CH - 1));
+          product(cur);
+          cur = ahead;
+          row += 4;
+        }
         if (leaves) {
 #pragma unroll 1
           for (int kx = -1; kx <= 2; ++kx) {  // (2: one-node grids only)
             const bool mine = kx != 0 && xv - kx * nx >= 0 && xv - kx * nx < nx;
             if (__ballot(mine) == 0ull) continue;
-            SpanPoly<SF> ox, oy, oz;
-            ox.set(s2, cubic_node_type(mine ? xv - kx * nx : 0, nx, 1), inv_h, mine ? 1.f : 0.f);
-            set_yz(kx, oy, oz);
-            for (int q = first; q < stop; q += 4) product(q - r0, ox, oy, oz);
+            px.set(s2, cubic_node_type(mine ? xv - kx * nx : 0, nx, 1), inv_h, mine ? 1.f : 0.f);
+            set_yz(kx);
+            for (int q = first; q < stop; q += 4) product(read_step(q - r0));
           }
+          px.set(s2, cubic_node_type(xv, nx, 1), inv_h, out_x ? 0.f : 1.f);
+          set_yz(0);
         }
       }
     }
@@ -1491,22 +1555,50 @@ __global__ __launch_bounds__(256) void p2g_mfma_kernel(pmpm_params prm, pmpm_gri
   }
 #pragma unroll
   for (int l = 0; l < SPAN - 1; ++l) flush(CELLS + l);
-  __syncthreads();
-  // slice node (ix, iy, iz): the columns of waves iz - SPAN + 1 .. iz
-  float *slice = partials + (int64_t)blockIdx.x * NV * M::NTN;
+  lds_barrier();
+  // the waves' columns: node (ix, iy, iz) lies in the rows iy - SPAN + 1 .. iy
+  // and the layers iz - SPAN + 1 .. iz; slices are stored y slowest
   if (t == 0) flags[blockIdx.x] = 1;
-  for (int i = t; i < M::NTN; i += 256) {
-    const int ix = i % M::BX, iy = (i / M::BX) % SPAN, iz = i / (M::BX * SPAN);
-    float sum[NV] = {};
+  float *slice = partials + (int64_t)blockIdx.x * NV * M::NTN;
+  constexpr int PL = M::BX * M::NZ;  // nodes of a y plane
+  for (int i = t; i < PL * NV; i += M::THREADS) {
+    const int ix = i % M::BX, iz = (i / M::BX) % M::NZ, f = i / PL;
+    float sum[M::NY];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int y = 0; y < M::NY; ++y) sum[y] = 0.f;
+#pragma unroll
+    for (int w = 0; w < M::TZ; ++w) {
       const int z = iz - w;
       if (z < 0 || z >= SPAN) continue;
 #pragma unroll
-      for (int f = 0; f < NV; ++f) sum[f] += block[w][f * BN + ix * M::XP + 4 * iy + z];
+      for (int r = 0; r < ROWS; ++r) {
+        const float4 q = *reinterpret_cast<const float4 *>(&block[r * M::TZ + w][f * BN + ix * M::XP + 4 * z]);
+        const float yj[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < SPAN; ++j) sum[r + j] += yj[j];
+      }
     }
 #pragma unroll
-    for (int f = 0; f < NV; ++f) slice[f * M::NTN + i] = sum[f];
+    for (int y = 0; y < M::NY; ++y) slice[f * M::NTN + y * PL + i % PL] = sum[y];
+  }
+  if (MODE != 2 && strays) {
+    // particles listed in this row but binned elsewhere (a partition of other
+    // positions): deposited over their own windows, straight to the node
+    // arrays (MODE 2 runs on a partition of the same positions). Walked again
+    // here, where the registers of the products are free.
+#pragma unroll 1
+    for (int q0 = 0; q0 < total; q0 += 64) {
+      Raw q;
+      float fr[3], fe[3] = {0.f, 0.f, 0.f};
+      load_raw(find(q0), q);
+      if (own_cell(q, fr) || !q.valid) continue;
+      Sym A = sym_zero();
+      if (MODE == 0) A = minus_v_sigma(q);
+      if (FEXT) planar_force<3>(prm, g, q.x, q.v, q.vol, q.m, fe);
+#pragma unroll 1
+      for (int sy = 0; sy < 4; ++sy)
+        p2g_stray<3, SF, MODE == 1 ? 1 : 0>(prm, g, nodes, in.x, n, q.slot, sy, q.m, q.v, A, fe);
+    }
   }
 }
 
@@ -1758,9 +1850,12 @@ struct TileGeom {
 // live tile covers skips the loads).
 // TG: the tiling's constants (Tiles3) in 3D, where the divisions then become
 // shifts; the runtime values of tg in 1D and 2D.
-template <int SPAN_, int CELLS_> struct Tiles3 {
-  static constexpr int SPAN = SPAN_, NLO = SPAN_ == 2 ? 0 : -1, COVER_Y = SPAN_;
-  static constexpr int T[3] = {CELLS_, 1, 4}, N[3] = {CELLS_ + SPAN_ - 1, SPAN_, 3 + SPAN_};
+template <int SPAN_, int CELLS_, int ROWS_> struct Tiles3 {
+  static constexpr int SPAN = SPAN_, NLO = SPAN_ == 2 ? 0 : -1;
+  static constexpr int T[3] = {CELLS_, ROWS_, 4}, N[3] = {CELLS_ + SPAN_ - 1, ROWS_ + SPAN_ - 1, 3 + SPAN_};
+  static constexpr int COVER_Y = (N[1] - 1) / T[1] + 1;
+  static_assert((N[0] - 1) / T[0] + 1 <= kCoverX && COVER_Y <= kCoverY && (N[2] - 1) / T[2] + 1 <= kCoverZ,
+                "the gather visits at most kCover tiles per axis");
 };
 struct TilesRuntime { static constexpr int COVER_Y = -1; };
 template <int D, int NV, class TG = TilesRuntime>
@@ -1805,8 +1900,9 @@ __device__ inline bool gather_partials(const TileGeom &tg, const float *partials
         const int tile = in ? bx + tg.tiles[0] * (by + tg.tiles[1] * bz) : 0;
         live[c] = in && flags[tile] != 0;
         int li = ids[0] - (bx * T[0] + nlo);
-        if (D > 1) li += N[0] * (ids[1] - (by * T[1] + nlo));
-        if (D > 2) li += N[0] * N[1] * (ids[2] - (bz * T[2] + nlo));
+        // (3D slices: y slowest)
+        if (D == 2) li += N[0] * (ids[1] - (by * T[1] + nlo));
+        if (D > 2) li += N[0] * (ids[2] - (bz * T[2] + nlo) + N[2] * (ids[1] - (by * T[1] + nlo)));
         off[c] = (int64_t)tile * NV * ntn + li;
       }
   bool any = false;
@@ -2692,18 +2788,20 @@ template <int D, int SF> TileGeom tile_geom_of(const pmpm_grid &g, int gather) {
   tg.nv = gather == 2 ? D : (gather == 3 ? 2 * D : 1 + 2 * D);  // 3: adjoint scatter
   return tg;
 }
-// Cells per wave of the 3D P2G tiles (MfmaGeom): 8, or 4 on small grids, where
-// eight cells per wave leave most of the chip idle. A function of the grid and
-// the particle count only: every pass of a step, and pmpm_step_noalloc, must
-// agree on it.
+// The 3D P2G tiles (MfmaGeom) of a scene. A function of the grid and the
+// particle count only: every pass of a step, and pmpm_step_noalloc, must agree
+// on it. Small scenes take small tiles (more waves, each with a short chain of
+// cells), the others larger ones (fewer nodes per cell in the slices).
+struct MfmaTiles { int cells, rows; };
 constexpr int kSmallGridNodes = 131072, kSmallParticles = 131072;
-static int mfma_cells(const pmpm_grid &g, int n) {
-  return g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles ? 4 : 8;
+static MfmaTiles mfma_tiles(const pmpm_grid &g, int n) {
+  if (g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles) return {4, 1};
+  return {8, 2};
 }
-static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, int cells) {
+static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, MfmaTiles m) {
   TileGeom tg{};
   const int span = sf == PMPM_SF_LINEAR ? 2 : 4;
-  const int T[3] = {cells, 1, 4}, N[3] = {cells + span - 1, span, 3 + span};
+  const int T[3] = {m.cells, m.rows, 4}, N[3] = {m.cells + span - 1, m.rows + span - 1, 3 + span};
   tg.nlo = sf == PMPM_SF_LINEAR ? 0 : -1;
   for (int a = 0; a < 3; ++a) {
     tg.T[a] = T[a];
@@ -2714,6 +2812,15 @@ static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, int cells
   tg.nv = gather == 2 ? 3 : (gather == 3 ? 6 : 7);
   return tg;
 }
+// M(args, Tiles3<..>) for the tiles of tg (3D).
+#define PMPM_WITH_TILES3(tg, M, ...)                            \
+  if ((tg).N[1] - (tg).T[1] == 1) {                             \
+    if ((tg).T[0] == 4) { M(__VA_ARGS__ Tiles3<2, 4, 1>); }     \
+    else { M(__VA_ARGS__ Tiles3<2, 8, 2>); }                    \
+  } else {                                                      \
+    if ((tg).T[0] == 4) { M(__VA_ARGS__ Tiles3<4, 4, 1>); }     \
+    else { M(__VA_ARGS__ Tiles3<4, 8, 2>); }                    \
+  }
 // The tiles of a P2G pass over n particles (gather: TileGeom::gather, or 3 for
 // the adjoint scatter).
 static TileGeom tile_geom(const pmpm_params &prm, const pmpm_grid &g, int gather, int n) {
@@ -2724,29 +2831,25 @@ static TileGeom tile_geom(const pmpm_params &prm, const pmpm_grid &g, int gather
     case 6: return tile_geom_of<2, PMPM_SF_LINEAR>(g, gather);
     case 7: return tile_geom_of<2, PMPM_SF_QUADRATIC>(g, gather);
     case 8: return tile_geom_of<2, PMPM_SF_CUBIC>(g, gather);
-    default: return mfma_tile_geom(prm.shape_fn, g, gather, mfma_cells(g, n));
+    default: return mfma_tile_geom(prm.shape_fn, g, gather, mfma_tiles(g, n));
   }
 }
 static size_t tile_count(const TileGeom &tg) { return (size_t)tg.tiles[0] * tg.tiles[1] * tg.tiles[2]; }
 
-template <int SF, int CELLS>
+template <int SF, int CELLS, int ROWS>
 static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
                             const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, int mode,
                             float *partials, int32_t *flags, hipStream_t s, const float *rec) {
-  const TileGeom mg = mfma_tile_geom(SF, g, mode + 1, CELLS);
-  const dim3 grid((unsigned)tile_count(mg)), block(256);
-  if (mode == 0 && has_planar(prm))
-    PMPM_LAUNCH((p2g_mfma_kernel<SF, 0, CELLS, true>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 0L, 1L})), grid,
-                block, 0, s, prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
-  else if (mode == 0)
-    PMPM_LAUNCH((p2g_mfma_kernel<SF, 0, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 0L})), grid, block, 0, s,
-                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
-  else if (mode == 1)
-    PMPM_LAUNCH((p2g_mfma_kernel<SF, 1, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 1L})), grid, block, 0, s,
-                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
-  else
-    PMPM_LAUNCH((p2g_mfma_kernel<SF, 2, CELLS>), (::pmpm::kname("p2g_mfma_kernel", {(long)SF, 2L})), grid, block, 0, s,
-                prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec);
+  const TileGeom mg = mfma_tile_geom(SF, g, mode + 1, MfmaTiles{CELLS, ROWS});
+  const dim3 grid((unsigned)tile_count(mg)), block(256 * ROWS);
+#define PMPM_MFMA(MODE, FEXT, ...)                                                                               \
+  PMPM_LAUNCH((p2g_mfma_kernel<SF, MODE, CELLS, ROWS, FEXT>), (::pmpm::kname("p2g_mfma_kernel", {__VA_ARGS__})), \
+              grid, block, 0, s, prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec)
+  if (mode == 0 && has_planar(prm)) PMPM_MFMA(0, true, (long)SF, 0L, 1L);
+  else if (mode == 0) PMPM_MFMA(0, false, (long)SF, 0L);
+  else if (mode == 1) PMPM_MFMA(1, false, (long)SF, 1L);
+  else PMPM_MFMA(2, false, (long)SF, 2L);
+#undef PMPM_MFMA
 }
 
 // mode 0: P2G, 1: MUSL first map + re-map, 2: adjoint scatter of the
@@ -2762,10 +2865,10 @@ void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles
     if (mode == 1 && in.n > 0)
       PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0,
                          s, prm, g, in, out, part, nodes, 1);
-    if (mfma_cells(g, in.n) == 4)
-      launch_p2g_mfma<SF, 4>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+    if (mfma_tiles(g, in.n).cells == 4)
+      launch_p2g_mfma<SF, 4, 1>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
     else
-      launch_p2g_mfma<SF, 8>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+      launch_p2g_mfma<SF, 8, 2>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
   } else {
     const TileGeom tg = tile_geom_of<D, SF>(g, 1);
     const dim3 grid((unsigned)tile_count(tg)), block(P2GGeom<D, SF>::THREADS);
@@ -2832,14 +2935,10 @@ int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
   if (gather == 0) PMPM_GRID_LAUNCH(D, 0, TilesRuntime);         \
   else if (gather == 1) PMPM_GRID_LAUNCH(D, 1, __VA_ARGS__);     \
   else PMPM_GRID_LAUNCH(D, 2, __VA_ARGS__)
-  const bool lin = prm.shape_fn == PMPM_SF_LINEAR, small = tg.T[0] == 4;
   if (prm.dim == 1) { PMPM_GRID_GATHER(1, TilesRuntime); }
   else if (prm.dim == 2) { PMPM_GRID_GATHER(2, TilesRuntime); }
   else if (prm.dim != 3) return PMPM_ERR_INVALID;
-  else if (lin && small) { PMPM_GRID_GATHER(3, Tiles3<2, 4>); }
-  else if (lin) { PMPM_GRID_GATHER(3, Tiles3<2, 8>); }
-  else if (small) { PMPM_GRID_GATHER(3, Tiles3<4, 4>); }
-  else { PMPM_GRID_GATHER(3, Tiles3<4, 8>); }
+  else PMPM_WITH_TILES3(tg, PMPM_GRID_GATHER, 3, )
 #undef PMPM_GRID_GATHER
 #undef PMPM_GRID_LAUNCH
   PMPM_LAUNCH_CHECK();
@@ -3909,16 +4008,10 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
 #define PMPM_GRID_ADJOINT(...)                                                                                   \
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
               dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
-  const bool lin = prm->shape_fn == PMPM_SF_LINEAR, small = tg.T[0] == 4;
   switch (D) {
     case 1: PMPM_GRID_ADJOINT(1, TilesRuntime); break;
     case 2: PMPM_GRID_ADJOINT(2, TilesRuntime); break;
-    default:
-      if (lin && small) PMPM_GRID_ADJOINT(3, Tiles3<2, 4>);
-      else if (lin) PMPM_GRID_ADJOINT(3, Tiles3<2, 8>);
-      else if (small) PMPM_GRID_ADJOINT(3, Tiles3<4, 4>);
-      else PMPM_GRID_ADJOINT(3, Tiles3<4, 8>);
-      break;
+    default: PMPM_WITH_TILES3(tg, PMPM_GRID_ADJOINT, 3, ) break;
   }
 #undef PMPM_GRID_ADJOINT
   PMPM_LAUNCH_CHECK();
