@@ -18,7 +18,7 @@ struct pmpm_context {
   int32_t *vals_tmp = nullptr;   // radix sort ping-pong values
   uint32_t *hist = nullptr;      // [radix][blocks] digit histograms
   size_t hist_len = 0;
-  uint32_t *counters = nullptr;  // [4]: out-of-grid particles, hint unsorted flag, movers, -
+  uint32_t *counters = nullptr;  // [4]: out-of-grid particles, hint unsorted flag (set, kept), heavy cells
   bool counters_clear = false;   // cleared once, by the first call that uses them
   // P2G tile partials: per tile, the LDS node block of each accumulated field
   // (plain stores; the grid kernel sums the <= 2^D tiles covering a node)
@@ -53,23 +53,22 @@ struct pmpm_context {
   size_t adj_pb_cap = 0;
   // partition from a sorted hint (the previous call's sorted keys): false
   // always runs the full radix sort (PMPM_PARTITION_RADIX=1 at creation);
-  // below hint_min_particles particles the radix sort runs too (its fewer
-  // launches win there; PMPM_PARTITION_HINT_MIN at creation)
+  // below hint_min_particles particles the radix sort runs too
+  // (PMPM_PARTITION_HINT_MIN at creation)
   bool sort_by_hint = true;
-  int32_t hint_min_particles = 131072;
+  int32_t hint_min_particles = 0;
   // per cell (ncells + 1, the last for the out-of-grid particles): counts
-  // of stayers and movers (zero between calls), and per block of 1024 cells
+  // of stayers and movers (zero between calls), and per block of 1024 cells;
+  // hint_clear: both have been cleared since they were allocated
   float *hint_cnt = nullptr;
   size_t hint_cnt_cap = 0;
   float *hint_cbt = nullptr;
   size_t hint_cbt_cap = 0;
+  bool hint_clear = false;
   // per cell: first slot, stayers before the cell, stayers, movers
   float *hint_info = nullptr;
   size_t hint_info_cap = 0;
-  // stayers per block of 1024 particles, then five arrays of n words:
-  // stayers before each particle (sign bit: a stayer), the movers' keys in
-  // slot order, the stayers before each mover, the sorted movers' keys and
-  // positions in the mover list
+  // per particle (HintLayout in partition.hip)
   float *hint_part = nullptr;
   size_t hint_part_cap = 0;
 };

@@ -94,25 +94,12 @@ __global__ void hash_kernel(const float *__restrict__ x, int n, pmpm_grid g, uin
 // step's G2P wrote the particles in cell order), so a wave's 64 consecutive
 // keys hold a few runs of one digit: the head lane of each run adds the
 // run's length, one LDS atomic per run instead of one per key.
-// Sorts of at most this many keys with a device-side count (the hint
-// partition's movers) run in one workgroup (small_sort_kernel); the
-// multi-block radix kernels skip them.
-constexpr int kSmallSort = 4096;
-
-// n_dev (optional): the key count is min(n, *n_dev), read on the device (the
-// grid is sized for n; the blocks past the count exit, and a count of at most
-// kSmallSort is left to small_sort_kernel).
 template <int RB>
 __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const uint32_t *__restrict__ keys, int n, int shift,
-                                                                uint32_t *__restrict__ hist, int nblocks,
-                                                                const uint32_t *__restrict__ n_dev) {
+                                                                uint32_t *__restrict__ hist, int nblocks) {
   constexpr int R = 1 << RB;
   __shared__ uint32_t h[R];
   const int t = threadIdx.x, lane = t & 63;
-  if (n_dev) {
-    n = min(n, (int)*n_dev);
-    if (n <= kSmallSort || (int64_t)blockIdx.x * kSortTile >= n) return;  // block-uniform
-  }
   for (int d = t; d < R; d += kSortBlock) h[d] = 0u;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * kSortTile;
@@ -137,20 +124,14 @@ __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const uint32_t *
 
 // Exclusive scan of each digit's column hist[d][0..nblocks) (one workgroup
 // per digit); the column total goes to totals[d].
-// With n_dev, only the columns' first ceil(*n_dev / kSortTile) entries (the
-// blocks that hold keys) are scanned, and nothing for a count of at most
-// kSmallSort.
 __global__ __launch_bounds__(256) void scan_columns_kernel(uint32_t *__restrict__ hist, int nblocks,
-                                                           uint32_t *__restrict__ totals,
-                                                           const uint32_t *__restrict__ n_dev) {
+                                                           uint32_t *__restrict__ totals) {
   __shared__ uint32_t part[256];
   const int t = threadIdx.x;
   uint32_t *col = hist + (int64_t)blockIdx.x * nblocks;
-  if (n_dev && *n_dev <= (uint32_t)kSmallSort) return;  // block-uniform
-  const int nb = n_dev ? min(nblocks, (int)(((int64_t)*n_dev + kSortTile - 1) / kSortTile)) : nblocks;
-  const int chunk = (nb + 255) / 256;
+  const int chunk = (nblocks + 255) / 256;
   const int b = t * chunk;
-  const int e = min(b + chunk, nb);
+  const int e = min(b + chunk, nblocks);
   uint32_t s = 0;
   for (int i = b; i < e; ++i) s += col[i];
   part[t] = s;
@@ -178,14 +159,9 @@ template <int RB>
 __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     const uint32_t *__restrict__ keys_in, const int32_t *__restrict__ vals_in, uint32_t *__restrict__ keys_out,
     int32_t *__restrict__ vals_out, int n, int shift, const uint32_t *__restrict__ hist, int nblocks,
-    const uint32_t *__restrict__ totals, const uint32_t *__restrict__ n_dev) {
+    const uint32_t *__restrict__ totals) {
   constexpr int R = 1 << RB, W = kSortBlock / 64;
   static_assert(R <= kSortBlock, "one digit per thread");
-  if (n_dev) {
-    n = min(n, (int)*n_dev);
-    if (n <= kSmallSort) return;  // block-uniform
-  }
-  if ((int64_t)blockIdx.x * kSortTile >= n) return;  // block-uniform: no keys here
   __shared__ uint32_t base[R];
   __shared__ uint32_t wcnt[W][R];
   __shared__ uint32_t wsum[W];
@@ -268,218 +244,96 @@ __global__ void cell_range_kernel(const uint32_t *__restrict__ hs, int n, uint32
   if (j == n - 1 || hs[j + 1] != h) cend[h] = j + 1;
 }
 
-// Stable LSD radix sort of at most kSmallSort keys in one workgroup, in LDS
-// (10-bit digits, `passes` of them; values = input positions): the hint
-// partition's movers when the count *n_dev is that small (the multi-block
-// kernels take larger counts). Thread d owns digit d; ranking within a round
-// of 1024 keys as in radix_scatter_kernel; only the rounds that hold keys run.
-__global__ __launch_bounds__(kSortBlock) void small_sort_kernel(const uint32_t *__restrict__ keys_in,
-                                                                const uint32_t *__restrict__ n_dev, int passes,
-                                                                uint32_t *__restrict__ keys_out,
-                                                                int32_t *__restrict__ vals_out) {
-  constexpr int RB = 10, R = 1 << RB, W = kSortBlock / 64;
-  static_assert(R == kSortBlock, "one digit per thread");
-  __shared__ uint32_t sk[2][kSmallSort];
-  __shared__ int32_t sv[2][kSmallSort];
-  __shared__ uint32_t wcnt[W][R];
-  __shared__ uint32_t wsum[W];
-  const uint32_t cnt = *n_dev;
-  if (cnt > (uint32_t)kSmallSort) return;  // block-uniform: the multi-block path
-  const int m = (int)cnt;
-  const int rounds = (m + kSortBlock - 1) / kSortBlock;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int r = 0; r < rounds; ++r) {
-    const int i = r * kSortBlock + t;
-    if (i < m) {
-      sk[0][i] = keys_in[i];
-      sv[0][i] = i;
-    }
-  }
-  int src = 0;
-  for (int p = 0; p < passes; ++p) {
-    const int shift = RB * p, dst = src ^ 1;
-    // digit totals (run lengths, as radix_hist_kernel), then their exclusive
-    // scan: thread t owns digit t
-#pragma unroll
-    for (int q = 0; q < W; ++q) wcnt[q][t] = 0u;
-    __syncthreads();
-    for (int r = 0; r < rounds; ++r) {
-      const int i = r * kSortBlock + t;
-      const bool valid = i < m;
-      const uint32_t d = valid ? (sk[src][i] >> shift) & (R - 1) : 0u;
-      const uint32_t prev = (uint32_t)__shfl_up((int)d, 1, 64);
-      const bool head = valid && (lane == 0 || prev != d);
-      const uint64_t heads = __ballot(head);
-      const int nvalid = __popcll(__ballot(valid));
-      if (head) {
-        const uint64_t later = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
-        const int next = later ? __ffsll((unsigned long long)later) - 1 : nvalid;
-        atomicAdd(&wcnt[0][d], (uint32_t)(next - lane));
-      }
-    }
-    __syncthreads();
-    const uint32_t tot = wcnt[0][t];
-    uint32_t incl = tot;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 64);
-      if (lane >= o) incl += u;
-    }
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    uint32_t before = 0u;
-    for (int q = 0; q < w; ++q) before += wsum[q];
-    uint32_t base = before + incl - tot;  // this thread's digit
-    for (int r = 0; r < rounds; ++r) {
-#pragma unroll
-      for (int q = 0; q < W; ++q) wcnt[q][t] = 0u;
-      __syncthreads();
-      const int i = r * kSortBlock + t;
-      const bool valid = i < m;
-      const uint32_t key = valid ? sk[src][i] : 0u;
-      const int32_t val = valid ? sv[src][i] : 0;
-      const uint32_t d = (key >> shift) & (R - 1);
-      uint64_t peers = __ballot(valid);
-#pragma unroll
-      for (int bit = 0; bit < RB; ++bit) {
-        const bool on = (d >> bit) & 1u;
-        const uint64_t mk = __ballot(on);
-        peers &= on ? mk : ~mk;
-      }
-      const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
-      if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-      __syncthreads();
-      {
-        uint32_t run = base;
-#pragma unroll
-        for (int q = 0; q < W; ++q) {
-          const uint32_t c = wcnt[q][t];
-          wcnt[q][t] = run;
-          run += c;
-        }
-        base = run;
-      }
-      __syncthreads();
-      if (valid) {
-        const uint32_t pos = wcnt[w][d] + rank;
-        if (pos < (uint32_t)m) {
-          sk[dst][pos] = key;
-          sv[dst][pos] = val;
-        }
-      }
-      __syncthreads();
-    }
-    src = dst;
-  }
-  for (int r = 0; r < rounds; ++r) {
-    const int i = r * kSortBlock + t;
-    if (i < m) {
-      keys_out[i] = sk[src][i];
-      vals_out[i] = sv[src][i];
-    }
-  }
-}
-
 // ---- Partition from a sorted hint ----------------------------------------
 // pmpm_step hands the particles to the next partition in the previous
 // partition's (cell, slot) order, and that partition's sorted keys are still
 // in hash_sorted. Used as a hint h[i], they equal the new key k[i] for every
 // particle that kept its cell. If h is sorted, the particles with k[i] ==
 // h[i] ("stayers") are in (key, slot) order among themselves already, so only
-// the others ("movers") need sorting, and the stable order is a merge per
-// cell c, with S[i] = stayers before slot i:
-//   first slot of c:         out_start[c] = particles with key < c
-//   stayer i:                out_start[c] + (S[i] - stayers with key < c)
-//                            + movers of c before slot i
-//   r-th mover (sorted):     out_start[c] + (r - movers with key < c)
-//                            + clamp(S[i] - stayers with key < c, 0, stayers of c)
+// the others ("movers") are ordered, per cell, and the stable order is a merge
+// per cell c, with S[i] = stayers before slot i:
+//   first slot of c: out_start[c] = particles with key < c
+//   stayer i:        out_start[c] + (S[i] - stayers with key < c) + movers of c before slot i
+//   mover i:         out_start[c] + movers of c before slot i
+//                    + clamp(S[i] - stayers with key < c, 0, stayers of c)
 // (stayers are sorted by key, so the first S[i] of them are those before i).
-// The movers are compacted in slot order and sorted by the radix passes; any
-// hint gives the stable sort (an unsorted hint makes every particle a mover),
-// a good one a short mover list.
-constexpr int kHintBlock = 1024;   // particles, or cells, per workgroup
-constexpr int kHintCellBits = 10;  // cells per block of the cell scan: 1 << 10
-constexpr int kHintSlots = 4;      // cell blocks a classify workgroup sums in LDS
-static_assert((1 << kHintCellBits) == kHintBlock, "one cell per thread in the cell scan");
+// An unsorted hint makes every particle a mover; any hint gives the stable
+// sort, a good one few movers.
+//
+// Four launches whatever the mover count: classify (keys, stay bits, counts
+// per cell), scan (cells), movers (each into its cell's part of a list, in any
+// order), place (a particle counts the movers of its cell with a smaller slot:
+// a step has a handful per 1000 particles). Cells with more than kHeavyMovers
+// movers get their part of the list in slot order from a workgroup that walks
+// all particles, and are searched by bisection, so no particle's count takes
+// more than kHeavyMovers reads. The movers used to be sorted, in one workgroup
+// up to 4,096 of them and by six multi-block radix launches otherwise, which
+// cost their launch also when they had nothing to do: ten launches and 50 us
+// at 1.08M particles, 39 us with these four. Small scenes gain most (17k
+// particles: 45 us of radix sort, 17 us).
+constexpr int kHintBlock = 256;     // particles per workgroup of classify and place
+constexpr int kHintCells = 1024;    // cells per workgroup of the scan
+constexpr int kHintCellBits = 10;
+constexpr int kHintSlots = 4;       // cell blocks a classify workgroup sums in LDS
+constexpr int kMoverBlock = 1024;   // threads of the movers pass
+constexpr int kHeavyMovers = 2048;
+static_assert((1 << kHintCellBits) == kHintCells, "one cell per thread in the cell scan");
 
-// Exclusive scan over a workgroup of kHintBlock threads; every thread gets its
-// prefix and the total. `w` holds kHintBlock / 64 words of LDS.
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *w, uint32_t &total) {
+// Exclusive scan over a workgroup of THREADS threads; every thread gets its
+// prefix and the total. `w` holds THREADS / 64 words of LDS.
+template <int THREADS, class T>
+__device__ inline T block_exclusive_scan(T v, T *w, T &total) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  uint32_t incl = v;
+  T incl = v;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 64);
+    const T u = (T)__shfl_up((unsigned long long)incl, o, 64);
     if (lane >= o) incl += u;
   }
   __syncthreads();  // w may still be read by an earlier call
   if (lane == 63) w[wv] = incl;
   __syncthreads();
-  uint32_t before = 0u, all = 0u;
+  T before = 0, all = 0;
 #pragma unroll
-  for (int q = 0; q < kHintBlock / 64; ++q) {
-    const uint32_t x = w[q];
-    before += q < wv ? x : 0u;
+  for (int q = 0; q < THREADS / 64; ++q) {
+    const T x = w[q];
+    before += q < wv ? x : (T)0;
     all += x;
   }
   total = all;
   return before + incl - v;
 }
 
-// Sum over a workgroup of kHintBlock threads (every thread gets it).
-__device__ inline uint32_t block_sum(uint32_t v, uint32_t *w) {
-  uint32_t total;
-  (void)block_exclusive_scan(v, w, total);
-  return total;
+template <int D>
+__device__ inline uint32_t cell_key(const float *__restrict__ x, int n, int i, const pmpm_grid &g, int *b) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) b[a] = (int)__fmul_rn(__fsub_rn(x[(int64_t)a * n + i], g.origin[a]), g.inv_cell_size);
+  int64_t h = b[0];
+  if (D > 1) h += (int64_t)b[1] * g.num_cells[0];
+  if (D > 2) h += (int64_t)b[2] * g.num_cells[0] * g.num_cells[1];
+  return (h < 0 || h >= g.num_cells_total) ? (uint32_t)g.num_cells_total : (uint32_t)h;
 }
 
-// The same scan of two 32-bit counts at once, packed as (high << 32) | low
-// (no carry crosses: each count stays below 2^31). `w` holds kHintBlock / 64
-// 64-bit words of LDS.
-__device__ inline uint64_t block_exclusive_scan2(uint64_t v, uint64_t *w, uint64_t &total) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  uint64_t incl = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t u = (uint64_t)__shfl_up((unsigned long long)incl, o, 64);
-    if (lane >= o) incl += u;
-  }
-  __syncthreads();  // w may still be read by an earlier call
-  if (lane == 63) w[wv] = incl;
-  __syncthreads();
-  uint64_t before = 0u, all = 0u;
-#pragma unroll
-  for (int q = 0; q < kHintBlock / 64; ++q) {
-    const uint64_t x = w[q];
-    before += q < wv ? x : 0u;
-    all += x;
-  }
-  total = all;
-  return before + incl - v;
-}
-
-// Cell key per particle (as hash_kernel), its class against the hint, and the
-// counts: per cell and per block of cells, stayers and movers (a run of lanes
-// with one key and one class adds its length once); stayers per workgroup.
-// flags[0] is set when the hint is not sorted. Blocks past the particles
-// only clear `clear`.
+// Cell key per particle (as hash_kernel), its class against the hint as a bit
+// (stay[i / 64]), and the counts: per cell and per block of cells, stayers and
+// movers (a run of lanes with one key and one class adds its length once);
+// stayers per workgroup. flags[0] is set when the hint is not sorted. Blocks
+// past the particles only clear `clear`.
 template <int D>
 __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
     const float *__restrict__ x, int n, pmpm_grid g, const uint32_t *__restrict__ hint, uint32_t *__restrict__ hash,
     int32_t *__restrict__ bins, uint32_t *__restrict__ cnt, uint32_t *__restrict__ cbt, uint32_t *__restrict__ pblk,
-    int npb, int ncb, uint32_t *__restrict__ flags, ZeroLists clear) {
-  __shared__ uint32_t w[kHintBlock / 64];
+    uint64_t *__restrict__ stay_bits, int npb, int ncb, uint32_t *__restrict__ flags, ZeroLists clear) {
   // per-class sums for the kHintSlots blocks of cells from the workgroup's
   // first key on (one global atomic per slot and class at the end: the
   // workgroups of a stretch of particles share these counters)
   __shared__ uint32_t slot_sum[kHintSlots][2];
+  __shared__ uint32_t stayers, first_block;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   for (int q = 0; q < clear.count; ++q)
     for (int64_t k = t; k < clear.n[q]; k += stride) clear.p[q][k] = 0u;
   if ((int)blockIdx.x >= npb) return;  // block-uniform
-  if (threadIdx.x < 2 * kHintSlots) (&slot_sum[0][0])[threadIdx.x] = 0u;
   const int lane = threadIdx.x & 63;
   const int i = (int)t;
   const bool valid = i < n;  // a prefix of each wave
@@ -487,35 +341,28 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
   bool stay = false;
   if (valid) {
     int b[3] = {0, 0, 0};
-#pragma unroll
-    for (int a = 0; a < D; ++a) b[a] = (int)__fmul_rn(__fsub_rn(x[a * n + i], g.origin[a]), g.inv_cell_size);
-    int64_t h = b[0];
-    if (D > 1) h += (int64_t)b[1] * g.num_cells[0];
-    if (D > 2) h += (int64_t)b[2] * g.num_cells[0] * g.num_cells[1];
-    key = (h < 0 || h >= g.num_cells_total) ? (uint32_t)g.num_cells_total : (uint32_t)h;
+    key = cell_key<D>(x, n, i, g, b);
     hash[i] = key;
     if (bins) {
 #pragma unroll
-      for (int a = 0; a < D; ++a) bins[a * n + i] = b[a];
+      for (int a = 0; a < D; ++a) bins[(int64_t)a * n + i] = b[a];
     }
     const uint32_t p = hint[i];
     if (i + 1 < n && p > hint[i + 1]) atomicOr(&flags[0], 1u);
     stay = key == p;
   }
-  // the cell block of the workgroup's first particle (i0 < n here)
-  const int i0 = (int)blockIdx.x * kHintBlock;
-  uint32_t k0;
-  {
-    int b0[3] = {0, 0, 0};
-#pragma unroll
-    for (int a = 0; a < D; ++a) b0[a] = (int)__fmul_rn(__fsub_rn(x[a * n + i0], g.origin[a]), g.inv_cell_size);
-    int64_t h0 = b0[0];
-    if (D > 1) h0 += (int64_t)b0[1] * g.num_cells[0];
-    if (D > 2) h0 += (int64_t)b0[2] * g.num_cells[0] * g.num_cells[1];
-    k0 = (h0 < 0 || h0 >= g.num_cells_total) ? (uint32_t)g.num_cells_total : (uint32_t)h0;
+  if (threadIdx.x < 2 * kHintSlots) (&slot_sum[0][0])[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) {
+    stayers = 0u;
+    first_block = key >> kHintCellBits;
   }
-  const uint32_t cb0 = k0 >> kHintCellBits;
-  __syncthreads();  // slot_sum cleared
+  __syncthreads();
+  const uint64_t bits = __ballot(stay);
+  if (lane == 0 && valid) {
+    stay_bits[i >> 6] = bits;
+    atomicAdd(&stayers, (uint32_t)__popcll(bits));
+  }
+  const uint32_t cb0 = first_block;
   const uint32_t pk = (uint32_t)__shfl_up((int)key, 1, 64);
   const int ps = __shfl_up((int)stay, 1, 64);
   const bool head = valid && (lane == 0 || pk != key || ps != (int)stay);
@@ -531,7 +378,7 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
     if (cb >= cb0 && cb - cb0 < (uint32_t)kHintSlots) atomicAdd(&slot_sum[cb - cb0][cls], len);
     else atomicAdd(&cbt[2 * (int64_t)cb + cls], len);
   }
-  const uint32_t stayers = block_sum(stay ? 1u : 0u, w);  // (its barriers order the slot sums)
+  __syncthreads();
   if (threadIdx.x == 0) pblk[blockIdx.x] = stayers;
   if (threadIdx.x < 2 * kHintSlots) {
     const uint32_t v = (&slot_sum[0][0])[threadIdx.x];
@@ -541,144 +388,252 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
   }
 }
 
-// Two kinds of workgroups, both after the classify pass:
-// - blocks [0, ncb): 1024 cells each (cells 0..ncells, the last holding the
-//   out-of-grid particles): the exclusive scans of the stayer and mover
-//   counts give each cell's record {first slot, stayers before, stayers,
-//   movers}, its range (cell_start/cell_end, 0 for an empty cell), and for
-//   the last cell the out-of-grid count (counters[0]) and the mover count
-//   (counters[2]); the per-cell counts are cleared for the next call.
-// - blocks [ncb, ncb + npb): 1024 particles each: S[i] (the stayers before
-//   slot i) with the stayer bit, and each mover's key and S[i] at its place
-//   i - S[i] in the slot-ordered mover list.
-// With an unsorted hint (flags[0]) every particle counts as a mover.
-__global__ __launch_bounds__(kHintBlock) void hint_scan_kernel(
-    int n, uint32_t ncells, int ncb, const uint32_t *__restrict__ hash, const uint32_t *__restrict__ hint,
-    uint32_t *__restrict__ cnt, const uint32_t *__restrict__ cbt, const uint32_t *__restrict__ pblk,
-    uint32_t *__restrict__ counters, int4 *__restrict__ info, int32_t *__restrict__ cstart,
-    int32_t *__restrict__ cend, int32_t *__restrict__ ss, uint32_t *__restrict__ mk, int32_t *__restrict__ sm) {
-  __shared__ uint64_t w2[kHintBlock / 64];
+// Block 0: the stayers before each particle block, and whether the hint was
+// unsorted (counters[2]; then every particle counts as a mover). Blocks 1 ..
+// ncb: 1024 cells each (cells 0..ncells, the last holding the out-of-grid
+// particles), four consecutive cells per thread: the exclusive scans of the
+// stayer and mover counts give each cell's record {first slot, stayers before,
+// stayers, movers}, its range (cell_start/cell_end, 0 for an empty cell), for
+// the last cell the out-of-grid count (counters[0]); the stayer counts are
+// cleared for the next call, the mover counts are left to the movers pass, and
+// cells with many movers are listed (counters[3] of them).
+constexpr int kScanThreads = kHintCells / 4;
+__global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(uint32_t ncells, int npb,
+                                                                 uint32_t *__restrict__ cnt,
+                                                                 const uint32_t *__restrict__ cbt,
+                                                                 uint32_t *__restrict__ pblk,
+                                                                 uint32_t *__restrict__ counters,
+                                                                 int4 *__restrict__ info, int32_t *__restrict__ cstart,
+                                                                 int32_t *__restrict__ cend, int32_t *__restrict__ heavy,
+                                                                 uint32_t heavy_cap) {
+  __shared__ uint64_t w2[kScanThreads / 64];
   const bool unsorted = counters[1] != 0u;
   const int t = threadIdx.x;
-  if ((int)blockIdx.x < ncb) {
-    const int b = blockIdx.x;
-    const int64_t c = (int64_t)b * kHintBlock + t;
-    const bool valid = c <= (int64_t)ncells;
-    uint32_t st = 0u, mv = 0u;
-    if (valid) {  // (loaded before the prefix sums' barriers)
-      st = cnt[2 * c];
-      mv = cnt[2 * c + 1];
+  if (blockIdx.x == 0) {
+    uint32_t base = 0u;
+    for (int b0 = 0; b0 < npb; b0 += 4 * kScanThreads) {
+      uint32_t v[4], sum = 0u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int b = b0 + 4 * t + q;
+        v[q] = b < npb ? pblk[b] : 0u;
+        sum += v[q];
+      }
+      uint64_t tot;
+      uint32_t at = base + (uint32_t)block_exclusive_scan<kScanThreads, uint64_t>(sum, w2, tot);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int b = b0 + 4 * t + q;
+        if (b < npb) pblk[b] = at;
+        at += v[q];
+      }
+      base += (uint32_t)tot;
     }
-    uint64_t pp = 0u;  // (stayers << 32) | movers of the cell blocks before this one
-    for (int j = t; j < b; j += kHintBlock) pp += ((uint64_t)cbt[2 * j] << 32) | cbt[2 * j + 1];
-    uint64_t pt;
-    (void)block_exclusive_scan2(pp, w2, pt);
-    uint32_t before_s = (uint32_t)(pt >> 32);
-    uint32_t before_m = (uint32_t)pt;
-    if (unsorted) {
-      before_m += before_s;
-      before_s = 0u;
-    }
-    if (valid) {
-      cnt[2 * c] = 0u;
-      cnt[2 * c + 1] = 0u;
-    }
-    if (unsorted) {
-      mv += st;
-      st = 0u;
-    }
-    uint64_t tot;
-    const uint64_t smx = block_exclusive_scan2(((uint64_t)st << 32) | mv, w2, tot);
-    const uint32_t sx = (uint32_t)(smx >> 32), mx = (uint32_t)smx;
-    if (!valid) return;
-    const uint32_t stay_before = before_s + sx, mover_before = before_m + mx;
-    const uint32_t start = stay_before + mover_before, count = st + mv;
-    info[c] = make_int4((int)start, (int)stay_before, (int)st, (int)mv);
-    if (c < (int64_t)ncells) {
-      cstart[c] = count ? (int32_t)start : 0;
-      cend[c] = count ? (int32_t)(start + count) : 0;
-    } else {
-      counters[0] = count;
-      counters[2] = mover_before + mv;
-    }
+    if (t == 0) counters[2] = unsorted ? 1u : 0u;
     return;
   }
-  const int b = (int)blockIdx.x - ncb;
-  const int i = b * kHintBlock + t;
-  const bool valid = i < n;
-  const uint32_t k = valid ? hash[i] : 0u;  // (loaded before the prefix sum's barriers)
-  const bool stay = valid && !unsorted && k == hint[i];
-  // (stayers of the blocks before << 32) | this thread's stayer flag, in one scan
-  uint64_t pv = stay ? 1u : 0u;
-  if (!unsorted)
-    for (int j = t; j < b; j += kHintBlock) pv += (uint64_t)pblk[j] << 32;
+  const int b = (int)blockIdx.x - 1;
+  const int64_t c0 = (int64_t)b * kHintCells + 4 * t;
+  uint32_t st[4], mv[4];  // (loaded before the prefix sums' barriers)
+  const bool all4 = c0 + 3 <= (int64_t)ncells;
+  if (all4) {
+    const uint4 u = *reinterpret_cast<const uint4 *>(cnt + 2 * c0), v = *reinterpret_cast<const uint4 *>(cnt + 2 * c0 + 4);
+    st[0] = u.x; mv[0] = u.y; st[1] = u.z; mv[1] = u.w;
+    st[2] = v.x; mv[2] = v.y; st[3] = v.z; mv[3] = v.w;
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool valid = c0 + q <= (int64_t)ncells;
+      st[q] = valid ? cnt[2 * (c0 + q)] : 0u;
+      mv[q] = valid ? cnt[2 * (c0 + q) + 1] : 0u;
+    }
+  }
+  uint64_t pp = 0u;  // (stayers << 32) | movers of the cell blocks before this one
+  for (int j = t; j < b; j += kScanThreads) {
+    const uint2 v = *reinterpret_cast<const uint2 *>(cbt + 2 * j);
+    pp += ((uint64_t)v.x << 32) | v.y;
+  }
+  uint64_t pt;
+  (void)block_exclusive_scan<kScanThreads, uint64_t>(pp, w2, pt);
+  uint32_t stay_before = (uint32_t)(pt >> 32);
+  uint32_t mover_before = (uint32_t)pt;
+  bool any = false;
+  uint64_t own = 0u;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    any = any || (st[q] | mv[q]) != 0u;
+    if (unsorted) {
+      mv[q] += st[q];
+      st[q] = 0u;
+    }
+    own += ((uint64_t)st[q] << 32) | mv[q];
+  }
+  if (unsorted) {
+    mover_before += stay_before;
+    stay_before = 0u;
+  }
   uint64_t tot;
-  const uint64_t ex = block_exclusive_scan2(pv, w2, tot);
-  const uint32_t S = (uint32_t)(tot >> 32) + (uint32_t)ex;
-  if (!valid) return;
-  ss[i] = (int32_t)(S | (stay ? 0x80000000u : 0u));
-  if (!stay) {
-    const uint32_t q = (uint32_t)i - S;
-    mk[q] = k;
-    sm[q] = (int32_t)S;
+  const uint64_t ex = block_exclusive_scan<kScanThreads, uint64_t>(own, w2, tot);
+  stay_before += (uint32_t)(ex >> 32);
+  mover_before += (uint32_t)ex;
+  int s4[4], e4[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t c = c0 + q;
+    const uint32_t start = stay_before + mover_before, count = st[q] + mv[q];
+    s4[q] = count ? (int)start : 0;
+    e4[q] = count ? (int)(start + count) : 0;
+    if (c <= (int64_t)ncells) {
+      if (any) *reinterpret_cast<uint2 *>(cnt + 2 * c) = make_uint2(0u, mv[q]);
+      info[c] = make_int4((int)start, (int)stay_before, (int)st[q], (int)mv[q]);
+      if (mv[q] > (uint32_t)kHeavyMovers) {
+        const uint32_t at = atomicAdd(&counters[3], 1u);
+        if (at < heavy_cap) heavy[at] = (int32_t)c;
+      }
+      if (c == (int64_t)ncells) counters[0] = count;
+    }
+    stay_before += st[q];
+    mover_before += mv[q];
+  }
+  const bool whole = c0 + 3 < (int64_t)ncells;
+  if (whole && ((reinterpret_cast<uintptr_t>(cstart) | reinterpret_cast<uintptr_t>(cend)) & 15u) == 0u) {
+    *reinterpret_cast<int4 *>(cstart + c0) = make_int4(s4[0], s4[1], s4[2], s4[3]);
+    *reinterpret_cast<int4 *>(cend + c0) = make_int4(e4[0], e4[1], e4[2], e4[3]);
+  } else {  // (the last cells, or caller's arrays that are not 16-byte aligned)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (c0 + q < (int64_t)ncells) {
+        cstart[c0 + q] = s4[q];
+        cend[c0 + q] = e4[q];
+      }
   }
 }
 
-// The merge: blocks [0, npb) place the stayers (slot order), the blocks
-// after them the sorted movers (mover r: key mkey[r], place mval[r] in the
-// slot-ordered list; a loop over the movers); writes sorted and hash_sorted.
-// Block 0 also clears the per-block cell counts and the unsorted flag for
-// the next call.
-__global__ __launch_bounds__(kHintBlock) void hint_place_kernel(
-    int n, uint32_t ncells, int npb, int ncb, const uint32_t *__restrict__ hash, const int32_t *__restrict__ ss,
-    const int4 *__restrict__ info, const uint32_t *__restrict__ mkey, const int32_t *__restrict__ mval,
-    const int32_t *__restrict__ sm, uint32_t *__restrict__ counters, uint32_t *__restrict__ cbt,
-    uint32_t *__restrict__ hash_sorted, int32_t *__restrict__ sorted) {
-  const int t = threadIdx.x;
+// Is particle i a mover? (stay bits of the classify pass)
+__device__ inline bool is_mover(const uint64_t *__restrict__ stay_bits, int i, bool unsorted) {
+  return unsorted || !((stay_bits[i >> 6] >> (i & 63)) & 1ull);
+}
+
+// Each mover's slot into its cell's part of `list` ([movers with a smaller
+// key] on): taken from the cell's count downward, in any order; heavy cells by
+// a workgroup each, in slot order. The counts end at zero, as the next call
+// needs them, and block 0 clears the per-block cell counts and the unsorted
+// flag.
+__global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_t ncells, int ncb, int words,
+                                                                  const uint32_t *__restrict__ hash,
+                                                                  const uint64_t *__restrict__ stay_bits,
+                                                                  const int4 *__restrict__ info,
+                                                                  uint32_t *__restrict__ cnt,
+                                                                  uint32_t *__restrict__ cbt,
+                                                                  uint32_t *__restrict__ counters,
+                                                                  const int32_t *__restrict__ heavy,
+                                                                  uint32_t heavy_cap, int32_t *__restrict__ list) {
+  __shared__ uint32_t w[kMoverBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const bool unsorted = counters[2] != 0u;
   if (blockIdx.x == 0) {
-    for (int j = t; j < 2 * ncb; j += kHintBlock) cbt[j] = 0u;
+    for (int j = t; j < 2 * ncb; j += kMoverBlock) cbt[j] = 0u;
     if (t == 0) counters[1] = 0u;
   }
-  const int m = (int)min(counters[2], (uint32_t)n);
-  if ((int)blockIdx.x < npb) {
-    const int i = (int)blockIdx.x * kHintBlock + t;
-    if (i >= n) return;
-    const int32_t v = ss[i];
-    if (v >= 0) return;  // a mover
-    const int S = v & 0x7fffffff;
-    const uint32_t k = hash[i];
-    if (k > ncells) return;
-    const int4 c = info[k];
-    const int mb = c.x - c.y;  // movers with a smaller key
-    // movers of this cell before slot i: their places in the slot-ordered
-    // list are below i - S (ascending within the cell)
-    const int lim = i - S;
-    int lo = 0, hi = c.w;
-    if (mb < 0 || mb + hi > m) return;  // (inconsistent counts: leave the slot)
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (mval[mb + mid] < lim) lo = mid + 1;
+  const uint32_t nheavy = min(counters[3], heavy_cap);
+  for (uint32_t h = blockIdx.x; h < nheavy; h += gridDim.x) {  // block-uniform
+    const uint32_t c = (uint32_t)heavy[h];
+    if (c > ncells) continue;
+    const int4 in = info[c];
+    const int base = in.x - in.y;
+    uint32_t done = 0u;
+    for (int i0 = 0; i0 < n; i0 += 4 * kMoverBlock) {
+      bool mine[4];
+      uint32_t m = 0u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = i0 + 4 * t + q;
+        mine[q] = i < n && hash[i] == c && is_mover(stay_bits, i, unsorted);
+        m += mine[q] ? 1u : 0u;
+      }
+      uint32_t all;
+      uint32_t at = done + block_exclusive_scan<kMoverBlock, uint32_t>(m, w, all);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (mine[q]) {
+          if (at < (uint32_t)in.w) list[base + (int)at] = i0 + 4 * t + q;
+          ++at;
+        }
+      done += all;
+    }
+    if (t == 0) cnt[2 * (int64_t)c + 1] = 0u;
+  }
+  // a wave takes `words` words of stay bits (at most 16)
+  const int first = ((int)blockIdx.x * (kMoverBlock / 64) + wv) * 64 * words;
+  if (first >= n) return;
+  const int word = (first >> 6) + lane;
+  const uint64_t bits = lane < words && word < (n + 63) / 64 ? stay_bits[word] : 0ull;
+  for (int q = 0; q < words; ++q) {
+    const int i = first + 64 * q + lane;
+    const uint64_t stay = (uint64_t)__shfl((unsigned long long)bits, q);
+    const bool mover = i < n && (unsorted || !((stay >> lane) & 1ull));
+    if (!__ballot(mover)) continue;
+    if (!mover) continue;
+    const uint32_t c = hash[i];
+    const int4 in = info[c];
+    if (in.w > kHeavyMovers) continue;
+    const int at = (int)atomicSub(&cnt[2 * (int64_t)c + 1], 1u) - 1;
+    if (at >= 0 && at < in.w) list[in.x - in.y + at] = i;
+  }
+}
+
+// The merge: each particle's place, written to sorted and hash_sorted. Block 0
+// also clears the count of heavy cells for the next call.
+__global__ __launch_bounds__(kHintBlock) void hint_place_kernel(int n, uint32_t ncells,
+                                                                const uint32_t *__restrict__ hash,
+                                                                const uint64_t *__restrict__ stay_bits,
+                                                                const uint32_t *__restrict__ pofs,
+                                                                const int4 *__restrict__ info,
+                                                                const int32_t *__restrict__ list,
+                                                                uint32_t *__restrict__ counters,
+                                                                uint32_t *__restrict__ hash_sorted,
+                                                                int32_t *__restrict__ sorted) {
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int i = (int)blockIdx.x * kHintBlock + t;
+  if (blockIdx.x == 0 && t == 0) counters[3] = 0u;
+  if (i >= n) return;
+  const uint32_t k = hash[i];
+  const bool unsorted = counters[2] != 0u;
+  const int4 c = info[k];
+  // stayers before this slot: those before the block, the block's waves
+  // before this one, the lanes before this one
+  const int w0 = (int)blockIdx.x * (kHintBlock / 64);
+  uint32_t S = 0u;
+  uint64_t bits = 0ull;
+  if (!unsorted) {
+    S = pofs[blockIdx.x];
+#pragma unroll
+    for (int q = 0; q < kHintBlock / 64; ++q) {
+      if (q > wv) break;
+      const uint64_t v = stay_bits[w0 + q];
+      if (q < wv) S += (uint32_t)__popcll(v);
+      else bits = v;
+    }
+    S += (uint32_t)__popcll(bits & ((1ull << lane) - 1ull));
+  }
+  // movers of this cell before this slot
+  const int32_t *part = list + (c.x - c.y);
+  int before = 0;
+  if (c.w <= kHeavyMovers) {
+    for (int r = 0; r < c.w; ++r) before += part[r] < i ? 1 : 0;
+  } else {
+    int hi = c.w;
+    while (before < hi) {
+      const int mid = (before + hi) >> 1;
+      if (part[mid] < i) before = mid + 1;
       else hi = mid;
     }
-    const int pos = c.x + (S - c.y) + lo;
-    if ((unsigned)pos >= (unsigned)n) return;
-    sorted[pos] = i;
-    hash_sorted[pos] = k;
-    return;
   }
-  const int nmw = ((int)gridDim.x - npb) * kHintBlock;  // mover threads
-  for (int r = ((int)blockIdx.x - npb) * kHintBlock + t; r < m; r += nmw) {
-    const int q = mval[r];
-    const uint32_t k = mkey[r];
-    if ((unsigned)q >= (unsigned)m || k > ncells) continue;
-    const int4 c = info[k];
-    const int S = sm[q];
-    const int st = min(max(S - c.y, 0), c.z);
-    const int pos = c.x + (r - (c.x - c.y)) + st;
-    if ((unsigned)pos >= (unsigned)n) continue;
-    sorted[pos] = S + q;
-    hash_sorted[pos] = k;
-  }
+  const int own = (int)S - c.y;
+  const int pos = c.x + before + ((bits >> lane) & 1ull ? own : min(max(own, 0), c.z));
+  if ((unsigned)pos >= (unsigned)n) return;  // (inconsistent counts)
+  sorted[pos] = i;
+  hash_sorted[pos] = k;
 }
 
 }  // namespace pmpm
@@ -753,7 +708,7 @@ extern "C" int pmpm_context_destroy(pmpm_context *ctx) {
   return PMPM_OK;
 }
 
-static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells, hipStream_t s);
+static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells);
 
 extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, int32_t max_cells) {
   if (!ctx || max_particles < 0 || max_cells < 0) return PMPM_ERR_INVALID;
@@ -773,11 +728,9 @@ extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, in
   if (max_cells > ctx->cap_cells) ctx->cap_cells = max_cells;
   if (ctx->sort_by_hint && max_particles >= ctx->hint_min_particles && max_particles > 0 && max_cells > 0) {
     // the hint partition's workspace too, so that stepping within these
-    // sizes allocates nothing (the counts are cleared on the null stream,
-    // which is waited for)
-    int rc = reserve_hint(ctx, max_particles, (uint32_t)max_cells, nullptr);
+    // sizes allocates nothing
+    int rc = reserve_hint(ctx, max_particles, (uint32_t)max_cells);
     if (rc != PMPM_OK) return rc;
-    PMPM_HIP_CHECK(hipStreamSynchronize(nullptr));
   }
   return PMPM_OK;
 }
@@ -803,11 +756,10 @@ extern "C" int pmpm_context_out_of_grid(pmpm_context *ctx, pmpm_stream_t stream,
 }
 
 // LSD radix sort of (key, position) pairs by keys in [0, ncells]: n keys
-// from kin (n_dev: the count is min(n, *n_dev), read on the device), values
-// = positions in kin; the passes alternate between (ktmp, vtmp) and (kdst,
+// from kin, values = positions in kin; the passes alternate between (ktmp, vtmp) and (kdst,
 // vdst), the last one writing (kdst, vdst). kin may alias neither.
 static int radix_sort_pairs(pmpm_context *ctx, const uint32_t *kin, uint32_t *ktmp, int32_t *vtmp, uint32_t *kdst,
-                            int32_t *vdst, int n, const uint32_t *n_dev, uint32_t ncells, hipStream_t s) {
+                            int32_t *vdst, int n, uint32_t ncells, hipStream_t s) {
   int bits = 1;
   while (bits < 32 && ((uint64_t)1 << bits) <= (uint64_t)ncells) ++bits;
   // 10-bit digits: 2 passes up to 2^20 cells (8-bit digits when one pass
@@ -824,20 +776,20 @@ static int radix_sort_pairs(pmpm_context *ctx, const uint32_t *kin, uint32_t *kt
     const int radix = 1 << rb;
     uint32_t *totals = ctx->hist + (size_t)radix * nblocks;
     if (rb == 8) {
-      PMPM_LAUNCH(radix_hist_kernel<8>, (::pmpm::kname("radix_hist_kernel", {(long)(8)})), dim3(nblocks), dim3(kSortBlock), 0, s, kin, n, shift, ctx->hist, nblocks, n_dev);
+      PMPM_LAUNCH(radix_hist_kernel<8>, (::pmpm::kname("radix_hist_kernel", {(long)(8)})), dim3(nblocks), dim3(kSortBlock), 0, s, kin, n, shift, ctx->hist, nblocks);
       PMPM_LAUNCH_CHECK();
-      PMPM_LAUNCH(scan_columns_kernel, (::pmpm::kname("scan_columns_kernel", {})), dim3(radix), dim3(256), 0, s, ctx->hist, nblocks, totals, n_dev);
+      PMPM_LAUNCH(scan_columns_kernel, (::pmpm::kname("scan_columns_kernel", {})), dim3(radix), dim3(256), 0, s, ctx->hist, nblocks, totals);
       PMPM_LAUNCH_CHECK();
       PMPM_LAUNCH(radix_scatter_kernel<8>, (::pmpm::kname("radix_scatter_kernel", {(long)(8)})), dim3(nblocks), dim3(kSortBlock), 0, s, kin, vin, kout, vout, n,
-                  shift, ctx->hist, nblocks, totals, n_dev);
+                  shift, ctx->hist, nblocks, totals);
     } else {
       PMPM_LAUNCH(radix_hist_kernel<10>, (::pmpm::kname("radix_hist_kernel", {(long)(10)})), dim3(nblocks), dim3(kSortBlock), 0, s, kin, n, shift, ctx->hist,
-                  nblocks, n_dev);
+                  nblocks);
       PMPM_LAUNCH_CHECK();
-      PMPM_LAUNCH(scan_columns_kernel, (::pmpm::kname("scan_columns_kernel", {})), dim3(radix), dim3(256), 0, s, ctx->hist, nblocks, totals, n_dev);
+      PMPM_LAUNCH(scan_columns_kernel, (::pmpm::kname("scan_columns_kernel", {})), dim3(radix), dim3(256), 0, s, ctx->hist, nblocks, totals);
       PMPM_LAUNCH_CHECK();
       PMPM_LAUNCH(radix_scatter_kernel<10>, (::pmpm::kname("radix_scatter_kernel", {(long)(10)})), dim3(nblocks), dim3(kSortBlock), 0, s, kin, vin, kout, vout, n,
-                  shift, ctx->hist, nblocks, totals, n_dev);
+                  shift, ctx->hist, nblocks, totals);
     }
     PMPM_LAUNCH_CHECK();
     kin = kout;
@@ -846,56 +798,58 @@ static int radix_sort_pairs(pmpm_context *ctx, const uint32_t *kin, uint32_t *kt
   return PMPM_OK;
 }
 
-// Grows a context buffer of 32-bit words; a new buffer is zero-filled on s
-// when `zero` (the counts that must be zero between calls).
-static int ensure_words(float *&buf, size_t &cap, size_t words, bool zero, hipStream_t s) {
-  if (words <= cap) return PMPM_OK;
-  int rc = ensure_buffer(buf, cap, words);
-  if (rc != PMPM_OK) return rc;
-  return zero ? zero_fill(buf, (int64_t)cap, s) : PMPM_OK;
+// The per-particle part of the hint workspace, in 32-bit words: the stay bits,
+// the stayers per particle block, the heavy cells, the movers by cell; each
+// starts on a 256-byte boundary.
+struct HintLayout {
+  size_t bits, pblk, heavy, list, words;
+  uint32_t heavy_cap;
+};
+static HintLayout hint_layout(int n) {
+  auto up = [](size_t w) { return (w + 63) / 64 * 64; };
+  HintLayout l;
+  l.heavy_cap = (uint32_t)(n / kHeavyMovers + 1);
+  l.bits = 0;
+  l.pblk = l.bits + up(2 * (size_t)ceil_div(n, 64));
+  l.heavy = l.pblk + up((size_t)ceil_div(n, kHintBlock));
+  l.list = l.heavy + up(l.heavy_cap);
+  l.words = l.list + up((size_t)n);
+  return l;
 }
 
-// Words of the per-particle hint workspace: the per-block stayer counts, then
-// five arrays of n words, each starting on a 256-byte boundary.
-static size_t hint_part_words(int n) {
-  const size_t npb = (size_t)ceil_div(n, kHintBlock);
-  return (npb + 63) / 64 * 64 + 4 * (((size_t)n + 63) / 64 * 64) + (size_t)n;
-}
-
-// Grows the hint workspace to n particles on ncells cells (the counts are
-// zero-filled on s when new).
-static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells, hipStream_t s) {
-  const int ncb = (int)ceil_div((int64_t)ncells + 1, kHintBlock);
-  const int npb = (int)ceil_div(n, kHintBlock);
+// Grows the hint workspace to n particles on ncells cells. The counts must be
+// zero between calls: new ones are marked and cleared by the partition that
+// uses them first, on its stream.
+static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells) {
+  const size_t cnt = 2 * ((size_t)ncells + 1), cbt = 2 * (size_t)ceil_div((int64_t)ncells + 1, kHintCells);
   int rc;
-  if ((rc = ensure_words(ctx->hint_cnt, ctx->hint_cnt_cap, 2 * ((size_t)ncells + 1), true, s)) != PMPM_OK) return rc;
-  if ((rc = ensure_words(ctx->hint_cbt, ctx->hint_cbt_cap, 2 * (size_t)ncb, true, s)) != PMPM_OK) return rc;
-  if ((rc = ensure_words(ctx->hint_info, ctx->hint_info_cap, 4 * ((size_t)ncells + 1), false, s)) != PMPM_OK)
-    return rc;
-  return ensure_words(ctx->hint_part, ctx->hint_part_cap, hint_part_words(n), false, s);
+  if (cnt > ctx->hint_cnt_cap || cbt > ctx->hint_cbt_cap) ctx->hint_clear = false;
+  if ((rc = ensure_buffer(ctx->hint_cnt, ctx->hint_cnt_cap, cnt)) != PMPM_OK) return rc;
+  if ((rc = ensure_buffer(ctx->hint_cbt, ctx->hint_cbt_cap, cbt)) != PMPM_OK) return rc;
+  if ((rc = ensure_buffer(ctx->hint_info, ctx->hint_info_cap, 4 * ((size_t)ncells + 1))) != PMPM_OK) return rc;
+  return ensure_buffer(ctx->hint_part, ctx->hint_part_cap, hint_layout(n).words);
 }
 
 // The partition from the hint in part->hash_sorted (see hint_classify_kernel).
 static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, const float *x, int n,
                              pmpm_spatial *part, hipStream_t s, const ZeroLists &extra) {
   const uint32_t ncells = (uint32_t)g.num_cells_total;
-  const int ncb = (int)ceil_div((int64_t)ncells + 1, kHintBlock);
+  const int ncb = (int)ceil_div((int64_t)ncells + 1, kHintCells);
   const int npb = (int)ceil_div(n, kHintBlock);
   int rc;
-  if ((rc = reserve_hint(ctx, n, ncells, s)) != PMPM_OK) return rc;
-  uint32_t *pblk = reinterpret_cast<uint32_t *>(ctx->hint_part);
-  const size_t o = ((size_t)npb + 63) / 64 * 64;  // 256-byte aligned arrays of n words
-  const size_t na = ((size_t)n + 63) / 64 * 64;
-  int32_t *ss = reinterpret_cast<int32_t *>(ctx->hint_part) + o;
-  uint32_t *mk = reinterpret_cast<uint32_t *>(ss + na);
-  int32_t *sm = reinterpret_cast<int32_t *>(mk + na);
-  uint32_t *k2 = reinterpret_cast<uint32_t *>(sm + na);
-  int32_t *v2 = reinterpret_cast<int32_t *>(k2 + na);
-  if ((size_t)((v2 + n) - reinterpret_cast<int32_t *>(ctx->hint_part)) != hint_part_words(n) ||
-      hint_part_words(n) > ctx->hint_part_cap) {
-    note_error("partition: hint workspace layout");
-    return PMPM_ERR_INVALID;
+  if ((rc = reserve_hint(ctx, n, ncells)) != PMPM_OK) return rc;
+  if (!ctx->hint_clear) {
+    ZeroLists z{};
+    z.add(ctx->hint_cnt, (int64_t)ctx->hint_cnt_cap);
+    z.add(ctx->hint_cbt, (int64_t)ctx->hint_cbt_cap);
+    if ((rc = zero_fill_lists(z, s)) != PMPM_OK) return rc;
+    ctx->hint_clear = true;
   }
+  const HintLayout l = hint_layout(n);
+  uint32_t *base = reinterpret_cast<uint32_t *>(ctx->hint_part);
+  uint64_t *bits = reinterpret_cast<uint64_t *>(base + l.bits);
+  uint32_t *pblk = base + l.pblk;
+  int32_t *heavy = reinterpret_cast<int32_t *>(base + l.heavy), *list = reinterpret_cast<int32_t *>(base + l.list);
   uint32_t *cnt = reinterpret_cast<uint32_t *>(ctx->hint_cnt);
   uint32_t *cbt = reinterpret_cast<uint32_t *>(ctx->hint_cbt);
   int4 *info = reinterpret_cast<int4 *>(ctx->hint_info);
@@ -904,29 +858,30 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   for (int q = 0; q < extra.count; ++q) words = extra.n[q] > words ? extra.n[q] : words;
   int64_t nb = npb;
   const int64_t nb_clear = ceil_div(words, (int64_t)kHintBlock * 4);
-  if (nb_clear > nb) nb = nb_clear < 4096 ? nb_clear : (nb > 4096 ? nb : 4096);
-  const unsigned blocks = (unsigned)nb;
+  if (nb_clear > nb) nb = nb_clear < 16384 ? nb_clear : (nb > 16384 ? nb : 16384);
+#define PMPM_CLASSIFY(D)                                                                                               \
+  PMPM_LAUNCH(hint_classify_kernel<D>, (::pmpm::kname("hint_classify_kernel", {(long)(D)})), dim3((unsigned)nb),       \
+              dim3(kHintBlock), 0, s, x, n, g, part->hash_sorted, part->hash, part->bins, cnt, cbt, pblk, bits, npb, ncb, \
+              ctx->counters + 1, extra)
   switch (dim) {
-    case 1: PMPM_LAUNCH(hint_classify_kernel<1>, (::pmpm::kname("hint_classify_kernel", {(long)(1)})), dim3(blocks), dim3(kHintBlock), 0, s, x, n, g, part->hash_sorted, part->hash, part->bins, cnt, cbt, pblk, npb, ncb, ctx->counters + 1, extra); break;
-    case 2: PMPM_LAUNCH(hint_classify_kernel<2>, (::pmpm::kname("hint_classify_kernel", {(long)(2)})), dim3(blocks), dim3(kHintBlock), 0, s, x, n, g, part->hash_sorted, part->hash, part->bins, cnt, cbt, pblk, npb, ncb, ctx->counters + 1, extra); break;
-    default: PMPM_LAUNCH(hint_classify_kernel<3>, (::pmpm::kname("hint_classify_kernel", {(long)(3)})), dim3(blocks), dim3(kHintBlock), 0, s, x, n, g, part->hash_sorted, part->hash, part->bins, cnt, cbt, pblk, npb, ncb, ctx->counters + 1, extra); break;
+    case 1: PMPM_CLASSIFY(1); break;
+    case 2: PMPM_CLASSIFY(2); break;
+    default: PMPM_CLASSIFY(3); break;
   }
+#undef PMPM_CLASSIFY
   PMPM_LAUNCH_CHECK();
-  PMPM_LAUNCH(hint_scan_kernel, (::pmpm::kname("hint_scan_kernel", {})), dim3((unsigned)(ncb + npb)), dim3(kHintBlock), 0, s, n, ncells, ncb, part->hash,
-              part->hash_sorted, cnt, cbt, pblk, ctx->counters, info, part->cell_start, part->cell_end, ss, mk, sm);
+  PMPM_LAUNCH(hint_scan_kernel, (::pmpm::kname("hint_scan_kernel", {})), dim3((unsigned)(ncb + 1)), dim3(kScanThreads), 0, s,
+              ncells, npb, cnt, cbt, pblk, ctx->counters, info, part->cell_start, part->cell_end, heavy, l.heavy_cap);
   PMPM_LAUNCH_CHECK();
-  // the movers sorted by (key, slot): one workgroup when at most kSmallSort
-  // of them, else the radix passes (each launch leaves the other case alone)
-  int bits = 1;
-  while (bits < 32 && ((uint64_t)1 << bits) <= (uint64_t)ncells) ++bits;
-  PMPM_LAUNCH(small_sort_kernel, (::pmpm::kname("small_sort_kernel", {})), dim3(1), dim3(kSortBlock), 0, s, mk, ctx->counters + 2, (bits + 9) / 10, k2, v2);
+  // a wave waits for each of its movers' chain of reads in turn: one word of
+  // stay bits per wave on small scenes (16 words at 40,000 particles: 14 us,
+  // one: 7), more where the waves alone would fill the chip many times over
+  const int mover_words = n < (1 << 18) ? 1 : (n < (1 << 22) ? n >> 18 : 16);
+  PMPM_LAUNCH(hint_movers_kernel, (::pmpm::kname("hint_movers_kernel", {})),
+              dim3((unsigned)ceil_div(n, (int64_t)mover_words * kMoverBlock)), dim3(kMoverBlock), 0, s, n, ncells, ncb, mover_words, part->hash, bits, info, cnt, cbt, ctx->counters, heavy, l.heavy_cap, list);
   PMPM_LAUNCH_CHECK();
-  if ((rc = radix_sort_pairs(ctx, mk, ctx->keys_tmp, ctx->vals_tmp, k2, v2, n, ctx->counters + 2, ncells, s)) !=
-      PMPM_OK)
-    return rc;
-  const int nmb = npb < 64 ? npb : 64;  // workgroups of the mover loop
-  PMPM_LAUNCH(hint_place_kernel, (::pmpm::kname("hint_place_kernel", {})), dim3((unsigned)(npb + nmb)), dim3(kHintBlock), 0, s, n, ncells, npb, ncb, part->hash,
-              ss, info, k2, v2, sm, ctx->counters, cbt, part->hash_sorted, part->sorted);
+  PMPM_LAUNCH(hint_place_kernel, (::pmpm::kname("hint_place_kernel", {})), dim3((unsigned)npb), dim3(kHintBlock), 0, s, n,
+              ncells, part->hash, bits, pblk, info, list, ctx->counters, part->hash_sorted, part->sorted);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -962,8 +917,8 @@ int pmpm::partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, 
     default: PMPM_LAUNCH(hash_kernel<3>, (::pmpm::kname("hash_kernel", {(long)(3)})), dim3(blocks), dim3(256), 0, s, x, n, g, part->hash, part->bins, part->cell_start, part->cell_end, extra); break;
   }
   PMPM_LAUNCH_CHECK();
-  if ((rc = radix_sort_pairs(ctx, part->hash, ctx->keys_tmp, ctx->vals_tmp, part->hash_sorted, part->sorted, n, nullptr,
-                             ncells, s)) != PMPM_OK)
+  if ((rc = radix_sort_pairs(ctx, part->hash, ctx->keys_tmp, ctx->vals_tmp, part->hash_sorted, part->sorted, n, ncells,
+                             s)) != PMPM_OK)
     return rc;
   PMPM_LAUNCH(cell_range_kernel, (::pmpm::kname("cell_range_kernel", {})), dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, part->hash_sorted, n, ncells,
                      part->cell_start, part->cell_end, ctx->counters);
