@@ -132,8 +132,10 @@ __device__ inline void cubic_span(float frac, int type, float inv_h, float &N, f
 // span form serves frac in [0, 1), every particle at t >= 0; a particle left
 // of the origin (t < 0, where trunc gives frac in (-1, 0)) takes the table
 // form, whose pieces then shift by one.
+// wrap: a node outside [0, n_axis) takes the type of the node one period away
+// (which the linear index reaches).
 __device__ inline void cubic_axis(float frac, int bin, int n_axis, int types_built, float inv_h, float *N, float *dN,
-                                  float *d2N = nullptr) {
+                                  float *d2N = nullptr, bool wrap = false) {
   if (!types_built) {  // untyped nodes: kCubic row 0
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -145,7 +147,11 @@ __device__ inline void cubic_axis(float frac, int bin, int n_axis, int types_bui
   }
   int type[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) type[e] = cubic_node_type(bin - 1 + e, n_axis, 1);
+  for (int e = 0; e < 4; ++e) {
+    int id = bin - 1 + e;
+    if (wrap) id += id < 0 ? n_axis : (id >= n_axis ? -n_axis : 0);
+    type[e] = cubic_node_type(id, n_axis, 1);
+  }
   if (frac >= 0.f) {
     cubic_span<0>(frac, type[0], inv_h, N[0], dN[0], d2N ? d2N + 0 : nullptr);
     cubic_span<1>(frac, type[1], inv_h, N[1], dN[1], d2N ? d2N + 1 : nullptr);

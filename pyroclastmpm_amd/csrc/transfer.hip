@@ -3546,60 +3546,57 @@ template <int D> __device__ inline void cofactor(const float *F, float *C) {
   C[8] = F[0] * F[4] - F[1] * F[3];
 }
 
-// Per particle: gather of the node adjoints through the P2G window (the same
-// entries as the forward deposit, linear-index wrap-around included) into the
-// adjoints of v, sigma, F (through V = det(F) V0) and x, plus the position
-// adjoint through the G2P weights, which walk the same window:
-//   xbar_c += sum_i grad_c w (vnt . vpb + dv . dvb) + sum_ab d2w/dx_c dx_a Lb_ab vnt_b
-// with vpb, dvb, Lb the records g2p_adjoint_kernel wrote. The in-grid entries
-// run branch-free (clamped node, zero weights outside, as gather_grid); the
-// wrap-around entries of boundary particles, which only the deposit reaches,
-// take a separate compact loop. Adds to ib.
-// LDS staging of the node records the 3D cubic adjoint P2G reads (one lane
-// per particle, kG2PThreads per workgroup, consecutive in cell order): as in
-// g2p_gather_staged, the workgroup's particles form runs (same y and z bins,
-// x bins not decreasing and within one 32-aligned block), whose windows lie
-// in 4 x 4 node rows over the run's x range - 1 .. + 2, at most 16 x 35
-// nodes; the runs are staged in rounds of at most kAdjStageNodes nodes, the
-// node adjoint record (8 floats) and velocity record (8 floats) of each
-// clamped node. gather(adj, vel, box0, X) is called by every live thread in
-// the round that holds its run: the node of window entry (ex, sy, sz) is
-// box0 + ex + X (sy + 4 sz) of adj and vel. Every thread of the workgroup
-// calls this (barriers); `live` is false past the particles.
+// LDS staging of the node records the 3D adjoint P2G reads (LANES lanes per
+// particle, particles consecutive in cell order): as in g2p_gather_staged, the
+// workgroup's particles form runs (same y and z bins, x bins not decreasing
+// and within one 32-aligned block), whose windows lie in 4 x 4 node rows over
+// the run's x range - 1 .. + 2, at most 16 x 35 nodes; the runs are staged in
+// rounds of at most kAdjStageNodes nodes, the node adjoint record (8 floats)
+// and velocity record (8 floats) of each. A node outside the grid carries the
+// adjoint of the node its linear index reaches (the wrap-around deposit's; zero
+// if none, or without wrap_quirk) and zero velocities (G2P never reads it).
+// gather(adj, vel, box0, X) is called by every live thread in the round that
+// holds its run: the node of window offset (ex, sy, sz) from bin - 1 is box0 +
+// ex + X (sy + 4 sz) of adj and vel. Every thread of the workgroup calls this
+// (barriers); `live` is false past the particles.
 constexpr int kAdjStageNodes = 576;  // 16 x 36: one run always fits
 static_assert(kAdjStageNodes >= 16 * (32 + 3), "a run spans at most 32 x bins");
 struct AdjRunTable {
   int y[kG2PThreads], z[kG2PThreads], x0[kG2PThreads], x1[kG2PThreads], base[kG2PThreads];
   int wave_sum[kG2PThreads / 64];
 };
-template <class PWT, class F>
+template <int LANES, class F>
 __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes &nodes,
-                                            const float *__restrict__ nbar, const PWT &w, bool live, F &&gather) {
-  constexpr int CAP = kAdjStageNodes;
+                                            const float *__restrict__ nbar, const int *bin, bool live,
+                                            bool wrap_quirk, F &&gather) {
+  constexpr int CAP = kAdjStageNodes, PPB = kG2PThreads / LANES;
   __shared__ float4 s_adj[CAP * 2], s_vel[CAP * 2];
   __shared__ AdjRunTable R;
-  __shared__ int rb[3][kG2PThreads];
-  const int t = (int)threadIdx.x;
+  __shared__ int rb[3][PPB];
+  const int t = (int)threadIdx.x, pl = t / LANES;
+  const bool lead = t % LANES == 0;  // the particle's first lane
+  if (lead) {
 #pragma unroll
-  for (int a = 0; a < 3; ++a) rb[a][t] = w.bin[a];
-  const int nv = __syncthreads_count(live);  // live threads are a prefix
+    for (int a = 0; a < 3; ++a) rb[a][pl] = bin[a];
+  }
+  const int nv = __syncthreads_count(live && lead);  // live particles are a prefix
   auto starts_at = [&](int q) {
     return rb[1][q - 1] != rb[1][q] || rb[2][q - 1] != rb[2][q] || rb[0][q] < rb[0][q - 1] ||
            (rb[0][q] >> 5) != (rb[0][q - 1] >> 5);
   };
   bool start = false, end = false;
-  if (live) {
-    start = t == 0 || starts_at(t);
-    end = t == nv - 1 || starts_at(t + 1);
+  if (live && lead) {
+    start = pl == 0 || starts_at(pl);
+    end = pl == nv - 1 || starts_at(pl + 1);
   }
   int nruns = 0;
   const int k = block_inclusive_sum(start ? 1 : 0, R.wave_sum, &nruns) - 1;
   if (start) {
-    R.y[k] = w.bin[1];
-    R.z[k] = w.bin[2];
-    R.x0[k] = w.bin[0];
+    R.y[k] = bin[1];
+    R.z[k] = bin[2];
+    R.x0[k] = bin[0];
   }
-  if (end) R.x1[k] = w.bin[0];
+  if (end) R.x1[k] = bin[0];
   __syncthreads();
   const int cnt = t < nruns ? 16 * (R.x1[t] - R.x0[t] + 4) : 0;
   int all = 0;
@@ -3607,6 +3604,7 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
   if (t < nruns) R.base[t] = incl - cnt;
   __syncthreads();
   const int myk = live ? k : -1;
+  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = g.num_cells[2];
   for (int k0 = 0; k0 < nruns;) {  // uniform over the workgroup
     const int b0 = R.base[k0];
     int k1 = k0 + 1;
@@ -3617,28 +3615,329 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
       while (kk + 1 < k1 && R.base[kk + 1] - b0 <= q) ++kk;
       const int X = R.x1[kk] - R.x0[kk] + 4, qq = q - (R.base[kk] - b0);
       const int row = qq / X, x = qq - row * X;  // row = sz * 4 + sy
-      const int ix = min(max(R.x0[kk] - 1 + x, 0), g.num_cells[0] - 1);
-      const int iy = min(max(R.y[kk] - 1 + (row & 3), 0), g.num_cells[1] - 1);
-      const int iz = min(max(R.z[kk] - 1 + (row >> 2), 0), g.num_cells[2] - 1);
-      const uint32_t node = (uint32_t)ix + (uint32_t)g.num_cells[0] * ((uint32_t)iy + (uint32_t)g.num_cells[1] * (uint32_t)iz);
-      const float4 *ar = reinterpret_cast<const float4 *>(nbar + 8 * (size_t)node);
-      const float4 *vr = reinterpret_cast<const float4 *>(nodes.vel + 8 * (size_t)node);
-      s_adj[2 * q] = ar[0];
-      s_adj[2 * q + 1] = ar[1];
-      s_vel[2 * q] = vr[0];
-      s_vel[2 * q + 1] = vr[1];
+      const int ix = R.x0[kk] - 1 + x, iy = R.y[kk] - 1 + (row & 3), iz = R.z[kk] - 1 + (row >> 2);
+      const bool in = ix >= 0 && ix < nx && iy >= 0 && iy < ny && iz >= 0 && iz < nz;
+      const int64_t lin = (int64_t)ix + (int64_t)nx * ((int64_t)iy + (int64_t)ny * (int64_t)iz);
+      const bool reaches = in || (wrap_quirk && lin >= 0 && lin < g.num_cells_total);
+      const size_t node = reaches ? (size_t)lin : 0;
+      const float4 *ar = reinterpret_cast<const float4 *>(nbar + 8 * node);
+      const float4 *vr = reinterpret_cast<const float4 *>(nodes.vel + 8 * node);
+      const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 a0 = ar[0], a1 = ar[1], v0 = vr[0], v1 = vr[1];
+      s_adj[2 * q] = reaches ? a0 : z4;
+      s_adj[2 * q + 1] = reaches ? a1 : z4;
+      s_vel[2 * q] = in ? v0 : z4;
+      s_vel[2 * q + 1] = in ? v1 : z4;
     }
     __syncthreads();
     if (myk >= k0 && myk < k1) {
       const int off = R.base[myk] - b0, X = R.x1[myk] - R.x0[myk] + 4;
-      gather(reinterpret_cast<const float *>(s_adj), reinterpret_cast<const float *>(s_vel),
-             off + (w.bin[0] - R.x0[myk]), X);
+      gather(s_adj, s_vel, off + (bin[0] - R.x0[myk]), X);
     }
     k0 = k1;
     __syncthreads();  // the next round overwrites the staging
   }
 }
 
+// Adjoint P2G of 3D scenes: p2g_adjoint_kernel's sums (below) in separable
+// form, the node records staged in LDS. Per node, with the particle's factors,
+//   gs = m (m_bar + v . P_bar) + v_nt . vpb + dv . dvb,  wv = L_bar v_nt - V sigma f_bar
+// and the sums over the window contract x first (weights N, dN, d2N of gs, wv,
+// P_bar, f_bar as each needs them), then y, then z: about 3,400 multiply-adds
+// per particle instead of 4,500 with a product of three weights per entry.
+// LANES = 1: a lane per particle; 4: a lane per z layer of the window, for
+// launches too small to fill the chip otherwise.
+// Wrap-around entries (deposit only): a node outside the grid holds the adjoint
+// of the node it reaches (see the staging), so it takes part as an ordinary
+// entry wherever its weight is a product of per-axis weights: always without
+// node types; with them if only x leaves the grid and the carry into y changes
+// no y type, or only y leaves and the carry into z changes no z type. The
+// particles of the remaining cells (the grid's edges) walk their outside
+// entries one by one.
+template <int SF, int LANES>
+__global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles st,
+                                                           pmpm_adjoint ib, pmpm_spatial part, pmpm_nodes nodes,
+                                                           const float *__restrict__ nbar,
+                                                           const float *__restrict__ rec) {
+  constexpr int E = Spline<SF>::ENTRIES;
+  constexpr bool TYPED = SF == PMPM_SF_CUBIC;
+  static_assert(LANES == 1 || LANES == 4, "lanes per particle");
+  const int n = st.n;
+  const int j = (int)blockIdx.x * (256 / LANES) + (int)threadIdx.x / LANES, sub = (int)threadIdx.x % LANES;
+  const bool live = j < n;  // a thread past the particles works on the last one and writes nothing
+  const uint32_t jj = (uint32_t)(live ? j : n - 1);
+  const uint32_t src = (uint32_t)part.sorted[jj];
+  const float inv_h = g.inv_cell_size;
+  // typed cubic: the y and z weights are formed per row from a table of the
+  // span polynomials (by node type; offset 4 is past the window), which costs
+  // what picking them from registers by offset would and saves 24 registers
+  __shared__ __attribute__((aligned(16))) float s_poly[TYPED ? 4 * 5 * 4 : 1];
+  if constexpr (TYPED) {
+    if (threadIdx.x < 80) {
+      const int e = (int)threadIdx.x;
+      s_poly[e] = (e / 4) % 5 < 4 ? kSpanCubic[e / 20][(e / 4) % 5][e % 4] : 0.f;
+    }  // (the staging's barriers come before the first use)
+  }
+  float t3[3], N[3][4], dN[3][4], d2N[3][4];
+  int bin[3], first[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) t3[a] = cell_coord(ld32(st.x + (int64_t)a * n, src), g.origin[a], inv_h);
+  bool out_axis[3] = {false, false, false};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    bin[a] = (int)t3[a];
+    const float frac = __fsub_rn(t3[a], (float)bin[a]);
+    first[a] = 0;
+    if constexpr (TYPED) {
+      first[a] = -1;
+      if (a == 0) cubic_axis(frac, bin[a], g.num_cells[a], prm.node_types_built, inv_h, N[a], dN[a], d2N[a], true);
+    } else {
+      axis_weights<SF>(t3[a], bin[a], g.num_cells[a], 0, inv_h, first[a], N[a], dN[a]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) d2N[a][e] = spline_d2<SF>(__fsub_rn(frac, (float)(first[a] + e)), 0, inv_h);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = bin[a] + first[a] + e;
+      out_axis[a] = out_axis[a] || i < 0 || i >= g.num_cells[a];
+    }
+  }
+  // may the outside entries take part in the separable sums?
+  const bool quirk = prm.wrap_quirk != 0;
+  bool joint = quirk;
+  if (TYPED) {
+    const bool own = t3[0] >= 0.f && t3[1] >= 0.f && t3[2] >= 0.f && bin[0] < g.num_cells[0] &&
+                     bin[1] < g.num_cells[1] && bin[2] < g.num_cells[2] && g.num_cells[0] >= 4 && g.num_cells[1] >= 4;
+    // (nodes bin - 2 .. bin + 3 away from the typed ones)
+    const bool y_plain = bin[1] >= 4 && bin[1] <= g.num_cells[1] - 5, z_plain = bin[2] >= 4 && bin[2] <= g.num_cells[2] - 5;
+    joint = quirk && own && (out_axis[0] ? !out_axis[1] && y_plain : out_axis[1] && z_plain);
+  }
+  const bool walk = TYPED && quirk && !joint && (out_axis[0] || out_axis[1]);
+#pragma unroll
+  for (int a = 0; a < (TYPED ? 1 : 3); ++a)
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = bin[a] + first[a] + e;
+      const bool drop = (i < 0 || i >= g.num_cells[a]) && !(joint && (a < 2 || !TYPED));
+      N[a][e] = drop ? 0.f : N[a][e];
+      dN[a][e] = drop ? 0.f : dN[a][e];
+      d2N[a][e] = drop ? 0.f : d2N[a][e];
+    }
+  const float m = ld32(st.mass, src), V = ld32(st.volume, src);
+  float v[3], vpb[3], dvb[3], Lb[9];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    v[a] = ld32(st.v + (int64_t)a * n, src);
+    vpb[a] = ld32(rec + (int64_t)a * n, jj);
+    dvb[a] = ld32(rec + (int64_t)(3 + a) * n, jj);
+  }
+#pragma unroll
+  for (int a = 0; a < 9; ++a) Lb[a] = ld32(rec + (int64_t)(6 + a) * n, jj);
+  Sym s;
+  {
+    const float *sg = st.stress;
+    s = Sym{ld32(sg, src), ld32(sg + (int64_t)n, src), ld32(sg + 2 * (int64_t)n, src),
+            ld32(sg + 3 * (int64_t)n, src), ld32(sg + 4 * (int64_t)n, src), ld32(sg + 5 * (int64_t)n, src)};
+  }
+  const Sym Sv{V * s.xx, V * s.yy, V * s.zz, V * s.xy, V * s.xz, V * s.yz};
+  const float mv[3] = {m * v[0], m * v[1], m * v[2]};
+  float xb[3] = {0.f, 0.f, 0.f}, vb[3] = {0.f, 0.f, 0.f}, G[3][3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) G[a][b] = 0.f;
+  auto pick = [](const float *a, int k) { return k == 0 ? a[0] : (k == 1 ? a[1] : (k == 2 ? a[2] : a[3])); };
+  // weight, derivative and second derivative at window offset e of axis a
+  auto axis_at = [&](int a, int e, float &w0, float &w1, float &w2) {
+    if constexpr (TYPED) {
+      const int cells = g.num_cells[a];
+      const float fr = __fsub_rn(t3[a], (float)bin[a]);
+      const bool left = fr < 0.f;  // t < 0: the pieces shift by one
+      const float f = left ? fr + 1.f : fr;
+      const int i = bin[a] - 1 + e;
+      const bool out = i < 0 || i >= cells;
+      const int id = a == 2 ? i : i + (i < 0 ? cells : (i >= cells ? -cells : 0));
+      const int type = out && !(joint && a < 2) ? 0 : cubic_node_type(id, cells, prm.node_types_built);
+      const float4 c = *reinterpret_cast<const float4 *>(&s_poly[(type * 5 + e + (left ? 1 : 0)) * 4]);
+      w0 = ((c.w * f + c.z) * f + c.y) * f + c.x;
+      w1 = inv_h * ((3.f * c.w * f + 2.f * c.z) * f + c.y);
+      w2 = inv_h * inv_h * (6.f * c.w * f + 2.f * c.z);
+    } else {
+      w0 = pick(N[a], e);
+      w1 = pick(dN[a], e);
+      w2 = pick(d2N[a], e);
+    }
+  };
+  adjoint_stage_rounds<LANES>(g, nodes, nbar, bin, live, quirk, [&](const float4 *adj, const float4 *vel, int box0,
+                                                                   int X) {
+    const int at0 = box0 + (first[0] + 1) + X * ((first[1] + 1) + 4 * (first[2] + 1));
+#pragma unroll 1
+    for (int sz = LANES == 1 ? 0 : sub; sz < (LANES == 1 ? E : min(sub + 1, E)); ++sz) {
+      // y-contracted sums of this layer: xb's terms by their z weight (N: yX,
+      // yY; dN: yZ, zX, zY; d2N: zZ), P_bar and f_bar by theirs
+      float yX = 0.f, yY = 0.f, yZ = 0.f, zX = 0.f, zY = 0.f, zZ = 0.f;
+      float yP[3] = {0.f, 0.f, 0.f}, fx[3] = {0.f, 0.f, 0.f}, fy[3] = {0.f, 0.f, 0.f}, fz[3] = {0.f, 0.f, 0.f};
+#pragma unroll(E > 2 ? 1 : 2)
+      for (int sy = 0; sy < E; ++sy) {  // (not unrolled: the next rows' records would fill the registers)
+        const int at = at0 + X * (sy + 4 * sz);
+        float g0 = 0.f, g1 = 0.f, wx1 = 0.f, wx2 = 0.f, wy0 = 0.f, wy1 = 0.f, wz0 = 0.f, wz1 = 0.f;
+        float P0[3] = {0.f, 0.f, 0.f}, f0[3] = {0.f, 0.f, 0.f}, f1[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ex = 0; ex < E; ++ex) {
+          const float4 a0 = adj[2 * (at + ex)], a1 = adj[2 * (at + ex) + 1];
+          const float4 u0 = vel[2 * (at + ex)], u1 = vel[2 * (at + ex) + 1];
+          const float P[3] = {a0.y, a0.z, a0.w}, f[3] = {a1.x, a1.y, a1.z};
+          const float vn[3] = {u0.x, u0.y, u0.z}, dv[3] = {u0.w, u1.x, u1.y};
+          float gs = m * a0.x;
+#pragma unroll
+          for (int a = 0; a < 3; ++a) gs += mv[a] * P[a];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) gs += vpb[a] * vn[a];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) gs += dvb[a] * dv[a];
+          const float wx = Lb[0] * vn[0] + Lb[1] * vn[1] + Lb[2] * vn[2] - (Sv.xx * f[0] + Sv.xy * f[1] + Sv.xz * f[2]);
+          const float wy = Lb[3] * vn[0] + Lb[4] * vn[1] + Lb[5] * vn[2] - (Sv.xy * f[0] + Sv.yy * f[1] + Sv.yz * f[2]);
+          const float wz = Lb[6] * vn[0] + Lb[7] * vn[1] + Lb[8] * vn[2] - (Sv.xz * f[0] + Sv.yz * f[1] + Sv.zz * f[2]);
+          const float n0 = N[0][ex], n1 = dN[0][ex], n2 = d2N[0][ex];
+          g0 += n0 * gs; g1 += n1 * gs;
+          wx1 += n1 * wx; wx2 += n2 * wx;
+          wy0 += n0 * wy; wy1 += n1 * wy;
+          wz0 += n0 * wz; wz1 += n1 * wz;
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            P0[a] += n0 * P[a];
+            f0[a] += n0 * f[a];
+            f1[a] += n1 * f[a];
+          }
+        }
+        float y0, y1, y2;
+        axis_at(1, sy, y0, y1, y2);
+        yX += y0 * (g1 + wx2) + y1 * wy1;
+        yY += y1 * (g0 + wx1) + y2 * wy0;
+        yZ += y0 * (g0 + wx1) + y1 * wy0;
+        zX += y0 * wz1;
+        zY += y1 * wz0;
+        zZ += y0 * wz0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          yP[a] += y0 * P0[a];
+          fx[a] += y0 * f1[a];
+          fy[a] += y1 * f0[a];
+          fz[a] += y0 * f0[a];
+        }
+      }
+      float z0, z1, z2;
+      axis_at(2, sz, z0, z1, z2);
+      xb[0] += z0 * yX + z1 * zX;
+      xb[1] += z0 * yY + z1 * zY;
+      xb[2] += z1 * yZ + z2 * zZ;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        vb[a] += z0 * yP[a];
+        G[a][0] += z0 * fx[a];
+        G[a][1] += z0 * fy[a];
+        G[a][2] += z1 * fz[a];
+      }
+    }
+  });
+#pragma unroll
+  for (int a = 0; a < 3; ++a) vb[a] *= m;
+  if (walk && (LANES == 1 || sub < E)) {
+    // outside entries one by one, with the types of the node each reaches
+#pragma unroll 1
+    for (int e = 0; e < E * E * (LANES == 1 ? E : 1); ++e) {
+      const int e3[3] = {e % E, (e / E) % E, LANES == 1 ? e / (E * E) : sub};
+      int nb[3];
+      bool inside = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        nb[a] = bin[a] + first[a] + e3[a];
+        inside = inside && nb[a] >= 0 && nb[a] < g.num_cells[a];
+      }
+      const int64_t lin = lin_index(g, nb, 3);
+      if (inside || lin < 0 || lin >= g.num_cells_total) continue;
+      int ids[3];
+      node_ids32<3>(g, (int)lin, ids);
+      float n3[3], d3[3], h3[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const int type = cubic_node_type(ids[a], g.num_cells[a], prm.node_types_built);
+        const float r = __fsub_rn(__fsub_rn(t3[a], (float)bin[a]), (float)(first[a] + e3[a]));
+        spline_eval<SF>(r, type, inv_h, n3[a], d3[a]);
+        h3[a] = spline_d2<SF>(r, type, inv_h);
+      }
+      float wgt, gr[3], H[6], mb, Pb[3], fb[3];
+      entry_derivs(n3, d3, h3, wgt, gr, H);
+      load_node_adj<3>(nbar, (int)lin, mb, Pb, fb);
+      const float gs = m * mb + mv[0] * Pb[0] + mv[1] * Pb[1] + mv[2] * Pb[2];
+      const float wv[3] = {-(Sv.xx * fb[0] + Sv.xy * fb[1] + Sv.xz * fb[2]),
+                           -(Sv.xy * fb[0] + Sv.yy * fb[1] + Sv.yz * fb[2]),
+                           -(Sv.xz * fb[0] + Sv.yz * fb[1] + Sv.zz * fb[2])};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        vb[a] += (m * wgt) * Pb[a];
+        float hs = 0.f;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+          G[a][b] += fb[a] * gr[b];
+          hs += H[sym_idx(a, b)] * wv[b];
+        }
+        xb[a] += gr[a] * gs + hs;
+      }
+    }
+  }
+  if constexpr (LANES > 1) {  // the particle's sums over its lanes; lane 0 goes on
+    auto sum_lanes = [](float u) {
+#pragma unroll
+      for (int o = 1; o < LANES; o <<= 1) u += __shfl_xor(u, o, 64);
+      return u;
+    };
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      xb[a] = sum_lanes(xb[a]);
+      vb[a] = sum_lanes(vb[a]);
+#pragma unroll
+      for (int b = 0; b < 3; ++b) G[a][b] = sum_lanes(G[a][b]);
+    }
+    if (sub != 0) return;
+  }
+  if (!live) return;
+  // M_bar = -V G, V_bar = -sigma : G
+  float Vb = 0.f;
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) Vb -= sym_at(s, a, b) * G[a][b];
+  float F[9], C[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) F[k] = ld32(st.F + (int64_t)k * n, src);
+  cofactor<3>(F, C);
+  const float VV = Vb * ld32(st.volume0, src);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    ib.x[(int64_t)a * n + src] += xb[a];
+    ib.v[(int64_t)a * n + src] += vb[a];
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) ib.F[(int64_t)k * n + src] += VV * C[k];
+  // sigma is stored symmetric: an off-diagonal component feeds both entries
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = a; b < 3; ++b)
+      ib.stress[(int64_t)sym_idx(a, b) * n + src] += a == b ? -V * G[a][a] : -V * G[a][b] + -V * G[b][a];
+}
+
+// Per particle: gather of the node adjoints through the P2G window (the same
+// entries as the forward deposit, linear-index wrap-around included) into the
+// adjoints of v, sigma, F (through V = det(F) V0) and x, plus the position
+// adjoint through the G2P weights, which walk the same window:
+//   xbar_c += sum_i grad_c w (vnt . vpb + dv . dvb) + sum_ab d2w/dx_c dx_a Lb_ab vnt_b
+// with vpb, dvb, Lb the records g2p_adjoint_kernel wrote. The in-grid entries
+// run branch-free (clamped node, zero weights outside, as gather_grid); the
+// wrap-around entries of boundary particles, which only the deposit reaches,
+// take a separate compact loop. Adds to ib.
+// 1D and 2D (3D: p2g_adjoint3_kernel).
 template <int D, int SF, int LANES>
 __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles st,
                                                           pmpm_adjoint ib, pmpm_spatial part, pmpm_nodes nodes,
@@ -3649,21 +3948,14 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
   const int n = st.n;
   const int nn = g.num_cells_total;
   // LANES = 1: one lane per particle, the window's y offsets in turn;
-  // LANES = 4: four consecutive lanes per particle, one y offset each;
-  // LANES = 16 (3D): sixteen lanes per particle, one (y, z) row of the window
-  // each. The particle's sums are combined by shuffles; the wider layouts are
-  // for launches too small to fill the chip otherwise.
-  static_assert(LANES == 1 || LANES == 4 || (LANES == 16 && D == 3), "lanes per particle");
-  // 3D cubic with one lane per particle: the workgroup's node records are
-  // staged in LDS (adjoint_stage_rounds), so every thread takes part in the
-  // staging barriers; a thread past the particles works on the last one and
-  // writes nothing
-  constexpr bool STAGED = D == 3 && LANES == 1 && SF == PMPM_SF_CUBIC;
+  // LANES = 4: four consecutive lanes per particle, one y offset each, the
+  // particle's sums combined by shuffles, for launches too small to fill the
+  // chip otherwise.
+  static_assert(D < 3 && (LANES == 1 || LANES == 4), "lanes per particle");
   const int j = (int)blockIdx.x * ((int)blockDim.x / LANES) + (int)threadIdx.x / LANES;
   const int sub0 = (int)threadIdx.x % LANES;
-  if (!STAGED && j >= n) return;  // (all lanes of a particle together)
-  const bool live = j < n;
-  const int jj = live ? j : n - 1;
+  if (j >= n) return;  // (all lanes of a particle together)
+  const int jj = j;
   const int src = part.sorted[jj];
   PW<D, SF> w;
   float xp[3];
@@ -3794,50 +4086,7 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
   // the window's offsets along y (and z) are picked by selects, so the
   // in-grid entries stay unrolled without indexing registers at run time
   auto pick = [](const auto *a, int k) { return k == 0 ? a[0] : (k == 1 ? a[1] : (k == 2 ? a[2] : a[3])); };
-  if constexpr (LANES == 16) {
-    const int sy = sub0 & 3, sz = sub0 >> 2;
-    if (sy < EY && sz < EZ) {
-      const int oyz = pick(off[1], sy) + pick(off[2], sz);
-      const float Ny = pick(N[1], sy), dNy = pick(dN[1], sy), d2Ny = pick(d2N[1], sy);
-      const float Nz = pick(N[2], sz), dNz = pick(dN[2], sz), d2Nz = pick(d2N[2], sz);
-#pragma unroll
-      for (int ex = 0; ex < E; ++ex) {
-        const float n3[3] = {N[0][ex], Ny, Nz}, d3[3] = {dN[0][ex], dNy, dNz}, h3[3] = {d2N[0][ex], d2Ny, d2Nz};
-        entry(nbar, nodes.vel, off[0][ex] + oyz, n3, d3, h3, true);
-      }
-      if (leaves && prm.wrap_quirk) {
-#pragma unroll 1
-        for (int ex = 0; ex < E; ++ex) {
-          const int e3[3] = {ex, sy, sz};
-          wrap_entry(e3);
-        }
-      }
-    }
-  } else if constexpr (STAGED) {
-    // in-grid entries from the LDS records of the workgroup's runs (the
-    // clamped nodes, as off[]), then the wrap-around entries
-    adjoint_stage_rounds(g, nodes, nbar, w, live, [&](const float *adj, const float *vel, int box0, int X) {
-#pragma unroll 1
-      for (int sy = 0; sy < 4; ++sy) {
-        const float Ny = pick(N[1], sy), dNy = pick(dN[1], sy), d2Ny = pick(d2N[1], sy);
-#pragma unroll
-        for (int ex = 0; ex < 4; ++ex)
-#pragma unroll
-          for (int ez = 0; ez < 4; ++ez) {
-            const float n3[3] = {N[0][ex], Ny, N[2][ez]}, d3[3] = {dN[0][ex], dNy, dN[2][ez]},
-                        h3[3] = {d2N[0][ex], d2Ny, d2N[2][ez]};
-            entry(adj, vel, box0 + ex + X * (sy + 4 * ez), n3, d3, h3, true);
-          }
-      }
-    });
-    if (leaves && prm.wrap_quirk) {
-#pragma unroll 1
-      for (int e = 0; e < 64; ++e) {
-        const int e3[3] = {e & 3, (e >> 2) & 3, e >> 4};
-        wrap_entry(e3);
-      }
-    }
-  } else {
+  {
 #pragma unroll 1
     for (int sub = sub0; sub < EY; sub += LANES) {
       const int oy = pick(off[1], sub);
@@ -3874,7 +4123,6 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
     }
     if (sub0 != 0) return;
   }
-  if (!live) return;  // (a staging helper past the particles)
   // M_bar = -V G, V_bar = -sigma : G
   float Mb[3][3], Vb = 0.f;
 #pragma unroll
@@ -3903,21 +4151,19 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
     for (int b = a; b < D; ++b) ib.stress[sym_idx(a, b) * n + src] += a == b ? Mb[a][a] : Mb[a][b] + Mb[b][a];
 }
 
-// Lanes per particle of the adjoint P2G: the fewest that still give three
-// waves per SIMD (256 CUs x 4 SIMDs x 64 lanes x 3 lanes in all), 16 only in
-// 3D. PMPM_ADJOINT_P2G_LANES=1, 4 or 16 in the environment overrides the
-// choice (read at every launch), so the layouts can be checked against each
-// other.
+// Lanes per particle of the adjoint P2G: one once that fills the chip
+// (kAdjointLanesWanted), else four. PMPM_ADJOINT_P2G_LANES=1, 4 or 16 (as 4)
+// in the environment overrides the choice (read at every launch), so the
+// layouts can be checked against each other.
 constexpr int kAdjointLanesWanted = 256 * 4 * 64 * 3;
-inline int adjoint_p2g_lanes(int n, int dim) {
+inline int adjoint_p2g_lanes(int n) {
   const char *e = getenv("PMPM_ADJOINT_P2G_LANES");
   if (e) {
     const int v = atoi(e);
-    if (v == 1 || v == 4 || (v == 16 && dim == 3)) return v;
+    if (v == 1) return 1;
+    if (v == 4 || v == 16) return 4;
   }
-  if (n >= kAdjointLanesWanted) return 1;
-  if ((int64_t)n * 4 >= kAdjointLanesWanted || dim != 3) return 4;
-  return 16;
+  return n >= kAdjointLanesWanted ? 1 : 4;
 }
 
 template <int D, int SF>
@@ -3925,23 +4171,24 @@ void launch_adjoint_particles(const pmpm_params &prm, const pmpm_grid &g, const 
                               const pmpm_adjoint &ob, const pmpm_adjoint &ib, const pmpm_spatial &part,
                               const pmpm_nodes &nodes, float *rec, float *pbar, int which, const float *nbar,
                               hipStream_t s) {
-  const unsigned blocks = (unsigned)ceil_div(st.n, 256);
-  if (which == 0)
-    PMPM_LAUNCH((g2p_adjoint_kernel<D, SF>), (::pmpm::kname("g2p_adjoint_kernel", {(long)(D), (long)(SF)})), dim3(blocks), dim3(256), 0, s, prm, g, st, ob, ib, part, nodes,
+  if (which == 0) {
+    PMPM_LAUNCH((g2p_adjoint_kernel<D, SF>), (::pmpm::kname("g2p_adjoint_kernel", {(long)(D), (long)(SF)})), dim3((unsigned)ceil_div(st.n, 256)), dim3(256), 0, s, prm, g, st, ob, ib, part, nodes,
                        rec, pbar);
-  else {
-    const int lanes = adjoint_p2g_lanes(st.n, D);
-    const dim3 grid((unsigned)ceil_div(st.n, 256 / lanes));
-    if (lanes == 1)
-      PMPM_LAUNCH((p2g_adjoint_kernel<D, SF, 1>), (::pmpm::kname("p2g_adjoint_kernel", {(long)(D), (long)(SF), (long)(1)})), grid, dim3(256), 0, s, prm, g, st, ib, part, nodes, nbar,
-                         rec);
-    else if (lanes == 4 || D != 3)
-      PMPM_LAUNCH((p2g_adjoint_kernel<D, SF, 4>), (::pmpm::kname("p2g_adjoint_kernel", {(long)(D), (long)(SF), (long)(4)})), grid, dim3(256), 0, s, prm, g, st, ib, part, nodes, nbar,
-                         rec);
-    else
-      PMPM_LAUNCH((p2g_adjoint_kernel<D, SF, D == 3 ? 16 : 4>), (::pmpm::kname("p2g_adjoint_kernel", {(long)(D), (long)(SF), (long)(D == 3 ? 16 : 4)})), grid, dim3(256), 0, s, prm, g, st, ib, part,
-                         nodes, nbar, rec);
+    return;
   }
+  const int lanes = adjoint_p2g_lanes(st.n);
+  const dim3 grid((unsigned)ceil_div(st.n, 256 / lanes));
+#define PMPM_P2G_ADJOINT(KERNEL)                                                                                 \
+  PMPM_LAUNCH((KERNEL), (::pmpm::kname("p2g_adjoint_kernel", {(long)(D), (long)(SF), (long)lanes})), grid, dim3(256), 0, \
+              s, prm, g, st, ib, part, nodes, nbar, rec)
+  if constexpr (D == 3) {
+    if (lanes == 1) { auto *k = &p2g_adjoint3_kernel<SF, 1>; PMPM_P2G_ADJOINT(*k); }
+    else { auto *k = &p2g_adjoint3_kernel<SF, 4>; PMPM_P2G_ADJOINT(*k); }
+  } else {
+    if (lanes == 1) { auto *k = &p2g_adjoint_kernel<D, SF, 1>; PMPM_P2G_ADJOINT(*k); }
+    else { auto *k = &p2g_adjoint_kernel<D, SF, 4>; PMPM_P2G_ADJOINT(*k); }
+  }
+#undef PMPM_P2G_ADJOINT
 }
 
 }  // namespace pmpm
