@@ -26,18 +26,6 @@ struct pmpm_context {
   size_t partials_cap = 0;       // floats
   int32_t *tile_flags = nullptr;  // 1 = tile had particles this launch
   size_t tile_flags_cap = 0;
-  // wrap-around sums of typed cubic splines: per (wrap cell, lane) records
-  // ([fields][cells][64] floats)
-  float *wrap_rec = nullptr;
-  size_t wrap_rec_cap = 0;
-  // a byte per node: the typed-cubic wrap-around sums reach it this pass
-  // (allocated in words of 4 bytes)
-  float *wrap_touch = nullptr;
-  size_t wrap_touch_cap = 0;
-  // the nodes the typed-cubic wrap-around sums reach this pass (each once):
-  // kWrapListShards counts, then as many parts of node indices
-  int32_t *wrap_list = nullptr;
-  size_t wrap_list_cap = 0;
   // a byte per node: the components the last grid pass's NodeDomain
   // condition set to zero (words of 4 bytes), read by the adjoint
   float *clamp_mask = nullptr;
@@ -161,7 +149,6 @@ class TimedRegion {
 // be captured in a HIP graph).
 int zero_fill(void *ptr, int64_t n_words, hipStream_t s);
 constexpr int kZeroLists = 6;
-constexpr int kWrapListShards = 32;  // parts of the wrap-around node list (a power of two)
 struct ZeroLists {  // buffers of 32-bit words to clear in one launch
   uint32_t *p[kZeroLists];
   int64_t n[kZeroLists];
@@ -180,10 +167,9 @@ bool params_ok(const pmpm_params *prm);
 bool step_args_ok(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *a, const pmpm_particles *b,
                   const pmpm_spatial *part, const pmpm_nodes *nodes);
 // Workspace the P2G passes of one step use on grid g: tile partials (floats)
-// and tile flags, the 2D typed-cubic wrap-around's records (floats), node
-// flags and node list (words), the clamp record (words).
+// and tile flags, the clamp record (words).
 struct P2GWorkspace {
-  size_t partial_floats, tiles, wrap_floats, touch_words, list_words, clamp_words;
+  size_t partial_floats, tiles, clamp_words;
 };
 void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w);
 // pmpm_partition whose first kernel also clears the buffers of `extra`.

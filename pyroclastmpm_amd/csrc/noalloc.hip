@@ -1,7 +1,7 @@
 // noalloc.hip -- pmpm_step_noalloc: the whole step without a context and
 // without allocating. Its workspace (the radix sort's ping-pong keys, slots and
-// digit histograms, the P2G tile partials and flags, the wrap-around records
-// and node flags, the grid pass's clamp record, the counters) is carved out of one file-scope device array of
+// digit histograms, the P2G tile partials and flags, the grid pass's clamp
+// record, the counters) is carved out of one file-scope device array of
 // kScratchBytes, which each GPU holds for the life of the process. Which steps
 // fit is decided by budget_bytes against PMPM_NOALLOC_SCRATCH_BYTES.
 // Every call on a GPU uses that GPU's copy: calls that overlap on one GPU race.
@@ -15,10 +15,11 @@
 namespace pmpm {
 namespace {
 
-// The budget's partials are those of 16-cell-wide 3D tiles; the tiles in use
-// are 4 or 8 cells wide and take up to 28/22 of that where the cubic budget
-// takes 8-cell tiles, so the array holds that much more than the budget.
-constexpr size_t kScratchBytes = (size_t)PMPM_NOALLOC_SCRATCH_BYTES / 64 * 84;
+// The budget's partials (budget_bytes) are those of other tiles than the ones
+// in use, which take up to 2.6 times as much (a 2D grid of a single row, linear
+// splines: tiles are four rows high; 28/22 in 3D), so the array holds that much
+// more than the budget.
+constexpr size_t kScratchBytes = (size_t)PMPM_NOALLOC_SCRATCH_BYTES / 64 * 168;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -52,32 +53,31 @@ struct Carver {
 };
 
 // The workspace a step is charged with: the sort's and the clamp record's own
-// sizes, and for 3D grids the partials of 16 x 1 x 4 cell tiles (32 x 1 x 4 for
-// linear splines; 8 x 1 x 4 where larger, typed cubic) with the typed-cubic
-// wrap-around's records, flags and node list. What a caller may ask for
+// sizes, the partials of tiles of 256 cells (1D), 64 x 1 cells (2D; 128 x 1 for
+// linear splines) or 16 x 1 x 4 cells (3D; 32 x 1 x 4 for linear splines, 8 x 1
+// x 4 where larger, typed cubic) and, typed cubic in 2D and 3D, the wrap-around's
+// records, flags and node list. What a caller may ask for
 // (PMPM_NOALLOC_SCRATCH_BYTES) must not move with the kernels' tilings.
 size_t budget_bytes(const pmpm_params &prm, const pmpm_grid &g, size_t n, size_t hist_len, const P2GWorkspace &w) {
   Carver c;
-  size_t floats = w.partial_floats, tiles = w.tiles, wrap_floats = w.wrap_floats, touch = w.touch_words,
-         list = w.list_words;
-  if (prm.dim == 3) {
-    auto tiling = [&](int tx, int span) {
-      const size_t t = (size_t)ceil_div(g.num_cells[0], tx) * g.num_cells[1] * ceil_div(g.num_cells[2], 4);
-      const size_t f = t * 7 * (size_t)((tx + span - 1) * span * (3 + span));
-      if (f > floats) floats = f;
-      if (t > tiles) tiles = t;
-    };
-    floats = tiles = 0;
-    const bool cubic = prm.shape_fn == PMPM_SF_CUBIC && prm.node_types_built;
-    if (prm.shape_fn == PMPM_SF_LINEAR) tiling(32, 2);
-    else tiling(16, 4);
-    if (cubic) tiling(8, 4);
-    const size_t cells = (size_t)wrap_cell_count<3>(g);
-    if (cubic && prm.wrap_quirk && cells > 0) {
-      wrap_floats = 8 * cells * 64;
-      touch = ((size_t)g.num_cells_total + 3) / 4;
-      list = (size_t)kWrapListShards * (1 + (size_t)wrap_target_count<3>(g));
-    }
+  const int dim = prm.dim, span = prm.shape_fn == PMPM_SF_LINEAR ? 2 : 4;
+  const bool cubic = prm.shape_fn == PMPM_SF_CUBIC && prm.node_types_built;
+  size_t floats = 0, tiles = 0, wrap_floats = 0, touch = 0, list = 0;
+  auto tiling = [&](int tx) {
+    const size_t t = (size_t)ceil_div(g.num_cells[0], tx) * (dim > 1 ? g.num_cells[1] : 1) *
+                     (dim > 2 ? ceil_div(g.num_cells[2], 4) : 1);
+    const size_t f = t * (1 + 2 * dim) * (size_t)((tx + span - 1) * (dim > 1 ? span : 1) * (dim > 2 ? 3 + span : 1));
+    if (f > floats) floats = f;
+    if (t > tiles) tiles = t;
+  };
+  if (dim == 1) tiling(256);
+  else tiling((dim == 2 ? 256 : 64) / span);
+  if (dim == 3 && cubic) tiling(8);
+  const size_t cells = dim == 3 ? (size_t)wrap_cell_count<3>(g) : (dim == 2 ? (size_t)wrap_cell_count<2>(g) : 0);
+  if (cubic && prm.wrap_quirk && cells > 0) {
+    wrap_floats = 8 * cells * 64;
+    touch = ((size_t)g.num_cells_total + 3) / 4;
+    list = 32 * (1 + cells);
   }
   for (const size_t bytes : {n * 4, n * 4, hist_len * 4, (size_t)16, floats * 4, tiles * 4, wrap_floats * 4, touch * 4,
                              list * 4, w.clamp_words * 4})
@@ -106,9 +106,6 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   const size_t o_counters = c.take(4 * sizeof(uint32_t));
   const size_t o_partials = c.take(w.partial_floats * sizeof(float));
   const size_t o_flags = c.take(w.tiles * sizeof(int32_t));
-  const size_t o_wrec = c.take(w.wrap_floats * sizeof(float));
-  const size_t o_touch = c.take(w.touch_words * sizeof(float));
-  const size_t o_list = c.take(w.list_words * sizeof(int32_t));
   const size_t o_clamp = c.take(w.clamp_words * sizeof(float));
   if (budget_bytes(*prm, *grid, n, hist_len, w) > (size_t)PMPM_NOALLOC_SCRATCH_BYTES || c.used > kScratchBytes) {
     note_error("pmpm_step_noalloc: the step needs more workspace than PMPM_NOALLOC_SCRATCH_BYTES "
@@ -135,14 +132,6 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   ctx.partials_cap = w.partial_floats;
   ctx.tile_flags = reinterpret_cast<int32_t *>(base + o_flags);
   ctx.tile_flags_cap = w.tiles;
-  ctx.wrap_rec = w.wrap_floats ? reinterpret_cast<float *>(base + o_wrec) : nullptr;
-  ctx.wrap_rec_cap = w.wrap_floats;
-  // (the step's first kernel clears the node flags and the list counters:
-  // the scratch holds whatever an earlier call left)
-  ctx.wrap_touch = w.touch_words ? reinterpret_cast<float *>(base + o_touch) : nullptr;
-  ctx.wrap_touch_cap = w.touch_words;
-  ctx.wrap_list = w.list_words ? reinterpret_cast<int32_t *>(base + o_list) : nullptr;
-  ctx.wrap_list_cap = w.list_words;
   ctx.clamp_mask = reinterpret_cast<float *>(base + o_clamp);
   ctx.clamp_mask_cap = w.clamp_words;
   // (the context is a plain struct on this stack frame: nothing frees the

@@ -692,9 +692,6 @@ extern "C" int pmpm_context_destroy(pmpm_context *ctx) {
   (void)hipFree(ctx->adj_pb);
   (void)hipFree(ctx->partials);
   (void)hipFree(ctx->tile_flags);
-  (void)hipFree(ctx->wrap_rec);
-  (void)hipFree(ctx->wrap_touch);
-  (void)hipFree(ctx->wrap_list);
   (void)hipFree(ctx->clamp_mask);
   (void)hipFree(ctx->hint_cnt);
   (void)hipFree(ctx->hint_cbt);

@@ -27,47 +27,9 @@
 
 namespace pmpm {
 
-// P2G workgroup. Lane = (cell, y node offset sy of the cell's node span); the
-// CX = 64 / SY cells of a wave lie along x. 3D: 4 waves on 4 consecutive z
-// layers (tile CX x 1 x 4 cells); ZH waves per layer would each take a share
-// of the z node offsets (fewer registers, more redundant weight work; 1 is
-// faster on gfx950). 1D/2D: 4 waves, 4 consecutive runs along x (tile
-// 4 CX x 1 cells).
-
-// LDS row pitch of the P2G node tile: at least nx, and an odd multiple of cx
-// so the SY rows of cx lanes that one flush instruction covers fall into
-// disjoint bank groups (64 banks of 4 bytes).
-__host__ __device__ constexpr int p2g_pitch(int nx, int cx, int sy) {
-  return sy <= 1 ? nx : (((nx + cx - 1) / cx) | 1) * cx;
-}
-
-// Tiles whose node block covers one node, at most, per axis: x and z tiles
-// are wider than the span overlap (T >= SPAN - 1), y tiles are one cell.
+// Tiles whose node block covers one node, at most, per axis (y: tiles of one
+// cell in small 3D scenes).
 constexpr int kCoverX = 2, kCoverY = 4, kCoverZ = 2;
-
-template <int D, int SF> struct P2GGeom {
-  static constexpr int SPAN = Spline<SF>::SPAN;  // node offsets a cell's particles reach, per axis
-  static constexpr int NLO = Spline<SF>::NLO;    // the first of them, relative to the cell
-  static constexpr int SY = D > 1 ? SPAN : 1;    // lanes per cell
-  static constexpr int SZ = D > 2 ? SPAN : 1;    // z node offsets per cell
-  static constexpr int ZH = 1;                   // waves sharing a z layer
-  static constexpr int SZH = SZ / ZH;            // z node offsets per lane
-  static constexpr int WAVES = 4;
-  static constexpr int THREADS = 64 * WAVES;
-  static constexpr int CX = 64 / SY;             // cells per wave
-  static constexpr int TX = D == 3 ? CX : CX * WAVES;
-  static constexpr int TY = 1;
-  static constexpr int TZ = D == 3 ? WAVES / ZH : 1;
-  static constexpr int NX = TX + SPAN - 1;       // tile nodes per axis
-  static constexpr int NY = D > 1 ? TY + SPAN - 1 : 1;
-  static constexpr int NZ = D > 2 ? TZ + SPAN - 1 : 1;
-  static constexpr int NXP = p2g_pitch(NX, CX, SY);
-  static constexpr int NT = NXP * NY * NZ;       // LDS nodes incl. padding
-  static constexpr int NTN = NX * NY * NZ;       // nodes of one partial slice
-  static_assert(CX * SY == 64 && SZH * ZH == SZ, "one wave = CX cells x SY lanes");
-  static_assert((NX - 1) / TX + 1 <= kCoverX && (NY - 1) / TY + 1 <= kCoverY && (NZ - 1) / TZ + 1 <= kCoverZ,
-                "the grid kernel's gather visits at most kCover tiles per axis");
-};
 
 __device__ inline int64_t lin_index(const pmpm_grid &g, const int *b, int D) {
   int64_t h = b[0];
@@ -386,78 +348,6 @@ __device__ inline void scatter_entry_global(const pmpm_params &prm, const pmpm_g
   }
 }
 
-// Weight of one particle at span offset S (node NLO + S relative to its cell)
-// along one axis, frac = t - bin in [0, 1): the same value as the window
-// weight (axis_weights), and 0 at an offset the window does not reach
-// (quadratic). `type` is the node's cubic type (shapefunction.cpp:108-122).
-// For the cubic spline (types 1-3; the caller handles unbuilt types),
-// r = frac - (S - 1) lies in piece 3 - S of the table (cubic.cuh:28-197)
-// except when frac = 1 - 2^-24, where rounding puts r on the next knot: at
-// S = 0 (r = 2) the weight is 0 as in cubic_eval; at S = 3 (r = -1) both
-// pieces meet there (the spline is C2), so the value agrees to rounding.
-template <int SF, int S>
-__device__ inline void span_eval(float frac, int type, float inv_h, float &N, float &dN) {
-  if (SF != PMPM_SF_CUBIC) {
-    spline_eval<SF>(__fsub_rn(frac, (float)(Spline<SF>::NLO + S)), 0, inv_h, N, dN);
-    return;
-  }
-  cubic_span<S>(frac, type, inv_h, N, dN);
-}
-
-// span_eval for the NS consecutive offsets S0 .. S0 + NS - 1.
-template <int SF, int S0, int NS>
-__device__ inline void span_evals(float frac, const int *type, float inv_h, float *N, float *dN) {
-  if constexpr (NS > 0) {
-    span_eval<SF, S0>(frac, type[0], inv_h, N[0], dN[0]);
-    span_evals<SF, S0 + 1, NS - 1>(frac, type + 1, inv_h, N + 1, dN + 1);
-  }
-}
-
-// Per-particle inputs of a P2G deposit.
-//   MODE 0: mass, velocity, -V sigma.
-//   MODE 1 (the re-map's wrap-around deposits): mass and v', read from out.v
-//   in cell order after the fused first map wrote it.
-//   MODE 2 (adjoint scatter): v = adjoint of the PIC velocity, dv = adjoint of
-//   the FLIP increment, Lb = adjoint of the velocity gradient (row-major 3x3),
-//   read from the record array `rec` in cell order.
-struct P2GRec {
-  float x[3], v[3], m;
-  Sym A;  // -V sigma (MODE 0)
-  float f[3];  // external force (MODE 0: the planar-domain walls, else 0)
-  float dv[3], Lb[9];
-};
-template <int D, int MODE>
-__device__ inline void p2g_load(const pmpm_params &prm, const pmpm_grid &g, bool planar, const pmpm_particles &in,
-                                const pmpm_particles &out, const float *rec, int n, int slot, int j, P2GRec &r) {
-  r.f[0] = r.f[1] = r.f[2] = 0.f;
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    r.x[a] = in.x[a * n + slot];
-    r.v[a] = MODE == 0 ? in.v[a * n + slot] : (MODE == 1 ? out.v[a * n + j] : rec[a * n + j]);
-  }
-  if (MODE == 2) {
-    r.m = 1.f;
-    r.A = sym_zero();
-#pragma unroll
-    for (int a = 0; a < D; ++a) r.dv[a] = rec[(3 + a) * n + j];
-#pragma unroll
-    for (int a = 0; a < D; ++a)
-#pragma unroll
-      for (int b = 0; b < D; ++b) r.Lb[3 * a + b] = rec[(6 + 3 * a + b) * n + j];
-    return;
-  }
-  r.m = in.mass[slot];
-  if (MODE == 0) {
-    const Sym s = load_sym(in.stress, n, slot);
-    const float vol = in.volume[slot];
-    const float mvol = -vol;
-    r.A = Sym{mvol * s.xx, mvol * s.yy, mvol * s.zz, mvol * s.xy, mvol * s.xz, mvol * s.yz};
-    if (planar) planar_force<D>(prm, g, r.x, r.v, vol, r.m, r.f);
-  } else {
-    r.A = sym_zero();
-  }
-}
-
 // P2G of a particle whose recomputed bin is not the cell it is listed in
 // (only possible when the partition was built from other positions): this
 // lane's y slice of its window goes straight to the node arrays.
@@ -486,36 +376,9 @@ __device__ void p2g_stray(const pmpm_params &prm, const pmpm_grid &g, const pmpm
     }
 }
 
-// Per-particle P2G inputs staged in LDS, one float (or int bits) per field,
-// field-major within a wave's region:
-//   frac[D]  position in the cell (t - bin, as the weights use it); MODE 1
-//            keeps the position itself (its first map moves it)
-//   lin      linear index of the particle's own bin (-1 outside the grid)
-//   m        mass (MODE 0/1)
-//   v[D]     velocity (MODE 0 and 1), adjoint of the PIC velocity (MODE 2)
-//   A        -V sigma, the D(D+1)/2 components used in D dimensions (MODE 0)
-//   dv[D], Lb[D*D]  adjoints of the FLIP increment and of L (MODE 2)
 // Fields per node of a P2G pass: MODE 0 mass, momentum, force; MODE 1 the
 // re-mapped momentum; MODE 2 the adjoints of v_nt and dv.
 template <int D, int MODE> constexpr int p2g_nv() { return MODE == 0 ? 1 + 2 * D : (MODE == 2 ? 2 * D : D); }
-
-template <int D, int MODE> struct P2GStage {
-  static constexpr int NA = D * (D + 1) / 2;
-  static constexpr int F_LIN = D, F_M = D + 1, F_V = D + 2, F_X = 2 * D + 2;  // F_X: A (MODE 0) or dv (MODE 2)
-  static constexpr int NF = MODE == 0 ? F_X + NA : (MODE == 2 ? F_X + D + D * D : F_X);
-};
-// Particles of one wave's run that fit its LDS region at once: the whole run
-// of 16 cells at the usual 27 particles per cell (longer runs take more
-// passes). MODE 0 leaves room for one workgroup per CU (the accumulators
-// allow 2 waves per SIMD at most), MODE 1 for two.
-template <int D, int SF, int MODE> constexpr int p2g_stage_cap() {
-  constexpr int NV = p2g_nv<D, MODE>();
-  constexpr int budget = MODE == 1 ? 18944 : 40448;  // floats per workgroup
-  constexpr int room = (budget - NV * P2GGeom<D, SF>::NT) / (P2GGeom<D, SF>::WAVES * P2GStage<D, MODE>::NF);
-  constexpr int cap = (room < 512 ? room : 512) / 64 * 64;
-  static_assert(cap >= 64, "LDS budget too small for the staging area");
-  return cap;
-}
 
 // LDS writes of a wave visible to all its lanes (and its earlier reads done)
 __device__ inline void wave_lds_sync() {
@@ -527,597 +390,10 @@ __device__ inline void wave_lds_sync() {
 // for the wave's global loads and stores in flight, which would drain a
 // kernel's prefetches.
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ inline int wave_min(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-  return v;
-}
 __device__ inline int wave_max(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
   return v;
-}
-
-// v_nt and dv gathered over one particle's own window: the rare path of the
-// fused MUSL map, kept as a compact loop (entries outside the grid skipped, as
-// the reference does) so it costs the fused pass no registers.
-template <int D, int SF>
-__device__ inline void gather_one(const pmpm_params &prm, const pmpm_grid &g, const float *x, int n, int slot,
-                                  const pmpm_nodes &nodes, float *vinc, float *dvinc) {
-  constexpr int SPAN = Spline<SF>::SPAN, NLO = Spline<SF>::NLO;
-  constexpr int NENT = D == 1 ? SPAN : (D == 2 ? SPAN * SPAN : SPAN * SPAN * SPAN);
-  const float inv_h = g.inv_cell_size;
-  float fr[3] = {0.f, 0.f, 0.f};
-  int b[3] = {0, 0, 0};
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    const float t = cell_coord(x[a * n + slot], g.origin[a], inv_h);
-    b[a] = (int)t;
-    fr[a] = __fsub_rn(t, (float)b[a]);
-  }
-#pragma unroll 1
-  for (int e = 0; e < NENT; ++e) {
-    int id[3] = {0, 0, 0};
-    float w = 1.f;
-    bool in = true;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      const int o = NLO + (a == 0 ? e % SPAN : (a == 1 ? (e / SPAN) % SPAN : e / (SPAN * SPAN)));
-      id[a] = b[a] + o;
-      in = in && id[a] >= 0 && id[a] < g.num_cells[a];
-      float N, dN;
-      spline_eval<SF>(__fsub_rn(fr[a], (float)o), cubic_node_type(id[a], g.num_cells[a], prm.node_types_built),
-                      inv_h, N, dN);
-      w *= N;
-    }
-    if (!in || w == 0.f) continue;
-    float v[3], dv[3];
-    load_node_vel<D, true>(nodes.vel, (int)lin_index(g, id, D), v, dv);
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      vinc[a] += w * v[a];
-      dvinc[a] += w * dv[a];
-    }
-  }
-}
-
-// Workgroups after the tiles of a MODE 1 launch: they run the first map of
-// the particles outside the grid, which sort last and belong to no cell.
-constexpr int kMuslTailBlocks = 4;
-template <int D, int SF>
-__device__ void musl_first_map_tail(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
-                                    const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes,
-                                    int tail_block) {
-  const int n = in.n;
-  const uint32_t nc = (uint32_t)g.num_cells_total;
-  if (n == 0 || part.hash_sorted[n - 1] < nc) return;  // none outside
-  int lo = 0, hi = n - 1;  // first j with hash_sorted[j] == nc
-  while (lo < hi) {
-    const int mid = lo + (hi - lo) / 2;
-    if (part.hash_sorted[mid] >= nc) hi = mid;
-    else lo = mid + 1;
-  }
-  const float am = (float)(1.0 - (double)prm.alpha);
-  for (int j = lo + tail_block * (int)blockDim.x + (int)threadIdx.x; j < n; j += kMuslTailBlocks * (int)blockDim.x) {
-    const int src = part.sorted[j];
-    PW<D, SF> w;
-    float xp[3];
-    particle_weights<D, SF>(prm, g, in.x, n, src, w, xp);
-    float vinc[3] = {0.f, 0.f, 0.f}, dvinc[3] = {0.f, 0.f, 0.f}, L[9];
-    gather_grid<D, SF, true, false>(g, node_src(g, nodes), w, vinc, dvinc, L);
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      out.v[a * n + j] = am * vinc[a] + prm.alpha * (in.v[a * n + src] + dvinc[a]);
-      out.x[a * n + j] = xp[a] + prm.dt * vinc[a];
-    }
-  }
-}
-
-// P2G of one tile of cells.
-//   MODE 0: mass, momentum and force (force accumulates in mom_nt).
-//   MODE 1: MUSL first map and re-map in one pass: each particle's v', x'
-//           from the node velocity records (written to slot j of `out`), then
-//           m v' deposited with the same weights (the reference's
-//           KERNEL_MUSL_G2P_DOUBLE_MAPPING and KERNEL_MUSL_P2G_DOUBLE_MAPPING,
-//           musl_kernels.cuh:33-60). Particles outside the grid are mapped by
-//           the kMuslTailBlocks workgroups after the tiles.
-//   MODE 2: adjoint scatter of the G2P record adjoints.
-// Lane (cell c, sy) walks the particles of c in sorted order and sums in
-// registers their contributions to its SPAN x SZ nodes c + NLO + (sx, sy, sz).
-// The sums then enter an LDS node tile in SPAN x SZ phases: within one phase
-// the lanes of the workgroup address distinct nodes, so a plain read-add-write
-// is race free (LDS float atomics are over an order of magnitude slower on
-// gfx950). The tile goes with plain stores to this workgroup's slice of
-// `partials` (flags[tile] marks the slice live) and the grid kernel sums the
-// slices covering each node.
-// A wave's cells are consecutive in the linear cell order, so their particles
-// form one run of the sorted order. The wave loads the run into LDS first,
-// lane = particle, with coalesced loads (fraction, own bin, and the products
-// each lane needs), then the register loop reads only LDS: every particle line
-// is fetched from HBM once instead of being re-fetched as the cells' lanes
-// step through it together.
-// Node offsets outside the grid: the reference bound-checks only the linear
-// node index (usl_inline.h:122-126, shapefunction.cpp:96-98), so such a
-// deposit lands on the wrapped node, weighted with that node's cubic types.
-// Those sums go to the node arrays with one global atomic per cell, node
-// offset and field (wrap_quirk), or are dropped.
-// Which P2G passes stage their particles in LDS: the MUSL map (8 floats per
-// particle, two workgroups per CU). The full P2G and the adjoint scatter
-// (14 and 20 floats) would fit one workgroup per CU only, and measured slower
-// that way than reading through L2 at two waves per SIMD.
-template <int MODE> constexpr bool p2g_staged() { return MODE == 1; }
-template <int D, int SF, int MODE> constexpr int p2g_lds_floats() {
-  constexpr int NV = p2g_nv<D, MODE>();
-  return NV * P2GGeom<D, SF>::NT +
-         (p2g_staged<MODE>() ? P2GGeom<D, SF>::WAVES * P2GStage<D, MODE>::NF * p2g_stage_cap<D, SF, MODE>() : 1);
-}
-// Waves per SIMD the LDS allows (4 waves per workgroup, 160 KB per CU); at 1
-// the register budget is the whole file.
-template <int D, int SF, int MODE> constexpr int p2g_waves_per_simd() {
-  return p2g_lds_floats<D, SF, MODE>() * 4 * 2 <= 163840 ? 2 : 1;
-}
-
-template <int D, int SF, int MODE>
-__global__ __launch_bounds__((P2GGeom<D, SF>::THREADS)) __attribute__((amdgpu_waves_per_eu(p2g_waves_per_simd<D, SF, MODE>()))) void p2g_kernel(pmpm_params prm, pmpm_grid g,
-                                                                      pmpm_particles in, pmpm_particles out,
-                                                                      pmpm_spatial part, pmpm_nodes nodes,
-                                                                      int tiles_x, int tiles_y,
-                                                                      float *__restrict__ partials,
-                                                                      int32_t *__restrict__ flags,
-                                                                      const float *__restrict__ rec) {
-  using G = P2GGeom<D, SF>;
-  constexpr int SPAN = G::SPAN, NLO = G::NLO, SZ = G::SZ, SZH = G::SZH, NE = SPAN * SZH;
-  constexpr int NV = p2g_nv<D, MODE>();
-  constexpr int NXP = G::NXP, NY = G::NY, NT = G::NT;
-  using ST = P2GStage<D, MODE>;
-  constexpr bool kStaged = p2g_staged<MODE>();
-  constexpr int NF = ST::NF, CW = p2g_stage_cap<D, SF, MODE>();
-  __shared__ float tile[NV * NT];
-  __shared__ float stage[kStaged ? G::WAVES * NF * CW : 1];
-
-  const int n = in.n;
-  const int nn = g.num_cells_total;
-  const float inv_h = g.inv_cell_size;
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int sy = D > 1 ? lane / G::CX : 0;
-  const int lx = (D == 3 ? 0 : wave * G::CX) + lane % G::CX;  // tile-local cell
-  const int lz = D == 3 ? wave / G::ZH : 0;
-  const int zh = D == 3 ? wave % G::ZH : 0;  // which half of the z node offsets
-  const int bx = blockIdx.x % tiles_x;
-  const int by = (blockIdx.x / tiles_x) % tiles_y;
-  const int bz = blockIdx.x / (tiles_x * tiles_y);
-  const int c[3] = {bx * G::TX + lx, D > 1 ? by : 0, D > 2 ? bz * G::TZ + lz : 0};
-
-  if constexpr (MODE == 1) {
-    if ((int)blockIdx.x >= (int)gridDim.x - kMuslTailBlocks) {
-      musl_first_map_tail<D, SF>(prm, g, in, out, part, nodes, (int)blockIdx.x - ((int)gridDim.x - kMuslTailBlocks));
-      return;
-    }
-  }
-  for (int i = t; i < NV * NT; i += G::THREADS) tile[i] = 0.f;
-
-  bool in_grid = c[0] < g.num_cells[0];
-  if (D > 1) in_grid = in_grid && c[1] < g.num_cells[1];
-  if (D > 2) in_grid = in_grid && c[2] < g.num_cells[2];
-  int cs = 0, ce = 0, cell = -2;
-  if (in_grid) {
-    cell = (int)lin_index(g, c, D);
-    ce = part.cell_end[cell];
-    cs = part.cell_start[cell];
-  }
-  // cubic weights without node types are zero (cubic.cuh: type 0): nothing
-  // to deposit
-  // (MODE 1 still moves the particles: its first map gathers zeros)
-  const bool none = SF == PMPM_SF_CUBIC && !prm.node_types_built;
-  const bool planar = MODE == 0 && has_planar(prm);  // wall forces on the particles
-  if (!__syncthreads_or(ce > cs) || (none && MODE != 1)) {
-    if (t == 0) flags[blockIdx.x] = 0;
-    return;
-  }
-
-  // which of this lane's nodes lie inside the grid
-  bool x_in[SPAN], z_in[SPAN];
-  const int yn = c[1] + NLO + sy;
-  const bool y_in = D < 2 || (yn >= 0 && yn < g.num_cells[1]);
-#pragma unroll
-  for (int s = 0; s < SPAN; ++s) {
-    const int xn = c[0] + NLO + s, zn = c[2] + NLO + s;
-    x_in[s] = xn >= 0 && xn < g.num_cells[0];
-    z_in[s] = D < 3 || (zn >= 0 && zn < g.num_cells[2]);
-  }
-
-  float acc[NE][NV];
-#pragma unroll
-  for (int e = 0; e < NE; ++e)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) acc[e][k] = 0.f;
-
-  // cubic node types of this lane's span nodes (own particles share them)
-  int tx[SPAN], tz[SZH];
-#pragma unroll
-  for (int s = 0; s < SPAN; ++s) tx[s] = cubic_node_type(c[0] + NLO + s, g.num_cells[0], prm.node_types_built);
-#pragma unroll
-  for (int s = 0; s < SZH; ++s)
-    tz[s] = D > 2 ? cubic_node_type(c[2] + NLO + zh * SZH + s, g.num_cells[2], prm.node_types_built) : 0;
-  // this lane's one y offset: its cubic piece (3 - sy) and the node's type
-  // fix the coefficients for every particle of the cell
-  const float ry0 = (float)(NLO + sy);
-  float yc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (SF == PMPM_SF_CUBIC && D > 1) {
-    const int ty = cubic_node_type(c[1] + NLO + sy, g.num_cells[1], prm.node_types_built);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) yc[k] = kCubic[ty][3 - sy][k];
-  }
-
-  // MODE 1: the velocity records of this lane's SPAN x SZH nodes, loaded once
-  // for all the cell's particles (zero outside the grid, as the gather skips
-  // such entries)
-  constexpr int NVN = MODE == 1 ? 2 * D : 1;
-  float vnode[SPAN][SZH][NVN];
-  if constexpr (MODE == 1) {
-#pragma unroll
-    for (int sx = 0; sx < SPAN; ++sx)
-#pragma unroll
-      for (int sz = 0; sz < SZH; ++sz) {
-        float v[3] = {0.f, 0.f, 0.f}, dv[3] = {0.f, 0.f, 0.f};
-        if (in_grid && x_in[sx] && y_in && z_in[zh * SZH + sz]) {
-          const int nb[3] = {c[0] + NLO + sx, c[1] + NLO + sy, c[2] + NLO + zh * SZH + sz};
-          load_node_vel<D, true>(nodes.vel, (int)lin_index(g, nb, D), v, dv);
-        }
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-          vnode[sx][sz][a] = v[a];
-          vnode[sx][sz][D + a] = dv[a];
-        }
-      }
-  }
-  const float am = (float)(1.0 - (double)prm.alpha);
-
-  // a particle's weights for this lane's nodes: Nx, Nz per span offset and
-  // the lane's one Ny (with derivatives)
-  struct Wts {
-    float Nx[SPAN], dNx[SPAN], Nz[SZH], dNz[SZH], Ny, dNy;
-  };
-  auto weights = [&](const float *frac, Wts &W) {
-    float *Nx = W.Nx, *dNx = W.dNx, *Nz = W.Nz, *dNz = W.dNz;
-    float Ny = 1.f, dNy = 0.f;
-    span_evals<SF, 0, SPAN>(frac[0], tx, inv_h, Nx, dNx);
-    if constexpr (D > 2) {
-      if constexpr (G::ZH == 1) {
-        span_evals<SF, 0, SZH>(frac[2], tz, inv_h, Nz, dNz);
-      } else {  // this wave's share of the z offsets (zh is uniform per wave)
-        if (zh == 0) span_evals<SF, 0, SZH>(frac[2], tz, inv_h, Nz, dNz);
-        else span_evals<SF, SZH, SZH>(frac[2], tz, inv_h, Nz, dNz);
-      }
-    } else {
-      Nz[0] = 1.f;
-      dNz[0] = 0.f;
-    }
-    if constexpr (D > 1) {
-      const float r = __fsub_rn(frac[1], ry0);
-      if (SF == PMPM_SF_CUBIC) {  // the Horner form of cubic_eval on this lane's piece
-        Ny = ((yc[3] * r + yc[2]) * r + yc[1]) * r + yc[0];
-        dNy = inv_h * ((3.f * yc[3] * r + 2.f * yc[2]) * r + yc[1]);
-        if (sy == 0 && !(r < 2.f)) Ny = dNy = 0.f;  // frac = 1 - 2^-24 (see span_eval)
-      } else {
-        spline_eval<SF>(r, 0, inv_h, Ny, dNy);
-      }
-    }
-    W.Ny = Ny;
-    W.dNy = dNy;
-  };
-  // one particle's contribution to this lane's register sums
-  auto deposit = [&](const P2GRec &cur, const Wts &W) {
-    const float *Nx = W.Nx, *dNx = W.dNx, *Nz = W.Nz, *dNz = W.dNz;
-    const float Ny = W.Ny, dNy = W.dNy;
-    const float m = cur.m;
-#pragma unroll
-    for (int sx = 0; sx < SPAN; ++sx) {
-      const float nxy = Nx[sx] * Ny;
-      const float nxym = nxy * m;
-      float mvxy[3], p[3], q[3];
-      // f_a = sum_b A_ab g_b with g = (dNx Ny Nz, Nx dNy Nz, Nx Ny dNz):
-      // f_a = p_a Nz + q_a dNz
-      const float dxy = dNx[sx] * Ny, dyx = dNy * Nx[sx];
-      float wd[3];
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        mvxy[a] = nxym * cur.v[a];
-        if (MODE == 2) {
-          // adjoint: sum_c Lb_ca g_c = p_a Nz + q_a dNz
-          wd[a] = nxy * cur.dv[a];
-          p[a] = cur.Lb[a] * dxy;
-          if (D > 1) p[a] += cur.Lb[3 + a] * dyx;
-          q[a] = D > 2 ? cur.Lb[6 + a] * nxy : 0.f;
-        } else {
-          p[a] = sym_at(cur.A, a, 0) * dxy;
-          if (D > 1) p[a] += sym_at(cur.A, a, 1) * dyx;
-          q[a] = D > 2 ? sym_at(cur.A, a, 2) * nxy : 0.f;
-          if (MODE == 0 && planar) p[a] += cur.f[a] * nxy;  // w f_ext (usl_inline.h:152-155)
-        }
-      }
-#pragma unroll
-      for (int sz = 0; sz < SZH; ++sz) {
-        float *r = acc[sx * SZH + sz];
-        if (MODE == 0) {
-          r[0] += nxym * Nz[sz];
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            r[1 + a] += mvxy[a] * Nz[sz];
-            r[1 + D + a] += p[a] * Nz[sz];
-            if (D > 2) r[1 + D + a] += q[a] * dNz[sz];
-          }
-        } else if (MODE == 2) {
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            r[a] += (mvxy[a] + p[a]) * Nz[sz];
-            if (D > 2) r[a] += q[a] * dNz[sz];
-            r[D + a] += wd[a] * Nz[sz];
-          }
-        } else {
-#pragma unroll
-          for (int a = 0; a < D; ++a) r[a] += mvxy[a] * Nz[sz];
-        }
-      }
-    }
-  };
-
-  if constexpr (!kStaged) {
-    // the next particle's inputs are loaded while the current one is summed
-    int j = cs;
-    int slot = j < ce ? part.sorted[j] : 0;
-    int slot_next = j + 1 < ce ? part.sorted[j + 1] : 0;
-    P2GRec cur;
-    if (j < ce) p2g_load<D, MODE>(prm, g, planar, in, out, rec, n, slot, j, cur);
-    for (; j < ce; ++j) {
-      const int jn = j + 1;
-      P2GRec nxt = cur;
-      if (jn < ce) p2g_load<D, MODE>(prm, g, planar, in, out, rec, n, slot_next, jn, nxt);
-      const int slot_cur = slot;
-      slot = slot_next;
-      slot_next = jn + 1 < ce ? part.sorted[jn + 1] : 0;
-      float frac[3] = {0.f, 0.f, 0.f};
-      bool own = true;
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        const float ta = cell_coord(cur.x[a], g.origin[a], inv_h);
-        const int ba = (int)ta;
-        own = own && ba == c[a] && ta >= 0.f;  // (t < 0: table form, stray path)
-        frac[a] = __fsub_rn(ta, (float)ba);
-      }
-      if (own) {
-        Wts W;
-        weights(frac, W);
-        deposit(cur, W);
-      } else if (MODE != 2 && zh == 0)  // (MODE 2 runs on a partition of the same positions)
-        p2g_stray<D, SF, MODE>(prm, g, nodes, in.x, n, slot_cur, sy, cur.m, cur.v, cur.A, cur.f);
-      cur = nxt;
-    }
-  } else {
-    // this wave's run [run_lo, run_hi) of the sorted order
-    const int run_lo = wave_min(ce > cs ? cs : 0x7fffffff);
-    const int run_hi = wave_max(ce > cs ? ce : 0);
-    float *st = stage + wave * (NF * CW);
-    for (int w0 = run_lo; w0 < run_hi; w0 += CW) {  // wave-uniform
-      const int wn = min(CW, run_hi - w0);
-      // straight-line staging: every slot, then every field load, so the loads
-      // of a lane's CW / 64 particles are in flight together (rounds past the
-      // window read particle w0 and fill LDS slots nobody reads)
-      constexpr int KR = CW / 64;
-      int slots[KR], js[KR];
-#pragma unroll
-      for (int r = 0; r < KR; ++r) {
-        const int q = lane + 64 * r;
-        js[r] = q < wn ? w0 + q : w0;
-        slots[r] = part.sorted[js[r]];
-      }
-#pragma unroll
-      for (int r = 0; r < KR; ++r) {
-        const int q = lane + 64 * r;
-        const int jj = js[r], slot = slots[r];
-        int b[3] = {0, 0, 0};
-        bool ing = true;
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-          const float ta = cell_coord(in.x[a * n + slot], g.origin[a], inv_h);
-          b[a] = (int)ta;
-          ing = ing && ta >= 0.f && b[a] < g.num_cells[a];  // (t < 0: stray path)
-          // (MODE 1 keeps the position itself: the first map moves it)
-          st[a * CW + q] = MODE == 1 ? in.x[a * n + slot] : __fsub_rn(ta, (float)b[a]);
-        }
-        st[ST::F_LIN * CW + q] = __int_as_float(ing ? (int)lin_index(g, b, D) : -1);
-        if (MODE != 2) st[ST::F_M * CW + q] = in.mass[slot];
-#pragma unroll
-        for (int a = 0; a < D; ++a)
-          st[(ST::F_V + a) * CW + q] = MODE != 2 ? in.v[a * n + slot] : rec[a * n + jj];
-        if constexpr (MODE == 0) {
-          const float mvol = -in.volume[slot];
-          const Sym sg = load_sym(in.stress, n, slot);
-          const float A6[6] = {mvol * sg.xx, mvol * sg.yy, mvol * sg.zz, mvol * sg.xy, mvol * sg.xz, mvol * sg.yz};
-          // D components in sym order: 1D xx; 2D xx yy xy; 3D all six
-          constexpr int pick[3][6] = {{0}, {0, 1, 3}, {0, 1, 2, 3, 4, 5}};
-#pragma unroll
-          for (int k = 0; k < ST::NA; ++k) st[(ST::F_X + k) * CW + q] = A6[pick[D - 1][k]];
-        } else if constexpr (MODE == 2) {
-#pragma unroll
-          for (int a = 0; a < D; ++a) st[(ST::F_X + a) * CW + q] = rec[(3 + a) * n + jj];
-#pragma unroll
-          for (int a = 0; a < D; ++a)
-#pragma unroll
-            for (int bb = 0; bb < D; ++bb) st[(ST::F_X + D + a * D + bb) * CW + q] = rec[(6 + 3 * a + bb) * n + jj];
-        }
-      }
-      wave_lds_sync();
-
-      // this lane's particles in the staged window
-      const int j0 = max(cs, w0), j1 = min(ce, w0 + wn);
-      auto read = [&](int q, P2GRec &r, float *fr, int &lin) {
-#pragma unroll
-        for (int a = 0; a < D; ++a) fr[a] = st[a * CW + q];
-        lin = __float_as_int(st[ST::F_LIN * CW + q]);
-        r.m = MODE == 2 ? 1.f : st[ST::F_M * CW + q];
-        r.f[0] = r.f[1] = r.f[2] = 0.f;  // (staged passes carry no force)
-#pragma unroll
-        for (int a = 0; a < D; ++a) r.v[a] = st[(ST::F_V + a) * CW + q];
-        r.A = sym_zero();
-        if constexpr (MODE == 0) {
-          if (D == 1) r.A.xx = st[ST::F_X * CW + q];
-          if (D == 2) {
-            r.A.xx = st[ST::F_X * CW + q]; r.A.yy = st[(ST::F_X + 1) * CW + q]; r.A.xy = st[(ST::F_X + 2) * CW + q];
-          }
-          if (D == 3) {
-            r.A.xx = st[ST::F_X * CW + q]; r.A.yy = st[(ST::F_X + 1) * CW + q]; r.A.zz = st[(ST::F_X + 2) * CW + q];
-            r.A.xy = st[(ST::F_X + 3) * CW + q]; r.A.xz = st[(ST::F_X + 4) * CW + q]; r.A.yz = st[(ST::F_X + 5) * CW + q];
-          }
-        } else if constexpr (MODE == 2) {
-#pragma unroll
-          for (int a = 0; a < D; ++a) r.dv[a] = st[(ST::F_X + a) * CW + q];
-#pragma unroll
-          for (int a = 0; a < D; ++a)
-#pragma unroll
-            for (int bb = 0; bb < D; ++bb) r.Lb[3 * a + bb] = st[(ST::F_X + D + a * D + bb) * CW + q];
-        }
-      };
-      // the next particle's inputs are read while the current one is summed
-      // (MODE 1 reads each in turn: its node records take the registers)
-      constexpr bool kPrefetch = MODE != 1;
-      P2GRec cur, nxt;
-      float fr[3] = {0.f, 0.f, 0.f}, fr_n[3] = {0.f, 0.f, 0.f};
-      int lin = -1, lin_n = -1;
-      if (kPrefetch && j0 < j1) read(j0 - w0, cur, fr, lin);
-      for (int j = j0; j < j1; ++j) {
-        if (!kPrefetch) read(j - w0, cur, fr, lin);
-        else if (j + 1 < j1) read(j + 1 - w0, nxt, fr_n, lin_n);
-        if constexpr (MODE == 1) {
-          // first map of particle j (fr holds its position): the cell's lanes
-          // each gather their y slice of the window, the butterfly over the
-          // cell's lanes completes the sums, then the re-map deposits m v'
-          float vinc[3] = {0.f, 0.f, 0.f}, dvinc[3] = {0.f, 0.f, 0.f};
-          const bool own = lin == cell;
-          Wts W;
-          if (own) {
-            float frac[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-            for (int a = 0; a < D; ++a) frac[a] = __fsub_rn(cell_coord(fr[a], g.origin[a], inv_h), (float)c[a]);
-            weights(frac, W);
-            if (!none) {
-#pragma unroll
-              for (int sx = 0; sx < SPAN; ++sx)
-#pragma unroll
-                for (int sz = 0; sz < SZH; ++sz) {
-                  const float wxz = W.Nx[sx] * W.Nz[sz];
-#pragma unroll
-                  for (int a = 0; a < D; ++a) {
-                    vinc[a] += wxz * vnode[sx][sz][a];
-                    dvinc[a] += wxz * vnode[sx][sz][D + a];
-                  }
-                }
-            }
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-              vinc[a] *= W.Ny;
-              dvinc[a] *= W.Ny;
-            }
-#pragma unroll
-            for (int o = G::CX; o < 64; o <<= 1)
-#pragma unroll
-              for (int a = 0; a < D; ++a) {
-                vinc[a] += __shfl_xor(vinc[a], o);
-                dvinc[a] += __shfl_xor(dvinc[a], o);
-              }
-          } else if (sy == 0) {
-            // a particle listed in this cell whose bin is another (only when
-            // the partition was built from other positions): its own window
-            gather_one<D, SF>(prm, g, in.x, n, part.sorted[j], nodes, vinc, dvinc);
-          }
-          float vn[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            if (!own) {  // the cell's sy = 0 lane gathered
-              vinc[a] = __shfl(vinc[a], lane % G::CX);
-              dvinc[a] = __shfl(dvinc[a], lane % G::CX);
-            }
-            vn[a] = am * vinc[a] + prm.alpha * (cur.v[a] + dvinc[a]);
-            if (a % G::SY == sy) {  // back into the particle's LDS slot (read above)
-              st[(ST::F_V + a) * CW + (j - w0)] = vn[a];
-              st[a * CW + (j - w0)] = fr[a] + prm.dt * vinc[a];
-            }
-          }
-          P2GRec rv = cur;
-#pragma unroll
-          for (int a = 0; a < D; ++a) rv.v[a] = vn[a];
-          if (own) {
-            if (!none) deposit(rv, W);
-          } else if (zh == 0) {
-            p2g_stray<D, SF, 1>(prm, g, nodes, in.x, n, part.sorted[j], sy, rv.m, rv.v, rv.A, rv.f);
-          }
-        } else if (lin != cell) {
-          // a particle listed in this cell whose bin is another (only when the
-          // partition was built from other positions); MODE 2 is only ever
-          // called on a partition of the same positions
-          if (MODE != 2 && zh == 0)
-            p2g_stray<D, SF, MODE>(prm, g, nodes, in.x, n, part.sorted[j], sy, cur.m, cur.v, cur.A, cur.f);
-        } else {
-          Wts W;
-          weights(fr, W);
-          deposit(cur, W);
-        }
-        if (kPrefetch) {
-          cur = nxt;
-          lin = lin_n;
-#pragma unroll
-          for (int a = 0; a < 3; ++a) fr[a] = fr_n[a];
-        }
-      }
-      wave_lds_sync();
-      if constexpr (MODE == 1) {
-        // the window's x', v' leave with coalesced stores (written from the
-        // cells' lanes they would land 16 lines per store, partly filled)
-        for (int q = lane; q < wn; q += 64)
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            out.x[a * n + w0 + q] = st[a * CW + q];
-            out.v[a * n + w0 + q] = st[(ST::F_V + a) * CW + q];
-          }
-        wave_lds_sync();
-      }
-    }
-  }
-
-  // sums into the LDS tile, one node offset (sx, sz) per phase; the waves
-  // holding that z offset write. Node offsets outside the grid stay in the
-  // tile too when the wrap-around is reproduced with weights that do not
-  // depend on node types (linear, quadratic): the grid kernel adds such a
-  // virtual node's sum to the node its linear index reaches, in a fixed
-  // order. With typed cubic splines the wrapped node's types change the
-  // weights, and p2g_wrap_kernel forms those sums instead. (MODE 2 transposes
-  // G2P, which never reads wrapped nodes.)
-  const bool keep_out = MODE != 2 && prm.wrap_quirk && !(SF == PMPM_SF_CUBIC && prm.node_types_built);
-#pragma unroll
-  for (int sx = 0; sx < SPAN; ++sx)
-#pragma unroll
-    for (int sz = 0; sz < SZ; ++sz) {
-      __syncthreads();
-      if (sz / SZH == zh && (keep_out || (x_in[sx] && y_in && z_in[sz]))) {
-        const int li = (lx + sx) + NXP * (sy + NY * (lz + sz));
-#pragma unroll
-        for (int k = 0; k < NV; ++k) tile[k * NT + li] += acc[sx * SZH + sz % SZH][k];
-      }
-    }
-
-  __syncthreads();
-  constexpr int NX = G::NX, NTN = G::NTN;
-  float *slice = partials + (int64_t)blockIdx.x * NV * NTN;
-  if (t == 0) flags[blockIdx.x] = 1;
-  for (int i = t; i < NTN; i += G::THREADS) {
-    const int ix = i % NX;
-    const int iy = (i / NX) % NY;
-    const int iz = i / (NX * NY);
-    const int li = ix + NXP * (iy + NY * iz);
-#pragma unroll
-    for (int k = 0; k < NV; ++k) slice[k * NTN + i] = tile[k * NT + li];
-  }
 }
 
 // Element i of a uniform base pointer through a 32-bit byte offset: the load
@@ -1194,6 +470,414 @@ template <> struct SpanPoly<PMPM_SF_LINEAR> {
   __device__ inline float N(float f) const { return c1 * f + c0; }
   __device__ inline float dN(float f) const { return f == 0.f ? d_at0 : d; }
 };
+
+// All weights of an interior particle along one axis (cubic: nodes of type 3),
+// and their derivatives times the cell size: SpanPoly with constant offsets.
+template <int SF> __device__ inline void inner_weights(float f, float *N, float *dN) {
+  if constexpr (SF == PMPM_SF_CUBIC) {
+    N[0] = ((-1.f / 6.f * f + 0.5f) * f - 0.5f) * f + 1.f / 6.f;
+    N[1] = (0.5f * f - 1.f) * f * f + 2.f / 3.f;
+    N[2] = ((-0.5f * f + 0.5f) * f + 0.5f) * f + 1.f / 6.f;
+    N[3] = 1.f / 6.f * f * f * f;
+    dN[0] = (-0.5f * f + 1.f) * f - 0.5f;
+    dN[1] = (1.5f * f - 2.f) * f;
+    dN[2] = (-1.5f * f + 1.f) * f + 0.5f;
+    dN[3] = 0.5f * f * f;
+  } else {
+#pragma unroll
+    for (int s = 0; s < Spline<SF>::SPAN; ++s) {
+      SpanPoly<SF> p;
+      p.set(s, 0, 1.f, 1.f);
+      N[s] = p.N(f);
+      dN[s] = p.dN(f);
+    }
+  }
+}
+
+// The P2G tiles of 1D and 2D scenes: CELLS x ROWS cells, one wave per row of
+// CELLS cells along x, lane = (y node offset, cell).
+template <int D, int SF> struct RowGeom {
+  static constexpr int SPAN = Spline<SF>::SPAN, NLO = Spline<SF>::NLO;
+  static constexpr int SY = D > 1 ? SPAN : 1, CELLS = 64 / SY, ROWS = D > 1 ? 4 : 1, THREADS = 64 * ROWS;
+  static constexpr int NX = CELLS + SPAN - 1, NY = ROWS + SY - 1, NTN = NX * NY;  // nodes of one partial slice
+};
+
+// P2G of one tile of a 1D or 2D scene. Modes as p2g_mfma_kernel.
+//
+// What bounds it: latency, not bandwidth or issue. A cell's particles are a
+// serial chain for its lanes (16 per cell at 4 x 4: about 70 vector
+// instructions each), so the chain must read LDS only: a round stages the next
+// KW particles of every cell of the row, two particles per lane, while the
+// fields of the round after and the slots of the one after that are in flight.
+// A lane evaluates the weights of its SPAN x node offsets and of its own y
+// offset, and sums its SPAN nodes in registers; a node column's sums are
+// added over the cells in LDS, phase by phase of x offset (distinct nodes
+// within a phase), and over the rows when the slice is stored. Tiles of 16 x 4
+// cells store 2.1 nodes per cell and a node lies in at most four of them
+// (64 x 1 cells: 4.2 and eight).
+//
+// Linear-index wrap-around as in p2g_mfma_kernel: a node offset outside the
+// grid is a virtual node of the tile with the spline types of the node its
+// linear index reaches, which the grid kernel adds. A carry out of x shifts y
+// by one, so in a row that touches an x face each x offset has y weights of
+// its own.
+template <int D, int SF, int MODE, bool FEXT = false>
+__global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
+    pmpm_params prm, pmpm_grid g, pmpm_particles in, pmpm_particles out, pmpm_spatial part, pmpm_nodes nodes,
+    int tiles_x, float *__restrict__ partials, int32_t *__restrict__ flags, const float *__restrict__ rec) {
+  using G = RowGeom<D, SF>;
+  static_assert(D == 1 || D == 2, "3D passes are p2g_mfma_kernel's");
+  static_assert(MODE == 0 || !FEXT, "only the P2G carries the wall force");
+  constexpr int SPAN = G::SPAN, NLO = G::NLO, SY = G::SY, CELLS = G::CELLS, ROWS = G::ROWS, NX = G::NX;
+  constexpr int NV = p2g_nv<D, MODE>();
+  constexpr bool TYPED = SF == PMPM_SF_CUBIC;
+  // a staged record: fractions, then MODE 0: m, m v, A = -V sigma (xx; yy, xy),
+  // wall force; MODE 1: m v'; MODE 2: adjoints of v_pic, dv and L's columns
+  constexpr int NF = MODE == 0 ? 2 * D + 1 + D * (D + 1) / 2 + (FEXT ? D : 0) : (MODE == 1 ? 2 * D : 3 * D + D * D);
+  constexpr int RS = (NF + 3) / 4 * 4;
+  constexpr int KW = 128 / CELLS;    // particles of a cell per round
+  constexpr int CP = KW * RS + 4;    // LDS words of a cell: the 16-byte reads of 16 cells fall into distinct banks
+  constexpr int WS = CELLS * CP > NV * SY * NX ? CELLS * CP : NV * SY * NX;
+  __shared__ __attribute__((aligned(16))) float smem[ROWS][WS];
+  __shared__ __attribute__((aligned(16))) float s_poly[TYPED ? 64 : 4];  // kSpanCubic
+
+  const int n = in.n;
+  const float inv_h = g.inv_cell_size;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lx = lane % CELLS, sy = lane / CELLS;
+  const int cx0 = ((int)blockIdx.x % tiles_x) * CELLS, cy = D > 1 ? ((int)blockIdx.x / tiles_x) * ROWS + wave : 0;
+  const int cx = cx0 + lx;
+  int cs = 0, ce = 0;
+  if (cx < g.num_cells[0] && (D < 2 || cy < g.num_cells[1])) {
+    const int cell = cx + (D > 1 ? g.num_cells[0] * cy : 0);
+    ce = part.cell_end[cell];
+    cs = part.cell_start[cell];
+  }
+  if (TYPED && t < 64) s_poly[t] = (&kSpanCubic[0][0][0])[t];
+  const bool none = TYPED && !prm.node_types_built;  // untyped cubic weights are zero
+  if (!__syncthreads_or(ce > cs) || none) {
+    if (t == 0) flags[blockIdx.x] = 0;
+    return;
+  }
+  float *st = &smem[wave][0];
+  const int most = wave_max(ce - cs);  // particles of the row's fullest cell
+
+  struct Raw {
+    int slot, cx;
+    bool valid;
+    float x[D], v[D], m, vol, sg[3], dv[D], Lb[D * D];
+  };
+  struct Where {
+    uint32_t j, slot;
+    bool valid;
+  };
+  // the two rows of this lane in a round: cell (lane + 64 r) / KW, its
+  // particle lane % KW
+  int rs[2], re[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int c = (lane + 64 * r) / KW;
+    rs[r] = __shfl(cs, c) + lane % KW;
+    re[r] = __shfl(ce, c);
+  }
+  auto find = [&](int k0, int r) {
+    Where w;
+    const int j = rs[r] + k0;
+    w.valid = j < re[r];
+    w.j = w.valid ? (uint32_t)j : 0u;
+    w.slot = __float_as_uint(ld32(reinterpret_cast<const float *>(part.sorted), w.j));
+    return w;
+  };
+  auto load_raw = [&](const Where &w, int r, Raw &q) {
+    const uint32_t jj = w.j, slot = w.slot;
+    q.valid = w.valid;
+    q.slot = (int)slot;
+    q.cx = cx0 + (lane + 64 * r) / KW;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const int64_t row_a = (int64_t)a * n;
+      q.x[a] = ld32(in.x + row_a, slot);
+      q.v[a] = MODE == 0 ? ld32(in.v + row_a, slot) : (MODE == 1 ? ld32(out.v + row_a, jj) : ld32(rec + row_a, jj));
+    }
+    q.m = MODE == 2 ? 1.f : ld32(in.mass, slot);
+    q.vol = MODE == 0 ? ld32(in.volume, slot) : 0.f;
+    if (MODE == 0) {  // xx, then yy and xy
+      q.sg[0] = ld32(in.stress, slot);
+      q.sg[1] = D > 1 ? ld32(in.stress + (int64_t)n, slot) : 0.f;
+      q.sg[2] = D > 1 ? ld32(in.stress + 3 * (int64_t)n, slot) : 0.f;
+    }
+    if (MODE == 2) {
+#pragma unroll
+      for (int a = 0; a < D; ++a) q.dv[a] = ld32(rec + (3 + a) * (int64_t)n, jj);
+#pragma unroll
+      for (int a = 0; a < D; ++a)
+#pragma unroll
+        for (int b = 0; b < D; ++b) q.Lb[D * a + b] = ld32(rec + (6 + 3 * a + b) * (int64_t)n, jj);
+    }
+  };
+  // is the particle in the cell it is listed in? fr: its fractions there
+  auto own_cell = [&](const Raw &q, float *fr) {
+    bool own = q.valid;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const float ta = cell_coord(q.x[a], g.origin[a], inv_h);
+      const int ba = (int)ta;
+      own = own && ta >= 0.f && ba == (a == 0 ? q.cx : cy);  // (t < 0: stray path)
+      fr[a] = __fsub_rn(ta, (float)ba);
+    }
+    return own;
+  };
+  bool strays = false;  // wave-uniform: some particle is listed in another cell than its own
+  auto stage_raw = [&](const Raw &q, int r) {
+    float fr[D], f[RS];
+    const bool own = own_cell(q, fr);
+    strays = strays || __ballot(q.valid && !own) != 0ull;
+#pragma unroll
+    for (int k = 0; k < RS; ++k) f[k] = 0.f;
+    // (a row without an own particle is zero even if the fields it loaded are
+    // not finite)
+    if (own) {
+#pragma unroll
+      for (int a = 0; a < D; ++a) f[a] = fr[a];
+      if (MODE == 0) {
+        f[D] = q.m;
+#pragma unroll
+        for (int a = 0; a < D; ++a) f[D + 1 + a] = q.m * q.v[a];
+#pragma unroll
+        for (int a = 0; a < D * (D + 1) / 2; ++a) f[2 * D + 1 + a] = -q.vol * q.sg[a];
+        if constexpr (FEXT) {
+          float fe[3] = {0.f, 0.f, 0.f};
+          planar_force<D>(prm, g, q.x, q.v, q.vol, q.m, fe);
+#pragma unroll
+          for (int a = 0; a < D; ++a) f[2 * D + 1 + D * (D + 1) / 2 + a] = fe[a];
+        }
+      } else if (MODE == 1) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) f[D + a] = q.m * q.v[a];
+      } else {
+#pragma unroll
+        for (int a = 0; a < D; ++a) { f[D + a] = q.v[a]; f[2 * D + a] = q.dv[a]; }
+#pragma unroll
+        for (int a = 0; a < D * D; ++a) f[3 * D + a] = q.Lb[a];
+      }
+    }
+    float4 *sp = reinterpret_cast<float4 *>(st + ((lane + 64 * r) / KW) * CP + (lane % KW) * RS);
+#pragma unroll
+    for (int k = 0; k < RS / 4; ++k) sp[k] = make_float4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
+  };
+
+  // this lane's y polynomial; x weights are those of interior nodes but in a
+  // row with cells near an x face (typed nodes), whose weights come from the
+  // table: the x type and, with a carry out of x, the y type per x offset
+  const int nx = g.num_cells[0], ny = g.num_cells[1];
+  const int yv = cy + NLO + sy;
+  SpanPoly<SF> py;
+  if (D > 1) py.set(sy, TYPED ? cubic_node_type(yv, ny, 1) : 0, inv_h, 1.f);
+  const bool faces = TYPED && __ballot(ce > cs && (cx < 3 || cx >= nx - 3)) != 0ull;  // wave-uniform
+  int xt[TYPED ? SPAN : 1] = {}, yt[TYPED ? SPAN : 1] = {};
+  if (TYPED && faces) {
+#pragma unroll
+    for (int s = 0; s < SPAN; ++s) {
+      int xv = cx + NLO + s, y = yv;
+      if (D > 1 && MODE != 2 && prm.wrap_quirk) {
+        while (xv < 0) { xv += nx; --y; }
+        while (xv >= nx) { xv -= nx; ++y; }
+      }
+      xt[s] = 4 * (4 * cubic_node_type(xv, nx, 1) + s);
+      yt[s] = D > 1 ? 4 * (4 * cubic_node_type(y, ny, 1) + sy) : 0;
+    }
+  }
+
+  float acc[SPAN][NV];
+#pragma unroll
+  for (int s = 0; s < SPAN; ++s)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[s][k] = 0.f;
+  const float *own = st + lx * CP;
+  auto read = [&](int k, float *f) {
+#pragma unroll
+    for (int q = 0; q < RS / 4; ++q) {
+      const float4 v = *reinterpret_cast<const float4 *>(own + k * RS + 4 * q);
+      f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
+    }
+  };
+  // the record's sums for one y weight: field k gets Nx c[k] + dNx d[k]
+  auto y_products = [&](const float *f, float Ny, float dNy, float *c, float *d) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) c[k] = d[k] = 0.f;
+    if constexpr (MODE == 0) {
+      constexpr int FA = 2 * D + 1, FE = FA + D * (D + 1) / 2;
+      c[0] = Ny * f[D];
+#pragma unroll
+      for (int a = 0; a < D; ++a) c[1 + a] = Ny * f[D + 1 + a];
+      if constexpr (D == 1) {
+        d[2] = f[FA];
+      } else {
+        d[3] = Ny * f[FA]; c[3] = dNy * f[FA + 2];
+        d[4] = Ny * f[FA + 2]; c[4] = dNy * f[FA + 1];
+      }
+      if constexpr (FEXT) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) c[1 + D + a] += Ny * f[FE + a];
+      }
+    } else if constexpr (MODE == 1) {
+#pragma unroll
+      for (int a = 0; a < D; ++a) c[a] = Ny * f[D + a];
+    } else {
+#pragma unroll
+      for (int a = 0; a < D; ++a) {
+        c[a] = Ny * f[D + a];
+        if (D > 1) c[a] += dNy * f[3 * D + D + a];
+        d[a] = Ny * f[3 * D + a];
+        c[D + a] = Ny * f[2 * D + a];
+      }
+    }
+  };
+  constexpr int DLO = MODE == 0 ? 1 + D : 0, DHI = MODE == 0 ? NV : (MODE == 1 ? 0 : D);  // fields with a dNx part
+  auto add = [&](int s, float Nx, float dNx, const float *c, const float *d) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      acc[s][k] += Nx * c[k];
+      if (k >= DLO && k < DHI) acc[s][k] += dNx * d[k];
+    }
+  };
+  auto product = [&](const float *f) {
+    float c[NV], d[NV], Nx[SPAN], dNx[SPAN];
+    float Ny = 1.f, dNy = 0.f;
+    if (D > 1) {
+      Ny = py.N(f[D - 1]);
+      dNy = MODE == 1 ? 0.f : py.dN(f[D - 1]);
+    }
+    y_products(f, Ny, dNy, c, d);
+#pragma unroll
+    for (int k = DLO; k < DHI; ++k) d[k] *= inv_h;
+    inner_weights<SF>(f[0], Nx, dNx);
+#pragma unroll
+    for (int s = 0; s < SPAN; ++s) add(s, Nx[s], dNx[s], c, d);
+  };
+  auto product_face = [&](const float *f) {
+    if constexpr (TYPED) {
+#pragma unroll
+      for (int s = 0; s < SPAN; ++s) {
+        __builtin_amdgcn_sched_barrier(0);  // (one offset's table reads at a time: registers)
+        const float x = f[0], y = f[D - 1];
+        const float4 p = *reinterpret_cast<const float4 *>(s_poly + xt[s]);
+        const float4 q = *reinterpret_cast<const float4 *>(s_poly + yt[s]);
+        const float Ny = D > 1 ? ((q.w * y + q.z) * y + q.y) * y + q.x : 1.f;
+        const float dNy = D > 1 ? inv_h * ((3.f * q.w * y + 2.f * q.z) * y + q.y) : 0.f;
+        float c[NV], d[NV];
+        y_products(f, Ny, dNy, c, d);
+        add(s, ((p.w * x + p.z) * x + p.y) * x + p.x, inv_h * ((3.f * p.w * x + 2.f * p.z) * x + p.y), c, d);
+      }
+    }
+  };
+
+  Raw raw[2];
+  Where ahead[2] = {};
+#pragma unroll
+  for (int r = 0; r < 2; ++r) ahead[r] = find(0, r);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) load_raw(ahead[r], r, raw[r]);
+  if (KW < most) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) ahead[r] = find(KW, r);
+  }
+#pragma unroll 1
+  for (int k0 = 0; k0 < most; k0 += KW) {  // wave-uniform
+    wave_lds_sync();  // the records staged before are read
+#pragma unroll
+    for (int r = 0; r < 2; ++r) stage_raw(raw[r], r);
+    if (k0 + KW < most) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r) load_raw(ahead[r], r, raw[r]);
+      if (k0 + 2 * KW < most) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) ahead[r] = find(k0 + 2 * KW, r);
+      }
+    }
+    wave_lds_sync();
+    const int rows = min(KW, most - k0);
+    float f[RS], f2[RS];
+    read(0, f);
+    // (two records per turn, each read while the one before is summed; past
+    // the last one a staged or older record is read and not used)
+    if (faces) {
+#pragma unroll 1
+      for (int k = 0; k < rows; ++k) {
+        product_face(f);
+        read((k + 1) & (KW - 1), f);
+      }
+    } else {
+#pragma unroll 1
+      for (int k = 0; k + 1 < rows; k += 2) {
+        read(k + 1, f2);
+        product(f);
+        read((k + 2) & (KW - 1), f);
+        product(f2);
+      }
+      if (rows & 1) product(f);
+    }
+  }
+
+  // sums over the row's cells, [field][y offset][x], in the staging area
+  float *blk = st;
+#pragma unroll
+  for (int s = 0; s < SPAN; ++s) {
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      float *b = blk + (k * SY + sy) * NX + lx;
+      if (s == 0) {
+        b[0] = acc[0][k];
+        if (lx < SPAN - 1) b[CELLS] = 0.f;
+      } else {
+        b[s] += acc[s][k];
+      }
+    }
+  }
+  lds_barrier();
+  if (t == 0) flags[blockIdx.x] = 1;
+  float *slice = partials + (int64_t)blockIdx.x * NV * G::NTN;
+  for (int i = t; i < G::NTN; i += G::THREADS) {
+    const int ix = i % NX, iy = i / NX;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const int y = iy - r;
+        if (y >= 0 && y < SY) sum += smem[r][(k * SY + y) * NX + ix];
+      }
+      slice[k * G::NTN + i] = sum;
+    }
+  }
+  if (MODE != 2 && strays) {
+    // as in p2g_mfma_kernel: particles listed in this row but binned elsewhere
+#pragma unroll 1
+    for (int k0 = 0; k0 < most; k0 += KW)
+#pragma unroll 1
+      for (int r = 0; r < 2; ++r) {
+        Raw q;
+        float fr[D], fe[3] = {0.f, 0.f, 0.f};
+        load_raw(find(k0, r), r, q);
+        if (own_cell(q, fr) || !q.valid) continue;
+        Sym A = sym_zero();
+        if (MODE == 0) {
+          const float mvol = -q.vol;
+          A.xx = mvol * q.sg[0];
+          A.yy = mvol * q.sg[1];
+          A.xy = mvol * q.sg[2];
+        }
+        if (FEXT) planar_force<D>(prm, g, q.x, q.v, q.vol, q.m, fe);
+        float v3[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int a = 0; a < D; ++a) v3[a] = q.v[a];
+#pragma unroll 1
+        for (int e = 0; e < SY; ++e)
+          p2g_stray<D, SF, MODE == 1 ? 1 : 0>(prm, g, nodes, in.x, n, q.slot, e, q.m, v3, A, fe);
+      }
+  }
+}
 
 // The matrix-core P2G of 3D scenes. Tile: CELLS x ROWS x 4 cells, one wave per
 // row of CELLS cells along x.
@@ -1602,227 +1286,6 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
   }
 }
 
-// Floats per (cell, offset) record of the wrap-around sums: the NV fields
-// padded to 16 or 32 bytes, so a record is one or two vector loads.
-__host__ __device__ constexpr int wrap_rec_stride(int nv) { return nv <= 4 ? 4 : 8; }
-
-// The wrap-around sums of one non-empty wrap cell c (index w), one lane per
-// node offset; writes the records of the offsets the gather reads.
-template <int D, int MODE, int NV, int NS>
-__device__ inline void wrap_cell_sums(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
-                                      const pmpm_particles &out, const pmpm_spatial &part, float *rec, int wcells,
-                                      int w, const int *c, int cs, int ce, int lane, float (*s_frac)[64],
-                                      float (*s_v)[64], float (*s_A)[64], float *s_m, int *s_own, int *s_list,
-                                      uint8_t *touch, int32_t *wlist) {
-  constexpr int SPAN = 4, NLO = -1;
-  const int nlanes = D == 3 ? 64 : (D == 2 ? 16 : 4);
-  const int nn = g.num_cells_total;
-  // the node of span offset o (o = sx + 4 (sy + 4 sz)); active: outside the
-  // grid with its linear index in range
-  auto offset_node = [&](int o, int *sv, int64_t &lin) {
-    sv[0] = o % SPAN;
-    sv[1] = D > 1 ? (o / SPAN) % SPAN : 0;
-    sv[2] = D > 2 ? o / (SPAN * SPAN) : 0;
-    int nb[3] = {0, 0, 0};
-    bool inside = true;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      nb[a] = c[a] + NLO + sv[a];
-      inside = inside && nb[a] >= 0 && nb[a] < g.num_cells[a];
-    }
-    lin = lin_index(g, nb, D);
-    return !inside && lin >= 0 && lin < nn;
-  };
-  int sv[3];
-  int64_t lin;
-  const bool active = lane < nlanes && offset_node(lane, sv, lin);
-  // the node's flag (one byte of a 32-bit word); the first writer also
-  // appends the node to the gather's list, so the list holds each reached
-  // node once. The list has kWrapListShards parts (counts wlist[0..S), part
-  // p's entries from wlist[S + p cap]); a wave appends to part w mod S, so
-  // the appends of the wrap cells spread over S counters
-  const int cap = wrap_target_count<D>(g), shard = w & (kWrapListShards - 1);
-  bool fresh = false;
-  if (active) {
-    const uint32_t bit = 1u << (8 * (int)(lin & 3));
-    fresh = (atomicOr(reinterpret_cast<uint32_t *>(touch) + (lin >> 2), bit) & bit) == 0u;
-  }
-  const uint64_t fm = __ballot(fresh);
-  if (fm) {  // wave-uniform
-    const int first = __ffsll((unsigned long long)fm) - 1;
-    int at = 0;
-    if (lane == first) at = atomicAdd(&wlist[shard], __popcll(fm));
-    at = __shfl(at, first);
-    const int idx = at + __popcll(fm & ((1ull << lane) - 1ull));
-    if (fresh && idx < cap) wlist[kWrapListShards + shard * cap + idx] = (int)lin;  // (at most cap nodes in all)
-  }
-  // the active offsets in order (s_list[rank] = offset)
-  const uint64_t act = __ballot(active);
-  const int nact = __popcll(act);
-  if (active) s_list[__popcll(act & ((1ull << lane) - 1ull))] = lane;
-  wave_lds_sync();
-
-  const int n = in.n;
-  const float inv_h = g.inv_cell_size;
-  const int q = lane & 3;  // a quarter of the cell's particles per lane
-  // rounds of 16 active offsets, four lanes per offset
-  for (int r0 = 0; r0 < nact; r0 += 16) {  // wave-uniform
-    const int idx = r0 + (lane >> 2);
-    const bool mine = idx < nact;
-    const int off = mine ? s_list[idx] : 0;
-    // r = frac - (NLO + s) lies in piece 3 - s of the wrapped node's spline
-    // (the same piece argument as span_eval): its coefficients are fixed per
-    // lane
-    float cf[3][4];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) cf[a][k] = 0.f;
-    int so[3] = {0, 0, 0};
-    if (mine) {
-      int64_t ln;
-      (void)offset_node(off, so, ln);
-      int ids[3];
-      node_ids<D>(g, ln, ids);
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        const int type = cubic_node_type(ids[a], g.num_cells[a], prm.node_types_built);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cf[a][k] = kCubic[type][3 - so[a]][k];
-      }
-    }
-    float acc[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = 0.f;
-    for (int base = cs; base < ce; base += 64) {
-      const int cnt = min(64, ce - base);
-      wave_lds_sync();  // the stage of the previous round is read
-      if (lane < cnt) {
-        const int j = base + lane;
-        const int slot = part.sorted[j];
-        bool own = true;
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-          const float ta = cell_coord(in.x[a * n + slot], g.origin[a], inv_h);
-          const int ba = (int)ta;
-          own = own && ta >= 0.f && ba == c[a];
-          s_frac[a][lane] = __fsub_rn(ta, (float)ba);
-        }
-        s_own[lane] = own;
-        P2GRec r;
-        p2g_load<D, MODE>(prm, g, MODE == 0 && has_planar(prm), in, out, nullptr, n, slot, j, r);
-        s_m[lane] = r.m;
-#pragma unroll
-        for (int a = 0; a < D; ++a) s_v[a][lane] = r.v[a];
-        if constexpr (MODE == 0) {
-          s_A[0][lane] = r.A.xx; s_A[1][lane] = r.A.yy; s_A[2][lane] = r.A.zz;
-          s_A[3][lane] = r.A.xy; s_A[4][lane] = r.A.xz; s_A[5][lane] = r.A.yz;
-          s_A[6][lane] = r.f[0]; s_A[7][lane] = r.f[1]; s_A[8][lane] = r.f[2];  // wall force
-        }
-      }
-      wave_lds_sync();
-      if (mine) {
-        for (int k = q; k < cnt; k += 4) {
-          if (!s_own[k]) continue;  // deposited whole by p2g_stray
-          float N[3] = {1.f, 1.f, 1.f}, dN[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            const float r = __fsub_rn(s_frac[a][k], (float)(NLO + so[a]));
-            N[a] = ((cf[a][3] * r + cf[a][2]) * r + cf[a][1]) * r + cf[a][0];
-            dN[a] = inv_h * ((3.f * cf[a][3] * r + 2.f * cf[a][2]) * r + cf[a][1]);
-            if (so[a] == 0 && !(r < 2.f)) N[a] = dN[a] = 0.f;  // frac = 1 - 2^-24
-          }
-          const float wk = (N[0] * N[1]) * N[2];
-          const float wm = wk * s_m[k];
-          const float gr[3] = {(dN[0] * N[1]) * N[2], (dN[1] * N[0]) * N[2], (dN[2] * N[0]) * N[1]};
-          if constexpr (MODE == 0) {
-            const Sym A{s_A[0][k], s_A[1][k], s_A[2][k], s_A[3][k], s_A[4][k], s_A[5][k]};
-            acc[0] += wm;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-              acc[1 + a] += wm * s_v[a][k];
-              acc[1 + D + a] += wk * s_A[6 + a][k];
-#pragma unroll
-              for (int b = 0; b < D; ++b) acc[1 + D + a] += sym_at(A, a, b) * gr[b];
-            }
-          } else {
-#pragma unroll
-            for (int a = 0; a < D; ++a) acc[a] += wm * s_v[a][k];
-          }
-        }
-      }
-    }
-    // the four quarters of an offset, combined in a fixed order
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      acc[k] += __shfl_xor(acc[k], 1);
-      acc[k] += __shfl_xor(acc[k], 2);
-    }
-    if (mine && q == 0) {  // one 16- or 32-byte record, fields past NV zero
-      constexpr int RST = wrap_rec_stride(NV);
-      float4 *dst = reinterpret_cast<float4 *>(rec + ((int64_t)w * 64 + off) * RST);
-#pragma unroll
-      for (int v = 0; v < RST / 4; ++v)
-        dst[v] = float4{4 * v + 0 < NV ? acc[4 * v + 0] : 0.f, 4 * v + 1 < NV ? acc[4 * v + 1] : 0.f,
-                        4 * v + 2 < NV ? acc[4 * v + 2] : 0.f, 4 * v + 3 < NV ? acc[4 * v + 3] : 0.f};
-    }
-  }
-}
-
-// Wrap-around sums of typed cubic splines: one wave per cell that can wrap
-// (four per workgroup). A node offset (sx, sy, sz) of the cell's span whose
-// node lies outside the grid but whose linear index is in range re-sums the
-// cell's particles with the types of the node that index reaches
-// (shapefunction.cpp:96-112); four lanes share such an offset, each summing a
-// quarter of the particles, and the quarters are combined in a fixed order.
-// The sums of a non-empty cell are stored per (cell, offset) in `rec`
-// ([wcells][64] records of wrap_rec_stride(NV) floats; only the offsets the
-// gather reads are written);
-// wrap_gather_kernel adds them to their nodes in a fixed order, so the node
-// sums do not depend on scheduling. Empty cells write nothing (the gather
-// skips them by their cell ranges). The cell's particles are first loaded
-// into LDS by the wave (lane = particle, up to 64 per round), so the per-node
-// loops read LDS instead of walking a chain of dependent global loads.
-constexpr int kWrapCellsPerBlock = 4;
-template <int D, int MODE>
-__global__ __launch_bounds__(64 * kWrapCellsPerBlock) void p2g_wrap_kernel(pmpm_params prm, pmpm_grid g,
-                                                                           pmpm_particles in, pmpm_particles out,
-                                                                           pmpm_spatial part, float *__restrict__ rec,
-                                                                           uint8_t *__restrict__ touch,
-                                                                           int32_t *__restrict__ wlist, int wcells) {
-  constexpr int NV = MODE == 0 ? 1 + 2 * D : D;
-  constexpr int NS = MODE == 0 ? 9 : 1;  // staged -V sigma (6) and wall force (3)
-  constexpr int WPB = kWrapCellsPerBlock;
-  __shared__ float s_frac_all[WPB][3][64], s_v_all[WPB][3][64], s_m_all[WPB][64], s_A_all[WPB][NS][64];
-  __shared__ int s_own_all[WPB][64], s_list_all[WPB][64];
-  // every wave works on its own cell; only wave-level synchronisation below
-  const int wv = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-  const int w = (int)blockIdx.x * WPB + wv;
-  int c[3] = {0, 0, 0};
-  if (w >= wcells || !wrap_cell<D>(g, w, c)) return;  // uniform over the wave
-  const int cell = (int)lin_index(g, c, D);
-  const int ce = part.cell_end[cell];
-  const int cs = part.cell_start[cell];
-  if (ce <= cs) return;
-  wrap_cell_sums<D, MODE, NV, NS>(prm, g, in, out, part, rec, wcells, w, c, cs, ce, lane, s_frac_all[wv],
-                                  s_v_all[wv], s_A_all[wv], s_m_all[wv], s_own_all[wv], s_list_all[wv], touch, wlist);
-}
-
-// The NV fields of the wrap record of (wrap cell w, offset rl).
-template <int NV>
-__device__ inline void wrap_rec_load(const float *wrec, int w, int rl, float *r) {
-  constexpr int RST = wrap_rec_stride(NV);
-  const float4 *src = reinterpret_cast<const float4 *>(wrec + ((int64_t)w * 64 + rl) * RST);
-#pragma unroll
-  for (int v = 0; v < RST / 4; ++v) {
-    const float4 q = src[v];
-    if (4 * v + 0 < NV) r[4 * v + 0] = q.x;
-    if (4 * v + 1 < NV) r[4 * v + 1] = q.y;
-    if (4 * v + 2 < NV) r[4 * v + 2] = q.z;
-    if (4 * v + 3 < NV) r[4 * v + 3] = q.w;
-  }
-}
-
 // Geometry of the P2G tiles for the grid kernel's gather.
 struct TileGeom {
   int tiles[3];  // tiles per axis
@@ -1831,14 +1294,6 @@ struct TileGeom {
   int nlo;       // first node offset of a tile block
   int nv;        // fields per node in the partials
   int gather;    // 0: none, 1: P2G (mass, momentum, force), 2: MUSL re-map (momentum)
-  // wrap-around sums (the reference bound-checks only the linear node index,
-  // usl_inline.h:122-126): 0 none; 1 the out-of-grid nodes of the tile
-  // partials (weights without node types); 2 the per-(cell, lane) records of
-  // p2g_wrap_kernel (typed cubic)
-  int wrap;
-  int wcells;
-  const float *wrec;
-  const int32_t *cstart, *cend;  // cell ranges: a non-empty wrap cell wrote its records
 };
 
 // Sums the NV fields of the partial slices of the tiles whose node block
@@ -1848,32 +1303,23 @@ struct TileGeom {
 // 0's first entries and adds zero), so a node waits for two loads in a row,
 // not one per tile. Returns whether any candidate tile was live (a node no
 // live tile covers skips the loads).
-// TG: the tiling's constants (Tiles3) in 3D, where the divisions then become
-// shifts; the runtime values of tg in 1D and 2D.
-template <int SPAN_, int CELLS_, int ROWS_> struct Tiles3 {
+// TG: the tiling's constants (the divisions then become shifts).
+template <int D, int SPAN_, int CELLS_, int ROWS_> struct Tiles {
   static constexpr int SPAN = SPAN_, NLO = SPAN_ == 2 ? 0 : -1;
-  static constexpr int T[3] = {CELLS_, ROWS_, 4}, N[3] = {CELLS_ + SPAN_ - 1, ROWS_ + SPAN_ - 1, 3 + SPAN_};
+  static constexpr int T[3] = {CELLS_, ROWS_, D > 2 ? 4 : 1};
+  static constexpr int N[3] = {CELLS_ + SPAN_ - 1, D > 1 ? ROWS_ + SPAN_ - 1 : 1, D > 2 ? 3 + SPAN_ : 1};
   static constexpr int COVER_Y = (N[1] - 1) / T[1] + 1;
   static_assert((N[0] - 1) / T[0] + 1 <= kCoverX && COVER_Y <= kCoverY && (N[2] - 1) / T[2] + 1 <= kCoverZ,
                 "the gather visits at most kCover tiles per axis");
 };
-struct TilesRuntime { static constexpr int COVER_Y = -1; };
-template <int D, int NV, class TG = TilesRuntime>
+template <int D, int NV, class TG>
 __device__ inline bool gather_partials(const TileGeom &tg, const float *partials, const int32_t *flags,
                                        const int *ids, float *acc) {
-  constexpr bool FIXED = D == 3;
-  constexpr int MX = kCoverX, MY = TG::COVER_Y < 0 ? (D > 1 ? kCoverY : 1) : TG::COVER_Y, MZ = D > 2 ? kCoverZ : 1;
-  constexpr int MC = MX * MY * MZ;
-  int T[3], N[3], nlo;
-  if constexpr (FIXED) {
-    nlo = TG::NLO;
+  constexpr int MX = kCoverX, MY = TG::COVER_Y, MZ = D > 2 ? kCoverZ : 1;
+  constexpr int MC = MX * MY * MZ, nlo = TG::NLO;
+  int T[3], N[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) { T[a] = TG::T[a]; N[a] = TG::N[a]; }
-  } else {
-    nlo = tg.nlo;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) { T[a] = tg.T[a]; N[a] = tg.N[a]; }
-  }
+  for (int a = 0; a < 3; ++a) { T[a] = TG::T[a]; N[a] = TG::N[a]; }
   int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
 #pragma unroll
   for (int a = 0; a < D; ++a) {
@@ -1921,238 +1367,6 @@ __device__ inline bool gather_partials(const TileGeom &tg, const float *partials
   return true;
 }
 
-// This lane's share of the wrap-around sums that land on node `node`: the
-// node vectors outside the grid whose linear index is `node` (x out of range,
-// or y in 3D), and for each the cells whose window holds it. Typed cubic
-// (tg.wrap == 2): lane = the window offset (sx, sy, sz) of the source cell,
-// whose record the wrap kernel left (empty cells wrote none and are skipped);
-// other splines (tg.wrap == 1): lane 0 sums the tile partials at the outside
-// node. Returns whether this lane added anything.
-template <int D, int NV>
-__device__ inline bool gather_wrapped_lane(const pmpm_grid &g, const TileGeom &tg, const float *partials,
-                                           const int32_t *flags, int node, int lane, float *acc) {
-  if (D < 2) return false;  // the only axis is the slowest: nothing wraps
-  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = D > 2 ? g.num_cells[2] : 1;
-  const int span = tg.N[0] - tg.T[0] + 1;
-  const int lo = tg.nlo, hi = tg.nlo + span - 1;
-  // node = tx + nx (ty + ny tz); an outside node (bx, by, bz) with the same
-  // linear index has bx = tx + kx nx and by + ny bz = rest - kx (32-bit
-  // arithmetic: grids stay below 2^27 nodes)
-  const int tx = node % nx, rest = node / nx;
-  const int sx = lane & 3, sy = (lane >> 2) & 3, sz = lane >> 4;
-  const bool my_lane = D > 2 || lane < 16;
-  bool found = false;
-#pragma unroll 1
-  for (int kx = -2; kx <= 2; ++kx) {  // wave-uniform loops over the outside nodes
-    const int bx = tx + kx * nx;
-    if (bx < lo || bx > nx - 1 + hi) continue;
-    const int q = rest - kx;
-    const int qy = ((q % ny) + ny) % ny, qz0 = (q - qy) / ny;  // q = qy + ny qz0, exactly
-#pragma unroll 1
-    for (int ky = -2; ky <= 2; ++ky) {
-      const int by = qy + ky * ny;
-      if (by < lo || by > ny - 1 + hi) continue;
-      const int qz = qz0 - ky;
-      if (D == 2 && qz != 0) continue;
-      if (D == 3 && (qz < lo || qz > nz - 1 + hi)) continue;
-      const int nb[3] = {bx, by, D > 2 ? qz : 0};
-      if (bx >= 0 && bx < nx && by >= 0 && by < ny && (D < 3 || (qz >= 0 && qz < nz))) continue;  // the node itself
-      if (tg.wrap == 1) {
-        if (lane == 0) found = gather_partials<D, NV>(tg, partials, flags, nb, acc) || found;
-        continue;
-      }
-      if (!my_lane) continue;
-      const int c[3] = {nb[0] + 1 - sx, nb[1] + 1 - sy, D > 2 ? nb[2] + 1 - sz : 0};
-      if (c[0] < 0 || c[0] >= nx || c[1] < 0 || c[1] >= ny || (D > 2 && (c[2] < 0 || c[2] >= nz))) continue;
-      const int w = wrap_index<D>(g, c);
-      if (w < 0) continue;
-      const int cl = c[0] + nx * (c[1] + ny * c[2]);
-      if (tg.cend[cl] <= tg.cstart[cl]) continue;
-      const int rl = sx + 4 * (sy + 4 * sz);
-      float r[NV];
-      wrap_rec_load<NV>(tg.wrec, w, rl, r);
-#pragma unroll
-      for (int k = 0; k < NV; ++k) acc[k] += r[k];
-      found = true;
-    }
-  }
-  return found;
-}
-// One wave per node the wrap-around can reach (wrap_target), four per
-// workgroup: the lanes gather their candidates in parallel, a butterfly over
-// the wave sums them (the same lanes in the same order every run) and lane 0
-// adds the result to the node arrays, which hold nothing else but the (rare)
-// stray deposits at this point; the grid kernel adds the tile partials next.
-// Fixed order, no atomics. With typed cubic splines (touch != nullptr) only
-// the nodes the wrap kernel flagged are gathered (and their flags cleared):
-// the others receive nothing this pass.
-template <int D, int NV>
-__global__ __launch_bounds__(256) void wrap_gather_kernel(pmpm_grid g, TileGeom tg, const float *__restrict__ partials,
-                                                          const int32_t *__restrict__ flags, pmpm_nodes nodes,
-                                                          uint8_t *__restrict__ touch) {
-  const int lane = (int)threadIdx.x & 63;
-  const int t = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6);  // wave-uniform
-  int ids[3] = {0, 0, 0};
-  if (t >= wrap_target_count<D>(g) || !wrap_target<D>(g, t, ids)) return;
-  const int nn = g.num_cells_total;
-  const int i = ids[0] + g.num_cells[0] * (ids[1] + (D > 2 ? g.num_cells[1] * ids[2] : 0));
-  if (touch) {
-    if (!touch[i]) return;  // uniform
-    if (lane == 0) touch[i] = 0;
-  }
-  float acc[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) acc[k] = 0.f;
-  const bool found = gather_wrapped_lane<D, NV>(g, tg, partials, flags, i, lane, acc);
-  if (!__ballot(found)) return;  // uniform: no wrap-around deposit reaches this node
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o);
-  if (lane != 0) return;
-  if constexpr (NV == 1 + 2 * D) {
-    nodes.mass[i] += acc[0];
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      nodes.mom[a * nn + i] += acc[1 + a];
-      nodes.mom_nt[a * nn + i] += acc[1 + D + a];
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < D; ++a) nodes.mom_nt[a * nn + i] += acc[a];
-  }
-}
-
-// gather_wrapped_lane for typed cubic records on grids of at least 3 cells
-// per axis, with one round of loads: there the outside nodes whose linear
-// index is `node` number at most four (at most two x images, x = tx or
-// tx -/+ nx, and for each at most two y images), so they are found first by
-// index arithmetic alone; then every lane issues the cell-range and record
-// loads of its (image, offset) pairs together, and an empty cell's (stale)
-// record is dropped by a select. The same pairs and summation order as
-// gather_wrapped_lane.
-template <int D, int NV>
-__device__ inline bool gather_wrapped_typed(const pmpm_grid &g, const TileGeom &tg, int node, int lane, float *acc) {
-  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = D > 2 ? g.num_cells[2] : 1;
-  constexpr int lo = -1, hi = 2;  // cubic spans: node offsets -1 .. +2
-  const int tx = node % nx, rest = node / nx;
-  int img[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, nimg = 0;
-#pragma unroll
-  for (int kx = -1; kx <= 1; ++kx) {
-    const int bx = tx + kx * nx;
-    if (bx < lo || bx > nx - 1 + hi) continue;
-    const int q = rest - kx;
-    const int qy = ((q % ny) + ny) % ny, qz0 = (q - qy) / ny;
-#pragma unroll
-    for (int ky = -1; ky <= 1; ++ky) {
-      const int by = qy + ky * ny;
-      if (by < lo || by > ny - 1 + hi) continue;
-      const int qz = qz0 - ky;
-      if (D == 2 && qz != 0) continue;
-      if (D == 3 && (qz < lo || qz > nz - 1 + hi)) continue;
-      if (bx >= 0 && bx < nx && by >= 0 && by < ny && (D < 3 || (qz >= 0 && qz < nz))) continue;  // the node itself
-      // (slot by selects: no indexed register array)
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (nimg == k) {
-          img[k][0] = bx;
-          img[k][1] = by;
-          img[k][2] = D > 2 ? qz : 0;
-        }
-      ++nimg;
-    }
-  }
-  const int sx = lane & 3, sy = (lane >> 2) & 3, sz = lane >> 4;
-  const bool my_lane = D > 2 || lane < 16;
-  int cl[4], wi[4];
-  bool ok[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int c[3] = {img[k][0] + 1 - sx, img[k][1] + 1 - sy, D > 2 ? img[k][2] + 1 - sz : 0};
-    ok[k] = k < nimg && my_lane && c[0] >= 0 && c[0] < nx && c[1] >= 0 && c[1] < ny &&
-            (D < 3 || (c[2] >= 0 && c[2] < nz));
-    wi[k] = ok[k] ? wrap_index<D>(g, c) : -1;
-    ok[k] = ok[k] && wi[k] >= 0;
-    cl[k] = ok[k] ? c[0] + nx * (c[1] + ny * c[2]) : 0;
-    if (!ok[k]) wi[k] = 0;
-  }
-  const int rl = sx + 4 * (sy + 4 * sz);
-  int cs[4], ce[4];
-  float r[4][NV];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    cs[k] = tg.cstart[cl[k]];
-    ce[k] = tg.cend[cl[k]];
-    wrap_rec_load<NV>(tg.wrec, wi[k], rl, r[k]);
-  }
-  bool found = false;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const bool use = ok[k] && ce[k] > cs[k];
-#pragma unroll
-    for (int f = 0; f < NV; ++f) acc[f] += use ? r[k][f] : 0.f;
-    found = found || use;
-  }
-  return found;
-}
-
-// The typed-cubic wrap-around sums, gathered for the nodes the wrap kernel
-// listed (each once; the grid pass that follows empties the list): wave e
-// takes list entry e (waves past the count exit after one load), gathers the
-// node's
-// candidates as wrap_gather_kernel does (same candidates, same order, so the
-// node sums do not depend on the list order) and clears its flag.
-template <int D, int NV>
-__global__ __launch_bounds__(256) void wrap_gather_list_kernel(pmpm_grid g, TileGeom tg,
-                                                               const float *__restrict__ partials,
-                                                               const int32_t *__restrict__ flags, pmpm_nodes nodes,
-                                                               uint8_t *__restrict__ touch, int32_t *__restrict__ wlist) {
-  const int lane = (int)threadIdx.x & 63;
-  const int wv = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), nw = (int)gridDim.x * 4;
-  const int nn = g.num_cells_total;
-  // the list's parts: lane p < S holds part p's count; entry e of the whole
-  // list is in the part whose inclusive count first exceeds e
-  const int cap = wrap_target_count<D>(g);
-  const int cnt = lane < kWrapListShards ? min(wlist[lane], cap) : 0;
-  int incl = cnt;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
-  const int count = __builtin_amdgcn_readlane(incl, 63);
-  // grids below 3 cells on an axis have more images per node: generic path
-  const bool small = g.num_cells[0] < 3 || g.num_cells[1] < 3 || (D > 2 && g.num_cells[2] < 3);
-  for (int e = wv; e < count; e += nw) {  // wave-uniform
-    const int part_e = __popcll(__ballot(lane < kWrapListShards && incl <= e));
-    const int before = __shfl(incl - cnt, part_e);
-    const int i = __builtin_amdgcn_readfirstlane(wlist[kWrapListShards + part_e * cap + (e - before)]);
-    float acc[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = 0.f;
-    const bool found = small ? gather_wrapped_lane<D, NV>(g, tg, partials, flags, i, lane, acc)
-                             : gather_wrapped_typed<D, NV>(g, tg, i, lane, acc);
-    if (lane == 0) touch[i] = 0;
-    if (!__ballot(found)) continue;  // uniform
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o);
-    if (lane != 0) continue;
-    if constexpr (NV == 1 + 2 * D) {
-      nodes.mass[i] += acc[0];
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        nodes.mom[a * nn + i] += acc[1 + a];
-        nodes.mom_nt[a * nn + i] += acc[1 + D + a];
-      }
-    } else {
-#pragma unroll
-      for (int a = 0; a < D; ++a) nodes.mom_nt[a * nn + i] += acc[a];
-    }
-  }
-}
-
 // Per node: cutoff + forward moment (finalize), boundary conditions
 // [bc_begin, bc_end) in list order, then the node velocities G2P reads.
 // remap_pass: mom_nt holds the MUSL re-mapped momentum; only kinematic
@@ -2162,20 +1376,18 @@ __global__ __launch_bounds__(256) void wrap_gather_list_kernel(pmpm_grid g, Tile
 // reads the forward moment but the velocity records written here).
 // clamp (optional): per node, the components a NodeDomain condition set to
 // zero (bit a: moment, bit 3 + a: forward moment; a slip clamp counts when
-// its input was not on the kept side), for the adjoint. wlist (optional): the
-// typed-cubic wrap-around node list of 2D, emptied here for the next pass (its
-// gather ran before this pass).
-// 3D (TG = Tiles3): the nodes the wrap-around can reach are left to the
-// launch's first nwrap workgroups, four lanes per node: the node itself and
-// the virtual nodes outside the grid that share its linear index (up to three
-// on grids of at least three nodes along x and y) are gathered by a lane each
+// its input was not on the kept side), for the adjoint.
+// 2D and 3D: the nodes the wrap-around can reach are left to the launch's
+// first nwrap workgroups, four lanes per node: the node itself and the virtual
+// nodes outside the grid that share its linear index (up to three on grids of
+// at least three nodes along x and y) are gathered by a lane each
 // and summed over the lanes in a fixed order. The workgroups after them take
 // the other nodes, one lane each.
 constexpr int kImageLanes = 4;
-template <int NV, class TG>
+template <int D, int NV, class TG>
 __device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, const float *partials,
                                      const int32_t *flags, const int *ids, int lane, float *acc) {
-  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = g.num_cells[2];
+  const int nx = g.num_cells[0], ny = g.num_cells[1], nz = D > 2 ? g.num_cells[2] : 1;
   constexpr int lo = TG::NLO, hi = TG::NLO + TG::SPAN - 1;
   const int kx_end = nx < 3 ? 2 : 1, ky_end = ny < 3 ? 2 : 1;
   int count = 0;
@@ -2189,6 +1401,15 @@ __device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, con
       const int vx = ids[0] + kx * nx;
       if (vx < lo || vx > nx - 1 + hi) continue;
       int qy = ids[1] - kx, qz = ids[2];
+      if (D == 2) {  // (a carry out of y leaves the grid)
+        if (qy < lo || qy > ny - 1 + hi) continue;
+        if (count++ == kImageLanes * round + lane) {
+          mine[0] = vx;
+          mine[1] = qy;
+          have = true;
+        }
+        continue;
+      }
       while (qy < 0) { qy += ny; --qz; }
       while (qy >= ny) { qy -= ny; ++qz; }
       for (int ky = -1; ky <= ky_end; ++ky) {
@@ -2202,7 +1423,7 @@ __device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, con
         }
       }
     }
-    if (have) gather_partials<3, NV, TG>(tg, partials, flags, mine, acc);
+    if (have) gather_partials<D, NV, TG>(tg, partials, flags, mine, acc);
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k)
@@ -2214,37 +1435,35 @@ template <int D, int GATHER, class TG>
 __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int finalize, int bc_begin, int bc_end,
                             int remap_pass, TileGeom tg, const float *__restrict__ partials,
                             const int32_t *__restrict__ flags, int clear_mom_nt, uint8_t *__restrict__ clamp,
-                            int32_t *__restrict__ wlist, int nwrap) {
+                            int nwrap) {
   const int nn = g.num_cells_total;
   int i = ((int)blockIdx.x - nwrap) * blockDim.x + threadIdx.x;
-  if (wlist && i == 0)  // the wrap-around list of this pass is consumed
-    for (int p2 = 0; p2 < kWrapListShards; ++p2) wlist[p2] = 0;
   int ids0[3] = {0, 0, 0};
   bool reached = false;  // a node the wrap-around can reach
-  if (D == 3 && (int)blockIdx.x < nwrap) {
+  if (D > 1 && (int)blockIdx.x < nwrap) {
     const int t = (blockIdx.x * blockDim.x + threadIdx.x) / kImageLanes;
     if (t >= wrap_target_count<D>(g) || !wrap_target<D>(g, t, ids0)) return;  // (a node's lanes together)
-    i = ids0[0] + g.num_cells[0] * (ids0[1] + g.num_cells[1] * ids0[2]);
+    i = ids0[0] + g.num_cells[0] * (ids0[1] + (D > 2 ? g.num_cells[1] * ids0[2] : 0));
     reached = true;
   } else {
     if (i >= nn) return;
     node_ids32<D>(g, i, ids0);
-    if (D == 3 && nwrap > 0 && (ids0[0] <= 1 || ids0[0] == g.num_cells[0] - 1 || ids0[1] <= 1 || ids0[1] == g.num_cells[1] - 1))
+    if (D > 1 && nwrap > 0 &&
+        (ids0[0] <= 1 || ids0[0] == g.num_cells[0] - 1 || (D > 2 && (ids0[1] <= 1 || ids0[1] == g.num_cells[1] - 1))))
       return;
   }
   float m = nodes.mass[i];
   float P[3] = {0.f, 0.f, 0.f}, Q[3] = {0.f, 0.f, 0.f};
   if constexpr (GATHER != 0) {
-    // node arrays hold the deposits of stray particles (and 2D's wrap-around
-    // sums); add the tile partials
+    // node arrays hold the deposits of stray particles; add the tile partials
     constexpr int NV = GATHER == 1 ? 1 + 2 * D : D;
     float acc[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) acc[k] = 0.f;
     if (reached) {
-      if constexpr (D == 3) {
+      if constexpr (D > 1) {
         const int lane = (int)threadIdx.x & (kImageLanes - 1);
-        gather_images<NV, TG>(g, tg, partials, flags, ids0, lane, acc);
+        gather_images<D, NV, TG>(g, tg, partials, flags, ids0, lane, acc);
         if (lane != 0) return;
       }
     } else {
@@ -2764,29 +1983,11 @@ __global__ void shape_function_kernel(pmpm_grid g, int types_built, const float 
     default: return PMPM_ERR_INVALID;                                             \
   }
 
-// How the wrap-around deposits of a P2G pass are summed (TileGeom::wrap): 1
-// from the virtual nodes of the tile partials (3D: in the grid kernel), 2 from
-// the records of p2g_wrap_kernel (2D, typed cubic).
-static int wrap_mode(const pmpm_params &prm, const pmpm_grid &g) {
-  if (!prm.wrap_quirk || prm.dim < 2) return 0;
-  if (prm.shape_fn == PMPM_SF_CUBIC && !prm.node_types_built) return 0;  // untyped cubic weights are zero
-  if (prm.shape_fn == PMPM_SF_CUBIC && prm.dim == 2) return wrap_cell_count<2>(g) > 0 ? 2 : 0;
-  return 1;
-}
-
-template <int D, int SF> TileGeom tile_geom_of(const pmpm_grid &g, int gather) {
-  using G = P2GGeom<D, SF>;
-  TileGeom tg{};
-  const int T[3] = {G::TX, G::TY, G::TZ}, N[3] = {G::NX, G::NY, G::NZ};
-  tg.nlo = G::NLO;
-  for (int a = 0; a < 3; ++a) {
-    tg.T[a] = a < D ? T[a] : 1;
-    tg.N[a] = a < D ? N[a] : 1;
-    tg.tiles[a] = a < D ? (int)ceil_div(g.num_cells[a], T[a]) : 1;
-  }
-  tg.gather = gather;
-  tg.nv = gather == 2 ? D : (gather == 3 ? 2 * D : 1 + 2 * D);  // 3: adjoint scatter
-  return tg;
+// Do virtual nodes of the tile partials land on grid nodes (the linear-index
+// wrap-around, summed by the grid kernel)?
+static bool wraps(const pmpm_params &prm) {
+  if (!prm.wrap_quirk || prm.dim < 2) return false;
+  return prm.shape_fn != PMPM_SF_CUBIC || prm.node_types_built;  // untyped cubic weights are zero
 }
 // The 3D P2G tiles (MfmaGeom) of a scene. A function of the grid and the
 // particle count only: every pass of a step, and pmpm_step_noalloc, must agree
@@ -2798,39 +1999,51 @@ static MfmaTiles mfma_tiles(const pmpm_grid &g, int n) {
   if (g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles) return {4, 1};
   return {8, 2};
 }
-static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, MfmaTiles m) {
+// Tiles of T cells and their node blocks over grid g.
+static TileGeom make_tiles(int dim, int sf, const pmpm_grid &g, int gather, const int *T) {
   TileGeom tg{};
   const int span = sf == PMPM_SF_LINEAR ? 2 : 4;
-  const int T[3] = {m.cells, m.rows, 4}, N[3] = {m.cells + span - 1, m.rows + span - 1, 3 + span};
-  tg.nlo = sf == PMPM_SF_LINEAR ? 0 : -1;
   for (int a = 0; a < 3; ++a) {
-    tg.T[a] = T[a];
-    tg.N[a] = N[a];
-    tg.tiles[a] = (int)ceil_div(g.num_cells[a], T[a]);
+    tg.T[a] = a < dim ? T[a] : 1;
+    tg.N[a] = a < dim ? T[a] + span - 1 : 1;
+    tg.tiles[a] = a < dim ? (int)ceil_div(g.num_cells[a], T[a]) : 1;
   }
-  tg.gather = gather;
-  tg.nv = gather == 2 ? 3 : (gather == 3 ? 6 : 7);
+  tg.nv = gather == 2 ? dim : (gather == 3 ? 2 * dim : 1 + 2 * dim);  // 3: adjoint scatter
   return tg;
 }
-// M(args, Tiles3<..>) for the tiles of tg (3D).
-#define PMPM_WITH_TILES3(tg, M, ...)                            \
-  if ((tg).N[1] - (tg).T[1] == 1) {                             \
-    if ((tg).T[0] == 4) { M(__VA_ARGS__ Tiles3<2, 4, 1>); }     \
-    else { M(__VA_ARGS__ Tiles3<2, 8, 2>); }                    \
-  } else {                                                      \
-    if ((tg).T[0] == 4) { M(__VA_ARGS__ Tiles3<4, 4, 1>); }     \
-    else { M(__VA_ARGS__ Tiles3<4, 8, 2>); }                    \
+static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, MfmaTiles m) {
+  const int T[3] = {m.cells, m.rows, 4};
+  return make_tiles(3, sf, g, gather, T);
+}
+template <int D, int SF> TileGeom row_tile_geom(const pmpm_grid &g, int gather) {
+  const int T[3] = {RowGeom<D, SF>::CELLS, RowGeom<D, SF>::ROWS, 1};
+  return make_tiles(D, SF, g, gather, T);
+}
+// M(D, Tiles<..>) for the tiles of tg: 1D and 2D, 3D.
+#define PMPM_WITH_ROWS(D, tg, M)                                                      \
+  if ((tg).N[0] - (tg).T[0] == 1) {                                                   \
+    M(D, Tiles<D, 2, RowGeom<D, PMPM_SF_LINEAR>::CELLS, RowGeom<D, PMPM_SF_LINEAR>::ROWS>); \
+  } else {                                                                            \
+    M(D, Tiles<D, 4, RowGeom<D, PMPM_SF_CUBIC>::CELLS, RowGeom<D, PMPM_SF_CUBIC>::ROWS>);   \
+  }
+#define PMPM_WITH_TILES3(tg, M)                      \
+  if ((tg).N[0] - (tg).T[0] == 1) {                  \
+    if ((tg).T[0] == 4) { M(3, Tiles<3, 2, 4, 1>); } \
+    else { M(3, Tiles<3, 2, 8, 2>); }                \
+  } else {                                           \
+    if ((tg).T[0] == 4) { M(3, Tiles<3, 4, 4, 1>); } \
+    else { M(3, Tiles<3, 4, 8, 2>); }                \
   }
 // The tiles of a P2G pass over n particles (gather: TileGeom::gather, or 3 for
 // the adjoint scatter).
 static TileGeom tile_geom(const pmpm_params &prm, const pmpm_grid &g, int gather, int n) {
   switch (prm.dim * 3 + prm.shape_fn) {
-    case 3: return tile_geom_of<1, PMPM_SF_LINEAR>(g, gather);
-    case 4: return tile_geom_of<1, PMPM_SF_QUADRATIC>(g, gather);
-    case 5: return tile_geom_of<1, PMPM_SF_CUBIC>(g, gather);
-    case 6: return tile_geom_of<2, PMPM_SF_LINEAR>(g, gather);
-    case 7: return tile_geom_of<2, PMPM_SF_QUADRATIC>(g, gather);
-    case 8: return tile_geom_of<2, PMPM_SF_CUBIC>(g, gather);
+    case 3: return row_tile_geom<1, PMPM_SF_LINEAR>(g, gather);
+    case 4: return row_tile_geom<1, PMPM_SF_QUADRATIC>(g, gather);
+    case 5: return row_tile_geom<1, PMPM_SF_CUBIC>(g, gather);
+    case 6: return row_tile_geom<2, PMPM_SF_LINEAR>(g, gather);
+    case 7: return row_tile_geom<2, PMPM_SF_QUADRATIC>(g, gather);
+    case 8: return row_tile_geom<2, PMPM_SF_CUBIC>(g, gather);
     default: return mfma_tile_geom(prm.shape_fn, g, gather, mfma_tiles(g, n));
   }
 }
@@ -2852,47 +2065,33 @@ static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pm
 #undef PMPM_MFMA
 }
 
-// mode 0: P2G, 1: MUSL first map + re-map, 2: adjoint scatter of the
-// records `rec` (never launched without them). 3D: the matrix-core tiles (the
-// re-map after a G2P-style first map); 1D and 2D: p2g_kernel.
+// mode 0: P2G, 1: MUSL first map (G2P-style) and re-map, 2: adjoint scatter of
+// the records `rec` (never launched without them). 3D: the matrix-core tiles;
+// 1D and 2D: tiles of rows.
 template <int D, int SF>
 void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in, const pmpm_particles &out,
                 const pmpm_spatial &part, const pmpm_nodes &nodes, int mode, float *partials, int32_t *flags,
-                float *wrec, uint8_t *wtouch, int32_t *wlist, hipStream_t s,
-                const float *rec = nullptr) {
+                hipStream_t s, const float *rec = nullptr) {
   if (mode == 2 && !rec) return;
+  if (mode == 1 && in.n > 0)
+    PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})),
+                dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0, s, prm, g, in, out, part, nodes, 1);
   if constexpr (D == 3) {
-    if (mode == 1 && in.n > 0)
-      PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0,
-                         s, prm, g, in, out, part, nodes, 1);
     if (mfma_tiles(g, in.n).cells == 4)
       launch_p2g_mfma<SF, 4, 1>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
     else
       launch_p2g_mfma<SF, 8, 2>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
   } else {
-    const TileGeom tg = tile_geom_of<D, SF>(g, 1);
-    const dim3 grid((unsigned)tile_count(tg)), block(P2GGeom<D, SF>::THREADS);
-    if (mode == 0)
-      PMPM_LAUNCH((p2g_kernel<D, SF, 0>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(0)})), grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0],
-                         tg.tiles[1], partials, flags, rec);
-    else if (mode == 1)
-      PMPM_LAUNCH((p2g_kernel<D, SF, 1>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(1)})), dim3((unsigned)tile_count(tg) + kMuslTailBlocks), block, 0, s, prm,
-                         g, in, out, part, nodes, tg.tiles[0], tg.tiles[1], partials, flags, rec);
-    else
-      PMPM_LAUNCH((p2g_kernel<D, SF, 2>), (::pmpm::kname("p2g_kernel", {(long)(D), (long)(SF), (long)(2)})), grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0],
-                         tg.tiles[1], partials, flags, rec);
-  }
-  if constexpr (D == 2) {
-    const int wcells = wrap_cell_count<D>(g);
-    if (mode != 2 && wrap_mode(prm, g) == 2 && wcells > 0) {
-      const dim3 wgrid((unsigned)ceil_div(wcells, kWrapCellsPerBlock)), wblock(64 * kWrapCellsPerBlock);
-      if (mode == 0)
-        PMPM_LAUNCH((p2g_wrap_kernel<D, 0>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(0)})), wgrid, wblock,
-                    0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
-      else
-        PMPM_LAUNCH((p2g_wrap_kernel<D, 1>), (::pmpm::kname("p2g_wrap_kernel", {(long)(D), (long)(1)})), wgrid, wblock,
-                    0, s, prm, g, in, out, part, wrec, wtouch, wlist, wcells);
-    }
+    const TileGeom tg = row_tile_geom<D, SF>(g, mode + 1);
+    const dim3 grid((unsigned)tile_count(tg)), block(RowGeom<D, SF>::THREADS);
+#define PMPM_ROWS(MODE, FEXT, ...)                                                                                 \
+  PMPM_LAUNCH((p2g_rows_kernel<D, SF, MODE, FEXT>), (::pmpm::kname("p2g_rows_kernel", {(long)D, __VA_ARGS__})),    \
+              grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0], partials, flags, rec)
+    if (mode == 0 && has_planar(prm)) PMPM_ROWS(0, true, (long)SF, 0L, 1L);
+    else if (mode == 0) PMPM_ROWS(0, false, (long)SF, 0L);
+    else if (mode == 1) PMPM_ROWS(1, false, (long)SF, 1L);
+    else PMPM_ROWS(2, false, (long)SF, 2L);
+#undef PMPM_ROWS
   }
 }
 template <int D, int SF>
@@ -2920,25 +2119,25 @@ int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
   const int32_t *flags = gather ? ctx->tile_flags : nullptr;
   // the clamp record of a pass that applies node conditions (not the MUSL
   // re-map pass), for pmpm_adjoint_step
-  int32_t *wl = (ctx && gather) ? ctx->wrap_list : nullptr;
   uint8_t *clamp = nullptr;
   if (!remap && b1 > b0)
     clamp = nodes.clamp ? nodes.clamp : (ctx ? reinterpret_cast<uint8_t *>(ctx->clamp_mask) : nullptr);
 
-  // 3D with the wrap-around: the workgroups of the nodes it can reach
-  const int nwrap = prm.dim == 3 && gather && wrap_mode(prm, g) ? (int)ceil_div((int64_t)wrap_target_count<3>(g) * kImageLanes, 256) : 0;
+  // with the wrap-around: the workgroups of the nodes it can reach
+  const int targets = !gather || !wraps(prm) ? 0 : (prm.dim == 2 ? wrap_target_count<2>(g) : wrap_target_count<3>(g));
+  const int nwrap = (int)ceil_div((int64_t)targets * kImageLanes, 256);
 #define PMPM_GRID_LAUNCH(...)                                                                                          \
   PMPM_LAUNCH((grid_kernel<__VA_ARGS__>), (::pmpm::kname("grid_kernel", {(long)prm.dim}) + " gather " + std::to_string(gather)), \
               dim3(blocks + (unsigned)nwrap), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags,      \
-              clear_mom_nt, clamp, wl, nwrap)
+              clear_mom_nt, clamp, nwrap)
 #define PMPM_GRID_GATHER(D, ...)                                 \
-  if (gather == 0) PMPM_GRID_LAUNCH(D, 0, TilesRuntime);         \
+  if (gather == 0) PMPM_GRID_LAUNCH(D, 0, __VA_ARGS__);          \
   else if (gather == 1) PMPM_GRID_LAUNCH(D, 1, __VA_ARGS__);     \
   else PMPM_GRID_LAUNCH(D, 2, __VA_ARGS__)
-  if (prm.dim == 1) { PMPM_GRID_GATHER(1, TilesRuntime); }
-  else if (prm.dim == 2) { PMPM_GRID_GATHER(2, TilesRuntime); }
-  else if (prm.dim != 3) return PMPM_ERR_INVALID;
-  else PMPM_WITH_TILES3(tg, PMPM_GRID_GATHER, 3, )
+  if (prm.dim == 1) { PMPM_WITH_ROWS(1, tg, PMPM_GRID_GATHER) }
+  else if (prm.dim == 2) { PMPM_WITH_ROWS(2, tg, PMPM_GRID_GATHER) }
+  else if (prm.dim == 3) { PMPM_WITH_TILES3(tg, PMPM_GRID_GATHER) }
+  else return PMPM_ERR_INVALID;
 #undef PMPM_GRID_GATHER
 #undef PMPM_GRID_LAUNCH
   PMPM_LAUNCH_CHECK();
@@ -2983,14 +2182,6 @@ static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, size_t *fl
     *floats = std::max(*floats, tile_count(tg) * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2]);
   }
 }
-// Words of the wrap-around node list (2D typed cubic): the part counts, then
-// kWrapListShards parts of wrap_target_count entries each.
-static size_t wrap_node_list_words(const pmpm_grid &g) {
-  return (size_t)kWrapListShards * (1 + (size_t)wrap_target_count<2>(g));
-}
-// (new flags and counts are cleared on s, the stream that uses them first: a
-// hipMemset on the null stream returns before the fill is done and is not
-// ordered before work on a non-blocking stream, such as a batch's lanes)
 static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, hipStream_t s) {
   size_t floats = 0, tiles = 0;
   partial_sizes(prm, g, &floats, &tiles);
@@ -2999,81 +2190,14 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   // the grid pass's clamp record (one byte per node, in words of 4)
   if ((rc = ensure_buffer(ctx->clamp_mask, ctx->clamp_mask_cap, ((size_t)g.num_cells_total + 3) / 4)) != PMPM_OK)
     return rc;
-  if (wrap_mode(prm, g) != 2) return rc;
-  const size_t wcells = (size_t)wrap_cell_count<2>(g);
-  if ((rc = ensure_buffer(ctx->wrap_rec, ctx->wrap_rec_cap, (size_t)wrap_rec_stride(1 + 2 * prm.dim) * wcells * 64)) != PMPM_OK)
-    return rc;
-  // node flags, one byte per node, cleared once here (the gather clears
-  // what it visits; a stale flag would only cost the gather a visit)
-  const size_t words = ((size_t)g.num_cells_total + 3) / 4;
-  if (words > ctx->wrap_touch_cap) {
-    if ((rc = ensure_buffer(ctx->wrap_touch, ctx->wrap_touch_cap, words)) != PMPM_OK) return rc;
-    if ((rc = zero_fill(ctx->wrap_touch, (int64_t)words, s)) != PMPM_OK) return rc;
-  }
-  // the gather's list: kWrapListShards counts, then as many parts of room
-  // for every node the wrap-around can reach
-  const size_t lwords = wrap_node_list_words(g);
-  if (lwords > ctx->wrap_list_cap) {
-    float *lb = reinterpret_cast<float *>(ctx->wrap_list);
-    size_t cap = ctx->wrap_list_cap;
-    if ((rc = ensure_buffer(lb, cap, lwords)) != PMPM_OK) return rc;
-    ctx->wrap_list = reinterpret_cast<int32_t *>(lb);
-    ctx->wrap_list_cap = cap;
-    if ((rc = zero_fill(ctx->wrap_list, kWrapListShards, s)) != PMPM_OK) return rc;
-  }
   return PMPM_OK;
 }
-static uint8_t *wrap_touch(pmpm_context *ctx) { return reinterpret_cast<uint8_t *>(ctx->wrap_touch); }
 
 void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w) {
   *w = P2GWorkspace{};
   partial_sizes(prm, g, &w->partial_floats, &w->tiles);
-  if (wrap_mode(prm, g) == 2) {
-    w->wrap_floats = (size_t)wrap_rec_stride(1 + 2 * prm.dim) * (size_t)wrap_cell_count<2>(g) * 64;
-    w->touch_words = ((size_t)g.num_cells_total + 3) / 4;
-    w->list_words = wrap_node_list_words(g);
-  }
   w->clamp_words = ((size_t)g.num_cells_total + 3) / 4;
 }
-
-// The wrap-around sums of a P2G pass (gather 1) or MUSL re-map (gather 2)
-// into the node arrays, after its tile kernel and wrap kernel.
-static int launch_wrap_gather(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_spatial &part,
-                              const pmpm_nodes &nodes, int gather, hipStream_t s) {
-  const int mode = wrap_mode(prm, g);
-  if (mode == 0 || prm.dim != 2) return PMPM_OK;  // (3D: the grid kernel adds them)
-  TileGeom tg = tile_geom(prm, g, gather, 0);
-  tg.wrap = mode;
-  tg.wcells = wrap_cell_count<2>(g);
-  tg.wrec = ctx->wrap_rec;
-  tg.cstart = part.cell_start;
-  tg.cend = part.cell_end;
-  const int targets = wrap_target_count<2>(g);
-  if (targets <= 0) return PMPM_OK;
-  if (mode == 2) {  // typed cubic: the nodes the wrap kernel listed
-    const dim3 lgrid((unsigned)ceil_div(targets, 4)), block(256);  // a wave per possible entry
-    uint8_t *touch = wrap_touch(ctx);
-    if (gather == 1)
-      PMPM_LAUNCH((wrap_gather_list_kernel<2, 5>), (std::string("wrap_gather_list_kernel<2, 5>")), lgrid, block, 0,
-                  s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-    else
-      PMPM_LAUNCH((wrap_gather_list_kernel<2, 2>), (std::string("wrap_gather_list_kernel<2, 2>")), lgrid, block, 0,
-                  s, g, tg, ctx->partials, ctx->tile_flags, nodes, touch, ctx->wrap_list);
-    PMPM_LAUNCH_CHECK();
-    return PMPM_OK;
-  }
-  uint8_t *touch = nullptr;
-  const dim3 grid((unsigned)ceil_div(targets, 4)), block(256);  // one wave per target node
-  if (gather == 1)
-    PMPM_LAUNCH((wrap_gather_kernel<2, 5>), (std::string("wrap_gather_kernel<2, 5>")), grid, block, 0, s, g, tg,
-                ctx->partials, ctx->tile_flags, nodes, touch);
-  else
-    PMPM_LAUNCH((wrap_gather_kernel<2, 2>), (std::string("wrap_gather_kernel<2, 2>")), grid, block, 0, s, g, tg,
-                ctx->partials, ctx->tile_flags, nodes, touch);
-  PMPM_LAUNCH_CHECK();
-  return PMPM_OK;
-}
-
 
 // Scatter into the tile partials (+ wrap-around deposits into the cleared
 // node arrays); a grid_kernel pass with gather = 1 completes the P2G.
@@ -3083,10 +2207,9 @@ int do_p2g(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const 
   int rc = reserve_tiles(ctx, prm, g, s);
   if (rc != PMPM_OK) return rc;
   if (!zeroed && (rc = do_zero_nodes(prm, g, nodes, s)) != PMPM_OK) return rc;
-  PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags,
-                    ctx->wrap_rec, wrap_touch(ctx), ctx->wrap_list, s);
+  PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags, s);
   PMPM_LAUNCH_CHECK();
-  return launch_wrap_gather(ctx, prm, g, part, nodes, 1, s);
+  return PMPM_OK;
 }
 
 // True when a material of the list runs after G2P; then the particles must
@@ -3131,9 +2254,9 @@ int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
   // for the re-map's wrap-around atomics first
   if (!zeroed && (rc = zero_fill(nodes.mom_nt, (int64_t)g.num_cells_total * prm.dim, s)) != PMPM_OK) return rc;
   PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, in, out, part, nodes, 1, ctx->partials,
-                    ctx->tile_flags, ctx->wrap_rec, wrap_touch(ctx), ctx->wrap_list, s);
+                    ctx->tile_flags, s);
   PMPM_LAUNCH_CHECK();
-  return launch_wrap_gather(ctx, prm, g, part, nodes, 2, s);
+  return PMPM_OK;
 }
 
 }  // namespace pmpm
@@ -3481,7 +2604,7 @@ __device__ inline void store_node_adj(float *__restrict__ nbar, int node, float 
 // -> adjoints of mass, moment and force. Boundary conditions in reverse list
 // order with the forward's active sets, which the forward grid pass recorded
 // per node in `clamp` (components a NodeDomain condition set to zero).
-template <int D, class TG = TilesRuntime>
+template <int D, class TG>
 __global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, TileGeom tg,
                                     const float *__restrict__ partials, const int32_t *__restrict__ flags,
                                     const uint8_t *__restrict__ clamp, float *__restrict__ nbar) {
@@ -4246,7 +3369,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
     PMPM_LAUNCH_CHECK();
   }
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_p2g, *prm, g, *state, *state, *part, *nodes, 2, ctx->partials,
-                    ctx->tile_flags, nullptr, nullptr, nullptr, s, ctx->adj_rec);
+                    ctx->tile_flags, s, ctx->adj_rec);
   PMPM_LAUNCH_CHECK();
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
@@ -4256,9 +3379,9 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
               dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
   switch (D) {
-    case 1: PMPM_GRID_ADJOINT(1, TilesRuntime); break;
-    case 2: PMPM_GRID_ADJOINT(2, TilesRuntime); break;
-    default: PMPM_WITH_TILES3(tg, PMPM_GRID_ADJOINT, 3, ) break;
+    case 1: PMPM_WITH_ROWS(1, tg, PMPM_GRID_ADJOINT) break;
+    case 2: PMPM_WITH_ROWS(2, tg, PMPM_GRID_ADJOINT) break;
+    default: PMPM_WITH_TILES3(tg, PMPM_GRID_ADJOINT) break;
   }
 #undef PMPM_GRID_ADJOINT
   PMPM_LAUNCH_CHECK();
