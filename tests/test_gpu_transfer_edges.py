@@ -1,0 +1,61 @@
+"""GPU parity of the P2G tilings at their edges, against the CPU oracle: grids
+smaller than a tile, one cell more than a tile and ragged in every axis, cells
+with no, one, a few and many particles (several staging rounds), particles in
+every boundary cell (node windows that leave the grid and wrap around through
+the linear index, usl_inline.h:122-126) and left of the origin (listed in cell
+0 with a negative fraction, deposited over their own windows).
+Bar: field-scaled relative error after 3 steps against the FP32 oracle <= 1e-4,
+as the other multi-step runs, or four times the FP32 oracle's own error against
+the FP64 oracle where that is larger (isolated particles of the sparse grid
+leave nodes of tiny mass)."""
+import numpy as np
+import pytest
+
+from tests import scenarios as S
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+
+
+def _spec(cells, sf, musl, seed):
+    rng = np.random.default_rng(seed)
+    dim, h = len(cells), 0.1
+    span = np.array(cells) * h
+    n = min(3000, 6 * int(np.prod(cells)) + 5)
+    pos = rng.uniform(0.002, 1.0, size=(n, dim)) * (span - 0.004)
+    many = min(90, n // 2)  # a full cell
+    pos[:many] = (np.array(cells) // 2 + rng.uniform(0.05, 0.95, size=(many, dim))) * h
+    pos[many:many + 4, 0] = rng.uniform(-0.09, -0.001, 4)
+    # a particle in every corner cell
+    for k in range(2 ** dim):
+        corner = np.array([(k >> a) & 1 for a in range(dim)])
+        pos[many + 4 + k] = np.where(corner, span - 0.04, 0.03)
+    return S.Spec(dim=dim, origin=[0.0] * dim, end=list((np.array(cells) - 0.75) * h), cell_size=h, shape_function=sf,
+                  dt=1e-4, ppc=2, positions=pos, velocities=rng.normal(0.0, 0.2, size=(n, dim)),
+                  materials=[("LinearElastic", {"density": 1000.0, "E": 1e5, "pois": 0.3})],
+                  bcs=[("Gravity", {"gravity": [0.0] * (dim - 1) + [-9.81]})], musl=musl)
+
+
+@pytest.mark.parametrize("sf", ["linear", "quadratic", "cubic"])
+@pytest.mark.parametrize("musl", [False, True])
+@pytest.mark.parametrize("cells", [(3,), (64,), (129,), (2, 3), (4, 2), (16, 4), (17, 9), (33, 5), (2, 3, 2),
+                                   (4, 2, 4), (9, 5, 5), (19, 3, 6), (53, 51, 50)])
+def test_transfer_tile_edges(oracle_mod, cells, musl, sf):
+    spec = _spec(cells, sf, musl, 17 + sum(cells))
+    print(f"\n[gpu-test] transfer edges cells={cells} {sf} {'MUSL' if musl else 'USL'}", flush=True)
+    pm, solver = S.build_product(spec)
+    sims = [S.build_oracle(oracle_mod, spec, prec) for prec in ("f32", "f64")]
+    solver.solve_nsteps(3)
+    for sim in sims:
+        for _ in range(3):
+            sim.step()
+    got, ref, exact = S.product_state(solver), *[S.oracle_state(sim) for sim in sims]
+    for k in S.FIELDS:
+        e, bar = S.max_rel_err(got[k], ref[k]), max(1e-4, 4 * S.max_rel_err(ref[k], exact[k]))
+        assert e <= bar, (k, e, bar)
