@@ -59,3 +59,31 @@ def test_transfer_tile_edges(oracle_mod, cells, musl, sf):
     for k in S.FIELDS:
         e, bar = S.max_rel_err(got[k], ref[k]), max(1e-4, 4 * S.max_rel_err(ref[k], exact[k]))
         assert e <= bar, (k, e, bar)
+
+
+@pytest.mark.parametrize("lanes", ["1", "4"])
+@pytest.mark.parametrize("sf", ["linear", "quadratic"])
+def test_adjoint_p2g_other_splines(oracle_mod, monkeypatch, sf, lanes):
+    """The 3D adjoint step with the splines whose derivative enters as
+    differences (the differentiable column is cubic), in both lane layouts of
+    the adjoint P2G: <adjoint, direction> against the FP64 oracle's finite
+    difference, with that check's bar (2e-3)."""
+    from pyroclastmpm_amd import capi, diff
+    from tests import test_gpu_adjoint as A
+
+    monkeypatch.setenv("PMPM_ADJOINT_P2G_LANES", lanes)
+    cubic = diff.DiffMPM.params
+
+    def params(self, theta):
+        prm = cubic(self, theta)
+        prm.shape_fn, prm.node_types_built = capi.SF[sf], 0
+        return prm
+
+    monkeypatch.setattr(diff.DiffMPM, "params", params)
+
+    class Oracle:  # the column's oracle with this spline
+        def __getattr__(self, name):
+            return lambda origin, end, h, _, dt, ppc: getattr(oracle_mod, name)(origin, end, h, sf, dt, ppc)
+
+    pos, geo = A._column_3d(h=0.05, per_axis=3)
+    A._one_step_check(Oracle(), pos, geo, label=f"{sf}, lanes {lanes}")
