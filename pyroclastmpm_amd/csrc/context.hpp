@@ -18,7 +18,7 @@ struct pmpm_context {
   int32_t *vals_tmp = nullptr;   // radix sort ping-pong values
   uint32_t *hist = nullptr;      // [radix][blocks] digit histograms
   size_t hist_len = 0;
-  uint32_t *counters = nullptr;  // [4]: out-of-grid particles, hint unsorted flag (set, kept), heavy cells
+  uint32_t *counters = nullptr;  // [8]: out-of-grid particles, hint unsorted flag (set, kept), heavy cells, stray flags (2)
   bool counters_clear = false;   // cleared once, by the first call that uses them
   // P2G tile partials: per tile, the LDS node block of each accumulated field
   // (plain stores; the grid kernel sums the <= 2^D tiles covering a node)
@@ -26,6 +26,12 @@ struct pmpm_context {
   size_t partials_cap = 0;       // floats
   int32_t *tile_flags = nullptr;  // 1 = tile had particles this launch
   size_t tile_flags_cap = 0;
+  // P2G sums of particles deposited over their own windows (mass, momentum,
+  // force per node), zero but between a P2G pass that sets its flag
+  // (stray_flags: P2G, re-map) and the grid pass after it
+  float *strays = nullptr;
+  size_t strays_cap = 0;
+  int32_t *stray_flags = nullptr;  // in counters
   // a byte per node: the components the last grid pass's NodeDomain
   // condition set to zero (words of 4 bytes), read by the adjoint
   float *clamp_mask = nullptr;
@@ -167,9 +173,9 @@ bool params_ok(const pmpm_params *prm);
 bool step_args_ok(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *a, const pmpm_particles *b,
                   const pmpm_spatial *part, const pmpm_nodes *nodes);
 // Workspace the P2G passes of one step use on grid g: tile partials (floats)
-// and tile flags, the clamp record (words).
+// and tile flags, the clamp record and the stray sums (words).
 struct P2GWorkspace {
-  size_t partial_floats, tiles, clamp_words;
+  size_t partial_floats, tiles, clamp_words, stray_words;
 };
 void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w);
 // pmpm_partition whose first kernel also clears the buffers of `extra`.

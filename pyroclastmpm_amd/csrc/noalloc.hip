@@ -17,9 +17,10 @@ namespace {
 
 // The budget's partials (budget_bytes) are those of other tiles than the ones
 // in use, which take up to 2.6 times as much (a 2D grid of a single row, linear
-// splines: tiles are four rows high; 28/22 in 3D), so the array holds that much
-// more than the budget.
-constexpr size_t kScratchBytes = (size_t)PMPM_NOALLOC_SCRATCH_BYTES / 64 * 168;
+// splines: tiles are four rows high; 28/22 in 3D), and the stray sums are not in
+// it (half as much again there), so the array holds that much more than the
+// budget.
+constexpr size_t kScratchBytes = (size_t)PMPM_NOALLOC_SCRATCH_BYTES / 64 * 200;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -103,10 +104,11 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   const size_t o_keys = c.take(n * sizeof(uint32_t));
   const size_t o_vals = c.take(n * sizeof(int32_t));
   const size_t o_hist = c.take(hist_len * sizeof(uint32_t));
-  const size_t o_counters = c.take(4 * sizeof(uint32_t));
+  const size_t o_counters = c.take(8 * sizeof(uint32_t));
   const size_t o_partials = c.take(w.partial_floats * sizeof(float));
   const size_t o_flags = c.take(w.tiles * sizeof(int32_t));
   const size_t o_clamp = c.take(w.clamp_words * sizeof(float));
+  const size_t o_strays = c.take(w.stray_words * sizeof(float));
   if (budget_bytes(*prm, *grid, n, hist_len, w) > (size_t)PMPM_NOALLOC_SCRATCH_BYTES || c.used > kScratchBytes) {
     note_error("pmpm_step_noalloc: the step needs more workspace than PMPM_NOALLOC_SCRATCH_BYTES "
                "(fewer particles or a smaller grid, or pmpm_step with a context)");
@@ -134,6 +136,11 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   ctx.tile_flags_cap = w.tiles;
   ctx.clamp_mask = reinterpret_cast<float *>(base + o_clamp);
   ctx.clamp_mask_cap = w.clamp_words;
+  ctx.strays = reinterpret_cast<float *>(base + o_strays);
+  ctx.strays_cap = w.stray_words;
+  ctx.stray_flags = reinterpret_cast<int32_t *>(ctx.counters + 4);
+  // (the scratch holds whatever an earlier call left)
+  if ((rc = zero_fill(ctx.strays, (int64_t)w.stray_words, (hipStream_t)stream)) != PMPM_OK) return rc;
   // (the context is a plain struct on this stack frame: nothing frees the
   // scratch pieces it points at)
   return step_on(&ctx, prm, grid, musl, a, b, part, nodes, (hipStream_t)stream);

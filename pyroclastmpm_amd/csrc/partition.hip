@@ -651,7 +651,8 @@ extern "C" int pmpm_context_create(pmpm_context **ctx) {
   c->sort_by_hint = !(radix_only && radix_only[0] == '1');
   const char *hint_min = getenv("PMPM_PARTITION_HINT_MIN");
   if (hint_min && hint_min[0]) c->hint_min_particles = (int32_t)strtol(hint_min, nullptr, 10);
-  if (!hip_ok(hipMalloc(&c->counters, 4 * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
+  if (!hip_ok(hipMalloc(&c->counters, 8 * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
+  c->stray_flags = reinterpret_cast<int32_t *>(c->counters + 4);
   *ctx = c;
   return PMPM_OK;
 }
@@ -701,6 +702,7 @@ extern "C" int pmpm_context_destroy(pmpm_context *ctx) {
   (void)hipFree(ctx->vals_tmp);
   (void)hipFree(ctx->hist);
   (void)hipFree(ctx->counters);
+  (void)hipFree(ctx->strays);
   delete ctx;
   return PMPM_OK;
 }

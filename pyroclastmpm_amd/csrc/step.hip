@@ -15,7 +15,7 @@ int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
                 const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s,
                 bool zeroed);
 int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, int finalize,
-                int b0, int b1, int remap, int gather, hipStream_t s, int n, int clear_mom_nt);
+                int b0, int b1, int remap, int gather, hipStream_t s, int n, int skip_mom_nt);
 }  // namespace pmpm
 
 using namespace pmpm;
@@ -24,13 +24,9 @@ using namespace pmpm;
 int pmpm::step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, int32_t musl,
                   const pmpm_particles *a, pmpm_particles *b, pmpm_spatial *part, pmpm_nodes *nodes,
                   hipStream_t s) {
-  // the partition's first kernel also clears the node arrays P2G sums into,
-  // and in MUSL the first grid pass leaves mom_nt cleared for the re-map
-  const int64_t nn = grid->num_cells_total;
+  // the partition's first kernel also clears the P2G passes' stray flags
   ZeroLists z{};
-  z.add(nodes->mass, nn);
-  z.add(nodes->mom, nn * prm->dim);
-  z.add(nodes->mom_nt, nn * prm->dim);
+  z.add(ctx->stray_flags, 2);
   int rc = partition_clearing(ctx, prm->dim, grid, a->x, a->n, part, s, z);
   if (rc != PMPM_OK) return rc;
   if ((rc = do_p2g(ctx, *prm, *grid, *a, *part, *nodes, s, true)) != PMPM_OK) return rc;

@@ -305,8 +305,16 @@ template <int D> __device__ inline void node_ids32(const pmpm_grid &g, int lin, 
 // through the linear index (wrap-around reproduced when wrap_quirk is set).
 // Used for particles whose bin is not their cell's coordinates and for the
 // entries of boundary particles that leave the grid on some axis.
+// Sums of the particles deposited over their own windows (p2g_stray): node
+// arrays of their own, zero between the passes, and a flag the pass sets when
+// it added something. The grid pass reads (and clears) them only then, so the
+// node arrays are neither cleared before a step nor read by its first grid pass.
+struct Strays {
+  float *mass, *mom, *mom_nt;
+  int32_t *flag;
+};
 template <int D, int SF, int MODE>
-__device__ inline void scatter_entry_global(const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes,
+__device__ inline void scatter_entry_global(const pmpm_params &prm, const pmpm_grid &g, const Strays &nodes,
                                             int nn, const PW<D, SF> &w, const int *e, float m, const float *mv,
                                             const float A[3][3], const float *fext) {
   int nb[3] = {0, 0, 0}, off[3] = {0, 0, 0};
@@ -350,9 +358,9 @@ __device__ inline void scatter_entry_global(const pmpm_params &prm, const pmpm_g
 
 // P2G of a particle whose recomputed bin is not the cell it is listed in
 // (only possible when the partition was built from other positions): this
-// lane's y slice of its window goes straight to the node arrays.
+// lane's y slice of its window goes straight to the stray sums.
 template <int D, int SF, int MODE>
-__device__ void p2g_stray(const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, const float *x, int n,
+__device__ void p2g_stray(const pmpm_params &prm, const pmpm_grid &g, const Strays &nodes, const float *x, int n,
                           int slot, int sy, float m, const float *v, const Sym &A, const float *fext) {
   constexpr int E = Spline<SF>::ENTRIES;
   constexpr int EZ = D > 2 ? E : 1;
@@ -523,7 +531,7 @@ template <int D, int SF> struct RowGeom {
 // its own.
 template <int D, int SF, int MODE, bool FEXT = false>
 __global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
-    pmpm_params prm, pmpm_grid g, pmpm_particles in, pmpm_particles out, pmpm_spatial part, pmpm_nodes nodes,
+    pmpm_params prm, pmpm_grid g, pmpm_particles in, pmpm_particles out, pmpm_spatial part, Strays nodes,
     int tiles_x, float *__restrict__ partials, int32_t *__restrict__ flags, const float *__restrict__ rec) {
   using G = RowGeom<D, SF>;
   static_assert(D == 1 || D == 2, "3D passes are p2g_mfma_kernel's");
@@ -852,6 +860,7 @@ __global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
     }
   }
   if (MODE != 2 && strays) {
+    if (lane == 0) *nodes.flag = 1;
     // as in p2g_mfma_kernel: particles listed in this row but binned elsewhere
 #pragma unroll 1
     for (int k0 = 0; k0 < most; k0 += KW)
@@ -936,7 +945,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // zero; the carry out of y only changes the lane's own z type.
 template <int SF, int MODE, int CELLS, int ROWS, bool FEXT = false>
 __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles in,
-                                                       pmpm_particles out, pmpm_spatial part, pmpm_nodes nodes,
+                                                       pmpm_particles out, pmpm_spatial part, Strays nodes,
                                                        int tiles_x, int tiles_y, float *__restrict__ partials,
                                                        int32_t *__restrict__ flags, const float *__restrict__ rec) {
   constexpr int NV = p2g_nv<3, MODE>();
@@ -1266,9 +1275,10 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
     for (int y = 0; y < M::NY; ++y) slice[f * M::NTN + y * PL + i % PL] = sum[y];
   }
   if (MODE != 2 && strays) {
+    if (lane == 0) *nodes.flag = 1;
     // particles listed in this row but binned elsewhere (a partition of other
-    // positions): deposited over their own windows, straight to the node
-    // arrays (MODE 2 runs on a partition of the same positions). Walked again
+    // positions): deposited over their own windows, straight to the stray
+    // sums (MODE 2 runs on a partition of the same positions). Walked again
     // here, where the registers of the products are free.
 #pragma unroll 1
     for (int q0 = 0; q0 < total; q0 += 64) {
@@ -1309,6 +1319,9 @@ template <int D, int SPAN_, int CELLS_, int ROWS_> struct Tiles {
   static constexpr int T[3] = {CELLS_, ROWS_, D > 2 ? 4 : 1};
   static constexpr int N[3] = {CELLS_ + SPAN_ - 1, D > 1 ? ROWS_ + SPAN_ - 1 : 1, D > 2 ? 3 + SPAN_ : 1};
   static constexpr int COVER_Y = (N[1] - 1) / T[1] + 1;
+  // a wave of the grid pass takes 64 nodes of one tile, in the tile's order
+  static constexpr bool BRICKS = T[0] * T[1] * T[2] % 64 == 0;
+  static constexpr int WAVES = BRICKS ? T[0] * T[1] * T[2] / 64 : 1;
   static_assert((N[0] - 1) / T[0] + 1 <= kCoverX && COVER_Y <= kCoverY && (N[2] - 1) / T[2] + 1 <= kCoverZ,
                 "the gather visits at most kCover tiles per axis");
 };
@@ -1367,13 +1380,39 @@ __device__ inline bool gather_partials(const TileGeom &tg, const float *partials
   return true;
 }
 
+// The node of thread t of a pass over all nodes (false: none). With tiles of
+// at least 64 cells a wave takes 64 nodes of one tile, so that the slice rows
+// its lanes read are the same or neighbours (64 nodes of one x row read a
+// 44-byte row of each of eight slices instead); with small tiles t is the
+// node's linear index.
+template <int D, class TG>
+__device__ inline bool pass_node(const pmpm_grid &g, const TileGeom &tg, int t, int *ids) {
+  if constexpr (TG::BRICKS) {
+    const int w = t >> 6;
+    int b = w / TG::WAVES, l = (w % TG::WAVES) * 64 + (t & 63);
+    if (b >= tg.tiles[0] * tg.tiles[1] * tg.tiles[2]) return false;
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      ids[a] = (a < D - 1 ? b % tg.tiles[a] : b) * TG::T[a] + l % TG::T[a];
+      b /= tg.tiles[a];
+      l /= TG::T[a];
+      in = in && ids[a] < g.num_cells[a];
+    }
+    return in;
+  } else {
+    if (t >= g.num_cells_total) return false;
+    node_ids32<D>(g, t, ids);
+    return true;
+  }
+}
 // Per node: cutoff + forward moment (finalize), boundary conditions
 // [bc_begin, bc_end) in list order, then the node velocities G2P reads.
 // remap_pass: mom_nt holds the MUSL re-mapped momentum; only kinematic
 // conditions apply (gravity already acted through the particle velocities).
-// clear_mom_nt: mom_nt is left at zero instead of the forward moment (the
-// MUSL step's first pass: the re-map accumulates into it next, and nothing
-// reads the forward moment but the velocity records written here).
+// skip_mom_nt: mom_nt is not written (the MUSL step's first pass: nothing reads
+// the forward moment but the velocity records written here, and the re-map's
+// pass writes it next).
 // clamp (optional): per node, the components a NodeDomain condition set to
 // zero (bit a: moment, bit 3 + a: forward moment; a slip clamp counts when
 // its input was not on the kept side), for the adjoint.
@@ -1434,28 +1473,35 @@ __device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, con
 template <int D, int GATHER, class TG>
 __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int finalize, int bc_begin, int bc_end,
                             int remap_pass, TileGeom tg, const float *__restrict__ partials,
-                            const int32_t *__restrict__ flags, int clear_mom_nt, uint8_t *__restrict__ clamp,
-                            int nwrap) {
+                            const int32_t *__restrict__ flags, int skip_mom_nt, uint8_t *__restrict__ clamp,
+                            int nwrap, Strays strays) {
   const int nn = g.num_cells_total;
-  int i = ((int)blockIdx.x - nwrap) * blockDim.x + threadIdx.x;
-  int ids0[3] = {0, 0, 0};
+  int i, ids0[3] = {0, 0, 0};
   bool reached = false;  // a node the wrap-around can reach
   if (D > 1 && (int)blockIdx.x < nwrap) {
     const int t = (blockIdx.x * blockDim.x + threadIdx.x) / kImageLanes;
     if (t >= wrap_target_count<D>(g) || !wrap_target<D>(g, t, ids0)) return;  // (a node's lanes together)
-    i = ids0[0] + g.num_cells[0] * (ids0[1] + (D > 2 ? g.num_cells[1] * ids0[2] : 0));
     reached = true;
   } else {
-    if (i >= nn) return;
-    node_ids32<D>(g, i, ids0);
+    if (!pass_node<D, TG>(g, tg, ((int)blockIdx.x - nwrap) * (int)blockDim.x + (int)threadIdx.x, ids0)) return;
     if (D > 1 && nwrap > 0 &&
         (ids0[0] <= 1 || ids0[0] == g.num_cells[0] - 1 || (D > 2 && (ids0[1] <= 1 || ids0[1] == g.num_cells[1] - 1))))
       return;
   }
-  float m = nodes.mass[i];
-  float P[3] = {0.f, 0.f, 0.f}, Q[3] = {0.f, 0.f, 0.f};
-  if constexpr (GATHER != 0) {
-    // node arrays hold the deposits of stray particles; add the tile partials
+  i = ids0[0] + (D > 1 ? g.num_cells[0] * (ids0[1] + (D > 2 ? g.num_cells[1] * ids0[2] : 0)) : 0);
+  // GATHER 1: mass, momentum and force are the sums gathered here; 2: the
+  // momentum mom_nt is; the rest (0: all) comes from the node arrays
+  float m = 0.f, P[3] = {0.f, 0.f, 0.f}, Q[3] = {0.f, 0.f, 0.f};
+  if constexpr (GATHER != 1) {
+    m = nodes.mass[i];
+#pragma unroll
+    for (int a = 0; a < D; ++a) P[a] = nodes.mom[a * nn + i];
+  }
+  const float P0[3] = {P[0], P[1], P[2]};
+  if constexpr (GATHER == 0) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) Q[a] = nodes.mom_nt[a * nn + i];
+  } else {
     constexpr int NV = GATHER == 1 ? 1 + 2 * D : D;
     float acc[NV];
 #pragma unroll
@@ -1469,17 +1515,25 @@ __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g,
     } else {
       gather_partials<D, NV, TG>(tg, partials, flags, ids0, acc);
     }
+    if (*strays.flag) {
+      float *a0 = GATHER == 1 ? strays.mass : strays.mom_nt;  // (mass, mom and mom_nt lie one after the other)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        acc[k] += a0[(int64_t)k * nn + i];
+        a0[(int64_t)k * nn + i] = 0.f;
+      }
+    }
     if constexpr (GATHER == 1) {
-      m += acc[0];
+      m = acc[0];
 #pragma unroll
       for (int a = 0; a < D; ++a) {
-        nodes.mom[a * nn + i] += acc[1 + a];
-        nodes.mom_nt[a * nn + i] += acc[1 + D + a];
+        P[a] = acc[1 + a];
+        Q[a] = acc[1 + D + a];
       }
-      nodes.mass[i] = m;
+      if (!(m <= prm.small_mass_cutoff)) nodes.mass[i] = m;  // (else written below)
     } else {
 #pragma unroll
-      for (int a = 0; a < D; ++a) nodes.mom_nt[a * nn + i] += acc[a];
+      for (int a = 0; a < D; ++a) Q[a] = acc[a];
     }
   }
   if ((finalize || remap_pass) && m <= prm.small_mass_cutoff) {
@@ -1506,11 +1560,6 @@ __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g,
     const float z[3] = {0.f, 0.f, 0.f};
     store_node_vel<D>(nodes.vel, i, z, z);
     return;
-  }
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    P[a] = nodes.mom[a * nn + i];
-    Q[a] = nodes.mom_nt[a * nn + i];
   }
   if (finalize) {
 #pragma unroll
@@ -1626,8 +1675,8 @@ __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g,
   }
 #pragma unroll
   for (int a = 0; a < D; ++a) {
-    nodes.mom[a * nn + i] = P[a];
-    nodes.mom_nt[a * nn + i] = clear_mom_nt ? 0.f : Q[a];
+    if (GATHER != 2 || P[a] != P0[a]) nodes.mom[a * nn + i] = P[a];  // (the re-map's pass rarely changes it)
+    if (!skip_mom_nt) nodes.mom_nt[a * nn + i] = Q[a];
   }
   if (clamp) clamp[i] = (uint8_t)cbits;
   const bool live = m > prm.small_mass_cutoff;
@@ -2051,13 +2100,13 @@ static size_t tile_count(const TileGeom &tg) { return (size_t)tg.tiles[0] * tg.t
 
 template <int SF, int CELLS, int ROWS>
 static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
-                            const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, int mode,
+                            const pmpm_particles &out, const pmpm_spatial &part, const Strays &strays, int mode,
                             float *partials, int32_t *flags, hipStream_t s, const float *rec) {
   const TileGeom mg = mfma_tile_geom(SF, g, mode + 1, MfmaTiles{CELLS, ROWS});
   const dim3 grid((unsigned)tile_count(mg)), block(256 * ROWS);
 #define PMPM_MFMA(MODE, FEXT, ...)                                                                               \
   PMPM_LAUNCH((p2g_mfma_kernel<SF, MODE, CELLS, ROWS, FEXT>), (::pmpm::kname("p2g_mfma_kernel", {__VA_ARGS__})), \
-              grid, block, 0, s, prm, g, in, out, part, nodes, mg.tiles[0], mg.tiles[1], partials, flags, rec)
+              grid, block, 0, s, prm, g, in, out, part, strays, mg.tiles[0], mg.tiles[1], partials, flags, rec)
   if (mode == 0 && has_planar(prm)) PMPM_MFMA(0, true, (long)SF, 0L, 1L);
   else if (mode == 0) PMPM_MFMA(0, false, (long)SF, 0L);
   else if (mode == 1) PMPM_MFMA(1, false, (long)SF, 1L);
@@ -2071,22 +2120,22 @@ static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pm
 template <int D, int SF>
 void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in, const pmpm_particles &out,
                 const pmpm_spatial &part, const pmpm_nodes &nodes, int mode, float *partials, int32_t *flags,
-                hipStream_t s, const float *rec = nullptr) {
+                const Strays &strays, hipStream_t s, const float *rec = nullptr) {
   if (mode == 2 && !rec) return;
   if (mode == 1 && in.n > 0)
     PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})),
                 dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0, s, prm, g, in, out, part, nodes, 1);
   if constexpr (D == 3) {
     if (mfma_tiles(g, in.n).cells == 4)
-      launch_p2g_mfma<SF, 4, 1>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+      launch_p2g_mfma<SF, 4, 1>(prm, g, in, out, part, strays, mode, partials, flags, s, rec);
     else
-      launch_p2g_mfma<SF, 8, 2>(prm, g, in, out, part, nodes, mode, partials, flags, s, rec);
+      launch_p2g_mfma<SF, 8, 2>(prm, g, in, out, part, strays, mode, partials, flags, s, rec);
   } else {
     const TileGeom tg = row_tile_geom<D, SF>(g, mode + 1);
     const dim3 grid((unsigned)tile_count(tg)), block(RowGeom<D, SF>::THREADS);
 #define PMPM_ROWS(MODE, FEXT, ...)                                                                                 \
   PMPM_LAUNCH((p2g_rows_kernel<D, SF, MODE, FEXT>), (::pmpm::kname("p2g_rows_kernel", {(long)D, __VA_ARGS__})),    \
-              grid, block, 0, s, prm, g, in, out, part, nodes, tg.tiles[0], partials, flags, rec)
+              grid, block, 0, s, prm, g, in, out, part, strays, tg.tiles[0], partials, flags, rec)
     if (mode == 0 && has_planar(prm)) PMPM_ROWS(0, true, (long)SF, 0L, 1L);
     else if (mode == 0) PMPM_ROWS(0, false, (long)SF, 0L);
     else if (mode == 1) PMPM_ROWS(1, false, (long)SF, 1L);
@@ -2109,12 +2158,23 @@ void launch_shape(const pmpm_grid &g, int types_built, const float *x, int n, fl
                      x, n, psi, dpsi);
 }
 
-// gather: 0 = node arrays only, 1 = add the P2G tile partials, 2 = add the
-// MUSL re-map tile partials (ctx holds them) of a pass over n particles.
+// Workgroups of 256 threads of a pass over all nodes (pass_node).
+static unsigned pass_blocks(const pmpm_grid &g, const TileGeom &tg) {
+  const int64_t cells = (int64_t)tg.T[0] * tg.T[1] * tg.T[2];
+  return (unsigned)ceil_div(cells % 64 == 0 ? (int64_t)tile_count(tg) * cells : (int64_t)g.num_cells_total, (int64_t)256);
+}
+// The stray sums of a P2G (mode 0) or re-map (mode 1) pass.
+static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, int mode) {
+  const int64_t nn = g.num_cells_total;
+  return {ctx->strays, ctx->strays + nn, ctx->strays + (1 + prm.dim) * nn, ctx->stray_flags + (mode == 1)};
+}
+// gather: 0 = node arrays only, 1 = from the P2G tile partials, 2 = mom_nt from
+// the MUSL re-map tile partials (ctx holds them) of a pass over n particles.
 int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, int finalize,
-                int b0, int b1, int remap, int gather, hipStream_t s, int n, int clear_mom_nt = 0) {
-  const unsigned blocks = (unsigned)ceil_div(g.num_cells_total, 256);
-  TileGeom tg = tile_geom(prm, g, gather, n);
+                int b0, int b1, int remap, int gather, hipStream_t s, int n, int skip_mom_nt = 0) {
+  const TileGeom tg = tile_geom(prm, g, gather, n);
+  const unsigned blocks = pass_blocks(g, tg);
+  const Strays strays = gather ? stray_sums(ctx, prm, g, gather - 1) : Strays{};
   const float *partials = gather ? ctx->partials : nullptr;
   const int32_t *flags = gather ? ctx->tile_flags : nullptr;
   // the clamp record of a pass that applies node conditions (not the MUSL
@@ -2129,7 +2189,7 @@ int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
 #define PMPM_GRID_LAUNCH(...)                                                                                          \
   PMPM_LAUNCH((grid_kernel<__VA_ARGS__>), (::pmpm::kname("grid_kernel", {(long)prm.dim}) + " gather " + std::to_string(gather)), \
               dim3(blocks + (unsigned)nwrap), dim3(256), 0, s, prm, g, nodes, finalize, b0, b1, remap, tg, partials, flags,      \
-              clear_mom_nt, clamp, nwrap)
+              skip_mom_nt, clamp, nwrap, strays)
 #define PMPM_GRID_GATHER(D, ...)                                 \
   if (gather == 0) PMPM_GRID_LAUNCH(D, 0, __VA_ARGS__);          \
   else if (gather == 1) PMPM_GRID_LAUNCH(D, 1, __VA_ARGS__);     \
@@ -2161,17 +2221,6 @@ static bool particles_ok(const pmpm_particles *p) {
                         p->flags && p->id));
 }
 
-int do_zero_nodes(const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, hipStream_t s) {
-  int rc;
-  const int64_t nn = g.num_cells_total;
-  ZeroLists z{};
-  z.add(nodes.mass, nn);
-  z.add(nodes.mom, nn * prm.dim);
-  z.add(nodes.mom_nt, nn * prm.dim);
-  if ((rc = zero_fill_lists(z, s)) != PMPM_OK) return rc;
-  return PMPM_OK;
-}
-
 // Partials and tile flags of the P2G passes on grid g, for any particle count
 // (a small grid's passes use either tile width).
 static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, size_t *floats, size_t *tiles) {
@@ -2190,24 +2239,32 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   // the grid pass's clamp record (one byte per node, in words of 4)
   if ((rc = ensure_buffer(ctx->clamp_mask, ctx->clamp_mask_cap, ((size_t)g.num_cells_total + 3) / 4)) != PMPM_OK)
     return rc;
+  // the stray sums are zero whenever no pass is under way
+  const size_t words = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
+  if (words > ctx->strays_cap) {
+    if ((rc = ensure_buffer(ctx->strays, ctx->strays_cap, words)) != PMPM_OK) return rc;
+    if ((rc = zero_fill(ctx->strays, (int64_t)words, s)) != PMPM_OK) return rc;
+  }
   return PMPM_OK;
 }
 
 void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w) {
   *w = P2GWorkspace{};
   partial_sizes(prm, g, &w->partial_floats, &w->tiles);
+  w->stray_words = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
   w->clamp_words = ((size_t)g.num_cells_total + 3) / 4;
 }
 
-// Scatter into the tile partials (+ wrap-around deposits into the cleared
-// node arrays); a grid_kernel pass with gather = 1 completes the P2G.
-// (zeroed: the caller has already cleared mass, mom and mom_nt)
+// Scatter into the tile partials (and the stray sums); a grid_kernel pass with
+// gather = 1 completes the P2G. (zeroed: the caller has already cleared the
+// stray flag)
 int do_p2g(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &p,
            const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s, bool zeroed = false) {
   int rc = reserve_tiles(ctx, prm, g, s);
   if (rc != PMPM_OK) return rc;
-  if (!zeroed && (rc = do_zero_nodes(prm, g, nodes, s)) != PMPM_OK) return rc;
-  PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags, s);
+  if (!zeroed && (rc = zero_fill(ctx->stray_flags, 1, s)) != PMPM_OK) return rc;
+  PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags,
+                    stray_sums(ctx, prm, g, 0), s);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -2244,17 +2301,15 @@ int do_g2p(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
 
 // First map (x, v into `out` in cell order) + re-map of m v into the tile
 // partials; a grid_kernel pass with gather = 2 completes mom_nt.
-// (zeroed: mom_nt is already zero, left so by the grid pass before)
+// (zeroed: as do_p2g)
 int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in,
                 const pmpm_particles &out, const pmpm_spatial &part, const pmpm_nodes &nodes, hipStream_t s,
                 bool zeroed = false) {
   int rc = reserve_tiles(ctx, prm, g, s);
   if (rc != PMPM_OK) return rc;
-  // the fused pass reads the node velocity records, never mom_nt: clear it
-  // for the re-map's wrap-around atomics first
-  if (!zeroed && (rc = zero_fill(nodes.mom_nt, (int64_t)g.num_cells_total * prm.dim, s)) != PMPM_OK) return rc;
+  if (!zeroed && (rc = zero_fill(ctx->stray_flags + 1, 1, s)) != PMPM_OK) return rc;
   PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, in, out, part, nodes, 1, ctx->partials,
-                    ctx->tile_flags, s);
+                    ctx->tile_flags, stray_sums(ctx, prm, g, 1), s);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -2609,10 +2664,9 @@ __global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm
                                     const float *__restrict__ partials, const int32_t *__restrict__ flags,
                                     const uint8_t *__restrict__ clamp, float *__restrict__ nbar) {
   const int nn = g.num_cells_total;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nn) return;
-  int ids[3];
-  node_ids32<D>(g, i, ids);
+  int ids[3] = {0, 0, 0};
+  if (!pass_node<D, TG>(g, tg, (int)(blockIdx.x * blockDim.x + threadIdx.x), ids)) return;
+  const int i = ids[0] + (D > 1 ? g.num_cells[0] * (ids[1] + (D > 2 ? g.num_cells[1] * ids[2] : 0)) : 0);
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   gather_partials<D, 2 * D, TG>(tg, partials, flags, ids, acc);
   const float m = nodes.mass[i];
@@ -3369,12 +3423,12 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
     PMPM_LAUNCH_CHECK();
   }
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_p2g, *prm, g, *state, *state, *part, *nodes, 2, ctx->partials,
-                    ctx->tile_flags, s, ctx->adj_rec);
+                    ctx->tile_flags, stray_sums(ctx, *prm, g, 0), s, ctx->adj_rec);
   PMPM_LAUNCH_CHECK();
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
   const TileGeom tg = tile_geom(*prm, g, 3, n);
-  const unsigned nblocks = (unsigned)ceil_div(g.num_cells_total, 256);
+  const unsigned nblocks = pass_blocks(g, tg);
 #define PMPM_GRID_ADJOINT(...)                                                                                   \
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
               dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
