@@ -1728,7 +1728,7 @@ __device__ inline int block_inclusive_sum(int v, int *wave_sum, int *total) {
     if (lane >= o) v += u;
   }
   if (lane == 63) wave_sum[wv] = v;
-  __syncthreads();
+  lds_barrier();
   int before = 0, all = 0;
 #pragma unroll
   for (int k = 0; k < kG2PThreads / 64; ++k) {
@@ -1758,7 +1758,7 @@ __device__ inline void g2p_gather_staged(const pmpm_grid &g, const pmpm_nodes &n
 #pragma unroll
     for (int a = 0; a < 3; ++a) rb[a * kG2PThreads + t] = w.bin[a];
   }
-  __syncthreads();
+  lds_barrier();
   // does a run start at lane q (after lane q - 1)?
   auto starts_at = [&](int q) {
     const int p0 = rb[q - 1], q0 = rb[q];
@@ -1778,12 +1778,12 @@ __device__ inline void g2p_gather_staged(const pmpm_grid &g, const pmpm_nodes &n
     R.x0[k] = w.bin[0];
   }
   if (end) R.x1[k] = w.bin[0];
-  __syncthreads();
+  lds_barrier();
   const int cnt = t < nruns ? 16 * (R.x1[t] - R.x0[t] + 4) : 0;
   int all = 0;
   const int incl = block_inclusive_sum(cnt, R.wave_sum, &all);
   if (t < nruns) R.base[t] = incl - cnt;
-  __syncthreads();
+  lds_barrier();
   const int myk = valid ? k : -1;
   for (int k0 = 0; k0 < nruns;) {
     const int b0 = R.base[k0];
@@ -1806,14 +1806,14 @@ __device__ inline void g2p_gather_staged(const pmpm_grid &g, const pmpm_nodes &n
         box2[q] = make_float2(b.x, b.y);
       }
     }
-    __syncthreads();
+    lds_barrier();
     if (myk >= k0 && myk < k1) {
       const int off = R.base[myk] - b0, X = R.x1[myk] - R.x0[myk] + 4;
       NodeSrc src{nodes.vel, box4 + off, box2 + off, {1, X, 4 * X}, {R.x0[myk] - 1, 0, 0}};
       gather_grid<D, SF, WANT_DV, WANT_L, true>(g, src, w, vinc, dvinc, L);
     }
     k0 = k1;
-    __syncthreads();  // the next round overwrites the staging
+    lds_barrier();  // the next round overwrites the staging
   }
 }
 
@@ -1833,6 +1833,28 @@ __global__ __launch_bounds__(kG2PThreads) void g2p_kernel(pmpm_params prm, pmpm_
   PW<D, SF> w;
   float xp[3];
   if (valid) particle_weights<D, SF>(prm, g, in.x, n, src, w, xp);
+  // The USL pass loads the particle's fields before the gather, whose barriers
+  // wait for LDS only: their latency passes behind it (3,276,800 particles:
+  // 245 -> 223 us). The MUSL second map loads them after it: its occupancy is
+  // worth more (1,080,000 particles: 65 us so, 70 us the other way).
+  float v0[3] = {0.f, 0.f, 0.f}, Fo[9], vol0 = 0.f, mass = 0.f;
+  int color = 0;
+  uint8_t pf = 0;
+  Sym s = sym_zero(), eps = sym_zero();
+  auto load_fields = [&]() {
+#pragma unroll
+    for (int k = 0; k < D * D; ++k) Fo[k] = in.F[k * n + src];
+    vol0 = in.volume0[src];
+    mass = in.mass[src];
+    color = in.color[src];
+    pf = in.flags[src];
+    s = load_sym(in.stress, n, src);
+  };
+  if (valid && MODE != 2) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) v0[a] = in.v[a * n + src];
+  }
+  if (valid && MODE == 0) load_fields();
   float vinc[3] = {0.f, 0.f, 0.f}, dvinc[3] = {0.f, 0.f, 0.f};
   float L[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if constexpr (D == 3) {
@@ -1849,15 +1871,14 @@ __global__ __launch_bounds__(kG2PThreads) void g2p_kernel(pmpm_params prm, pmpm_
     const float am = (float)(1.0 - (double)prm.alpha);
 #pragma unroll
     for (int a = 0; a < D; ++a) {
-      out.v[a * n + to] = am * vinc[a] + prm.alpha * (in.v[a * n + src] + dvinc[a]);
+      out.v[a * n + to] = am * vinc[a] + prm.alpha * (v0[a] + dvinc[a]);
       out.x[a * n + to] = xp[a] + prm.dt * vinc[a];
     }
     if (MODE == 1) return;
   }
+  if (MODE == 2) load_fields();
   // F = (I + L dt) F, V = det(F) V0
-  float Fo[9], Fn[9];
-#pragma unroll
-  for (int k = 0; k < D * D; ++k) Fo[k] = in.F[k * n + src];
+  float Fn[9];
 #pragma unroll
   for (int a = 0; a < D; ++a)
 #pragma unroll
@@ -1867,7 +1888,6 @@ __global__ __launch_bounds__(kG2PThreads) void g2p_kernel(pmpm_params prm, pmpm_
       for (int k = 0; k < D; ++k) acc += ((a == k ? 1.f : 0.f) + L[3 * a + k] * prm.dt) * Fo[k * D + b];
       Fn[a * D + b] = acc;
     }
-  const float vol0 = in.volume0[src];
   const float vol = det_dd<D>(Fn) * vol0;
 #pragma unroll
   for (int k = 0; k < D * D; ++k) out.F[k * n + dst] = Fn[k];
@@ -1879,11 +1899,7 @@ __global__ __launch_bounds__(kG2PThreads) void g2p_kernel(pmpm_params prm, pmpm_
       for (int b = 0; b < D; ++b) out.L[(a * D + b) * n + dst] = L[3 * a + b];
   }
   // return map of the particle's material
-  const int color = in.color[src];
-  const uint8_t pf = in.flags[src];
-  const float mass = in.mass[src];
-  Sym s = load_sym(in.stress, n, src);
-  Sym eps = in.eps_e ? load_sym(in.eps_e, n, src) : sym_zero();
+  if (in.eps_e) eps = load_sym(in.eps_e, n, src);
   Sym sref = sym_zero();
   if (in.stress_ref && color < prm.num_materials && (prm.materials[color].flags & PMPM_MATF_HAS_STRESS_REF))
     sref = load_sym(in.stress_ref, n, src);
@@ -2459,7 +2475,7 @@ __device__ inline float wave_sum(float v) {
 // Per particle (cell order j, state slot src): return-map VJP, F, v, x, and
 // the records (vpic adjoint, FLIP adjoint, L adjoint) for the node scatter.
 template <int D, int SF>
-__global__ __launch_bounds__(256) void g2p_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles st,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? 4 : 1))) void g2p_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles st,
                                                           pmpm_adjoint ob, pmpm_adjoint ib, pmpm_spatial part,
                                                           pmpm_nodes nodes, float *__restrict__ rec,
                                                           float *__restrict__ pbar) {
@@ -2473,19 +2489,11 @@ __global__ __launch_bounds__(256) void g2p_adjoint_kernel(pmpm_params prm, pmpm_
   PW<D, SF> w;
   float xp[3];
   if (valid) particle_weights<D, SF>(prm, g, st.x, n, src, w, xp);
-  float vpic[3] = {0.f, 0.f, 0.f}, dvp[3] = {0.f, 0.f, 0.f};
-  float L[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if constexpr (D == 3) {  // the forward G2P's gather, node rows staged in LDS
-    static_assert(kG2PThreads == 256, "the workgroup of the staged gather");
-    __shared__ __attribute__((aligned(16))) char lds[g2p_stage_bytes<true>()];
-    const int nv = min(n - (int)blockIdx.x * kG2PThreads, kG2PThreads);
-    g2p_gather_staged<D, SF, true, true>(g, nodes, w, nv, lds, vpic, dvp, L);
-  } else if (valid) {
-    gather_grid<D, SF, true, true>(g, node_src(g, nodes), w, vpic, dvp, L);
-  }
+  // (loaded before the gather, whose barriers wait for LDS only, at four waves
+  // per SIMD: 1,080,000 particles 123 -> 110 us)
+  float xo[3] = {0.f, 0.f, 0.f}, vo[3] = {0.f, 0.f, 0.f}, Fo[9], F[9], so6[6], eo6[6], s6[6], e6[6], sr6[6];
+  uint8_t pf = 0;
   if (valid) {
-
-    float xo[3] = {0.f, 0.f, 0.f}, vo[3] = {0.f, 0.f, 0.f}, Fo[9], F[9], so6[6], eo6[6], s6[6], e6[6], sr6[6];
 #pragma unroll
     for (int a = 0; a < D; ++a) {
       xo[a] = ob.x[a * n + j];
@@ -2505,8 +2513,19 @@ __global__ __launch_bounds__(256) void g2p_adjoint_kernel(pmpm_params prm, pmpm_
       sr6[k] = 0.f;
     }
     color = st.color[src];
-    const uint8_t pf = st.flags[src];
-
+    pf = st.flags[src];
+  }
+  float vpic[3] = {0.f, 0.f, 0.f}, dvp[3] = {0.f, 0.f, 0.f};
+  float L[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if constexpr (D == 3) {  // the forward G2P's gather, node rows staged in LDS
+    static_assert(kG2PThreads == 256, "the workgroup of the staged gather");
+    __shared__ __attribute__((aligned(16))) char lds[g2p_stage_bytes<true>()];
+    const int nv = min(n - (int)blockIdx.x * kG2PThreads, kG2PThreads);
+    g2p_gather_staged<D, SF, true, true>(g, nodes, w, nv, lds, vpic, dvp, L);
+  } else if (valid) {
+    gather_grid<D, SF, true, true>(g, node_src(g, nodes), w, vpic, dvp, L);
+  }
+  if (valid) {
     // return map (stress and elastic strain pass through unless updated)
     float Lb[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sb6[6], eb6[6];
 #pragma unroll
@@ -2732,9 +2751,9 @@ template <int D> __device__ inline void cofactor(const float *F, float *C) {
 // and velocity record (8 floats) of each. A node outside the grid carries the
 // adjoint of the node its linear index reaches (the wrap-around deposit's; zero
 // if none, or without wrap_quirk) and zero velocities (G2P never reads it).
-// gather(adj, vel, box0, X) is called by every live thread in the round that
-// holds its run: the node of window offset (ex, sy, sz) from bin - 1 is box0 +
-// ex + X (sy + 4 sz) of adj and vel. Every thread of the workgroup calls this
+// gather(rec, dvz, box0, X) is called by every live thread in the round that
+// holds its run: the node of window offset (ex, sy, sz) from bin - 1 is entry
+// box0 + ex + X (sy + 4 sz) of rec (three float4) and dvz. Every thread of the workgroup calls this
 // (barriers); `live` is false past the particles.
 constexpr int kAdjStageNodes = 576;  // 16 x 36: one run always fits
 static_assert(kAdjStageNodes >= 16 * (32 + 3), "a run spans at most 32 x bins");
@@ -2747,9 +2766,13 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
                                             const float *__restrict__ nbar, const int *bin, bool live,
                                             bool wrap_quirk, F &&gather) {
   constexpr int CAP = kAdjStageNodes, PPB = kG2PThreads / LANES;
-  __shared__ float4 s_adj[CAP * 2], s_vel[CAP * 2];
+  // a node's 13 floats: mass and momentum adjoint, force adjoint and v.x, (v.y,
+  // v.z, dv.x, dv.y); dv.z (packed so: four workgroups' staging per CU)
+  __shared__ float4 s_rec[CAP * 3];
+  __shared__ float s_dvz[CAP];
   __shared__ AdjRunTable R;
-  __shared__ int rb[3][PPB];
+  static_assert(CAP * 48 >= 3 * PPB * 4, "the lane bins fit the staging");
+  int(*rb)[PPB] = reinterpret_cast<int(*)[PPB]>(s_rec);  // before staging
   const int t = (int)threadIdx.x, pl = t / LANES;
   const bool lead = t % LANES == 0;  // the particle's first lane
   if (lead) {
@@ -2774,12 +2797,12 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
     R.x0[k] = bin[0];
   }
   if (end) R.x1[k] = bin[0];
-  __syncthreads();
+  lds_barrier();
   const int cnt = t < nruns ? 16 * (R.x1[t] - R.x0[t] + 4) : 0;
   int all = 0;
   const int incl = block_inclusive_sum(cnt, R.wave_sum, &all);
   if (t < nruns) R.base[t] = incl - cnt;
-  __syncthreads();
+  lds_barrier();
   const int myk = live ? k : -1;
   const int nx = g.num_cells[0], ny = g.num_cells[1], nz = g.num_cells[2];
   for (int k0 = 0; k0 < nruns;) {  // uniform over the workgroup
@@ -2801,18 +2824,18 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
       const float4 *vr = reinterpret_cast<const float4 *>(nodes.vel + 8 * node);
       const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
       const float4 a0 = ar[0], a1 = ar[1], v0 = vr[0], v1 = vr[1];
-      s_adj[2 * q] = reaches ? a0 : z4;
-      s_adj[2 * q + 1] = reaches ? a1 : z4;
-      s_vel[2 * q] = in ? v0 : z4;
-      s_vel[2 * q + 1] = in ? v1 : z4;
+      s_rec[3 * q] = reaches ? a0 : z4;
+      s_rec[3 * q + 1] = make_float4(reaches ? a1.x : 0.f, reaches ? a1.y : 0.f, reaches ? a1.z : 0.f, in ? v0.x : 0.f);
+      s_rec[3 * q + 2] = in ? make_float4(v0.y, v0.z, v0.w, v1.x) : z4;
+      s_dvz[q] = in ? v1.y : 0.f;
     }
-    __syncthreads();
+    lds_barrier();
     if (myk >= k0 && myk < k1) {
       const int off = R.base[myk] - b0, X = R.x1[myk] - R.x0[myk] + 4;
-      gather(s_adj, s_vel, off + (bin[0] - R.x0[myk]), X);
+      gather(s_rec, s_dvz, off + (bin[0] - R.x0[myk]), X);
     }
     k0 = k1;
-    __syncthreads();  // the next round overwrites the staging
+    lds_barrier();  // the next round overwrites the staging
   }
 }
 
@@ -2822,6 +2845,8 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
 // and the sums over the window contract x first (weights N, dN, d2N of gs, wv,
 // P_bar, f_bar as each needs them), then y, then z: about 3,400 multiply-adds
 // per particle instead of 4,500 with a product of three weights per entry.
+// Bound by vector issue (1,080,000 particles: 230 us, of which 136 us are issue
+// at three waves per SIMD; capped to 128 registers for four it spills, 272 us).
 // LANES = 1: a lane per particle; 4: a lane per z layer of the window, for
 // launches too small to fill the chip otherwise.
 // Wrap-around entries (deposit only): a node outside the grid holds the adjoint
@@ -2945,7 +2970,7 @@ __global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm
       w2 = pick(d2N[a], e);
     }
   };
-  adjoint_stage_rounds<LANES>(g, nodes, nbar, bin, live, quirk, [&](const float4 *adj, const float4 *vel, int box0,
+  adjoint_stage_rounds<LANES>(g, nodes, nbar, bin, live, quirk, [&](const float4 *nrec, const float *dvz, int box0,
                                                                    int X) {
     const int at0 = box0 + (first[0] + 1) + X * ((first[1] + 1) + 4 * (first[2] + 1));
 #pragma unroll 1
@@ -2961,10 +2986,9 @@ __global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm
         float P0[3] = {0.f, 0.f, 0.f}, f0[3] = {0.f, 0.f, 0.f}, f1[3] = {0.f, 0.f, 0.f};
 #pragma unroll
         for (int ex = 0; ex < E; ++ex) {
-          const float4 a0 = adj[2 * (at + ex)], a1 = adj[2 * (at + ex) + 1];
-          const float4 u0 = vel[2 * (at + ex)], u1 = vel[2 * (at + ex) + 1];
+          const float4 a0 = nrec[3 * (at + ex)], a1 = nrec[3 * (at + ex) + 1], u = nrec[3 * (at + ex) + 2];
           const float P[3] = {a0.y, a0.z, a0.w}, f[3] = {a1.x, a1.y, a1.z};
-          const float vn[3] = {u0.x, u0.y, u0.z}, dv[3] = {u0.w, u1.x, u1.y};
+          const float vn[3] = {a1.w, u.x, u.y}, dv[3] = {u.z, u.w, dvz[at + ex]};
           float gs = m * a0.x;
 #pragma unroll
           for (int a = 0; a < 3; ++a) gs += mv[a] * P[a];
