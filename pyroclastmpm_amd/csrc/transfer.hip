@@ -1319,9 +1319,7 @@ template <int D, int SPAN_, int CELLS_, int ROWS_> struct Tiles {
   static constexpr int T[3] = {CELLS_, ROWS_, D > 2 ? 4 : 1};
   static constexpr int N[3] = {CELLS_ + SPAN_ - 1, D > 1 ? ROWS_ + SPAN_ - 1 : 1, D > 2 ? 3 + SPAN_ : 1};
   static constexpr int COVER_Y = (N[1] - 1) / T[1] + 1;
-  // a wave of the grid pass takes 64 nodes of one tile, in the tile's order
-  static constexpr bool BRICKS = T[0] * T[1] * T[2] % 64 == 0;
-  static constexpr int WAVES = BRICKS ? T[0] * T[1] * T[2] / 64 : 1;
+  static constexpr int CELLS = T[0] * T[1] * T[2];
   static_assert((N[0] - 1) / T[0] + 1 <= kCoverX && COVER_Y <= kCoverY && (N[2] - 1) / T[2] + 1 <= kCoverZ,
                 "the gather visits at most kCover tiles per axis");
 };
@@ -1380,31 +1378,23 @@ __device__ inline bool gather_partials(const TileGeom &tg, const float *partials
   return true;
 }
 
-// The node of thread t of a pass over all nodes (false: none). With tiles of
-// at least 64 cells a wave takes 64 nodes of one tile, so that the slice rows
-// its lanes read are the same or neighbours (64 nodes of one x row read a
-// 44-byte row of each of eight slices instead); with small tiles t is the
-// node's linear index.
+// The node of thread t of a pass over all nodes (false: none): tile by tile, a
+// tile's nodes in x, y, z order, so that the slice rows a wave's lanes read are
+// the same or neighbours (64 nodes of one x row would read a short row of each
+// of 8 or 16 slices).
 template <int D, class TG>
 __device__ inline bool pass_node(const pmpm_grid &g, const TileGeom &tg, int t, int *ids) {
-  if constexpr (TG::BRICKS) {
-    const int w = t >> 6;
-    int b = w / TG::WAVES, l = (w % TG::WAVES) * 64 + (t & 63);
-    if (b >= tg.tiles[0] * tg.tiles[1] * tg.tiles[2]) return false;
-    bool in = true;
+  int b = t / TG::CELLS, l = t % TG::CELLS;
+  if (b >= tg.tiles[0] * tg.tiles[1] * tg.tiles[2]) return false;
+  bool in = true;
 #pragma unroll
-    for (int a = 0; a < D; ++a) {
-      ids[a] = (a < D - 1 ? b % tg.tiles[a] : b) * TG::T[a] + l % TG::T[a];
-      b /= tg.tiles[a];
-      l /= TG::T[a];
-      in = in && ids[a] < g.num_cells[a];
-    }
-    return in;
-  } else {
-    if (t >= g.num_cells_total) return false;
-    node_ids32<D>(g, t, ids);
-    return true;
+  for (int a = 0; a < D; ++a) {
+    ids[a] = (a < D - 1 ? b % tg.tiles[a] : b) * TG::T[a] + l % TG::T[a];
+    b /= tg.tiles[a];
+    l /= TG::T[a];
+    in = in && ids[a] < g.num_cells[a];
   }
+  return in;
 }
 // Per node: cutoff + forward moment (finalize), boundary conditions
 // [bc_begin, bc_end) in list order, then the node velocities G2P reads.
@@ -2175,9 +2165,8 @@ void launch_shape(const pmpm_grid &g, int types_built, const float *x, int n, fl
 }
 
 // Workgroups of 256 threads of a pass over all nodes (pass_node).
-static unsigned pass_blocks(const pmpm_grid &g, const TileGeom &tg) {
-  const int64_t cells = (int64_t)tg.T[0] * tg.T[1] * tg.T[2];
-  return (unsigned)ceil_div(cells % 64 == 0 ? (int64_t)tile_count(tg) * cells : (int64_t)g.num_cells_total, (int64_t)256);
+static unsigned pass_blocks(const TileGeom &tg) {
+  return (unsigned)ceil_div((int64_t)tile_count(tg) * tg.T[0] * tg.T[1] * tg.T[2], (int64_t)256);
 }
 // The stray sums of a P2G (mode 0) or re-map (mode 1) pass.
 static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, int mode) {
@@ -2189,7 +2178,7 @@ static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const 
 int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes, int finalize,
                 int b0, int b1, int remap, int gather, hipStream_t s, int n, int skip_mom_nt = 0) {
   const TileGeom tg = tile_geom(prm, g, gather, n);
-  const unsigned blocks = pass_blocks(g, tg);
+  const unsigned blocks = pass_blocks(tg);
   const Strays strays = gather ? stray_sums(ctx, prm, g, gather - 1) : Strays{};
   const float *partials = gather ? ctx->partials : nullptr;
   const int32_t *flags = gather ? ctx->tile_flags : nullptr;
@@ -3452,7 +3441,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
   const TileGeom tg = tile_geom(*prm, g, 3, n);
-  const unsigned nblocks = pass_blocks(g, tg);
+  const unsigned nblocks = pass_blocks(tg);
 #define PMPM_GRID_ADJOINT(...)                                                                                   \
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
               dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
