@@ -429,9 +429,10 @@ __device__ __constant__ static const float kSpanCubic[4][4][4] = {
 template <int SF> struct SpanPoly;
 template <> struct SpanPoly<PMPM_SF_CUBIC> {
   float a0, a1, a2, a3, d1, d2, d3;
-  // offset s, type of the node there; keep = 0 drops the offset
-  __device__ inline void set(int s, int type, float inv_h, float keep) {
-    const float4 c = *reinterpret_cast<const float4 *>(&kSpanCubic[type][s][0]);
+  // offset s, type of the node there; keep = 0 drops the offset. table:
+  // kSpanCubic in LDS (a load from memory here would be a round trip per cell)
+  __device__ inline void set(const float *table, int s, int type, float inv_h, float keep) {
+    const float4 c = *reinterpret_cast<const float4 *>(table + 4 * (4 * type + s));
     a0 = keep * c.x; a1 = keep * c.y; a2 = keep * c.z; a3 = keep * c.w;
     d1 = inv_h * a1; d2 = inv_h * (2.f * a2); d3 = inv_h * (3.f * a3);
   }
@@ -442,7 +443,7 @@ template <> struct SpanPoly<PMPM_SF_CUBIC> {
 // one above. Offset s is 0 where the particle's window does not reach it.
 template <> struct SpanPoly<PMPM_SF_QUADRATIC> {
   float e[2], c0[2], c1[2], d1[2];
-  __device__ inline void set(int s, int, float inv_h, float keep) {
+  __device__ inline void set(const float *, int s, int, float inv_h, float keep) {
     // f < 1/2: 0.5 (f - 0.5)^2, 0.75 - f^2, 0.5 (f + 0.5)^2, 0
     // else:    0, 0.5 (f - 1.5)^2, 0.75 - (f - 1)^2, 0.5 (f - 0.5)^2
     e[0] = s == 0 ? 0.5f : (s == 2 ? -0.5f : 0.f);
@@ -468,7 +469,7 @@ template <> struct SpanPoly<PMPM_SF_QUADRATIC> {
 // Linear: N = c0 + c1 f; the derivative is 0 on a node (linear_eval).
 template <> struct SpanPoly<PMPM_SF_LINEAR> {
   float c0, c1, d, d_at0;
-  __device__ inline void set(int s, int, float inv_h, float keep) {
+  __device__ inline void set(const float *, int s, int, float inv_h, float keep) {
     const float k = s > 1 ? 0.f : keep;
     c0 = s == 0 ? k : 0.f;
     c1 = s == 0 ? -k : k;
@@ -495,7 +496,7 @@ template <int SF> __device__ inline void inner_weights(float f, float *N, float 
 #pragma unroll
     for (int s = 0; s < Spline<SF>::SPAN; ++s) {
       SpanPoly<SF> p;
-      p.set(s, 0, 1.f, 1.f);
+      p.set(nullptr, s, 0, 1.f, 1.f);
       N[s] = p.N(f);
       dN[s] = p.dN(f);
     }
@@ -680,7 +681,7 @@ __global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
   const int nx = g.num_cells[0], ny = g.num_cells[1];
   const int yv = cy + NLO + sy;
   SpanPoly<SF> py;
-  if (D > 1) py.set(sy, TYPED ? cubic_node_type(yv, ny, 1) : 0, inv_h, 1.f);
+  if (D > 1) py.set(s_poly, sy, TYPED ? cubic_node_type(yv, ny, 1) : 0, inv_h, 1.f);
   const bool faces = TYPED && __ballot(ce > cs && (cx < 3 || cx >= nx - 3)) != 0ull;  // wave-uniform
   int xt[TYPED ? SPAN : 1] = {}, yt[TYPED ? SPAN : 1] = {};
   if (TYPED && faces) {
@@ -961,6 +962,8 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
   __shared__ __attribute__((aligned(16))) float block[M::WAVES][NV * BN];
   __shared__ __attribute__((aligned(16))) float stage[M::WAVES][CH * RS];
 
+  __shared__ __attribute__((aligned(16))) float s_poly[TYPED ? 64 : 4];  // kSpanCubic
+
   const int n = in.n;
   const float inv_h = g.inv_cell_size;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -978,6 +981,7 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
       cs = part.cell_start[cell];
     }
   }
+  if (TYPED && t < 64) s_poly[t] = (&kSpanCubic[0][0][0])[t];
   const bool none = TYPED && !prm.node_types_built;  // untyped cubic weights are zero
   if (!__syncthreads_or(ce > cs) || none) {
     if (t == 0) flags[blockIdx.x] = 0;
@@ -1117,8 +1121,8 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
       ty = cubic_node_type(yv, g.num_cells[1], 1);
       tz = cubic_node_type(zv, g.num_cells[2], 1);
     }
-    py.set(s1, ty, inv_h, 1.f);
-    pz.set(s2, tz, inv_h, 1.f);
+    py.set(s_poly, s1, ty, inv_h, 1.f);
+    pz.set(s_poly, s2, tz, inv_h, 1.f);
   };
   set_yz(0);
 
@@ -1198,7 +1202,7 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
       const int xv = cx + NLO + s2;  // this lane's x node
       const bool out_x = xv < 0 || xv >= nx;
       if (!inx || !inner_x) {
-        px.set(s2, TYPED ? cubic_node_type(xv, nx, 1) : 0, inv_h, TYPED && out_x ? 0.f : 1.f);
+        px.set(s_poly, s2, TYPED ? cubic_node_type(xv, nx, 1) : 0, inv_h, TYPED && out_x ? 0.f : 1.f);
         inner_x = inx;
       }
       const bool leaves = TYPED && MODE != 2 && !inx && prm.wrap_quirk && __ballot(out_x) != 0ull;
@@ -1235,11 +1239,11 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
           for (int kx = -1; kx <= 2; ++kx) {  // (2: one-node grids only)
             const bool mine = kx != 0 && xv - kx * nx >= 0 && xv - kx * nx < nx;
             if (__ballot(mine) == 0ull) continue;
-            px.set(s2, cubic_node_type(mine ? xv - kx * nx : 0, nx, 1), inv_h, mine ? 1.f : 0.f);
+            px.set(s_poly, s2, cubic_node_type(mine ? xv - kx * nx : 0, nx, 1), inv_h, mine ? 1.f : 0.f);
             set_yz(kx);
             for (int q = first; q < stop; q += 4) product(read_step(q - r0));
           }
-          px.set(s2, cubic_node_type(xv, nx, 1), inv_h, out_x ? 0.f : 1.f);
+          px.set(s_poly, s2, cubic_node_type(xv, nx, 1), inv_h, out_x ? 0.f : 1.f);
           set_yz(0);
         }
       }
