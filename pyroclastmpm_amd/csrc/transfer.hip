@@ -2840,7 +2840,8 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
 // per particle instead of 4,500 with a product of three weights per entry.
 // Bound by vector issue (1,080,000 particles: 230 us, of which 136 us are issue
 // at three waves per SIMD; capped to 128 registers for four it spills, 272 us).
-// LANES = 1: a lane per particle; 4: a lane per z layer of the window, for
+// LANES = 1: a lane per particle; 4: a lane per z layer of the window, 16: per
+// row of it, for
 // launches too small to fill the chip otherwise.
 // Wrap-around entries (deposit only): a node outside the grid holds the adjoint
 // of the node it reaches (see the staging), so it takes part as an ordinary
@@ -2856,7 +2857,7 @@ __global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm
                                                            const float *__restrict__ rec) {
   constexpr int E = Spline<SF>::ENTRIES;
   constexpr bool TYPED = SF == PMPM_SF_CUBIC;
-  static_assert(LANES == 1 || LANES == 4, "lanes per particle");
+  static_assert(LANES == 1 || LANES == 4 || LANES == 16, "lanes per particle");
   const int n = st.n;
   const int j = (int)blockIdx.x * (256 / LANES) + (int)threadIdx.x / LANES, sub = (int)threadIdx.x % LANES;
   const bool live = j < n;  // a thread past the particles works on the last one and writes nothing
@@ -2963,17 +2964,20 @@ __global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm
       w2 = pick(d2N[a], e);
     }
   };
+  // this lane's window offsets along z and y
+  const int z0_lane = LANES == 1 ? 0 : (LANES == 4 ? sub : sub >> 2), z1_lane = LANES == 1 ? E : min(z0_lane + 1, E);
+  const int y0_lane = LANES == 16 ? sub & 3 : 0, y1_lane = LANES == 16 ? min(y0_lane + 1, E) : E;
   adjoint_stage_rounds<LANES>(g, nodes, nbar, bin, live, quirk, [&](const float4 *nrec, const float *dvz, int box0,
                                                                    int X) {
     const int at0 = box0 + (first[0] + 1) + X * ((first[1] + 1) + 4 * (first[2] + 1));
 #pragma unroll 1
-    for (int sz = LANES == 1 ? 0 : sub; sz < (LANES == 1 ? E : min(sub + 1, E)); ++sz) {
+    for (int sz = z0_lane; sz < z1_lane; ++sz) {
       // y-contracted sums of this layer: xb's terms by their z weight (N: yX,
       // yY; dN: yZ, zX, zY; d2N: zZ), P_bar and f_bar by theirs
       float yX = 0.f, yY = 0.f, yZ = 0.f, zX = 0.f, zY = 0.f, zZ = 0.f;
       float yP[3] = {0.f, 0.f, 0.f}, fx[3] = {0.f, 0.f, 0.f}, fy[3] = {0.f, 0.f, 0.f}, fz[3] = {0.f, 0.f, 0.f};
-#pragma unroll(E > 2 ? 1 : 2)
-      for (int sy = 0; sy < E; ++sy) {  // (not unrolled: the next rows' records would fill the registers)
+#pragma unroll(E > 2 || LANES == 16 ? 1 : 2)
+      for (int sy = y0_lane; sy < y1_lane; ++sy) {  // (not unrolled: the next rows' records would fill the registers)
         const int at = at0 + X * (sy + 4 * sz);
         float g0 = 0.f, g1 = 0.f, wx1 = 0.f, wx2 = 0.f, wy0 = 0.f, wy1 = 0.f, wz0 = 0.f, wz1 = 0.f;
         float P0[3] = {0.f, 0.f, 0.f}, f0[3] = {0.f, 0.f, 0.f}, f1[3] = {0.f, 0.f, 0.f};
@@ -3036,11 +3040,11 @@ __global__ __launch_bounds__(256) void p2g_adjoint3_kernel(pmpm_params prm, pmpm
   });
 #pragma unroll
   for (int a = 0; a < 3; ++a) vb[a] *= m;
-  if (walk && (LANES == 1 || sub < E)) {
+  if (walk) {
     // outside entries one by one, with the types of the node each reaches
 #pragma unroll 1
-    for (int e = 0; e < E * E * (LANES == 1 ? E : 1); ++e) {
-      const int e3[3] = {e % E, (e / E) % E, LANES == 1 ? e / (E * E) : sub};
+    for (int e = E * (y0_lane + E * z0_lane); e < E * (y1_lane + E * (z1_lane - 1)); ++e) {  // (z, y, x)
+      const int e3[3] = {e % E, (e / E) % E, e / (E * E)};
       int nb[3];
       bool inside = true;
 #pragma unroll
@@ -3346,18 +3350,20 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
 }
 
 // Lanes per particle of the adjoint P2G: one once that fills the chip
-// (kAdjointLanesWanted), else four. PMPM_ADJOINT_P2G_LANES=1, 4 or 16 (as 4)
-// in the environment overrides the choice (read at every launch), so the
+// (kAdjointLanesWanted), four below, sixteen while a lane's chain is what counts
+// (3D, windows of 3 and 4; adjoint step, cubic: 1,152 particles 54 us with four
+// and 49 with sixteen, 14,784: 55 and 52, 25,088: 62 and 70). PMPM_ADJOINT_P2G_LANES=1, 4 or 16 in the environment overrides the choice (read at every launch), so the
 // layouts can be checked against each other.
 constexpr int kAdjointLanesWanted = 256 * 4 * 64 * 3;
+constexpr int kAdjointRowLanes = 16384;
 inline int adjoint_p2g_lanes(int n) {
   const char *e = getenv("PMPM_ADJOINT_P2G_LANES");
   if (e) {
     const int v = atoi(e);
     if (v == 1) return 1;
-    if (v == 4 || v == 16) return 4;
+    if (v == 4 || v == 16) return v;
   }
-  return n >= kAdjointLanesWanted ? 1 : 4;
+  return n >= kAdjointLanesWanted ? 1 : (n > kAdjointRowLanes ? 4 : 16);
 }
 
 template <int D, int SF>
@@ -3370,14 +3376,15 @@ void launch_adjoint_particles(const pmpm_params &prm, const pmpm_grid &g, const 
                        rec, pbar);
     return;
   }
-  const int lanes = adjoint_p2g_lanes(st.n);
+  const int lanes = std::min(adjoint_p2g_lanes(st.n), D == 3 && SF != PMPM_SF_LINEAR ? 16 : 4);
   const dim3 grid((unsigned)ceil_div(st.n, 256 / lanes));
 #define PMPM_P2G_ADJOINT(KERNEL)                                                                                 \
   PMPM_LAUNCH((KERNEL), (::pmpm::kname("p2g_adjoint_kernel", {(long)(D), (long)(SF), (long)lanes})), grid, dim3(256), 0, \
               s, prm, g, st, ib, part, nodes, nbar, rec)
   if constexpr (D == 3) {
     if (lanes == 1) { auto *k = &p2g_adjoint3_kernel<SF, 1>; PMPM_P2G_ADJOINT(*k); }
-    else { auto *k = &p2g_adjoint3_kernel<SF, 4>; PMPM_P2G_ADJOINT(*k); }
+    else if (lanes == 4) { auto *k = &p2g_adjoint3_kernel<SF, 4>; PMPM_P2G_ADJOINT(*k); }
+    else if constexpr (SF != PMPM_SF_LINEAR) { auto *k = &p2g_adjoint3_kernel<SF, 16>; PMPM_P2G_ADJOINT(*k); }
   } else {
     if (lanes == 1) { auto *k = &p2g_adjoint_kernel<D, SF, 1>; PMPM_P2G_ADJOINT(*k); }
     else { auto *k = &p2g_adjoint_kernel<D, SF, 4>; PMPM_P2G_ADJOINT(*k); }

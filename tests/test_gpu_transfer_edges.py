@@ -61,11 +61,11 @@ def test_transfer_tile_edges(oracle_mod, cells, musl, sf):
         assert e <= bar, (k, e, bar)
 
 
-@pytest.mark.parametrize("lanes", ["1", "4"])
+@pytest.mark.parametrize("lanes", ["1", "4", "16"])
 @pytest.mark.parametrize("sf", ["linear", "quadratic"])
 def test_adjoint_p2g_other_splines(oracle_mod, monkeypatch, sf, lanes):
     """The 3D adjoint step with the splines whose derivative enters as
-    differences (the differentiable column is cubic), in both lane layouts of
+    differences (the differentiable column is cubic), in the lane layouts of
     the adjoint P2G: <adjoint, direction> against the FP64 oracle's finite
     difference, with that check's bar (2e-3)."""
     from pyroclastmpm_amd import capi, diff
