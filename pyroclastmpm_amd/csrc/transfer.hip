@@ -2598,7 +2598,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? 4 
   }
   // material parameter adjoints: the workgroup's sum per material and
   // parameter (waves in a fixed order), reduced over workgroups in a fixed
-  // order by param_bar_reduce_kernel, so the gradient does not depend on
+  // order by the grid adjoint pass, so the gradient does not depend on
   // scheduling
   __shared__ float wsum[4][4 * PMPM_MAX_MATERIALS];
   const int wave = threadIdx.x >> 6;
@@ -2617,10 +2617,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? 4 
 // param_bar[e] += the sum over workgroups of part[b * entries + e]: one
 // workgroup per entry, each lane summing a fixed stride of workgroups, then a
 // fixed tree.
-__global__ __launch_bounds__(256) void param_bar_reduce_kernel(const float *__restrict__ part, int groups,
-                                                               int entries, float *__restrict__ param_bar) {
+__device__ inline void param_bar_reduce(const float *__restrict__ part, int groups, int entries, int e,
+                                        float *__restrict__ param_bar) {
   __shared__ float red[256];
-  const int e = blockIdx.x;
   float s = 0.f;
   for (int b = threadIdx.x; b < groups; b += 256) s += part[(size_t)b * entries + e];
   red[threadIdx.x] = s;
@@ -2670,14 +2669,23 @@ __device__ inline void store_node_adj(float *__restrict__ nbar, int node, float 
 // Per node: adjoints of the node velocities (scattered in the tile partials)
 // -> adjoints of mass, moment and force. Boundary conditions in reverse list
 // order with the forward's active sets, which the forward grid pass recorded
-// per node in `clamp` (components a NodeDomain condition set to zero).
+// per node in `clamp` (components a NodeDomain condition set to zero). The
+// launch's first `entries` workgroups sum the material parameters' adjoints
+// that g2p_adjoint_kernel left per workgroup in `pb` (a launch of their own was
+// 4 us of a small scene's 33).
 template <int D, class TG>
 __global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, TileGeom tg,
                                     const float *__restrict__ partials, const int32_t *__restrict__ flags,
-                                    const uint8_t *__restrict__ clamp, float *__restrict__ nbar) {
+                                    const uint8_t *__restrict__ clamp, float *__restrict__ nbar,
+                                    const float *__restrict__ pb, int groups, int entries,
+                                    float *__restrict__ param_bar) {
   const int nn = g.num_cells_total;
+  if ((int)blockIdx.x < entries) {
+    param_bar_reduce(pb, groups, entries, (int)blockIdx.x, param_bar);
+    return;
+  }
   int ids[3] = {0, 0, 0};
-  if (!pass_node<D, TG>(g, tg, (int)(blockIdx.x * blockDim.x + threadIdx.x), ids)) return;
+  if (!pass_node<D, TG>(g, tg, ((int)blockIdx.x - entries) * (int)blockDim.x + (int)threadIdx.x, ids)) return;
   const int i = ids[0] + (D > 1 ? g.num_cells[0] * (ids[1] + (D > 2 ? g.num_cells[1] * ids[2] : 0)) : 0);
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   gather_partials<D, 2 * D, TG>(tg, partials, flags, ids, acc);
@@ -3441,21 +3449,17 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_adjoint_particles, *prm, g, *state, *out_bar, *in_bar, *part, *nodes,
                     ctx->adj_rec, ctx->adj_pb, 0, nullptr, s);
   PMPM_LAUNCH_CHECK();
-  if (entries > 0) {
-    PMPM_LAUNCH(param_bar_reduce_kernel, (::pmpm::kname("param_bar_reduce_kernel", {})), dim3((unsigned)entries), dim3(256), 0, s, ctx->adj_pb, groups,
-                       entries, param_bar);
-    PMPM_LAUNCH_CHECK();
-  }
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_p2g, *prm, g, *state, *state, *part, *nodes, 2, ctx->partials,
                     ctx->tile_flags, stray_sums(ctx, *prm, g, 0), s, ctx->adj_rec);
   PMPM_LAUNCH_CHECK();
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
   const TileGeom tg = tile_geom(*prm, g, 3, n);
-  const unsigned nblocks = pass_blocks(tg);
+  const unsigned nblocks = pass_blocks(tg) + (unsigned)entries;
 #define PMPM_GRID_ADJOINT(...)                                                                                   \
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
-              dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes)
+              dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes, ctx->adj_pb, \
+              groups, entries, param_bar)
   switch (D) {
     case 1: PMPM_WITH_ROWS(1, tg, PMPM_GRID_ADJOINT) break;
     case 2: PMPM_WITH_ROWS(2, tg, PMPM_GRID_ADJOINT) break;
