@@ -49,16 +49,16 @@ BYTES_PER_PARTICLE = {
 # Algorithmic HBM bytes of each kernel of the step, per particle and per grid
 # node of one launch (the compulsory reads and writes of a fused design).
 KERNEL_BYTES = {
-    "hash_kernel<3>": (16, 36),             # x 12 in, key 4 out; clears cell ranges 8 + node m, P, Q 28
-    "radix_hist_kernel<10>": (4, 0),        # key 4
-    "radix_scatter_kernel<10>": (16, 0),    # key + slot 8 in, 8 out
-    "cell_range_kernel": (4, 0),            # sorted key 4
+    "hint_classify_kernel<3>": (20, 8),     # x 12, hint 4 in, key 4 out; counts 8
+    "hint_scan_kernel": (0, 32),            # counts 8 in; cell record 16, range 8 out
+    "hint_movers_kernel": (0, 0),           # (the few particles that changed cell)
+    "hint_place_kernel": (12, 16),          # key 4 in, slot 4, sorted key 4 out; cell record 16
     "p2g_mfma_kernel<2, 0>": (56, 0),       # x 12, v 12, m 4, V 4, stress 24 (P2G of the particle state)
-    "p2g_mfma_kernel<2, 1>": (36, 0),       # re-map: sorted 4, hash 4, x 12, m 4, v' 12
+    "p2g_mfma_kernel<2, 1>": (32, 0),       # re-map: sorted 4, x 12, m 4, v' 12
     "g2p_kernel<3, 2, 1>": (52, 0),         # first map: sorted 4, x 12, v 12 in; x 12, v 12 out
     "g2p_kernel<3, 2, 2>": (252, 0),        # second map + return map (entry musl_g2p above)
-    "grid_kernel<3> gather 1": (0, 88),     # m, P, Q in 28; m, P, Q out 28, velocity record 32
-    "grid_kernel<3> gather 2": (0, 72),     # m, P, Q in 28; Q out 12, velocity record 32
+    "grid_kernel<3> gather 1": (0, 48),     # m, P out 16, velocity record 32
+    "grid_kernel<3> gather 2": (0, 60),     # m, P in 16; Q out 12, velocity record 32
 }
 # The step's algorithmic bytes per particle (compulsory traffic of a fused
 # step: sort 16, P2G 56, MUSL map 52, second map + return map 188 + L 36,

@@ -303,9 +303,9 @@ int pmpm_step(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, 
  * capture, tight serving loops, harnesses that forbid hipMalloc). It runs the
  * step pmpm_step runs, with the same arguments minus the context: the
  * workspace (sort keys and slots, digit histograms, P2G tile partials and
- * flags, wrap-around records and cell list, counters) comes from a file-scope
- * device array of PMPM_NOALLOC_SCRATCH_BYTES that each GPU holds until the
- * process ends. A step that needs more returns PMPM_ERR_WORKSPACE (see
+ * flags, stray sums, counters) comes from a file-scope device array that each
+ * GPU holds until the process ends. A step is charged by its particle count
+ * and grid against PMPM_NOALLOC_SCRATCH_BYTES; one that needs more returns PMPM_ERR_WORKSPACE (see
  * pmpm_last_error); it calls no allocator. All calls on one GPU share that
  * GPU's array: calls that overlap on one GPU race. */
 #define PMPM_NOALLOC_SCRATCH_BYTES (64u << 20)
