@@ -2413,7 +2413,7 @@ extern "C" int pmpm_stress_update(const pmpm_params *prm, int32_t mat_id, pmpm_p
 //                            F' = (I + dt L) F, (sigma', eps') = return map
 // The adjoint runs these backwards: g2p_adjoint_kernel (per particle: return
 // map VJP, F, v, and the records of the PIC/FLIP/L adjoints), the adjoint
-// scatter (p2g_kernel MODE 2) of those records to the nodes,
+// scatter (the P2G tiles, MODE 2) of those records to the nodes,
 // grid_adjoint_kernel (per node: velocities, BCs, forward moment), and
 // p2g_adjoint_kernel (per particle: gather of the node adjoints into v, sigma,
 // V = det(F) V0 and x, together with the position adjoint of the G2P weights
