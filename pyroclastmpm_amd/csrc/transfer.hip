@@ -927,6 +927,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // on to the next cell is a register rotation: only the leftmost node column
 // leaves, and each column of the wave's row is written once, complete.
 //
+// 1,080,000 particles, 27 per cell, cubic: P2G 81 -> 70 us (and 32 us of
+// wrap-around launches less), re-map 40 -> 36 (23), adjoint scatter 159 -> 67.
 // What bounds it: instruction issue. Per four particles there are 4 (MODE 1:
 // 1) matrix instructions of 32 cycles and about 45 vector instructions, so
 // the weights are evaluated here from per-lane coefficients (about 20
@@ -2056,9 +2058,12 @@ static bool wraps(const pmpm_params &prm) {
 // The 3D P2G tiles (MfmaGeom) of a scene. A function of the grid and the
 // particle count only: every pass of a step, and pmpm_step_noalloc, must agree
 // on it. Small scenes take small tiles (more waves, each with a short chain of
-// cells), the others larger ones (fewer nodes per cell in the slices).
+// cells), the others larger ones (fewer nodes per cell in the slices). Small
+// and large tiles, a step or adjoint step: 1,300 particles 35.5 and 37.3 us,
+// 2,016: 36.5 and 38.3, 8,320: 36.6 and 38.9, 14,784: 49.9 and 51.1, 17,000:
+// 73.2 and 69.8, 40,000: 46.7 and 46.4, 275,000: 101.7 and 96.0.
 struct MfmaTiles { int cells, rows; };
-constexpr int kSmallGridNodes = 131072, kSmallParticles = 131072;
+constexpr int kSmallGridNodes = 131072, kSmallParticles = 16384;
 static MfmaTiles mfma_tiles(const pmpm_grid &g, int n) {
   if (g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles) return {4, 1};
   return {8, 2};
