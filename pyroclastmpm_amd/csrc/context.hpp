@@ -18,8 +18,10 @@ struct pmpm_context {
   int32_t *vals_tmp = nullptr;   // radix sort ping-pong values
   uint32_t *hist = nullptr;      // [radix][blocks] digit histograms
   size_t hist_len = 0;
-  uint32_t *counters = nullptr;  // [8]: out-of-grid particles, hint unsorted flag (set, kept), heavy cells, stray flags (2)
-  bool counters_clear = false;   // cleared once, by the first call that uses them
+  // [kCounters]: out-of-grid particles, hint unsorted flag (set, kept), heavy
+  // cells, stray flags (2); counters_clear: cleared since they were allocated
+  uint32_t *counters = nullptr;
+  bool counters_clear = false;
   // P2G tile partials: per tile, the LDS node block of each accumulated field
   // (plain stores; the grid kernel sums the <= 2^D tiles covering a node)
   float *partials = nullptr;
@@ -31,6 +33,7 @@ struct pmpm_context {
   // (stray_flags: P2G, re-map) and the grid pass after it
   float *strays = nullptr;
   size_t strays_cap = 0;
+  bool strays_clear = false;       // cleared since they were allocated
   int32_t *stray_flags = nullptr;  // in counters
   // a byte per node: the components the last grid pass's NodeDomain
   // condition set to zero (words of 4 bytes), read by the adjoint
@@ -77,6 +80,7 @@ int ensure_buffer(float *&buf, size_t &cap, size_t floats);
 
 namespace pmpm {
 
+constexpr int kCounters = 8;  // words of pmpm_context::counters
 constexpr int kSortBlock = 1024;  // 16 waves rank 1024 keys per round
 constexpr int kSortItems = 4;
 constexpr int kSortTile = kSortBlock * kSortItems;
@@ -164,6 +168,11 @@ struct ZeroLists {  // buffers of 32-bit words to clear in one launch
   }
 };
 int zero_fill_lists(const ZeroLists &z, hipStream_t s);
+// Clears buffers that must be zero between a context's calls, once (`clear`),
+// on the stream of the call that uses them first. A clear that is only being
+// recorded into a graph does not count: the graph may not have been replayed
+// when the next call comes.
+int clear_on_stream(const ZeroLists &z, bool &clear, hipStream_t s);
 // One step on the workspace of ctx (arguments already checked by
 // step_args_ok); the body of pmpm_step.
 int step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, int32_t musl,

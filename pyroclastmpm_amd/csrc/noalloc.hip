@@ -104,7 +104,7 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   const size_t o_keys = c.take(n * sizeof(uint32_t));
   const size_t o_vals = c.take(n * sizeof(int32_t));
   const size_t o_hist = c.take(hist_len * sizeof(uint32_t));
-  const size_t o_counters = c.take(8 * sizeof(uint32_t));
+  const size_t o_counters = c.take(kCounters * sizeof(uint32_t));
   const size_t o_partials = c.take(w.partial_floats * sizeof(float));
   const size_t o_flags = c.take(w.tiles * sizeof(int32_t));
   const size_t o_clamp = c.take(w.clamp_words * sizeof(float));
@@ -141,6 +141,7 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   ctx.stray_flags = reinterpret_cast<int32_t *>(ctx.counters + 4);
   // (the scratch holds whatever an earlier call left)
   if ((rc = zero_fill(ctx.strays, (int64_t)w.stray_words, (hipStream_t)stream)) != PMPM_OK) return rc;
+  ctx.strays_clear = true;
   // (the context is a plain struct on this stack frame: nothing frees the
   // scratch pieces it points at)
   return step_on(&ctx, prm, grid, musl, a, b, part, nodes, (hipStream_t)stream);

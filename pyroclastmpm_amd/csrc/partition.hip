@@ -768,7 +768,7 @@ extern "C" int pmpm_context_create(pmpm_context **ctx) {
   c->sort_by_hint = !(radix_only && radix_only[0] == '1');
   const char *hint_min = getenv("PMPM_PARTITION_HINT_MIN");
   if (hint_min && hint_min[0]) c->hint_min_particles = (int32_t)strtol(hint_min, nullptr, 10);
-  if (!hip_ok(hipMalloc(&c->counters, 8 * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
+  if (!hip_ok(hipMalloc(&c->counters, kCounters * sizeof(uint32_t)), "hipMalloc")) { delete c; return PMPM_ERR_HIP; }
   c->stray_flags = reinterpret_cast<int32_t *>(c->counters + 4);
   *ctx = c;
   return PMPM_OK;
@@ -848,16 +848,37 @@ extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, in
     int rc = reserve_hint(ctx, max_particles, (uint32_t)max_cells);
     if (rc != PMPM_OK) return rc;
   }
+  // what must be zero between calls is so when this returns, whatever stream
+  // uses it first, and also if that use is only recorded (a captured graph)
+  if (!ctx->counters_clear || (ctx->hint_cnt && !ctx->hint_clear)) {
+    ZeroLists z{};
+    z.add(ctx->counters, kCounters);
+    z.add(ctx->hint_cnt, (int64_t)ctx->hint_cnt_cap);
+    z.add(ctx->hint_cbt, (int64_t)ctx->hint_cbt_cap);
+    int rc = zero_fill_lists(z, nullptr);
+    if (rc != PMPM_OK) return rc;
+    PMPM_HIP_CHECK(hipStreamSynchronize(nullptr));
+    ctx->counters_clear = true;
+    ctx->hint_clear = ctx->hint_cnt != nullptr;
+  }
   return PMPM_OK;
 }
 
-// A new context's counters, cleared on the stream that uses them first (a
-// hipMemset on the null stream is not ordered before a non-blocking stream).
+int pmpm::clear_on_stream(const ZeroLists &z, bool &clear, hipStream_t s) {
+  if (clear) return PMPM_OK;
+  int rc = zero_fill_lists(z, s);
+  if (rc != PMPM_OK) return rc;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  PMPM_HIP_CHECK(hipStreamIsCapturing(s, &capture));
+  clear = capture == hipStreamCaptureStatusNone;
+  return PMPM_OK;
+}
+
+// The counters of a context that was not reserved for anything yet.
 static int clear_counters(pmpm_context *ctx, hipStream_t s) {
-  if (ctx->counters_clear) return PMPM_OK;
-  int rc = zero_fill(ctx->counters, 4, s);
-  if (rc == PMPM_OK) ctx->counters_clear = true;
-  return rc;
+  ZeroLists z{};
+  z.add(ctx->counters, kCounters);
+  return clear_on_stream(z, ctx->counters_clear, s);
 }
 
 extern "C" int pmpm_context_out_of_grid(pmpm_context *ctx, pmpm_stream_t stream, int32_t *count) {
@@ -934,8 +955,8 @@ static HintLayout hint_layout(int n) {
 }
 
 // Grows the hint workspace to n particles on ncells cells. The counts must be
-// zero between calls: new ones are marked and cleared by the partition that
-// uses them first, on its stream.
+// zero between calls: new ones are marked, and cleared by pmpm_context_reserve
+// or, if they grew in a partition, by that partition on its stream.
 static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells) {
   const size_t cnt = 2 * ((size_t)ncells + 1), cbt = 2 * (size_t)ceil_div((int64_t)ncells + 1, kHintCells);
   int rc;
@@ -976,8 +997,7 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
     ZeroLists z{};
     z.add(ctx->hint_cnt, (int64_t)ctx->hint_cnt_cap);
     z.add(ctx->hint_cbt, (int64_t)ctx->hint_cbt_cap);
-    if ((rc = zero_fill_lists(z, s)) != PMPM_OK) return rc;
-    ctx->hint_clear = true;
+    if ((rc = clear_on_stream(z, ctx->hint_clear, s)) != PMPM_OK) return rc;
   }
   const HintLayout l = hint_layout(n);
   uint32_t *base = reinterpret_cast<uint32_t *>(ctx->hint_part);

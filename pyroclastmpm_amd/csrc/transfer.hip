@@ -2261,10 +2261,12 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   // the stray sums are zero whenever no pass is under way
   const size_t words = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
   if (words > ctx->strays_cap) {
+    ctx->strays_clear = false;
     if ((rc = ensure_buffer(ctx->strays, ctx->strays_cap, words)) != PMPM_OK) return rc;
-    if ((rc = zero_fill(ctx->strays, (int64_t)words, s)) != PMPM_OK) return rc;
   }
-  return PMPM_OK;
+  ZeroLists z{};
+  z.add(ctx->strays, (int64_t)ctx->strays_cap);
+  return clear_on_stream(z, ctx->strays_clear, s);
 }
 
 void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w) {
