@@ -19,7 +19,7 @@ struct pmpm_context {
   uint32_t *hist = nullptr;      // [radix][blocks] digit histograms
   size_t hist_len = 0;
   // [kCounters]: out-of-grid particles, hint unsorted flag (set, kept), heavy
-  // cells, stray flags (2); counters_clear: cleared since they were allocated
+  // cells, stray flags (3); counters_clear: cleared since they were allocated
   uint32_t *counters = nullptr;
   bool counters_clear = false;
   // P2G tile partials: per tile, the LDS node block of each accumulated field
@@ -29,8 +29,9 @@ struct pmpm_context {
   int32_t *tile_flags = nullptr;  // 1 = tile had particles this launch
   size_t tile_flags_cap = 0;
   // P2G sums of particles deposited over their own windows (mass, momentum,
-  // force per node), zero but between a P2G pass that sets its flag
-  // (stray_flags: P2G, re-map) and the grid pass after it
+  // force per node; the adjoint scatter's fields), zero but between a pass that
+  // sets its flag (stray_flags: P2G, re-map, adjoint scatter) and the grid pass
+  // after it
   float *strays = nullptr;
   size_t strays_cap = 0;
   bool strays_clear = false;       // cleared since they were allocated

@@ -303,12 +303,12 @@ template <int D> __device__ inline void node_ids32(const pmpm_grid &g, int lin, 
 
 // Slow path of the scatter: every entry goes straight to global memory,
 // through the linear index (wrap-around reproduced when wrap_quirk is set).
-// Used for particles whose bin is not their cell's coordinates and for the
-// entries of boundary particles that leave the grid on some axis.
-// Sums of the particles deposited over their own windows (p2g_stray): node
-// arrays of their own, zero between the passes, and a flag the pass sets when
-// it added something. The grid pass reads (and clears) them only then, so the
-// node arrays are neither cleared before a step nor read by its first grid pass.
+// Used for the particles that are not in the cell they are listed in (see
+// p2g_stray).
+// Strays: their sums, in node arrays of their own that are zero between the
+// passes, and a flag the pass sets when it added something. The grid pass reads
+// (and clears) them only then, so the node arrays are neither cleared before a
+// step nor read by its first grid pass.
 struct Strays {
   float *mass, *mom, *mom_nt;
   int32_t *flag;
@@ -356,9 +356,10 @@ __device__ inline void scatter_entry_global(const pmpm_params &prm, const pmpm_g
   }
 }
 
-// P2G of a particle whose recomputed bin is not the cell it is listed in
-// (only possible when the partition was built from other positions): this
-// lane's y slice of its window goes straight to the stray sums.
+// P2G of a particle that is not in the cell it is listed in: one left of the
+// origin (its coordinate truncates to cell 0, its fraction is negative), or any
+// other where the partition was built from other positions. This lane's y slice
+// of its window goes straight to the stray sums.
 template <int D, int SF, int MODE>
 __device__ void p2g_stray(const pmpm_params &prm, const pmpm_grid &g, const Strays &nodes, const float *x, int n,
                           int slot, int sy, float m, const float *v, const Sym &A, const float *fext) {
@@ -382,6 +383,47 @@ __device__ void p2g_stray(const pmpm_params &prm, const pmpm_grid &g, const Stra
       const int e3[3] = {ex, sy, ez};
       scatter_entry_global<D, SF, MODE>(prm, g, nodes, g.num_cells_total, w, e3, m, mv, A3, fext);
     }
+}
+
+// The same for the adjoint scatter (MODE 2): the records' adjoints (v_pic: vpb,
+// dv: dvb, L: row a from Lb + LROW a) over the entries the G2P gathered, those
+// inside the grid, into the first 2 D stray arrays.
+template <int D, int SF, int LROW>
+__device__ void adjoint_stray(const pmpm_params &prm, const pmpm_grid &g, const Strays &nodes, const float *x, int n,
+                              int slot, const float *vpb, const float *dvb, const float *Lb) {
+  constexpr int E = Spline<SF>::ENTRIES, EY = D > 1 ? E : 1, EZ = D > 2 ? E : 1;
+  PW<D, SF> w;
+  float xp[3];
+  particle_weights<D, SF>(prm, g, x, n, slot, w, xp);
+#pragma unroll 1
+  for (int e = 0; e < E * EY * EZ; ++e) {
+    const int e3[3] = {e % E, (e / E) % EY, e / (E * EY)};
+    float N[3] = {1.f, 1.f, 1.f}, dN[3] = {0.f, 0.f, 0.f};
+    int id[3] = {0, 0, 0};
+    bool inside = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      id[a] = w.bin[a] + w.first[a] + e3[a];
+      inside = inside && id[a] >= 0 && id[a] < g.num_cells[a];
+#pragma unroll
+      for (int k = 0; k < E; ++k) {  // (picked by compares: no indexed registers)
+        N[a] = e3[a] == k ? w.N[a][k] : N[a];
+        dN[a] = e3[a] == k ? w.dN[a][k] : dN[a];
+      }
+    }
+    if (!inside) continue;
+    const int node = (int)lin_index(g, id, D), nn = g.num_cells_total;
+    const float wgt = (N[0] * N[1]) * N[2];
+    const float gr[3] = {(dN[0] * N[1]) * N[2], (dN[1] * N[0]) * N[2], (dN[2] * N[0]) * N[1]};
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      float v = wgt * vpb[a];
+#pragma unroll
+      for (int c = 0; c < D; ++c) v += gr[c] * Lb[LROW * c + a];
+      unsafeAtomicAdd(&nodes.mass[(int64_t)a * nn + node], v);
+      unsafeAtomicAdd(&nodes.mass[(int64_t)(D + a) * nn + node], wgt * dvb[a]);
+    }
+  }
 }
 
 // Fields per node of a P2G pass: MODE 0 mass, momentum, force; MODE 1 the
@@ -862,9 +904,9 @@ __global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
       slice[k * G::NTN + i] = sum;
     }
   }
-  if (MODE != 2 && strays) {
+  if (strays) {
     if (lane == 0) *nodes.flag = 1;
-    // as in p2g_mfma_kernel: particles listed in this row but binned elsewhere
+    // as in p2g_mfma_kernel: particles listed in this row that are not in their cell
 #pragma unroll 1
     for (int k0 = 0; k0 < most; k0 += KW)
 #pragma unroll 1
@@ -873,6 +915,10 @@ __global__ __launch_bounds__((RowGeom<D, SF>::THREADS)) void p2g_rows_kernel(
         float fr[D], fe[3] = {0.f, 0.f, 0.f};
         load_raw(find(k0, r), r, q);
         if (own_cell(q, fr) || !q.valid) continue;
+        if constexpr (MODE == 2) {
+          adjoint_stray<D, SF, D>(prm, g, nodes, in.x, n, q.slot, q.v, q.dv, q.Lb);
+          continue;
+        }
         Sym A = sym_zero();
         if (MODE == 0) {
           const float mvol = -q.vol;
@@ -1282,18 +1328,22 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
 #pragma unroll
     for (int y = 0; y < M::NY; ++y) slice[f * M::NTN + y * PL + i % PL] = sum[y];
   }
-  if (MODE != 2 && strays) {
+  if (strays) {
     if (lane == 0) *nodes.flag = 1;
-    // particles listed in this row but binned elsewhere (a partition of other
-    // positions): deposited over their own windows, straight to the stray
-    // sums (MODE 2 runs on a partition of the same positions). Walked again
-    // here, where the registers of the products are free.
+    // particles listed in this row that are not in their cell (left of the
+    // origin, or a partition of other positions): deposited over their own
+    // windows, straight to the stray sums. Walked again here, where the
+    // registers of the products are free.
 #pragma unroll 1
     for (int q0 = 0; q0 < total; q0 += 64) {
       Raw q;
       float fr[3], fe[3] = {0.f, 0.f, 0.f};
       load_raw(find(q0), q);
       if (own_cell(q, fr) || !q.valid) continue;
+      if constexpr (MODE == 2) {
+        adjoint_stray<3, SF, 3>(prm, g, nodes, in.x, n, q.slot, q.v, q.dv, q.Lb);
+        continue;
+      }
       Sym A = sym_zero();
       if (MODE == 0) A = minus_v_sigma(q);
       if (FEXT) planar_force<3>(prm, g, q.x, q.v, q.vol, q.m, fe);
@@ -2182,10 +2232,10 @@ void launch_shape(const pmpm_grid &g, int types_built, const float *x, int n, fl
 static unsigned pass_blocks(const TileGeom &tg) {
   return (unsigned)ceil_div((int64_t)tile_count(tg) * tg.T[0] * tg.T[1] * tg.T[2], (int64_t)256);
 }
-// The stray sums of a P2G (mode 0) or re-map (mode 1) pass.
+// The stray sums of a P2G (mode 0), re-map (mode 1) or adjoint scatter (mode 2).
 static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, int mode) {
   const int64_t nn = g.num_cells_total;
-  return {ctx->strays, ctx->strays + nn, ctx->strays + (1 + prm.dim) * nn, ctx->stray_flags + (mode == 1)};
+  return {ctx->strays, ctx->strays + nn, ctx->strays + (1 + prm.dim) * nn, ctx->stray_flags + mode};
 }
 // gather: 0 = node arrays only, 1 = from the P2G tile partials, 2 = mom_nt from
 // the MUSL re-map tile partials (ctx holds them) of a pass over n particles.
@@ -2483,10 +2533,11 @@ template <int D, int SF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? 4 : 1))) void g2p_adjoint_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles st,
                                                           pmpm_adjoint ob, pmpm_adjoint ib, pmpm_spatial part,
                                                           pmpm_nodes nodes, float *__restrict__ rec,
-                                                          float *__restrict__ pbar) {
+                                                          float *__restrict__ pbar, int32_t *stray_flag) {
   const int n = st.n;
   const int nn = g.num_cells_total;
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j == 0) *stray_flag = 0;  // of the scatter that follows
   const bool valid = j < n;
   float pb[4] = {0.f, 0.f, 0.f, 0.f};
   int color = -1;
@@ -2690,7 +2741,7 @@ __global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm
                                     const float *__restrict__ partials, const int32_t *__restrict__ flags,
                                     const uint8_t *__restrict__ clamp, float *__restrict__ nbar,
                                     const float *__restrict__ pb, int groups, int entries,
-                                    float *__restrict__ param_bar) {
+                                    float *__restrict__ param_bar, Strays strays) {
   const int nn = g.num_cells_total;
   if ((int)blockIdx.x < entries) {
     param_bar_reduce(pb, groups, entries, (int)blockIdx.x, param_bar);
@@ -2701,6 +2752,13 @@ __global__ __launch_bounds__(256) void grid_adjoint_kernel(pmpm_params prm, pmpm
   const int i = ids[0] + (D > 1 ? g.num_cells[0] * (ids[1] + (D > 2 ? g.num_cells[1] * ids[2] : 0)) : 0);
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   gather_partials<D, 2 * D, TG>(tg, partials, flags, ids, acc);
+  if (*strays.flag) {
+#pragma unroll
+    for (int k = 0; k < 2 * D; ++k) {
+      acc[k] += strays.mass[(int64_t)k * nn + i];
+      strays.mass[(int64_t)k * nn + i] = 0.f;
+    }
+  }
   const float m = nodes.mass[i];
   float mb = 0.f, Pb[3] = {0.f, 0.f, 0.f}, Qb[3] = {0.f, 0.f, 0.f}, fb[3] = {0.f, 0.f, 0.f};
   if (m > prm.small_mass_cutoff) {
@@ -3390,10 +3448,10 @@ template <int D, int SF>
 void launch_adjoint_particles(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &st,
                               const pmpm_adjoint &ob, const pmpm_adjoint &ib, const pmpm_spatial &part,
                               const pmpm_nodes &nodes, float *rec, float *pbar, int which, const float *nbar,
-                              hipStream_t s) {
+                              int32_t *stray_flag, hipStream_t s) {
   if (which == 0) {
     PMPM_LAUNCH((g2p_adjoint_kernel<D, SF>), (::pmpm::kname("g2p_adjoint_kernel", {(long)(D), (long)(SF)})), dim3((unsigned)ceil_div(st.n, 256)), dim3(256), 0, s, prm, g, st, ob, ib, part, nodes,
-                       rec, pbar);
+                       rec, pbar, stray_flag);
     return;
   }
   const int lanes = std::min(adjoint_p2g_lanes(st.n), D == 3 && SF != PMPM_SF_LINEAR ? 16 : 4);
@@ -3456,13 +3514,14 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
     return rc;
   const int groups = ceil_div(n, 256), entries = 4 * prm->num_materials;
   if ((rc = ensure_buffer(ctx->adj_pb, ctx->adj_pb_cap, (size_t)groups * entries)) != PMPM_OK) return rc;
+  const Strays strays = stray_sums(ctx, *prm, g, 2);
   // G2P adjoint (material parameter adjoints per workgroup, then summed into
   // param_bar), then the scatter of its records to the nodes
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_adjoint_particles, *prm, g, *state, *out_bar, *in_bar, *part, *nodes,
-                    ctx->adj_rec, ctx->adj_pb, 0, nullptr, s);
+                    ctx->adj_rec, ctx->adj_pb, 0, nullptr, strays.flag, s);
   PMPM_LAUNCH_CHECK();
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_p2g, *prm, g, *state, *state, *part, *nodes, 2, ctx->partials,
-                    ctx->tile_flags, stray_sums(ctx, *prm, g, 0), s, ctx->adj_rec);
+                    ctx->tile_flags, strays, s, ctx->adj_rec);
   PMPM_LAUNCH_CHECK();
   // grid adjoint, with the forward grid pass's clamp record
   const uint8_t *clamp = nodes->clamp ? nodes->clamp : reinterpret_cast<const uint8_t *>(ctx->clamp_mask);
@@ -3471,7 +3530,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
 #define PMPM_GRID_ADJOINT(...)                                                                                   \
   PMPM_LAUNCH((grid_adjoint_kernel<__VA_ARGS__>), (::pmpm::kname("grid_adjoint_kernel", {(long)D})), dim3(nblocks), \
               dim3(256), 0, s, *prm, g, *nodes, tg, ctx->partials, ctx->tile_flags, clamp, ctx->adj_nodes, ctx->adj_pb, \
-              groups, entries, param_bar)
+              groups, entries, param_bar, strays)
   switch (D) {
     case 1: PMPM_WITH_ROWS(1, tg, PMPM_GRID_ADJOINT) break;
     case 2: PMPM_WITH_ROWS(2, tg, PMPM_GRID_ADJOINT) break;
@@ -3481,7 +3540,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
   PMPM_LAUNCH_CHECK();
   // P2G adjoint
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_adjoint_particles, *prm, g, *state, *out_bar, *in_bar, *part, *nodes,
-                    ctx->adj_rec, param_bar, 1, ctx->adj_nodes, s);
+                    ctx->adj_rec, param_bar, 1, ctx->adj_nodes, strays.flag, s);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
