@@ -1220,14 +1220,19 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
       C1 = __builtin_amdgcn_mfma_f32_16x16x4f32(v ? Nx * q.A.w : 0.f, b3, C1, 0, 0, 0);
     }
   };
-  // node column lx of the wave's row is complete: out of the accumulators
+  // node column lx of the wave's row is complete: out of the accumulators (linear
+  // splines: the columns past the span hold products with zero weights, which
+  // are not zero where a field is not finite)
+  auto shifted = [](const v4f &C) {
+    return v4f{C[1], SPAN > 2 ? C[2] : 0.f, SPAN > 3 ? C[3] : 0.f, 0.f};
+  };
   auto flush = [&](int lx) {
     float *b = blk + lx * M::XP + 4 * s2 + s1;
     if (MODE != 1 || pk < 3) b[pk * BN] = C1[0];
-    C1 = v4f{C1[1], C1[2], C1[3], 0.f};
+    C1 = shifted(C1);
     if (MODE != 1) {
       if (pk < (MODE == 0 ? 3 : 2)) b[(4 + pk) * BN] = C2[0];
-      C2 = v4f{C2[1], C2[2], C2[3], 0.f};
+      C2 = shifted(C2);
     }
   };
 
