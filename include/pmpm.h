@@ -303,11 +303,14 @@ int pmpm_step(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, 
  * capture, tight serving loops, harnesses that forbid hipMalloc). It runs the
  * step pmpm_step runs, with the same arguments minus the context: the
  * workspace (sort keys and slots, digit histograms, P2G tile partials and
- * flags, stray sums, counters) comes from a file-scope device array that each
- * GPU holds until the process ends. A step is charged by its particle count
- * and grid against PMPM_NOALLOC_SCRATCH_BYTES; one that needs more returns PMPM_ERR_WORKSPACE (see
- * pmpm_last_error); it calls no allocator. All calls on one GPU share that
- * GPU's array: calls that overlap on one GPU race. */
+ * flags, counters) comes from a file-scope device array of
+ * PMPM_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends. A step
+ * is charged by its particle count and grid (a fixed rule, not the present
+ * kernels' arrays); one that is charged more than the array holds returns
+ * PMPM_ERR_WORKSPACE (see pmpm_last_error); it calls no allocator. On grids of
+ * one to five nodes along y or z a step near that limit sums its particles by
+ * atomics, equal to pmpm_step's sums to float rounding. All calls on one GPU
+ * share that GPU's array: calls that overlap on one GPU race. */
 #define PMPM_NOALLOC_SCRATCH_BYTES (64u << 20)
 int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, int32_t musl, const pmpm_particles *a,
                       pmpm_particles *b, pmpm_spatial *part, pmpm_nodes *nodes, pmpm_stream_t stream);

@@ -36,6 +36,10 @@ struct pmpm_context {
   size_t strays_cap = 0;
   bool strays_clear = false;       // cleared since they were allocated
   int32_t *stray_flags = nullptr;  // in counters
+  // the workspace is the caller's and never grows (pmpm_step_noalloc): the
+  // stray sums are then the step's node arrays, cleared before it, and without
+  // room for the partials every particle is deposited over its own window
+  bool fixed_workspace = false;
   // a byte per node: the components the last grid pass's NodeDomain
   // condition set to zero (words of 4 bytes), read by the adjoint
   float *clamp_mask = nullptr;
@@ -159,7 +163,7 @@ class TimedRegion {
 // Fill n floats/ints with zero (a kernel, not hipMemsetAsync, so the step can
 // be captured in a HIP graph).
 int zero_fill(void *ptr, int64_t n_words, hipStream_t s);
-constexpr int kZeroLists = 6;
+constexpr int kZeroLists = 8;  // (four of a step, three of an empty partition)
 struct ZeroLists {  // buffers of 32-bit words to clear in one launch
   uint32_t *p[kZeroLists];
   int64_t n[kZeroLists];
@@ -182,12 +186,12 @@ int step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, in
 bool params_ok(const pmpm_params *prm);
 bool step_args_ok(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *a, const pmpm_particles *b,
                   const pmpm_spatial *part, const pmpm_nodes *nodes);
-// Workspace the P2G passes of one step use on grid g: tile partials (floats)
-// and tile flags, the clamp record and the stray sums (words).
+// Workspace the P2G passes of one step of n particles use on grid g: tile
+// partials (floats) and tile flags, and the clamp record (words).
 struct P2GWorkspace {
-  size_t partial_floats, tiles, clamp_words, stray_words;
+  size_t partial_floats, tiles, clamp_words;
 };
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w);
+void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n, P2GWorkspace *w);
 // pmpm_partition whose first kernel also clears the buffers of `extra`.
 int partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, const float *x, int n, pmpm_spatial *part,
                        hipStream_t s, const ZeroLists &extra);

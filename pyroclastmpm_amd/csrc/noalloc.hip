@@ -2,11 +2,12 @@
 // without allocating. Its workspace (the radix sort's ping-pong keys, slots and
 // digit histograms, the P2G tile partials and flags, the grid pass's clamp
 // record, the counters) is carved out of one file-scope device array of
-// kScratchBytes, which each GPU holds for the life of the process. Which steps
-// fit is decided by budget_bytes against PMPM_NOALLOC_SCRATCH_BYTES.
+// PMPM_NOALLOC_SCRATCH_BYTES, which each GPU holds for the life of the process.
+// Which steps fit is decided by budget_bytes.
 // Every call on a GPU uses that GPU's copy: calls that overlap on one GPU race.
 #include <hip/hip_runtime.h>
 
+#include <cstdio>
 #include <mutex>
 
 #include "context.hpp"
@@ -15,13 +16,7 @@
 namespace pmpm {
 namespace {
 
-// The budget's partials (budget_bytes) are those of other tiles than the ones
-// in use, which take up to 2.6 times as much (a 2D grid of a single row, linear
-// splines: tiles are four rows high; 28/22 in 3D), and the stray sums are not in
-// it (half as much again there), so the array holds that much more than the
-// budget.
-constexpr size_t kScratchBytes = (size_t)PMPM_NOALLOC_SCRATCH_BYTES / 64 * 200;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[PMPM_NOALLOC_SCRATCH_BYTES];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
@@ -56,10 +51,14 @@ struct Carver {
 // The workspace a step is charged with: the sort's and the clamp record's own
 // sizes, the partials of tiles of 256 cells (1D), 64 x 1 cells (2D; 128 x 1 for
 // linear splines) or 16 x 1 x 4 cells (3D; 32 x 1 x 4 for linear splines, 8 x 1
-// x 4 where larger, typed cubic) and, typed cubic in 2D and 3D, the wrap-around's
-// records, flags and node list. What a caller may ask for
-// (PMPM_NOALLOC_SCRATCH_BYTES) must not move with the kernels' tilings.
-size_t budget_bytes(const pmpm_params &prm, const pmpm_grid &g, size_t n, size_t hist_len, const P2GWorkspace &w) {
+// x 4 where larger, typed cubic) and, typed cubic in 2D and 3D, 64 records of 8
+// floats per cell whose window wraps around, a byte per node and 32 lists of
+// those cells. These are not the kernels' present arrays: what a caller may ask
+// for must not move with their tilings. The present tiles' partials take less
+// but on grids of one to five nodes along y or z, where they take up to twice as
+// much (a single row of 2D cells; in 3D 1.6 times); those steps go without
+// partials once the array is full (p2g_direct_kernel).
+size_t budget_bytes(const pmpm_params &prm, const pmpm_grid &g, size_t n, size_t hist_len, size_t clamp_words) {
   Carver c;
   const int dim = prm.dim, span = prm.shape_fn == PMPM_SF_LINEAR ? 2 : 4;
   const bool cubic = prm.shape_fn == PMPM_SF_CUBIC && prm.node_types_built;
@@ -81,7 +80,7 @@ size_t budget_bytes(const pmpm_params &prm, const pmpm_grid &g, size_t n, size_t
     list = 32 * (1 + cells);
   }
   for (const size_t bytes : {n * 4, n * 4, hist_len * 4, (size_t)16, floats * 4, tiles * 4, wrap_floats * 4, touch * 4,
-                             list * 4, w.clamp_words * 4})
+                             list * 4, clamp_words * 4})
     (void)c.take(bytes);
   return c.used;
 }
@@ -99,25 +98,30 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   const size_t nblocks = (size_t)ceil_div((int64_t)n, kSortTile);
   const size_t hist_len = (size_t)kMaxRadix * nblocks + kMaxRadix;
   P2GWorkspace w;
-  p2g_workspace(*prm, *grid, &w);
+  p2g_workspace(*prm, *grid, (int)a->n, &w);
   Carver c;
   const size_t o_keys = c.take(n * sizeof(uint32_t));
   const size_t o_vals = c.take(n * sizeof(int32_t));
   const size_t o_hist = c.take(hist_len * sizeof(uint32_t));
   const size_t o_counters = c.take(kCounters * sizeof(uint32_t));
-  const size_t o_partials = c.take(w.partial_floats * sizeof(float));
   const size_t o_flags = c.take(w.tiles * sizeof(int32_t));
   const size_t o_clamp = c.take(w.clamp_words * sizeof(float));
-  const size_t o_strays = c.take(w.stray_words * sizeof(float));
-  if (budget_bytes(*prm, *grid, n, hist_len, w) > (size_t)PMPM_NOALLOC_SCRATCH_BYTES || c.used > kScratchBytes) {
-    note_error("pmpm_step_noalloc: the step needs more workspace than PMPM_NOALLOC_SCRATCH_BYTES "
-               "(fewer particles or a smaller grid, or pmpm_step with a context)");
+  const size_t o_partials = c.used;
+  const size_t charge = budget_bytes(*prm, *grid, n, hist_len, w.clamp_words);
+  if (charge > (size_t)PMPM_NOALLOC_SCRATCH_BYTES || c.used > (size_t)PMPM_NOALLOC_SCRATCH_BYTES) {
+    char why[200];
+    snprintf(why, sizeof(why),
+             "pmpm_step_noalloc: the step is charged %zu bytes of workspace, PMPM_NOALLOC_SCRATCH_BYTES is %zu "
+             "(fewer particles or a smaller grid, or pmpm_step with a context)",
+             charge, (size_t)PMPM_NOALLOC_SCRATCH_BYTES);
+    note_error(why);
     return PMPM_ERR_WORKSPACE;
   }
+  const bool tiled = o_partials + w.partial_floats * sizeof(float) <= (size_t)PMPM_NOALLOC_SCRATCH_BYTES;
   unsigned char *base = nullptr;
   int rc = scratch_of_current_device(&base);
   if (rc != PMPM_OK) return rc;
-  // a context over the scratch; every capacity is what this call needs, so no
+  // a context over the scratch, which holds whatever an earlier call left; no
   // entry point below grows (allocates) anything
   pmpm_context ctx;
   PMPM_HIP_CHECK(hipGetDevice(&ctx.device));
@@ -130,18 +134,14 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   ctx.counters = reinterpret_cast<uint32_t *>(base + o_counters);
   ctx.counters_clear = true;  // (the radix path writes what it reads)
   ctx.sort_by_hint = false;  // the full radix sort: its workspace is all carved above
-  ctx.partials = reinterpret_cast<float *>(base + o_partials);
-  ctx.partials_cap = w.partial_floats;
+  ctx.partials = tiled ? reinterpret_cast<float *>(base + o_partials) : nullptr;
+  ctx.partials_cap = tiled ? w.partial_floats : 0;
   ctx.tile_flags = reinterpret_cast<int32_t *>(base + o_flags);
   ctx.tile_flags_cap = w.tiles;
   ctx.clamp_mask = reinterpret_cast<float *>(base + o_clamp);
   ctx.clamp_mask_cap = w.clamp_words;
-  ctx.strays = reinterpret_cast<float *>(base + o_strays);
-  ctx.strays_cap = w.stray_words;
   ctx.stray_flags = reinterpret_cast<int32_t *>(ctx.counters + 4);
-  // (the scratch holds whatever an earlier call left)
-  if ((rc = zero_fill(ctx.strays, (int64_t)w.stray_words, (hipStream_t)stream)) != PMPM_OK) return rc;
-  ctx.strays_clear = true;
+  ctx.fixed_workspace = true;
   // (the context is a plain struct on this stack frame: nothing frees the
   // scratch pieces it points at)
   return step_on(&ctx, prm, grid, musl, a, b, part, nodes, (hipStream_t)stream);

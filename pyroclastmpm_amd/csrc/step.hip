@@ -27,6 +27,12 @@ int pmpm::step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *gr
   // the partition's first kernel also clears the P2G passes' stray flags
   ZeroLists z{};
   z.add(ctx->stray_flags, 2);
+  if (ctx->fixed_workspace) {  // (the stray sums are the node arrays)
+    const int64_t nn = grid->num_cells_total;
+    z.add(nodes->mass, nn);
+    z.add(nodes->mom, nn * prm->dim);
+    z.add(nodes->mom_nt, nn * prm->dim);
+  }
   int rc = partition_clearing(ctx, prm->dim, grid, a->x, a->n, part, s, z);
   if (rc != PMPM_OK) return rc;
   if ((rc = do_p2g(ctx, *prm, *grid, *a, *part, *nodes, s, true)) != PMPM_OK) return rc;

@@ -1359,6 +1359,37 @@ __global__ __launch_bounds__(256 * ROWS) void p2g_mfma_kernel(pmpm_params prm, p
   }
 }
 
+// P2G (MODE 0) or MUSL re-map (MODE 1) of every particle over its own window,
+// straight to the stray sums: for steps whose workspace has no room for the tile
+// partials (pmpm_step_noalloc). Bound by its global atomics, up to 64
+// nodes of 7 fields per particle.
+template <int D, int SF, int MODE>
+__global__ __launch_bounds__(256) void p2g_direct_kernel(pmpm_params prm, pmpm_grid g, pmpm_particles in,
+                                                         pmpm_particles out, pmpm_spatial part, Strays nodes,
+                                                         int fext) {
+  const int n = in.n, j = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (j == 0) *nodes.flag = 1;
+  if (j >= n) return;
+  const int slot = part.sorted[j];
+  if (part.hash[slot] >= (uint32_t)g.num_cells_total) return;  // (in no cell: not deposited)
+  const float m = in.mass[slot];
+  float x[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, fe[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    x[a] = in.x[(int64_t)a * n + slot];
+    v[a] = MODE == 0 ? in.v[(int64_t)a * n + slot] : out.v[(int64_t)a * n + j];
+  }
+  Sym A = sym_zero();
+  if (MODE == 0) {
+    const float vol = in.volume[slot];
+    const Sym s = load_sym(in.stress, n, slot);
+    A = Sym{-vol * s.xx, -vol * s.yy, -vol * s.zz, -vol * s.xy, -vol * s.xz, -vol * s.yz};
+    if (fext) planar_force<D>(prm, g, x, v, vol, m, fe);
+  }
+#pragma unroll 1
+  for (int sy = 0; sy < 4; ++sy) p2g_stray<D, SF, MODE>(prm, g, nodes, in.x, n, slot, sy, m, v, A, fe);
+}
+
 // Geometry of the P2G tiles for the grid kernel's gather.
 struct TileGeom {
   int tiles[3];  // tiles per axis
@@ -1573,11 +1604,14 @@ __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g,
       gather_partials<D, NV, TG>(tg, partials, flags, ids0, acc);
     }
     if (*strays.flag) {
-      float *a0 = GATHER == 1 ? strays.mass : strays.mom_nt;  // (mass, mom and mom_nt lie one after the other)
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
-        acc[k] += a0[(int64_t)k * nn + i];
-        a0[(int64_t)k * nn + i] = 0.f;
+        // (mass, momentum, force)
+        float *a0 = GATHER == 1 && k == 0 ? strays.mass
+                                          : (GATHER == 1 && k <= D ? strays.mom + (int64_t)(k - 1) * nn
+                                                                   : strays.mom_nt + (int64_t)(GATHER == 1 ? k - 1 - D : k) * nn);
+        acc[k] += a0[i];
+        a0[i] = 0.f;
       }
     }
     if constexpr (GATHER == 1) {
@@ -2191,7 +2225,7 @@ static void launch_p2g_mfma(const pmpm_params &prm, const pmpm_grid &g, const pm
 
 // mode 0: P2G, 1: MUSL first map (G2P-style) and re-map, 2: adjoint scatter of
 // the records `rec` (never launched without them). 3D: the matrix-core tiles;
-// 1D and 2D: tiles of rows.
+// 1D and 2D: tiles of rows. Without partials: every particle by itself.
 template <int D, int SF>
 void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles &in, const pmpm_particles &out,
                 const pmpm_spatial &part, const pmpm_nodes &nodes, int mode, float *partials, int32_t *flags,
@@ -2200,6 +2234,17 @@ void launch_p2g(const pmpm_params &prm, const pmpm_grid &g, const pmpm_particles
   if (mode == 1 && in.n > 0)
     PMPM_LAUNCH((g2p_kernel<D, SF, 1>), (::pmpm::kname("g2p_kernel", {(long)(D), (long)(SF), (long)(1)})),
                 dim3((unsigned)ceil_div(in.n, kG2PThreads)), dim3(kG2PThreads), 0, s, prm, g, in, out, part, nodes, 1);
+  if (!partials) {  // (the caller has cleared the tile flags)
+    const dim3 grid((unsigned)ceil_div(in.n, 256)), block(256);
+    if (in.n <= 0) return;
+    if (mode == 0)
+      PMPM_LAUNCH((p2g_direct_kernel<D, SF, 0>), (::pmpm::kname("p2g_direct_kernel", {(long)D, (long)SF, 0L})), grid,
+                  block, 0, s, prm, g, in, out, part, strays, has_planar(prm) ? 1 : 0);
+    else
+      PMPM_LAUNCH((p2g_direct_kernel<D, SF, 1>), (::pmpm::kname("p2g_direct_kernel", {(long)D, (long)SF, 1L})), grid,
+                  block, 0, s, prm, g, in, out, part, strays, 0);
+    return;
+  }
   if constexpr (D == 3) {
     if (mfma_tiles(g, in.n).cells == 4)
       launch_p2g_mfma<SF, 4, 1>(prm, g, in, out, part, strays, mode, partials, flags, s, rec);
@@ -2238,8 +2283,10 @@ static unsigned pass_blocks(const TileGeom &tg) {
   return (unsigned)ceil_div((int64_t)tile_count(tg) * tg.T[0] * tg.T[1] * tg.T[2], (int64_t)256);
 }
 // The stray sums of a P2G (mode 0), re-map (mode 1) or adjoint scatter (mode 2).
-static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, int mode) {
+static Strays stray_sums(const pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const pmpm_nodes &nodes,
+                         int mode) {
   const int64_t nn = g.num_cells_total;
+  if (ctx->fixed_workspace) return {nodes.mass, nodes.mom, nodes.mom_nt, ctx->stray_flags + mode};
   return {ctx->strays, ctx->strays + nn, ctx->strays + (1 + prm.dim) * nn, ctx->stray_flags + mode};
 }
 // gather: 0 = node arrays only, 1 = from the P2G tile partials, 2 = mom_nt from
@@ -2248,7 +2295,7 @@ int launch_grid(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
                 int b0, int b1, int remap, int gather, hipStream_t s, int n, int skip_mom_nt = 0) {
   const TileGeom tg = tile_geom(prm, g, gather, n);
   const unsigned blocks = pass_blocks(tg);
-  const Strays strays = gather ? stray_sums(ctx, prm, g, gather - 1) : Strays{};
+  const Strays strays = gather ? stray_sums(ctx, prm, g, nodes, gather - 1) : Strays{};
   const float *partials = gather ? ctx->partials : nullptr;
   const int32_t *flags = gather ? ctx->tile_flags : nullptr;
   // the clamp record of a pass that applies node conditions (not the MUSL
@@ -2295,19 +2342,16 @@ static bool particles_ok(const pmpm_particles *p) {
                         p->flags && p->id));
 }
 
-// Partials and tile flags of the P2G passes on grid g, for any particle count
-// (a small grid's passes use either tile width).
-static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, size_t *floats, size_t *tiles) {
-  *tiles = *floats = 0;
-  for (const int n : {0, kSmallParticles + 1}) {
-    const TileGeom tg = tile_geom(prm, g, 1, n);
-    *tiles = std::max(*tiles, tile_count(tg));
-    *floats = std::max(*floats, tile_count(tg) * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2]);
-  }
+// Partials and tile flags of the P2G passes of n particles on grid g.
+static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, int n, size_t *floats, size_t *tiles) {
+  const TileGeom tg = tile_geom(prm, g, 1, n);
+  *tiles = std::max(*tiles, tile_count(tg));
+  *floats = std::max(*floats, tile_count(tg) * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2]);
 }
 static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, hipStream_t s) {
+  if (ctx->fixed_workspace) return ctx->partials ? PMPM_OK : zero_fill(ctx->tile_flags, (int64_t)ctx->tile_flags_cap, s);
   size_t floats = 0, tiles = 0;
-  partial_sizes(prm, g, &floats, &tiles);
+  for (const int n : {0, kSmallParticles + 1}) partial_sizes(prm, g, n, &floats, &tiles);  // (any particle count)
   int rc = ensure_partials(ctx, floats, tiles);
   if (rc != PMPM_OK) return rc;
   // the grid pass's clamp record (one byte per node, in words of 4)
@@ -2324,10 +2368,9 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   return clear_on_stream(z, ctx->strays_clear, s);
 }
 
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, P2GWorkspace *w) {
+void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n, P2GWorkspace *w) {
   *w = P2GWorkspace{};
-  partial_sizes(prm, g, &w->partial_floats, &w->tiles);
-  w->stray_words = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
+  partial_sizes(prm, g, n, &w->partial_floats, &w->tiles);
   w->clamp_words = ((size_t)g.num_cells_total + 3) / 4;
 }
 
@@ -2340,7 +2383,7 @@ int do_p2g(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, const 
   if (rc != PMPM_OK) return rc;
   if (!zeroed && (rc = zero_fill(ctx->stray_flags, 1, s)) != PMPM_OK) return rc;
   PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, p, p, part, nodes, 0, ctx->partials, ctx->tile_flags,
-                    stray_sums(ctx, prm, g, 0), s);
+                    stray_sums(ctx, prm, g, nodes, 0), s);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -2385,7 +2428,7 @@ int do_musl_map(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, c
   if (rc != PMPM_OK) return rc;
   if (!zeroed && (rc = zero_fill(ctx->stray_flags + 1, 1, s)) != PMPM_OK) return rc;
   PMPM_DISPATCH_DSF(prm.dim, prm.shape_fn, launch_p2g, prm, g, in, out, part, nodes, 1, ctx->partials,
-                    ctx->tile_flags, stray_sums(ctx, prm, g, 1), s);
+                    ctx->tile_flags, stray_sums(ctx, prm, g, nodes, 1), s);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }
@@ -3519,7 +3562,7 @@ extern "C" int pmpm_adjoint_step(pmpm_context *ctx, const pmpm_params *prm, cons
     return rc;
   const int groups = ceil_div(n, 256), entries = 4 * prm->num_materials;
   if ((rc = ensure_buffer(ctx->adj_pb, ctx->adj_pb_cap, (size_t)groups * entries)) != PMPM_OK) return rc;
-  const Strays strays = stray_sums(ctx, *prm, g, 2);
+  const Strays strays = stray_sums(ctx, *prm, g, *nodes, 2);
   // G2P adjoint (material parameter adjoints per workgroup, then summed into
   // param_bar), then the scatter of its records to the nodes
   PMPM_DISPATCH_DSF(D, prm->shape_fn, launch_adjoint_particles, *prm, g, *state, *out_bar, *in_bar, *part, *nodes,
