@@ -10,6 +10,17 @@
 
 namespace pmpm {
 
+// LDS writes of a wave visible to all its lanes (and its earlier reads done)
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// A workgroup barrier that orders LDS accesses only: __syncthreads also waits
+// for the wave's global loads and stores in flight, which would drain a
+// kernel's prefetches.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // ---------------------------------------------------------------------------
 // Spline traits. SPAN = node extent per cell (tile halo), ENTRIES = nodes one
 // particle touches per axis. NLO = first node offset relative to the cell.

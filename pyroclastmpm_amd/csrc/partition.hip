@@ -4,6 +4,8 @@
 // (spatialpartition_inline.h:49-115, spatialpartition.cpp:77-136).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -151,25 +153,78 @@ __global__ __launch_bounds__(256) void scan_columns_kernel(uint32_t *__restrict_
   if (t == 255) totals[blockIdx.x] = part[255];
 }
 
-// Stable scatter of one radix pass (digits of RB bits). Within a round of
-// kSortBlock keys (thread order == input order) a lane's rank among
-// same-digit lanes of its wave comes from RB ballots; per-wave counts are
-// combined per digit in LDS (thread d owns digit d).
+// Stable scatter of the keys [first, end) by a digit of RB bits, each digit's
+// next place in base[]. Within a round of kSortBlock keys (thread order == input
+// order) a lane's rank among same-digit lanes of its wave comes from RB ballots;
+// per-wave counts are combined per digit in LDS (thread d owns digit d).
+template <int RB> struct ScatterLds {
+  uint32_t base[1 << RB];
+  uint32_t wcnt[kSortBlock / 64][1 << RB];
+};
+template <int RB>
+__device__ inline void scatter_tile(const uint32_t *__restrict__ keys_in, const int32_t *__restrict__ vals_in,
+                                    uint32_t *__restrict__ keys_out, int32_t *__restrict__ vals_out, int64_t first,
+                                    int64_t end, int shift, ScatterLds<RB> &lds) {
+  constexpr int R = 1 << RB, W = kSortBlock / 64;
+  static_assert(R <= kSortBlock, "one digit per thread");
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int w = t >> 6;
+  const bool owner = t < R;
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (int64_t r = first; r < end; r += kSortBlock) {
+    if (owner) {
+#pragma unroll
+      for (int q = 0; q < W; ++q) lds.wcnt[q][t] = 0u;
+    }
+    __syncthreads();
+    const int64_t i = r + t;
+    const bool valid = i < end;
+    const uint32_t key = valid ? keys_in[i] : 0u;
+    const uint32_t d = (key >> shift) & (R - 1);
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int bit = 0; bit < RB; ++bit) {
+      const bool on = (d >> bit) & 1u;
+      const uint64_t m = __ballot(on);
+      peers &= on ? m : ~m;
+    }
+    const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
+    if (valid && rank == 0) lds.wcnt[w][d] = (uint32_t)__popcll(peers);
+    __syncthreads();
+    if (owner) {
+      uint32_t run = lds.base[t];
+#pragma unroll
+      for (int q = 0; q < W; ++q) {
+        const uint32_t c = lds.wcnt[q][t];
+        lds.wcnt[q][t] = run;
+        run += c;
+      }
+      lds.base[t] = run;
+    }
+    __syncthreads();
+    if (valid) {
+      const uint32_t pos = lds.wcnt[w][d] + rank;
+      keys_out[pos] = key;
+      vals_out[pos] = vals_in ? vals_in[i] : (int32_t)i;
+    }
+    __syncthreads();
+  }
+}
+
+// One radix pass: the digit bases, then the tile's scatter.
 template <int RB>
 __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     const uint32_t *__restrict__ keys_in, const int32_t *__restrict__ vals_in, uint32_t *__restrict__ keys_out,
     int32_t *__restrict__ vals_out, int n, int shift, const uint32_t *__restrict__ hist, int nblocks,
     const uint32_t *__restrict__ totals) {
   constexpr int R = 1 << RB, W = kSortBlock / 64;
-  static_assert(R <= kSortBlock, "one digit per thread");
-  __shared__ uint32_t base[R];
-  __shared__ uint32_t wcnt[W][R];
+  __shared__ ScatterLds<RB> lds;
   __shared__ uint32_t wsum[W];
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int w = t >> 6;
   const bool owner = t < R;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // digit bases: exclusive scan of the R column totals (thread d owns digit
   // d): a shuffle scan within each wave, then the wave totals before it
   const uint32_t tot = owner ? totals[t] : 0u;
@@ -183,46 +238,9 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
   __syncthreads();
   uint32_t before = 0u;
   for (int q = 0; q < w; ++q) before += wsum[q];
-  if (owner) base[t] = before + incl - tot + hist[(int64_t)t * nblocks + blockIdx.x];
+  if (owner) lds.base[t] = before + incl - tot + hist[(int64_t)t * nblocks + blockIdx.x];
   const int64_t tile = (int64_t)blockIdx.x * kSortTile;
-  for (int r = 0; r < kSortItems; ++r) {
-    if (owner) {
-#pragma unroll
-      for (int q = 0; q < W; ++q) wcnt[q][t] = 0u;
-    }
-    __syncthreads();
-    const int64_t i = tile + (int64_t)r * kSortBlock + t;
-    const bool valid = i < n;
-    const uint32_t key = valid ? keys_in[i] : 0u;
-    const uint32_t d = (key >> shift) & (R - 1);
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int bit = 0; bit < RB; ++bit) {
-      const bool on = (d >> bit) & 1u;
-      const uint64_t m = __ballot(on);
-      peers &= on ? m : ~m;
-    }
-    const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
-    if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    if (owner) {
-      uint32_t run = base[t];
-#pragma unroll
-      for (int q = 0; q < W; ++q) {
-        const uint32_t c = wcnt[q][t];
-        wcnt[q][t] = run;
-        run += c;
-      }
-      base[t] = run;
-    }
-    __syncthreads();
-    if (valid) {
-      const uint32_t pos = wcnt[w][d] + rank;
-      keys_out[pos] = key;
-      vals_out[pos] = vals_in ? vals_in[i] : (int32_t)i;
-    }
-    __syncthreads();
-  }
+  scatter_tile<RB>(keys_in, vals_in, keys_out, vals_out, tile, min(tile + kSortTile, (int64_t)n), shift, lds);
 }
 
 // Cell ranges over the sorted hashes (spatialpartition_inline.h:85-115);
@@ -257,8 +275,6 @@ __global__ void cell_range_kernel(const uint32_t *__restrict__ hs, int n, uint32
 //   mover i:         out_start[c] + movers of c before slot i
 //                    + clamp(S[i] - stayers with key < c, 0, stayers of c)
 // (stayers are sorted by key, so the first S[i] of them are those before i).
-// An unsorted hint makes every particle a mover; any hint gives the stable
-// sort, a good one few movers.
 //
 // Four launches whatever the mover count: classify (keys, stay bits, counts
 // per cell), scan (cells), movers (each into its cell's part of a list, in any
@@ -271,6 +287,15 @@ __global__ void cell_range_kernel(const uint32_t *__restrict__ hs, int n, uint32
 // cost their launch also when they had nothing to do: ten launches and 50 us
 // at 1.08M particles, 39 us with these four. Small scenes gain most (17k
 // particles: 45 us of radix sort, 17 us).
+//
+// A hint that says little (the first call on new buffers, particles in another
+// order, most of them in another cell) is not merged: the same launches then
+// sort all particles by their keys' high and low digits ("cold"; see
+// hint_scan_kernel). Per-cell counts cost such a call an atomic per particle on
+// a few cache lines, and ranking within a cell the square of its particles:
+// partition of 20,000 particles in random order, 8 per cell, from a zero hint 70
+// -> 39 us (radix sort: 51), 2,000 per cell 302 -> 38 (29, one digit); of
+// 1,000,000, 27 per cell 819 -> 90 (75), 2,000 per cell 10,500 -> 104 (69).
 constexpr int kHintBlock = 256;     // particles per workgroup of classify and place
 constexpr int kHintCells = 1024;    // cells per workgroup of the scan
 constexpr int kHintCellBits = 10;
@@ -278,6 +303,27 @@ constexpr int kHintSlots = 4;       // cell blocks a classify workgroup sums in 
 constexpr int kMoverBlock = 1024;   // threads of the movers pass
 constexpr int kHeavyMovers = 2048;
 static_assert((1 << kHintCellBits) == kHintCells, "one cell per thread in the cell scan");
+// A classify workgroup is cold when over half of its particles moved; the call
+// is cold when the hint is unsorted or flat or over a sixteenth of the workgroups
+// are, but no more than kColdLimit (counting 256 scattered particles costs
+// atomics: 1,000,000 in random order, 244 workgroups counted: classify 61 us, 32:
+// 29).
+constexpr uint32_t kUnsorted = 0x80000000u;
+constexpr int kColdLimit = 32;
+constexpr int kColdBits = 10, kColdBuckets = 1 << kColdBits;  // high digit of a cold sort
+constexpr int kColdCells = 1024;    // cells of a bucket that a place workgroup counts at a time
+static_assert(kMoverBlock == kSortBlock && kColdBits <= kMaxRadixBits, "the cold scatter is a radix pass");
+// (a hint that is one key throughout, as new buffers' are, is told by its ends)
+__device__ inline bool flat_hint(const uint32_t *__restrict__ hint, int n) { return hint[0] == hint[n - 1]; }
+struct Cold {
+  uint32_t limit;            // cold workgroups of a call that is still merged
+  int shift, buckets;        // bucket of a key: key >> shift
+  int tile, tiles;           // particles per tile of the cold sort
+  uint32_t *hist;            // [tiles][kColdBuckets] particles per tile and bucket, then each bucket's first place
+  uint32_t *keys;            // the particles by bucket, in slot order
+  int32_t *slots;
+  __device__ bool is(uint32_t count) const { return count > limit; }
+};
 
 // Exclusive scan over a workgroup of THREADS threads; every thread gets its
 // prefix and the total. `w` holds THREADS / 64 words of LDS.
@@ -317,18 +363,22 @@ __device__ inline uint32_t cell_key(const float *__restrict__ x, int n, int i, c
 // Cell key per particle (as hash_kernel), its class against the hint as a bit
 // (stay[i / 64]), and the counts: per cell and per block of cells, stayers and
 // movers (a run of lanes with one key and one class adds its length once);
-// stayers per workgroup. flags[0] is set when the hint is not sorted. Blocks
-// past the particles only clear `clear`.
+// stayers per workgroup. *cold counts the cold workgroups (kUnsorted: the hint
+// is not sorted); once the call is cold, what is left of the counting is
+// skipped. Blocks past the particles only clear `clear`.
 template <int D>
 __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
     const float *__restrict__ x, int n, pmpm_grid g, const uint32_t *__restrict__ hint, uint32_t *__restrict__ hash,
     int32_t *__restrict__ bins, uint32_t *__restrict__ cnt, uint32_t *__restrict__ cbt, uint32_t *__restrict__ pblk,
-    uint64_t *__restrict__ stay_bits, int npb, int ncb, uint32_t *__restrict__ flags, ZeroLists clear) {
+    uint64_t *__restrict__ stay_bits, int npb, int ncb, uint32_t *__restrict__ cold, Cold cd, ZeroLists clear) {
   // per-class sums for the kHintSlots blocks of cells from the workgroup's
   // first key on (one global atomic per slot and class at the end: the
   // workgroups of a stretch of particles share these counters)
   __shared__ uint32_t slot_sum[kHintSlots][2];
-  __shared__ uint32_t stayers, first_block;
+  // the waves' stayers, kUnsorted in the top bit (read as one word of four)
+  __shared__ __attribute__((aligned(16))) uint32_t wave_stay[kHintBlock / 64];
+  __shared__ uint32_t first_block, skip;
+  static_assert(kHintBlock == 256, "four waves");
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   for (int q = 0; q < clear.count; ++q)
@@ -338,7 +388,7 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
   const int i = (int)t;
   const bool valid = i < n;  // a prefix of each wave
   uint32_t key = 0u;
-  bool stay = false;
+  bool stay = false, falls = false;
   if (valid) {
     int b[3] = {0, 0, 0};
     key = cell_key<D>(x, n, i, g, b);
@@ -348,19 +398,32 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
       for (int a = 0; a < D; ++a) bins[(int64_t)a * n + i] = b[a];
     }
     const uint32_t p = hint[i];
-    if (i + 1 < n && p > hint[i + 1]) atomicOr(&flags[0], 1u);
+    falls = i + 1 < n && p > hint[i + 1];
     stay = key == p;
   }
-  if (threadIdx.x < 2 * kHintSlots) (&slot_sum[0][0])[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) {
-    stayers = 0u;
-    first_block = key >> kHintCellBits;
+  const uint64_t bits = __ballot(stay), fall_bits = __ballot(falls);
+  if (lane == 0) {
+    if (valid) stay_bits[i >> 6] = bits;
+    wave_stay[threadIdx.x >> 6] = (uint32_t)__popcll(bits) | (fall_bits ? kUnsorted : 0u);
   }
+  if (threadIdx.x < 2 * kHintSlots) (&slot_sum[0][0])[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) first_block = key >> kHintCellBits;
   __syncthreads();
-  const uint64_t bits = __ballot(stay);
-  if (lane == 0 && valid) {
-    stay_bits[i >> 6] = bits;
-    atomicAdd(&stayers, (uint32_t)__popcll(bits));
+  const uint4 ws = *reinterpret_cast<const uint4 *>(wave_stay);
+  const uint32_t unsorted = (ws.x | ws.y | ws.z | ws.w) & kUnsorted;
+  const uint32_t stayers = (ws.x + ws.y + ws.z + ws.w) & 0xffffu;
+  const int movers = min(n - (int)blockIdx.x * kHintBlock, kHintBlock) - (int)stayers;
+  if (flat_hint(hint, n)) return;  // block-uniform
+  if (movers > kHintBlock / 2 || unsorted) {  // block-uniform
+    if (threadIdx.x == 0) {
+      // (the count only grows, so a workgroup that sees it past the limit may
+      // stop: the call is cold)
+      bool stop = cd.is(__hip_atomic_load(cold, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      if (!stop) stop = cd.is(unsorted ? atomicOr(cold, kUnsorted) | kUnsorted : atomicAdd(cold, 1u) + 1u);
+      skip = stop ? 1u : 0u;
+    }
+    __syncthreads();
+    if (skip) return;
   }
   const uint32_t cb0 = first_block;
   const uint32_t pk = (uint32_t)__shfl_up((int)key, 1, 64);
@@ -388,27 +451,50 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
   }
 }
 
-// Block 0: the stayers before each particle block, and whether the hint was
-// unsorted (counters[2]; then every particle counts as a mover). Blocks 1 ..
-// ncb: 1024 cells each (cells 0..ncells, the last holding the out-of-grid
-// particles), four consecutive cells per thread: the exclusive scans of the
-// stayer and mover counts give each cell's record {first slot, stayers before,
-// stayers, movers}, its range (cell_start/cell_end, 0 for an empty cell), for
-// the last cell the out-of-grid count (counters[0]); the stayer counts are
-// cleared for the next call, the mover counts are left to the movers pass, and
-// cells with many movers are listed (counters[3] of them).
+// Block 0: the stayers before each particle block, and whether the call is cold
+// (counters[2]). Blocks 1 .. ncb: 1024 cells each (cells 0..ncells, the last
+// holding the out-of-grid particles), four consecutive cells per thread: the
+// exclusive scans of the stayer and mover counts give each cell's record {first
+// slot, stayers before, stayers, movers}, its range (cell_start/cell_end, 0 for
+// an empty cell), for the last cell the out-of-grid count (counters[0]); the
+// stayer counts are cleared for the next call, the mover counts are left to the
+// movers pass, and cells with many movers are listed (counters[3] of them).
+//
+// Cold: the particles are sorted here and in the two launches after, by the high
+// digit of their keys (kColdBuckets buckets at most) and then, a workgroup per
+// bucket, by cell. This pass counts each tile's particles per bucket; the movers
+// pass scatters the tiles stably to the buckets (every workgroup adds up the
+// tiles before its own); the place pass counts and places a bucket's particles
+// cell by cell in LDS and writes the cells' ranges. No global atomics, and the
+// time does not depend on the particles per cell. What the classify pass had
+// counted is cleared on the way.
 constexpr int kScanThreads = kHintCells / 4;
-__global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(uint32_t ncells, int npb,
+__global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(int n, uint32_t ncells, int npb, int ncb,
                                                                  uint32_t *__restrict__ cnt,
                                                                  const uint32_t *__restrict__ cbt,
                                                                  uint32_t *__restrict__ pblk,
                                                                  uint32_t *__restrict__ counters,
                                                                  int4 *__restrict__ info, int32_t *__restrict__ cstart,
                                                                  int32_t *__restrict__ cend, int32_t *__restrict__ heavy,
-                                                                 uint32_t heavy_cap) {
+                                                                 uint32_t heavy_cap, const uint32_t *__restrict__ hash,
+                                                                 const uint32_t *__restrict__ hint, Cold cd) {
   __shared__ uint64_t w2[kScanThreads / 64];
-  const bool unsorted = counters[1] != 0u;
+  __shared__ uint32_t bucket[kColdBuckets];
+  const bool cold = cd.is(counters[1]) || flat_hint(hint, n);
   const int t = threadIdx.x;
+  if (cold) {
+    for (int tile = (int)blockIdx.x; tile < cd.tiles; tile += (int)gridDim.x) {
+      for (int k = t; k < kColdBuckets; k += kScanThreads) bucket[k] = 0u;
+      __syncthreads();
+      const int64_t first = (int64_t)tile * cd.tile, end = min(first + cd.tile, (int64_t)n);
+      for (int64_t i = first + t; i < end; i += kScanThreads) atomicAdd(&bucket[hash[i] >> cd.shift], 1u);
+      __syncthreads();
+      for (int k = t; k < kColdBuckets; k += kScanThreads) cd.hist[(size_t)tile * kColdBuckets + k] = bucket[k];
+      __syncthreads();
+    }
+    if (blockIdx.x == 0 && t == 0) counters[2] = 1u;
+    return;
+  }
   if (blockIdx.x == 0) {
     uint32_t base = 0u;
     for (int b0 = 0; b0 < npb; b0 += 4 * kScanThreads) {
@@ -429,9 +515,10 @@ __global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(uint32_t ncells
       }
       base += (uint32_t)tot;
     }
-    if (t == 0) counters[2] = unsorted ? 1u : 0u;
+    if (t == 0) counters[2] = 0u;
     return;
   }
+  if ((int)blockIdx.x > ncb) return;  // (a cold call's tiles)
   const int b = (int)blockIdx.x - 1;
   const int64_t c0 = (int64_t)b * kHintCells + 4 * t;
   uint32_t st[4], mv[4];  // (loaded before the prefix sums' barriers)
@@ -462,15 +549,7 @@ __global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(uint32_t ncells
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     any = any || (st[q] | mv[q]) != 0u;
-    if (unsorted) {
-      mv[q] += st[q];
-      st[q] = 0u;
-    }
     own += ((uint64_t)st[q] << 32) | mv[q];
-  }
-  if (unsorted) {
-    mover_before += stay_before;
-    stay_before = 0u;
   }
   uint64_t tot;
   const uint64_t ex = block_exclusive_scan<kScanThreads, uint64_t>(own, w2, tot);
@@ -510,16 +589,16 @@ __global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(uint32_t ncells
 }
 
 // Is particle i a mover? (stay bits of the classify pass)
-__device__ inline bool is_mover(const uint64_t *__restrict__ stay_bits, int i, bool unsorted) {
-  return unsorted || !((stay_bits[i >> 6] >> (i & 63)) & 1ull);
+__device__ inline bool is_mover(const uint64_t *__restrict__ stay_bits, int i) {
+  return !((stay_bits[i >> 6] >> (i & 63)) & 1ull);
 }
 
 // Each mover's slot into its cell's part of `list` ([movers with a smaller
 // key] on): taken from the cell's count downward, in any order; heavy cells by
 // a workgroup each, in slot order. The counts end at zero, as the next call
-// needs them, and block 0 clears the per-block cell counts and the unsorted
-// flag.
-__global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_t ncells, int ncb, int words,
+// needs them, and block 0 clears the per-block cell counts and the count of cold
+// workgroups. Cold: the scatter of a tile to the buckets.
+__global__ __launch_bounds__(kMoverBlock, 8) void hint_movers_kernel(int n, uint32_t ncells, int ncb, int words,
                                                                   const uint32_t *__restrict__ hash,
                                                                   const uint64_t *__restrict__ stay_bits,
                                                                   const int4 *__restrict__ info,
@@ -527,13 +606,38 @@ __global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_
                                                                   uint32_t *__restrict__ cbt,
                                                                   uint32_t *__restrict__ counters,
                                                                   const int32_t *__restrict__ heavy,
-                                                                  uint32_t heavy_cap, int32_t *__restrict__ list) {
+                                                                  uint32_t heavy_cap, int32_t *__restrict__ list,
+                                                                  Cold cd) {
   __shared__ uint32_t w[kMoverBlock / 64];
+  __shared__ ScatterLds<kColdBits> lds;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const bool unsorted = counters[2] != 0u;
   if (blockIdx.x == 0) {
     for (int j = t; j < 2 * ncb; j += kMoverBlock) cbt[j] = 0u;
     if (t == 0) counters[1] = 0u;
+  }
+  if (counters[2] != 0u) {  // cold
+    const int tile = (int)blockIdx.x;
+    if (tile >= cd.tiles) return;
+    // a bucket's first place, and this tile's: thread t's bucket is t
+    // (sixteen rows in flight: each is a trip to memory)
+    uint32_t total = 0u, mine = 0u;
+    for (int j = 0; j < cd.tiles; j += 16) {
+      uint32_t v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = cd.hist[(size_t)min(j + q, cd.tiles - 1) * kColdBuckets + t];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        mine += j + q < tile ? v[q] : 0u;
+        total += j + q < cd.tiles ? v[q] : 0u;
+      }
+    }
+    uint32_t all;
+    const uint32_t first = block_exclusive_scan<kMoverBlock, uint32_t>(total, w, all);
+    if (tile == 0) cd.hist[(size_t)cd.tiles * kColdBuckets + t] = first;
+    lds.base[t] = first + mine;
+    const int64_t i0 = (int64_t)tile * cd.tile;
+    scatter_tile<kColdBits>(hash, nullptr, cd.keys, cd.slots, i0, min(i0 + cd.tile, (int64_t)n), cd.shift, lds);
+    return;
   }
   const uint32_t nheavy = min(counters[3], heavy_cap);
   for (uint32_t h = blockIdx.x; h < nheavy; h += gridDim.x) {  // block-uniform
@@ -548,7 +652,7 @@ __global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int i = i0 + 4 * t + q;
-        mine[q] = i < n && hash[i] == c && is_mover(stay_bits, i, unsorted);
+        mine[q] = i < n && hash[i] == c && is_mover(stay_bits, i);
         m += mine[q] ? 1u : 0u;
       }
       uint32_t all;
@@ -571,7 +675,7 @@ __global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_
   for (int q = 0; q < words; ++q) {
     const int i = first + 64 * q + lane;
     const uint64_t stay = (uint64_t)__shfl((unsigned long long)bits, q);
-    const bool mover = i < n && (unsorted || !((stay >> lane) & 1ull));
+    const bool mover = i < n && !((stay >> lane) & 1ull);
     if (!__ballot(mover)) continue;
     if (!mover) continue;
     const uint32_t c = hash[i];
@@ -582,9 +686,126 @@ __global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_
   }
 }
 
+// The place pass of a cold call: one bucket's particles (in slot order) counted
+// per cell, the cells' ranges, and the particles to their places; kColdCells of
+// the bucket's cells at a time. Each wave takes a quarter of the particles with
+// counters of its own, so the waves need no barrier while they place: a lane's
+// rank among its wave's particles of the same cell comes from ballots over the
+// cell's bits.
+struct ColdCounters {
+  uint32_t next[kHintBlock / 64][kColdCells];
+};
+__device__ inline void place_bucket(int bucket, int n, uint32_t ncells, const Cold &cd, uint32_t *__restrict__ cnt,
+                                    uint32_t *__restrict__ counters, int32_t *__restrict__ cstart,
+                                    int32_t *__restrict__ cend, uint32_t *__restrict__ hash_sorted,
+                                    int32_t *__restrict__ sorted, ColdCounters &lds, uint32_t *w) {
+  constexpr int W = kHintBlock / 64, F = 2;  // F: rounds whose loads are in flight together
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const uint32_t *starts = cd.hist + (size_t)cd.tiles * kColdBuckets;
+  const int first = (int)starts[bucket], end = bucket + 1 < cd.buckets ? (int)starts[bucket + 1] : n;
+  const int quarter = (end - first + W - 1) / W;
+  const int j_first = min(first + wv * quarter, end), j_end = min(j_first + quarter, end);
+  const int64_t cells_end = min((int64_t)(bucket + 1) << cd.shift, (int64_t)ncells + 1);
+  uint32_t *next = lds.next[wv];
+  uint32_t placed = (uint32_t)first;
+  for (int64_t r0 = (int64_t)bucket << cd.shift; r0 < cells_end; r0 += kColdCells) {  // block-uniform
+    const int m = (int)min(cells_end - r0, (int64_t)kColdCells);
+    const uint32_t c0 = (uint32_t)r0;
+    const int per = (m + kHintBlock - 1) / kHintBlock;  // cells of a thread
+    __syncthreads();  // (the counters of the range before are read)
+    for (int c = t; c < per * kHintBlock; c += kHintBlock)
+#pragma unroll
+      for (int q = 0; q < W; ++q) lds.next[q][c] = 0u;
+    __syncthreads();
+    for (int j = j_first + lane; j < j_end; j += 64 * F) {
+      uint32_t c[F];
+#pragma unroll
+      for (int q = 0; q < F; ++q) c[q] = j + 64 * q < j_end ? cd.keys[j + 64 * q] - c0 : 0xffffffffu;
+#pragma unroll
+      for (int q = 0; q < F; ++q)
+        if (c[q] < (uint32_t)m) atomicAdd(&next[c[q]], 1u);
+    }
+    __syncthreads();
+    uint32_t sum = 0u;
+    for (int c = t * per; c < (t + 1) * per; ++c)
+#pragma unroll
+      for (int q = 0; q < W; ++q) sum += lds.next[q][c];
+    uint32_t all;
+    uint32_t at = placed + block_exclusive_scan<kHintBlock, uint32_t>(sum, w, all);
+    placed += all;
+    for (int c = t * per; c < (t + 1) * per; ++c) {
+      const uint32_t start = at;
+#pragma unroll
+      for (int q = 0; q < W; ++q) {
+        const uint32_t count = lds.next[q][c];
+        lds.next[q][c] = at;
+        at += count;
+      }
+      if (c < m) {
+        const int64_t cell = r0 + c;
+        *reinterpret_cast<uint2 *>(cnt + 2 * cell) = make_uint2(0u, 0u);
+        if (cell < (int64_t)ncells) {
+          cstart[cell] = at > start ? (int32_t)start : 0;
+          cend[cell] = at > start ? (int32_t)at : 0;
+        } else {
+          counters[0] = at - start;  // out-of-grid particles
+        }
+      }
+    }
+    __syncthreads();
+    const int cell_bits = 32 - __clz(m - 1);  // (0 for one cell: __clz(0) is 32)
+    uint32_t key[F];
+    int slot[F];
+    auto load = [&](int j) {
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        const bool valid = j + 64 * q < j_end;
+        key[q] = valid ? cd.keys[j + 64 * q] : 0xffffffffu;  // (in no cell)
+        slot[q] = valid ? cd.slots[j + 64 * q] : 0;
+      }
+    };
+    load(j_first + lane);
+    for (int j0 = j_first; j0 < j_end; j0 += 64 * F) {  // wave-uniform
+      uint32_t k[F];
+      int i[F];
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        k[q] = key[q];
+        i[q] = slot[q];
+      }
+      load(j0 + 64 * F + lane);  // (the next rounds', in flight meanwhile)
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        const uint32_t c = k[q] - c0;
+        const bool mine = c < (uint32_t)m;
+        uint64_t peers = __ballot(mine);
+        if (!peers) continue;
+        for (int bit = 0; bit < cell_bits; ++bit) {
+          const bool on = (c >> bit) & 1u;
+          const uint64_t v = __ballot(on);
+          peers &= on ? v : ~v;
+        }
+        const int rank = __popcll(peers & ((1ull << lane) - 1ull));
+        const int leader = mine ? __ffsll((unsigned long long)peers) - 1 : lane;
+        uint32_t pos = 0u;
+        if (mine && rank == 0) {
+          pos = next[c];
+          next[c] = pos + (uint32_t)__popcll(peers);
+        }
+        wave_lds_sync();  // (the next round's leaders are other lanes)
+        pos = (uint32_t)__shfl((int)pos, leader) + (uint32_t)rank;
+        if (mine && pos < (uint32_t)n) {
+          sorted[pos] = i[q];
+          hash_sorted[pos] = k[q];
+        }
+      }
+    }
+  }
+}
+
 // The merge: each particle's place, written to sorted and hash_sorted. Block 0
-// also clears the count of heavy cells for the next call.
-__global__ __launch_bounds__(kHintBlock) void hint_place_kernel(int n, uint32_t ncells,
+// also clears the count of heavy cells for the next call. Cold: the buckets.
+__global__ __launch_bounds__(kHintBlock, 8) void hint_place_kernel(int n, uint32_t ncells,
                                                                 const uint32_t *__restrict__ hash,
                                                                 const uint64_t *__restrict__ stay_bits,
                                                                 const uint32_t *__restrict__ pofs,
@@ -592,30 +813,37 @@ __global__ __launch_bounds__(kHintBlock) void hint_place_kernel(int n, uint32_t 
                                                                 const int32_t *__restrict__ list,
                                                                 uint32_t *__restrict__ counters,
                                                                 uint32_t *__restrict__ hash_sorted,
-                                                                int32_t *__restrict__ sorted) {
+                                                                int32_t *__restrict__ sorted,
+                                                                uint32_t *__restrict__ cnt, int32_t *__restrict__ cstart,
+                                                                int32_t *__restrict__ cend, Cold cd) {
+  __shared__ ColdCounters lds;  // (eight workgroups of it fit a CU)
+  __shared__ uint32_t w[kHintBlock / 64];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int i = (int)blockIdx.x * kHintBlock + t;
+  const uint32_t cold = counters[2];
   if (blockIdx.x == 0 && t == 0) counters[3] = 0u;
+  uint32_t k = hash[min(i, n - 1)];
+  asm volatile("" : "+v"(k));  // (or this load waits for the flag's)
+  if (cold != 0u) {
+    for (int b = (int)blockIdx.x; b < cd.buckets; b += (int)gridDim.x)
+      place_bucket(b, n, ncells, cd, cnt, counters, cstart, cend, hash_sorted, sorted, lds, w);
+    return;
+  }
   if (i >= n) return;
-  const uint32_t k = hash[i];
-  const bool unsorted = counters[2] != 0u;
   const int4 c = info[k];
   // stayers before this slot: those before the block, the block's waves
   // before this one, the lanes before this one
   const int w0 = (int)blockIdx.x * (kHintBlock / 64);
-  uint32_t S = 0u;
+  uint32_t S = pofs[blockIdx.x];
   uint64_t bits = 0ull;
-  if (!unsorted) {
-    S = pofs[blockIdx.x];
 #pragma unroll
-    for (int q = 0; q < kHintBlock / 64; ++q) {
-      if (q > wv) break;
-      const uint64_t v = stay_bits[w0 + q];
-      if (q < wv) S += (uint32_t)__popcll(v);
-      else bits = v;
-    }
-    S += (uint32_t)__popcll(bits & ((1ull << lane) - 1ull));
+  for (int q = 0; q < kHintBlock / 64; ++q) {
+    if (q > wv) break;
+    const uint64_t v = stay_bits[w0 + q];
+    if (q < wv) S += (uint32_t)__popcll(v);
+    else bits = v;
   }
+  S += (uint32_t)__popcll(bits & ((1ull << lane) - 1ull));
   // movers of this cell before this slot
   const int32_t *part = list + (c.x - c.y);
   int before = 0;
@@ -1007,6 +1235,31 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   uint32_t *cnt = reinterpret_cast<uint32_t *>(ctx->hint_cnt);
   uint32_t *cbt = reinterpret_cast<uint32_t *>(ctx->hint_cbt);
   int4 *info = reinterpret_cast<int4 *>(ctx->hint_info);
+  // a wave waits for each of its movers' chain of reads in turn: one word of
+  // stay bits per wave on small scenes (16 words at 40,000 particles: 14 us,
+  // one: 7), more where the waves alone would fill the chip many times over
+  const int mover_words = n < (1 << 18) ? 1 : (n < (1 << 22) ? n >> 18 : 16);
+  const int mover_blocks = (int)ceil_div(n, (int64_t)mover_words * kMoverBlock);
+  // a cold call's buckets: as many as the high digit has, for short chains in
+  // the place pass; its tiles: one per movers workgroup
+  Cold cd;
+  cd.limit = (uint32_t)std::min(npb / 16, kColdLimit);
+  cd.shift = 0;
+  while ((ncells >> cd.shift) >= (uint32_t)kColdBuckets) ++cd.shift;
+  cd.buckets = (int)(ncells >> cd.shift) + 1;
+  // (a movers workgroup reads every tile's counts, so their bytes grow with the
+  // square of the tiles; fewer tiles are longer chains. The sum is least near the
+  // cube root: movers pass of 4,000,000 particles 109 -> 80 us against tiles as
+  // small as the workgroups allow)
+  cd.tile = kMoverBlock * std::max({mover_words, kSortItems, (int)(n / (1024.0 * std::cbrt(2.4 * n))) + 1});
+  cd.tiles = (int)ceil_div(n, cd.tile);
+  cd.hist = ctx->hist;
+  cd.keys = ctx->keys_tmp;
+  cd.slots = ctx->vals_tmp;
+  if ((size_t)(cd.tiles + 1) * kColdBuckets > ctx->hist_len) {
+    note_error("partition: histogram workspace");
+    return PMPM_ERR_WORKSPACE;
+  }
   // classify: enough workgroups for the particles and for the clears
   int64_t words = 0;
   for (int q = 0; q < extra.count; ++q) words = extra.n[q] > words ? extra.n[q] : words;
@@ -1016,7 +1269,7 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
 #define PMPM_CLASSIFY(D)                                                                                               \
   PMPM_LAUNCH(hint_classify_kernel<D>, (::pmpm::kname("hint_classify_kernel", {(long)(D)})), dim3((unsigned)nb),       \
               dim3(kHintBlock), 0, s, x, n, g, part->hash_sorted, part->hash, part->bins, cnt, cbt, pblk, bits, npb, ncb, \
-              ctx->counters + 1, extra)
+              ctx->counters + 1, cd, extra)
   switch (dim) {
     case 1: PMPM_CLASSIFY(1); break;
     case 2: PMPM_CLASSIFY(2); break;
@@ -1024,18 +1277,19 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   }
 #undef PMPM_CLASSIFY
   PMPM_LAUNCH_CHECK();
-  PMPM_LAUNCH(hint_scan_kernel, (::pmpm::kname("hint_scan_kernel", {})), dim3((unsigned)(ncb + 1)), dim3(kScanThreads), 0, s,
-              ncells, npb, cnt, cbt, pblk, ctx->counters, info, part->cell_start, part->cell_end, heavy, l.heavy_cap);
+  PMPM_LAUNCH(hint_scan_kernel, (::pmpm::kname("hint_scan_kernel", {})), dim3((unsigned)std::max(ncb + 1, cd.tiles)),
+              dim3(kScanThreads), 0, s, n, ncells, npb, ncb, cnt, cbt, pblk, ctx->counters, info, part->cell_start,
+              part->cell_end, heavy, l.heavy_cap, part->hash, part->hash_sorted, cd);
   PMPM_LAUNCH_CHECK();
-  // a wave waits for each of its movers' chain of reads in turn: one word of
-  // stay bits per wave on small scenes (16 words at 40,000 particles: 14 us,
-  // one: 7), more where the waves alone would fill the chip many times over
-  const int mover_words = n < (1 << 18) ? 1 : (n < (1 << 22) ? n >> 18 : 16);
-  PMPM_LAUNCH(hint_movers_kernel, (::pmpm::kname("hint_movers_kernel", {})),
-              dim3((unsigned)ceil_div(n, (int64_t)mover_words * kMoverBlock)), dim3(kMoverBlock), 0, s, n, ncells, ncb, mover_words, part->hash, bits, info, cnt, cbt, ctx->counters, heavy, l.heavy_cap, list);
+  PMPM_LAUNCH(hint_movers_kernel, (::pmpm::kname("hint_movers_kernel", {})), dim3((unsigned)mover_blocks),
+              dim3(kMoverBlock), 0, s, n, ncells, ncb, mover_words, part->hash, bits, info, cnt, cbt, ctx->counters, heavy,
+              l.heavy_cap, list, cd);
   PMPM_LAUNCH_CHECK();
-  PMPM_LAUNCH(hint_place_kernel, (::pmpm::kname("hint_place_kernel", {})), dim3((unsigned)npb), dim3(kHintBlock), 0, s, n,
-              ncells, part->hash, bits, pblk, info, list, ctx->counters, part->hash_sorted, part->sorted);
+  // (a cold call of few particles: up to four buckets per workgroup)
+  PMPM_LAUNCH(hint_place_kernel, (::pmpm::kname("hint_place_kernel", {})),
+              dim3((unsigned)std::max(npb, std::min(cd.buckets, kColdBuckets / 4))),
+              dim3(kHintBlock), 0, s, n, ncells, part->hash, bits, pblk, info, list, ctx->counters, part->hash_sorted,
+              part->sorted, cnt, part->cell_start, part->cell_end, cd);
   PMPM_LAUNCH_CHECK();
   return PMPM_OK;
 }

@@ -430,16 +430,6 @@ __device__ void adjoint_stray(const pmpm_params &prm, const pmpm_grid &g, const 
 // re-mapped momentum; MODE 2 the adjoints of v_nt and dv.
 template <int D, int MODE> constexpr int p2g_nv() { return MODE == 0 ? 1 + 2 * D : (MODE == 2 ? 2 * D : D); }
 
-// LDS writes of a wave visible to all its lanes (and its earlier reads done)
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// A workgroup barrier that orders LDS accesses only: __syncthreads also waits
-// for the wave's global loads and stores in flight, which would drain a
-// kernel's prefetches.
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ inline int wave_max(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));

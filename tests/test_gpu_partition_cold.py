@@ -1,0 +1,107 @@
+"""GPU: the partition where the hint says little (the first call on new
+buffers, another order, most particles in another cell), which sorts by the
+keys' digits instead of merging, and where it only just says enough. Bar:
+bit-exact against numpy's stable argsort of the cell keys
+(thrust::stable_sort_by_key, spatialpartition.cpp:113-117). Every case is a
+sequence on one context (cold, merged, cold again), so a count that one way of
+sorting leaves behind shows in the next."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+
+
+class _Run:
+    def __init__(self, n, nodes):
+        from pyroclastmpm_amd import capi
+        self.capi, self.n, self.nodes, self.dev = capi, n, nodes, torch.device("cuda")
+        self.g = capi.make_grid([0, 0, 0], [c - 0.75 for c in nodes] + [0], 1.0, 2)
+        self.nc = self.g.num_cells_total
+        assert self.nc == nodes[0] * nodes[1]
+        self.ctx = capi.Context(n, self.nc)
+
+    def check(self, keys, hint, what):
+        capi, n, nc = self.capi, self.n, self.nc
+        keys = np.asarray(keys, dtype=np.int64)
+        x = np.stack([keys % self.nodes[0] + 0.5, keys // self.nodes[0] + 0.5]).astype(np.float32)
+        x[:, keys == nc] = 1e7  # past the last cell
+        xs = torch.from_numpy(x).to(self.dev)
+        hs = torch.from_numpy(np.asarray(hint).astype(np.uint32).view(np.int32).copy()).to(self.dev)
+        i32 = lambda m: torch.full((m,), 7, dtype=torch.int32, device=self.dev)
+        ha, so, cs, ce = i32(n), i32(n), i32(nc), i32(nc)
+        sp = capi.Spatial(ha.data_ptr(), hs.data_ptr(), so.data_ptr(), cs.data_ptr(), ce.data_ptr(), None)
+        s = torch.cuda.current_stream().cuda_stream
+        capi.check(capi.lib().pmpm_partition(self.ctx.ptr, 2, C.byref(self.g), xs.data_ptr(), n, C.byref(sp), s))
+        out = C.c_int32(-1)
+        capi.check(capi.lib().pmpm_context_out_of_grid(self.ctx.ptr, s, C.byref(out)))
+        torch.cuda.synchronize()
+        order = np.argsort(keys, kind="stable")
+        cnt = np.bincount(keys, minlength=nc + 1)[:nc]
+        end = np.cumsum(cnt)
+        np.testing.assert_array_equal(ha.cpu().numpy(), keys, err_msg=what)
+        np.testing.assert_array_equal(so.cpu().numpy(), order, err_msg=what)
+        np.testing.assert_array_equal(hs.cpu().numpy(), keys[order], err_msg=what)
+        np.testing.assert_array_equal(ce.cpu().numpy(), np.where(cnt > 0, end, 0), err_msg=what)
+        np.testing.assert_array_equal(cs.cpu().numpy(), np.where(cnt > 0, end - cnt, 0), err_msg=what)
+        assert out.value == int((keys == nc).sum()), what
+        return keys[order]
+
+
+# particle counts: one tile and one more, remainders of 256, 1024 and 4096; grids: one cell, fewer cells than buckets, a
+# bucket of one range of counters, of one more, of many
+@pytest.mark.parametrize("n", [2049, 4096, 4097, 12345, 270001])
+@pytest.mark.parametrize("nodes", [(1, 1), (19, 15), (181, 170), (1031, 1021), (2600, 2400)])
+def test_cold_then_merged_then_cold(n, nodes):
+    rng = np.random.default_rng(n + nodes[0])
+    run = _Run(n, nodes)
+    nc = run.nc
+    dense = rng.integers(0, min(nc, 5), n) * max(1, nc // 7)     # a few cells hold everything
+    some_out = np.where(rng.random(n) < 0.05, nc, rng.integers(0, nc, n))
+    hints = {"zero": np.zeros(n, np.int64), "garbage": rng.integers(0, 2 ** 32 - 1, n),
+             "sorted": np.sort(rng.integers(0, nc + 1, n))}
+    for name, hint in hints.items():
+        for keys in (rng.integers(0, nc, n), np.minimum(dense, nc - 1), np.sort(some_out), some_out):
+            prev = run.check(keys, hint, f"cold, hint {name}")
+            moved = prev.copy()  # the sorted keys as hint, a few of them changed since
+            at = rng.integers(0, n, max(1, n // 100))
+            moved[at] = np.clip(moved[at] + rng.integers(-2, 3, at.size), 0, nc)
+            run.check(moved, prev, f"merged after cold, hint {name}")
+    run.check(np.full(n, nc), hints["zero"], "all outside")
+
+
+@pytest.mark.parametrize("share", [0.4, 0.498, 0.502, 0.6])
+@pytest.mark.parametrize("n", [2304, 40000, 41234])
+def test_about_half_of_the_particles_moved(n, share):
+    """Around the share of movers from which a workgroup, and a call, is cold."""
+    rng = np.random.default_rng(n)
+    run = _Run(n, (211, 190))
+    prev = np.sort(rng.integers(0, run.nc, n))
+    for k in range(3):
+        at = rng.random(n) < share
+        if k == 1:  # some workgroups only
+            at &= (np.arange(n) // 256) % 17 == 3
+        moved = np.where(at, rng.integers(0, run.nc, n), prev)
+        run.check(moved, prev, f"{share} moved, {k}")
+
+
+def test_many_movers_into_one_cell_are_merged():
+    """More movers than a cell's list is counted through (kHeavyMovers), a few
+    from each workgroup: the call stays merged and bisects."""
+    rng = np.random.default_rng(2)
+    n = 60000
+    run = _Run(n, (300, 200))
+    prev = np.sort(rng.integers(0, run.nc, n))
+    for target in (0, 12345, run.nc - 1, run.nc):
+        moved = np.where(rng.random(n) < 0.1, target, prev)
+        assert (moved == target).sum() > 4096
+        run.check(moved, prev, f"movers into {target}")
+    run.check(rng.permutation(prev), np.zeros(n, np.int64), "cold after it")
