@@ -451,6 +451,36 @@ __global__ __launch_bounds__(kHintBlock) void hint_classify_kernel(
   }
 }
 
+// The stayers and movers before each block of cells, by one workgroup, for grids
+// of more than kScanBlocks such blocks: on smaller ones every scan workgroup adds
+// up the blocks before its own, whose reads grow with the square of the cells
+// (2^24 nodes, 1,000,000 particles: partition 278 us so, 254 with this launch;
+// 2^25: 574 and 419; 2^22: 82 so, 90 with it).
+constexpr int kScanBlocks = 4096;
+__global__ __launch_bounds__(kMoverBlock) void hint_blocks_kernel(int ncb, const uint32_t *__restrict__ cbt,
+                                                                  uint32_t *__restrict__ before) {
+  __shared__ uint64_t w[kMoverBlock / 64];
+  uint64_t base = 0u;
+  for (int b0 = 0; b0 < ncb; b0 += 4 * kMoverBlock) {  // block-uniform
+    uint64_t v[4], sum = 0u, tot;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int b = b0 + 4 * (int)threadIdx.x + q;
+      const uint2 u = b < ncb ? *reinterpret_cast<const uint2 *>(cbt + 2 * (int64_t)b) : make_uint2(0u, 0u);
+      v[q] = ((uint64_t)u.x << 32) | u.y;
+      sum += v[q];
+    }
+    uint64_t at = base + block_exclusive_scan<kMoverBlock, uint64_t>(sum, w, tot);
+    base += tot;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int b = b0 + 4 * (int)threadIdx.x + q;
+      if (b < ncb) *reinterpret_cast<uint2 *>(before + 2 * (int64_t)b) = make_uint2((uint32_t)(at >> 32), (uint32_t)at);
+      at += v[q];
+    }
+  }
+}
+
 // Block 0: the stayers before each particle block, and whether the call is cold
 // (counters[2]). Blocks 1 .. ncb: 1024 cells each (cells 0..ncells, the last
 // holding the out-of-grid particles), four consecutive cells per thread: the
@@ -477,7 +507,8 @@ __global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(int n, uint32_t
                                                                  int4 *__restrict__ info, int32_t *__restrict__ cstart,
                                                                  int32_t *__restrict__ cend, int32_t *__restrict__ heavy,
                                                                  uint32_t heavy_cap, const uint32_t *__restrict__ hash,
-                                                                 const uint32_t *__restrict__ hint, Cold cd) {
+                                                                 const uint32_t *__restrict__ hint,
+                                                                 const uint32_t *__restrict__ before, Cold cd) {
   __shared__ uint64_t w2[kScanThreads / 64];
   __shared__ uint32_t bucket[kColdBuckets];
   const bool cold = cd.is(counters[1]) || flat_hint(hint, n);
@@ -535,13 +566,18 @@ __global__ __launch_bounds__(kScanThreads) void hint_scan_kernel(int n, uint32_t
       mv[q] = valid ? cnt[2 * (c0 + q) + 1] : 0u;
     }
   }
-  uint64_t pp = 0u;  // (stayers << 32) | movers of the cell blocks before this one
-  for (int j = t; j < b; j += kScanThreads) {
-    const uint2 v = *reinterpret_cast<const uint2 *>(cbt + 2 * j);
-    pp += ((uint64_t)v.x << 32) | v.y;
+  uint64_t pt;  // (stayers << 32) | movers of the cell blocks before this one
+  if (before) {
+    const uint2 v = *reinterpret_cast<const uint2 *>(before + 2 * (int64_t)b);
+    pt = ((uint64_t)v.x << 32) | v.y;
+  } else {
+    uint64_t pp = 0u;
+    for (int j = t; j < b; j += kScanThreads) {
+      const uint2 v = *reinterpret_cast<const uint2 *>(cbt + 2 * j);
+      pp += ((uint64_t)v.x << 32) | v.y;
+    }
+    (void)block_exclusive_scan<kScanThreads, uint64_t>(pp, w2, pt);
   }
-  uint64_t pt;
-  (void)block_exclusive_scan<kScanThreads, uint64_t>(pp, w2, pt);
   uint32_t stay_before = (uint32_t)(pt >> 32);
   uint32_t mover_before = (uint32_t)pt;
   bool any = false;
@@ -1052,6 +1088,16 @@ extern "C" int pmpm_context_destroy(pmpm_context *ctx) {
   return PMPM_OK;
 }
 
+// Is the partition of n particles on ncells cells from the hint? Its scan writes
+// 32 bytes per cell, the radix sort's clear 8, so few particles on a large grid
+// are sorted. Merged and sorted, us: 2^22 nodes, 3,000 particles 52 and 66,
+// 1,000,000: 90 and 114; 2^23, 3,000: 78 and 69, 1,000,000: 143 and 122,
+// 4,000,000: 196 and 298; 2^24, 1,000,000: 254 and 137, 4,000,000: 382 and 326,
+// 16,000,000: 499 and 1,123; 2^26, 16,000,000: 1,395 and 1,461.
+constexpr int64_t kHintNodes = 1 << 22, kHintNodesPerParticle = 3;
+static bool use_hint(const pmpm_context *ctx, int n, int64_t ncells) {
+  return ctx->sort_by_hint && n >= ctx->hint_min_particles && ncells <= kHintNodes + kHintNodesPerParticle * n;
+}
 static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells);
 
 extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, int32_t max_cells) {
@@ -1070,10 +1116,12 @@ extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, in
     ctx->cap_particles = max_particles;
   }
   if (max_cells > ctx->cap_cells) ctx->cap_cells = max_cells;
-  if (ctx->sort_by_hint && max_particles >= ctx->hint_min_particles && max_particles > 0 && max_cells > 0) {
-    // the hint partition's workspace too, so that stepping within these
-    // sizes allocates nothing
-    int rc = reserve_hint(ctx, max_particles, (uint32_t)max_cells);
+  if (ctx->sort_by_hint && max_particles >= ctx->hint_min_particles && max_particles > 0 && max_cells > 0 &&
+      (max_particles > kSmallParticles || max_cells > kSmallCells)) {
+    // the hint partition's workspace too, for the grids it is used on, so that
+    // stepping within these sizes allocates nothing
+    const int64_t cells = std::min<int64_t>(max_cells, kHintNodes + kHintNodesPerParticle * max_particles);
+    int rc = reserve_hint(ctx, max_particles, (uint32_t)cells);
     if (rc != PMPM_OK) return rc;
   }
   // what must be zero between calls is so when this returns, whatever stream
@@ -1186,7 +1234,8 @@ static HintLayout hint_layout(int n) {
 // zero between calls: new ones are marked, and cleared by pmpm_context_reserve
 // or, if they grew in a partition, by that partition on its stream.
 static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells) {
-  const size_t cnt = 2 * ((size_t)ncells + 1), cbt = 2 * (size_t)ceil_div((int64_t)ncells + 1, kHintCells);
+  // (the blocks' counts, and where hint_blocks_kernel leaves their sums)
+  const size_t cnt = 2 * ((size_t)ncells + 1), cbt = 4 * (size_t)ceil_div((int64_t)ncells + 1, kHintCells);
   int rc;
   if (cnt > ctx->hint_cnt_cap || cbt > ctx->hint_cbt_cap) ctx->hint_clear = false;
   if ((rc = ensure_buffer(ctx->hint_cnt, ctx->hint_cnt_cap, cnt)) != PMPM_OK) return rc;
@@ -1277,9 +1326,16 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   }
 #undef PMPM_CLASSIFY
   PMPM_LAUNCH_CHECK();
+  uint32_t *before = nullptr;
+  if (ncb > kScanBlocks) {
+    before = cbt + ctx->hint_cbt_cap / 2;
+    PMPM_LAUNCH(hint_blocks_kernel, (::pmpm::kname("hint_blocks_kernel", {})), dim3(1), dim3(kMoverBlock), 0, s, ncb, cbt,
+                before);
+    PMPM_LAUNCH_CHECK();
+  }
   PMPM_LAUNCH(hint_scan_kernel, (::pmpm::kname("hint_scan_kernel", {})), dim3((unsigned)std::max(ncb + 1, cd.tiles)),
               dim3(kScanThreads), 0, s, n, ncells, npb, ncb, cnt, cbt, pblk, ctx->counters, info, part->cell_start,
-              part->cell_end, heavy, l.heavy_cap, part->hash, part->hash_sorted, cd);
+              part->cell_end, heavy, l.heavy_cap, part->hash, part->hash_sorted, before, cd);
   PMPM_LAUNCH_CHECK();
   PMPM_LAUNCH(hint_movers_kernel, (::pmpm::kname("hint_movers_kernel", {})), dim3((unsigned)mover_blocks),
               dim3(kMoverBlock), 0, s, n, ncells, ncb, mover_words, part->hash, bits, info, cnt, cbt, ctx->counters, heavy,
@@ -1316,7 +1372,7 @@ int pmpm::partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, 
     if (n <= 1024) return partition_small<1, 1024>(ctx, dim, g, x, n, part, s, extra);
     return partition_small<2, 1024>(ctx, dim, g, x, n, part, s, extra);
   }
-  if (ctx->sort_by_hint && n >= ctx->hint_min_particles) return partition_by_hint(ctx, dim, g, x, n, part, s, extra);
+  if (use_hint(ctx, n, ncells)) return partition_by_hint(ctx, dim, g, x, n, part, s, extra);
   // enough threads for the particles, and for the clears at 4 words each
   int64_t words = ncells;
   for (int q = 0; q < extra.count; ++q) words = extra.n[q] > words ? extra.n[q] : words;
