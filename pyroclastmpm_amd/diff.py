@@ -53,12 +53,14 @@ class ParticleSet:
 
 class StepBuffers:
     """The partition (pmpm_spatial) and node arrays (pmpm_nodes) one step
-    uses."""
+    uses. hash_sorted: the sorted keys of another step's buffers, to share
+    them: a partition reads the last one's as its hint, and nothing but the
+    next partition reads them."""
 
-    def __init__(self, n, nn, dim, device="cuda"):
+    def __init__(self, n, nn, dim, device="cuda", hash_sorted=None):
         i32 = lambda m: torch.zeros(m, dtype=torch.int32, device=device)
-        self.sp = {"hash": i32(n), "hash_sorted": i32(n), "sorted": i32(n), "cell_start": i32(nn),
-                   "cell_end": i32(nn)}
+        self.sp = {"hash": i32(n), "hash_sorted": i32(n) if hash_sorted is None else hash_sorted, "sorted": i32(n),
+                   "cell_start": i32(nn), "cell_end": i32(nn)}
         self.spatial = capi.Spatial(*[self.sp[k].data_ptr() for k in ["hash", "hash_sorted", "sorted",
                                                                       "cell_start", "cell_end"]], None)
         f = lambda m: torch.zeros(m, dtype=torch.float32, device=device)
@@ -212,11 +214,13 @@ class DiffMPM:
         """K - 1 particle sets and K partition/node sets, reused by every
         segment: step k of a segment reads state k (state 0 is the checkpoint
         itself, which a USL step only reads) and keeps its partition and nodes
-        in work k for the adjoint of the same step."""
+        in work k for the adjoint of the same step. The sorted keys are shared,
+        so every partition has the one before it as its hint."""
         if self._segment is None:
             nn = self.grid.num_cells_total
             states = [ParticleSet(self.n, self.dim, self.device) for _ in range(self.K - 1)]
-            work = [self.work] + [StepBuffers(self.n, nn, self.dim, self.device) for _ in range(self.K - 1)]
+            work = [self.work] + [StepBuffers(self.n, nn, self.dim, self.device, self.sp["hash_sorted"])
+                                  for _ in range(self.K - 1)]
             self._segment = (states, work)
         return self._segment
 
