@@ -10,6 +10,14 @@
 
 #include "../../include/pmpm.h"
 
+namespace pmpm {
+// Words of the P2G workspace: tile partials, tile flags, the clamp record (a byte
+// per node) and the stray sums.
+struct TileSizes {
+  size_t partials = 0, flags = 0, clamp = 0, strays = 0;
+};
+}  // namespace pmpm
+
 struct pmpm_context {
   int device = 0;
   int32_t cap_particles = 0;
@@ -22,28 +30,27 @@ struct pmpm_context {
   // cells, stray flags (3); counters_clear: cleared since they were allocated
   uint32_t *counters = nullptr;
   bool counters_clear = false;
-  // P2G tile partials: per tile, the LDS node block of each accumulated field
-  // (plain stores; the grid kernel sums the <= 2^D tiles covering a node)
+  // the P2G workspace, one allocation (tile_mem): tile partials (per tile, the
+  // node block of each accumulated field; the grid kernel sums the tiles covering
+  // a node), tile flags (1 = the tile had particles this launch), and
+  // - a byte per node: the components the last grid pass's NodeDomain condition
+  //   set to zero, read by the adjoint
+  // - the sums of particles deposited over their own windows (mass, momentum,
+  //   force per node; the adjoint scatter's fields), zero but between a pass that
+  //   sets its flag (stray_flags: P2G, re-map, adjoint scatter) and the grid pass
+  //   after it (strays_clear: cleared since they were allocated)
+  float *tile_mem = nullptr;
+  pmpm::TileSizes tile_cap;
   float *partials = nullptr;
-  size_t partials_cap = 0;       // floats
-  int32_t *tile_flags = nullptr;  // 1 = tile had particles this launch
-  size_t tile_flags_cap = 0;
-  // P2G sums of particles deposited over their own windows (mass, momentum,
-  // force per node; the adjoint scatter's fields), zero but between a pass that
-  // sets its flag (stray_flags: P2G, re-map, adjoint scatter) and the grid pass
-  // after it
+  int32_t *tile_flags = nullptr;
+  float *clamp_mask = nullptr;
   float *strays = nullptr;
-  size_t strays_cap = 0;
-  bool strays_clear = false;       // cleared since they were allocated
+  bool strays_clear = false;
   int32_t *stray_flags = nullptr;  // in counters
   // the workspace is the caller's and never grows (pmpm_step_noalloc): the
   // stray sums are then the step's node arrays, cleared before it, and without
   // room for the partials every particle is deposited over its own window
   bool fixed_workspace = false;
-  // a byte per node: the components the last grid pass's NodeDomain
-  // condition set to zero (words of 4 bytes), read by the adjoint
-  float *clamp_mask = nullptr;
-  size_t clamp_mask_cap = 0;
   // adjoint step: per-particle scatter records (15 floats, cell order) and
   // node adjoints (one record of 8 floats per node, 4 in 1D)
   float *adj_rec = nullptr;
@@ -59,26 +66,21 @@ struct pmpm_context {
   // (PMPM_PARTITION_HINT_MIN at creation)
   bool sort_by_hint = true;
   int32_t hint_min_particles = 0;
-  // per cell (ncells + 1, the last for the out-of-grid particles): counts
-  // of stayers and movers (zero between calls), and per block of 1024 cells;
-  // hint_clear: both have been cleared since they were allocated
-  float *hint_cnt = nullptr;
-  size_t hint_cnt_cap = 0;
-  float *hint_cbt = nullptr;
-  size_t hint_cbt_cap = 0;
+  // its workspace, one allocation. Per cell (the last for the out-of-grid
+  // particles): counts of stayers and movers, and per block of 1024 cells (both
+  // zero between calls; hint_clear: cleared since they were allocated), the
+  // blocks' sums, and per cell the first slot, stayers before the cell, stayers,
+  // movers; then the arrays per particle (HintLayout in partition.hip)
+  uint32_t *hint_mem = nullptr;
+  uint32_t *hint_cnt = nullptr, *hint_cbt = nullptr, *hint_sums = nullptr, *hint_info = nullptr, *hint_part = nullptr;
+  size_t hint_zero_words = 0, hint_part_cap = 0, hint_cells_cap = 0;
   bool hint_clear = false;
-  // per cell: first slot, stayers before the cell, stayers, movers
-  float *hint_info = nullptr;
-  size_t hint_info_cap = 0;
-  // per particle (HintLayout in partition.hip)
-  float *hint_part = nullptr;
-  size_t hint_part_cap = 0;
 };
 
 namespace pmpm {
-// Grows the tile-partial workspace (hipMalloc on first use of a larger grid;
-// run one step before capturing a graph).
-int ensure_partials(pmpm_context *ctx, size_t floats, size_t tiles);
+// Grows the P2G workspace (hipMalloc on first use of a larger grid; run one step
+// before capturing a graph).
+int ensure_tiles(pmpm_context *ctx, const TileSizes &want);
 // Grows a context-owned float buffer to at least `floats`.
 int ensure_buffer(float *&buf, size_t &cap, size_t floats);
 }  // namespace pmpm
@@ -186,12 +188,8 @@ int step_on(pmpm_context *ctx, const pmpm_params *prm, const pmpm_grid *grid, in
 bool params_ok(const pmpm_params *prm);
 bool step_args_ok(const pmpm_params *prm, const pmpm_grid *grid, const pmpm_particles *a, const pmpm_particles *b,
                   const pmpm_spatial *part, const pmpm_nodes *nodes);
-// Workspace the P2G passes of one step of n particles use on grid g: tile
-// partials (floats) and tile flags, and the clamp record (words).
-struct P2GWorkspace {
-  size_t partial_floats, tiles, clamp_words;
-};
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n, P2GWorkspace *w);
+// The P2G workspace of a step of n particles on grid g (without stray sums).
+TileSizes p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n);
 // pmpm_partition whose first kernel also clears the buffers of `extra`.
 int partition_clearing(pmpm_context *ctx, int dim, const pmpm_grid *grid, const float *x, int n, pmpm_spatial *part,
                        hipStream_t s, const ZeroLists &extra);

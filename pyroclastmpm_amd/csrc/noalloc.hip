@@ -97,17 +97,16 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   const size_t n = (size_t)(a->n > 0 ? a->n : 1);
   const size_t nblocks = (size_t)ceil_div((int64_t)n, kSortTile);
   const size_t hist_len = (size_t)kMaxRadix * nblocks + kMaxRadix;
-  P2GWorkspace w;
-  p2g_workspace(*prm, *grid, (int)a->n, &w);
+  const TileSizes w = p2g_workspace(*prm, *grid, (int)a->n);
   Carver c;
   const size_t o_keys = c.take(n * sizeof(uint32_t));
   const size_t o_vals = c.take(n * sizeof(int32_t));
   const size_t o_hist = c.take(hist_len * sizeof(uint32_t));
   const size_t o_counters = c.take(kCounters * sizeof(uint32_t));
-  const size_t o_flags = c.take(w.tiles * sizeof(int32_t));
-  const size_t o_clamp = c.take(w.clamp_words * sizeof(float));
+  const size_t o_flags = c.take(w.flags * sizeof(int32_t));
+  const size_t o_clamp = c.take(w.clamp * sizeof(float));
   const size_t o_partials = c.used;
-  const size_t charge = budget_bytes(*prm, *grid, n, hist_len, w.clamp_words);
+  const size_t charge = budget_bytes(*prm, *grid, n, hist_len, w.clamp);
   if (charge > (size_t)PMPM_NOALLOC_SCRATCH_BYTES || c.used > (size_t)PMPM_NOALLOC_SCRATCH_BYTES) {
     char why[200];
     snprintf(why, sizeof(why),
@@ -117,7 +116,7 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
     note_error(why);
     return PMPM_ERR_WORKSPACE;
   }
-  const bool tiled = o_partials + w.partial_floats * sizeof(float) <= (size_t)PMPM_NOALLOC_SCRATCH_BYTES;
+  const bool tiled = o_partials + w.partials * sizeof(float) <= (size_t)PMPM_NOALLOC_SCRATCH_BYTES;
   unsigned char *base = nullptr;
   int rc = scratch_of_current_device(&base);
   if (rc != PMPM_OK) return rc;
@@ -135,11 +134,9 @@ extern "C" int pmpm_step_noalloc(const pmpm_params *prm, const pmpm_grid *grid, 
   ctx.counters_clear = true;  // (the radix path writes what it reads)
   ctx.sort_by_hint = false;  // the full radix sort: its workspace is all carved above
   ctx.partials = tiled ? reinterpret_cast<float *>(base + o_partials) : nullptr;
-  ctx.partials_cap = tiled ? w.partial_floats : 0;
   ctx.tile_flags = reinterpret_cast<int32_t *>(base + o_flags);
-  ctx.tile_flags_cap = w.tiles;
   ctx.clamp_mask = reinterpret_cast<float *>(base + o_clamp);
-  ctx.clamp_mask_cap = w.clamp_words;
+  ctx.tile_cap = w;
   ctx.stray_flags = reinterpret_cast<int32_t *>(ctx.counters + 4);
   ctx.fixed_workspace = true;
   // (the context is a plain struct on this stack frame: nothing frees the

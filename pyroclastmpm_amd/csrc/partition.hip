@@ -1038,21 +1038,25 @@ extern "C" int pmpm_context_create(pmpm_context **ctx) {
   return PMPM_OK;
 }
 
-int pmpm::ensure_partials(pmpm_context *ctx, size_t floats, size_t tiles) {
-  if (floats > ctx->partials_cap) {
-    (void)hipFree(ctx->partials);
-    ctx->partials = nullptr;
-    ctx->partials_cap = 0;
-    PMPM_HIP_CHECK(hipMalloc(&ctx->partials, floats * sizeof(float)));
-    ctx->partials_cap = floats;
-  }
-  if (tiles > ctx->tile_flags_cap) {
-    (void)hipFree(ctx->tile_flags);
-    ctx->tile_flags = nullptr;
-    ctx->tile_flags_cap = 0;
-    PMPM_HIP_CHECK(hipMalloc(&ctx->tile_flags, tiles * sizeof(int32_t)));
-    ctx->tile_flags_cap = tiles;
-  }
+int pmpm::ensure_tiles(pmpm_context *ctx, const TileSizes &want) {
+  TileSizes &cap = ctx->tile_cap;
+  if (want.partials <= cap.partials && want.flags <= cap.flags && want.clamp <= cap.clamp && want.strays <= cap.strays)
+    return PMPM_OK;
+  const TileSizes to{std::max(want.partials, cap.partials), std::max(want.flags, cap.flags),
+                     std::max(want.clamp, cap.clamp), std::max(want.strays, cap.strays)};
+  (void)hipFree(ctx->tile_mem);
+  ctx->tile_mem = ctx->partials = ctx->clamp_mask = ctx->strays = nullptr;
+  ctx->tile_flags = nullptr;
+  cap = TileSizes{};
+  auto up = [](size_t w) { return (w + 63) / 64 * 64; };
+  PMPM_HIP_CHECK(hipMalloc(&ctx->tile_mem,
+                           (up(to.flags) + up(to.clamp) + up(to.strays) + to.partials) * sizeof(float)));
+  ctx->tile_flags = reinterpret_cast<int32_t *>(ctx->tile_mem);
+  ctx->clamp_mask = ctx->tile_mem + up(to.flags);
+  ctx->strays = ctx->clamp_mask + up(to.clamp);
+  ctx->partials = ctx->strays + up(to.strays);
+  ctx->strays_clear = false;
+  cap = to;
   return PMPM_OK;
 }
 
@@ -1072,18 +1076,12 @@ extern "C" int pmpm_context_destroy(pmpm_context *ctx) {
   (void)hipFree(ctx->adj_rec);
   (void)hipFree(ctx->adj_nodes);
   (void)hipFree(ctx->adj_pb);
-  (void)hipFree(ctx->partials);
-  (void)hipFree(ctx->tile_flags);
-  (void)hipFree(ctx->clamp_mask);
-  (void)hipFree(ctx->hint_cnt);
-  (void)hipFree(ctx->hint_cbt);
-  (void)hipFree(ctx->hint_info);
-  (void)hipFree(ctx->hint_part);
+  (void)hipFree(ctx->tile_mem);
+  (void)hipFree(ctx->hint_mem);
   (void)hipFree(ctx->keys_tmp);
   (void)hipFree(ctx->vals_tmp);
   (void)hipFree(ctx->hist);
   (void)hipFree(ctx->counters);
-  (void)hipFree(ctx->strays);
   delete ctx;
   return PMPM_OK;
 }
@@ -1126,16 +1124,15 @@ extern "C" int pmpm_context_reserve(pmpm_context *ctx, int32_t max_particles, in
   }
   // what must be zero between calls is so when this returns, whatever stream
   // uses it first, and also if that use is only recorded (a captured graph)
-  if (!ctx->counters_clear || (ctx->hint_cnt && !ctx->hint_clear)) {
+  if (!ctx->counters_clear || (ctx->hint_mem && !ctx->hint_clear)) {
     ZeroLists z{};
     z.add(ctx->counters, kCounters);
-    z.add(ctx->hint_cnt, (int64_t)ctx->hint_cnt_cap);
-    z.add(ctx->hint_cbt, (int64_t)ctx->hint_cbt_cap);
+    z.add(ctx->hint_mem, (int64_t)ctx->hint_zero_words);
     int rc = zero_fill_lists(z, nullptr);
     if (rc != PMPM_OK) return rc;
     PMPM_HIP_CHECK(hipStreamSynchronize(nullptr));
     ctx->counters_clear = true;
-    ctx->hint_clear = ctx->hint_cnt != nullptr;
+    ctx->hint_clear = ctx->hint_mem != nullptr;
   }
   return PMPM_OK;
 }
@@ -1230,18 +1227,33 @@ static HintLayout hint_layout(int n) {
   return l;
 }
 
-// Grows the hint workspace to n particles on ncells cells. The counts must be
-// zero between calls: new ones are marked, and cleared by pmpm_context_reserve
-// or, if they grew in a partition, by that partition on its stream.
+// Grows the hint workspace to n particles on ncells cells (one allocation). The
+// counts must be zero between calls: new ones are marked, and cleared by
+// pmpm_context_reserve or, if they grew in a partition, by that partition on its
+// stream.
 static int reserve_hint(pmpm_context *ctx, int n, uint32_t ncells) {
+  const size_t words = hint_layout(n).words, cells = (size_t)ncells + 1;
+  if (words <= ctx->hint_part_cap && cells <= ctx->hint_cells_cap) return PMPM_OK;
+  const size_t to_words = std::max(words, ctx->hint_part_cap), to_cells = std::max(cells, ctx->hint_cells_cap);
+  (void)hipFree(ctx->hint_mem);
+  ctx->hint_mem = nullptr;
+  ctx->hint_part_cap = ctx->hint_cells_cap = 0;
+  ctx->hint_clear = false;
+  auto up = [](size_t w) { return (w + 63) / 64 * 64; };
   // (the blocks' counts, and where hint_blocks_kernel leaves their sums)
-  const size_t cnt = 2 * ((size_t)ncells + 1), cbt = 4 * (size_t)ceil_div((int64_t)ncells + 1, kHintCells);
-  int rc;
-  if (cnt > ctx->hint_cnt_cap || cbt > ctx->hint_cbt_cap) ctx->hint_clear = false;
-  if ((rc = ensure_buffer(ctx->hint_cnt, ctx->hint_cnt_cap, cnt)) != PMPM_OK) return rc;
-  if ((rc = ensure_buffer(ctx->hint_cbt, ctx->hint_cbt_cap, cbt)) != PMPM_OK) return rc;
-  if ((rc = ensure_buffer(ctx->hint_info, ctx->hint_info_cap, 4 * ((size_t)ncells + 1))) != PMPM_OK) return rc;
-  return ensure_buffer(ctx->hint_part, ctx->hint_part_cap, hint_layout(n).words);
+  const size_t blocks = (size_t)ceil_div((int64_t)to_cells, kHintCells);
+  const size_t o_cbt = up(2 * to_cells), o_sums = o_cbt + up(2 * blocks), o_info = o_sums + up(2 * blocks),
+               o_part = o_info + up(4 * to_cells);
+  PMPM_HIP_CHECK(hipMalloc(&ctx->hint_mem, (o_part + to_words) * sizeof(uint32_t)));
+  ctx->hint_cnt = ctx->hint_mem;
+  ctx->hint_cbt = ctx->hint_mem + o_cbt;
+  ctx->hint_sums = ctx->hint_mem + o_sums;
+  ctx->hint_info = ctx->hint_mem + o_info;
+  ctx->hint_part = ctx->hint_mem + o_part;
+  ctx->hint_zero_words = o_sums;  // (cnt and cbt)
+  ctx->hint_part_cap = to_words;
+  ctx->hint_cells_cap = to_cells;
+  return PMPM_OK;
 }
 
 // The one-workgroup partition (small_partition_kernel).
@@ -1272,17 +1284,15 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   if ((rc = reserve_hint(ctx, n, ncells)) != PMPM_OK) return rc;
   if (!ctx->hint_clear) {
     ZeroLists z{};
-    z.add(ctx->hint_cnt, (int64_t)ctx->hint_cnt_cap);
-    z.add(ctx->hint_cbt, (int64_t)ctx->hint_cbt_cap);
+    z.add(ctx->hint_mem, (int64_t)ctx->hint_zero_words);
     if ((rc = clear_on_stream(z, ctx->hint_clear, s)) != PMPM_OK) return rc;
   }
   const HintLayout l = hint_layout(n);
-  uint32_t *base = reinterpret_cast<uint32_t *>(ctx->hint_part);
+  uint32_t *base = ctx->hint_part;
   uint64_t *bits = reinterpret_cast<uint64_t *>(base + l.bits);
   uint32_t *pblk = base + l.pblk;
   int32_t *heavy = reinterpret_cast<int32_t *>(base + l.heavy), *list = reinterpret_cast<int32_t *>(base + l.list);
-  uint32_t *cnt = reinterpret_cast<uint32_t *>(ctx->hint_cnt);
-  uint32_t *cbt = reinterpret_cast<uint32_t *>(ctx->hint_cbt);
+  uint32_t *cnt = ctx->hint_cnt, *cbt = ctx->hint_cbt;
   int4 *info = reinterpret_cast<int4 *>(ctx->hint_info);
   // a wave waits for each of its movers' chain of reads in turn: one word of
   // stay bits per wave on small scenes (16 words at 40,000 particles: 14 us,
@@ -1328,7 +1338,7 @@ static int partition_by_hint(pmpm_context *ctx, int dim, const pmpm_grid &g, con
   PMPM_LAUNCH_CHECK();
   uint32_t *before = nullptr;
   if (ncb > kScanBlocks) {
-    before = cbt + ctx->hint_cbt_cap / 2;
+    before = ctx->hint_sums;
     PMPM_LAUNCH(hint_blocks_kernel, (::pmpm::kname("hint_blocks_kernel", {})), dim3(1), dim3(kMoverBlock), 0, s, ncb, cbt,
                 before);
     PMPM_LAUNCH_CHECK();

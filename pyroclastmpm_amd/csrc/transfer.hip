@@ -2332,36 +2332,28 @@ static bool particles_ok(const pmpm_particles *p) {
                         p->flags && p->id));
 }
 
-// Partials and tile flags of the P2G passes of n particles on grid g.
-static void partial_sizes(const pmpm_params &prm, const pmpm_grid &g, int n, size_t *floats, size_t *tiles) {
+TileSizes p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n) {
   const TileGeom tg = tile_geom(prm, g, 1, n);
-  *tiles = std::max(*tiles, tile_count(tg));
-  *floats = std::max(*floats, tile_count(tg) * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2]);
+  TileSizes w;
+  w.flags = tile_count(tg);
+  w.partials = w.flags * tg.nv * (size_t)tg.N[0] * tg.N[1] * tg.N[2];
+  w.clamp = ((size_t)g.num_cells_total + 3) / 4;
+  return w;
 }
 static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_grid &g, hipStream_t s) {
-  if (ctx->fixed_workspace) return ctx->partials ? PMPM_OK : zero_fill(ctx->tile_flags, (int64_t)ctx->tile_flags_cap, s);
-  size_t floats = 0, tiles = 0;
-  for (const int n : {0, kSmallParticles + 1}) partial_sizes(prm, g, n, &floats, &tiles);  // (any particle count)
-  int rc = ensure_partials(ctx, floats, tiles);
+  if (ctx->fixed_workspace) return ctx->partials ? PMPM_OK : zero_fill(ctx->tile_flags, (int64_t)ctx->tile_cap.flags, s);
+  // (any particle count: a small grid's passes use either tiles)
+  TileSizes w = p2g_workspace(prm, g, 0);
+  const TileSizes large = p2g_workspace(prm, g, kSmallParticles + 1);
+  w.partials = std::max(w.partials, large.partials);
+  w.flags = std::max(w.flags, large.flags);
+  w.strays = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
+  int rc = ensure_tiles(ctx, w);
   if (rc != PMPM_OK) return rc;
-  // the grid pass's clamp record (one byte per node, in words of 4)
-  if ((rc = ensure_buffer(ctx->clamp_mask, ctx->clamp_mask_cap, ((size_t)g.num_cells_total + 3) / 4)) != PMPM_OK)
-    return rc;
   // the stray sums are zero whenever no pass is under way
-  const size_t words = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
-  if (words > ctx->strays_cap) {
-    ctx->strays_clear = false;
-    if ((rc = ensure_buffer(ctx->strays, ctx->strays_cap, words)) != PMPM_OK) return rc;
-  }
   ZeroLists z{};
-  z.add(ctx->strays, (int64_t)ctx->strays_cap);
+  z.add(ctx->strays, (int64_t)ctx->tile_cap.strays);
   return clear_on_stream(z, ctx->strays_clear, s);
-}
-
-void p2g_workspace(const pmpm_params &prm, const pmpm_grid &g, int n, P2GWorkspace *w) {
-  *w = P2GWorkspace{};
-  partial_sizes(prm, g, n, &w->partial_floats, &w->tiles);
-  w->clamp_words = ((size_t)g.num_cells_total + 3) / 4;
 }
 
 // Scatter into the tile partials (and the stray sums); a grid_kernel pass with
