@@ -634,7 +634,7 @@ __device__ inline bool is_mover(const uint64_t *__restrict__ stay_bits, int i) {
 // a workgroup each, in slot order. The counts end at zero, as the next call
 // needs them, and block 0 clears the per-block cell counts and the count of cold
 // workgroups. Cold: the scatter of a tile to the buckets.
-__global__ __launch_bounds__(kMoverBlock, 8) void hint_movers_kernel(int n, uint32_t ncells, int ncb, int words,
+__global__ __launch_bounds__(kMoverBlock) void hint_movers_kernel(int n, uint32_t ncells, int ncb, int words,
                                                                   const uint32_t *__restrict__ hash,
                                                                   const uint64_t *__restrict__ stay_bits,
                                                                   const int4 *__restrict__ info,

@@ -2923,11 +2923,14 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
       const size_t node = reaches ? (size_t)lin : 0;
       const float4 *ar = reinterpret_cast<const float4 *>(nbar + 8 * node);
       const float4 *vr = reinterpret_cast<const float4 *>(nodes.vel + 8 * node);
-      const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
       const float4 a0 = ar[0], a1 = ar[1], v0 = vr[0], v1 = vr[1];
-      s_rec[3 * q] = reaches ? a0 : z4;
+      // (component by component: a choice between two vectors goes through memory)
+      auto keep = [](bool c, float x, float y, float z, float w) {
+        return make_float4(c ? x : 0.f, c ? y : 0.f, c ? z : 0.f, c ? w : 0.f);
+      };
+      s_rec[3 * q] = keep(reaches, a0.x, a0.y, a0.z, a0.w);
       s_rec[3 * q + 1] = make_float4(reaches ? a1.x : 0.f, reaches ? a1.y : 0.f, reaches ? a1.z : 0.f, in ? v0.x : 0.f);
-      s_rec[3 * q + 2] = in ? make_float4(v0.y, v0.z, v0.w, v1.x) : z4;
+      s_rec[3 * q + 2] = keep(in, v0.y, v0.z, v0.w, v1.x);
       s_dvz[q] = in ? v1.y : 0.f;
     }
     lds_barrier();
