@@ -58,10 +58,11 @@ class _Run:
 
 # particle counts: one tile and one more, remainders of 256, 1024 and 4096; grids: one cell, fewer cells than buckets, a
 # bucket of one range of counters, of one more, of many (the last grid: with the cells' blocks summed by a launch of their
-# own, and with too few particles for a hint to be read at all)
+# own, and with too few particles for a hint to be read at all); a handful of particles on more nodes than one workgroup
+# sorts
 @pytest.mark.parametrize("n, nodes", [(n, nodes) for n in (2049, 4096, 4097, 12345, 270001)
                                       for nodes in ((1, 1), (19, 15), (181, 170), (1031, 1021))]
-                         + [(4097, (2600, 2400)), (681899, (2600, 2400))])
+                         + [(n, (181, 170)) for n in (1, 2, 5, 259, 1031)] + [(4097, (2600, 2400)), (681899, (2600, 2400))])
 def test_cold_then_merged_then_cold(n, nodes):
     rng = np.random.default_rng(n + nodes[0])
     run = _Run(n, nodes)
