@@ -183,7 +183,9 @@ typedef struct pmpm_context pmpm_context;
 /* ---- context / workspace -------------------------------------------------
  * A context owns the scratch memory of the spatial sort for up to
  * max_particles particles and max_cells cells on the current device (and the
- * P2G, wrap-around and adjoint workspace, grown on first use). Its work is
+ * P2G, stray and adjoint workspace, grown on first use). pmpm_context_reserve
+ * allocates, clears the counts that must be zero between calls and waits for
+ * that, so it does not belong into a captured graph. A context's work is
  * stream-ordered: calls on one context must be issued to one stream, or
  * ordered between streams by the caller; overlapping calls on one context
  * race on its workspace. Independent scenes take a context each. */

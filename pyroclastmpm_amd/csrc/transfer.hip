@@ -965,12 +965,17 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 //
 // 1,080,000 particles, 27 per cell, cubic: P2G 81 -> 70 us (and 32 us of
 // wrap-around launches less), re-map 40 -> 36 (23), adjoint scatter 159 -> 67.
-// What bounds it: instruction issue. Per four particles there are 4 (MODE 1:
-// 1) matrix instructions of 32 cycles and about 45 vector instructions, so
-// the weights are evaluated here from per-lane coefficients (about 20
-// multiply-adds) instead of being staged: a particle's LDS record is 20
-// floats written by one lane and read with two 16-byte broadcasts and one
-// word. The rows of a round are the wave's particles in sorted order, each
+// What bounds it (P2G, 70 us there): waiting, in workgroups that do not come
+// out even. Vector instructions take 26 us of issue and the matrix cores are
+// busy 15 us; a workgroup's 80,896 bytes of LDS let two run per CU, so the
+// column's 750 tiles with particles take the 512 places in two rounds, the
+// second half full, among the 3,644 empty tiles, which hold a place for the
+// length of a cell-range read; within a wave the rounds are a chain of slots,
+// fields, LDS and products. Per four particles there are 4 (MODE 1: 1) matrix
+// instructions of 32 cycles and about 45 vector instructions; the weights are
+// evaluated from per-lane coefficients (about 20 multiply-adds) instead of
+// being staged: a particle's LDS record is 20 floats written by one lane and
+// read with two 16-byte broadcasts and one word. The rows of a round are the wave's particles in sorted order, each
 // cell padded to a multiple of four, so a round fills its 64 lanes whatever
 // the particles per cell (at 8 per cell staging cell by cell left 3 of 4
 // lanes idle); the next round's fields load while a round is multiplied, the
@@ -1385,9 +1390,7 @@ struct TileGeom {
   int tiles[3];  // tiles per axis
   int T[3];      // cells per tile per axis
   int N[3];      // nodes per tile block per axis (T + SPAN - 1)
-  int nlo;       // first node offset of a tile block
   int nv;        // fields per node in the partials
-  int gather;    // 0: none, 1: P2G (mass, momentum, force), 2: MUSL re-map (momentum)
 };
 
 // Sums the NV fields of the partial slices of the tiles whose node block
@@ -1547,7 +1550,7 @@ __device__ inline void gather_images(const pmpm_grid &g, const TileGeom &tg, con
 #pragma unroll
     for (int o = 1; o < kImageLanes; o <<= 1) acc[k] += __shfl_xor(acc[k], o);
 }
-// GATHER as TileGeom::gather (fixed per instance: it sets the fields gathered).
+// GATHER as make_tiles' `gather` (fixed per instance: it sets the fields gathered).
 template <int D, int GATHER, class TG>
 __global__ __launch_bounds__(256) void grid_kernel(pmpm_params prm, pmpm_grid g, pmpm_nodes nodes, int finalize, int bc_begin, int bc_end,
                             int remap_pass, TileGeom tg, const float *__restrict__ partials,
@@ -2142,12 +2145,13 @@ static bool wraps(const pmpm_params &prm) {
 // 2,016: 36.5 and 38.3, 8,320: 36.6 and 38.9, 14,784: 49.9 and 51.1, 17,000:
 // 73.2 and 69.8, 40,000: 46.7 and 46.4, 275,000: 101.7 and 96.0.
 struct MfmaTiles { int cells, rows; };
-constexpr int kSmallGridNodes = 131072, kSmallParticles = 16384;
+constexpr int kSmallGridNodes = 131072, kSmallTileParticles = 16384;
 static MfmaTiles mfma_tiles(const pmpm_grid &g, int n) {
-  if (g.num_cells_total <= kSmallGridNodes && n <= kSmallParticles) return {4, 1};
+  if (g.num_cells_total <= kSmallGridNodes && n <= kSmallTileParticles) return {4, 1};
   return {8, 2};
 }
-// Tiles of T cells and their node blocks over grid g.
+// Tiles of T cells and their node blocks over grid g. gather: 1: P2G (mass,
+// momentum, force), 2: MUSL re-map (momentum), 3: adjoint scatter.
 static TileGeom make_tiles(int dim, int sf, const pmpm_grid &g, int gather, const int *T) {
   TileGeom tg{};
   const int span = sf == PMPM_SF_LINEAR ? 2 : 4;
@@ -2156,7 +2160,7 @@ static TileGeom make_tiles(int dim, int sf, const pmpm_grid &g, int gather, cons
     tg.N[a] = a < dim ? T[a] + span - 1 : 1;
     tg.tiles[a] = a < dim ? (int)ceil_div(g.num_cells[a], T[a]) : 1;
   }
-  tg.nv = gather == 2 ? dim : (gather == 3 ? 2 * dim : 1 + 2 * dim);  // 3: adjoint scatter
+  tg.nv = gather == 2 ? dim : (gather == 3 ? 2 * dim : 1 + 2 * dim);
   return tg;
 }
 static TileGeom mfma_tile_geom(int sf, const pmpm_grid &g, int gather, MfmaTiles m) {
@@ -2344,7 +2348,7 @@ static int reserve_tiles(pmpm_context *ctx, const pmpm_params &prm, const pmpm_g
   if (ctx->fixed_workspace) return ctx->partials ? PMPM_OK : zero_fill(ctx->tile_flags, (int64_t)ctx->tile_cap.flags, s);
   // (any particle count: a small grid's passes use either tiles)
   TileSizes w = p2g_workspace(prm, g, 0);
-  const TileSizes large = p2g_workspace(prm, g, kSmallParticles + 1);
+  const TileSizes large = p2g_workspace(prm, g, kSmallTileParticles + 1);
   w.partials = std::max(w.partials, large.partials);
   w.flags = std::max(w.flags, large.flags);
   w.strays = (size_t)g.num_cells_total * (1 + 2 * prm.dim);
@@ -2949,11 +2953,10 @@ __device__ inline void adjoint_stage_rounds(const pmpm_grid &g, const pmpm_nodes
 // and the sums over the window contract x first (weights N, dN, d2N of gs, wv,
 // P_bar, f_bar as each needs them), then y, then z: about 3,400 multiply-adds
 // per particle instead of 4,500 with a product of three weights per entry.
-// Bound by vector issue (1,080,000 particles: 230 us, of which 136 us are issue
+// Bound by vector issue (1,080,000 particles: 225 us, of which 136 us are issue
 // at three waves per SIMD; capped to 128 registers for four it spills, 272 us).
 // LANES = 1: a lane per particle; 4: a lane per z layer of the window, 16: per
-// row of it, for
-// launches too small to fill the chip otherwise.
+// row of it, for launches too small to fill the chip otherwise.
 // Wrap-around entries (deposit only): a node outside the grid holds the adjoint
 // of the node it reaches (see the staging), so it takes part as an ordinary
 // entry wherever its weight is a product of per-axis weights: always without
@@ -3253,7 +3256,6 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
                                                           const float *__restrict__ nbar, const float *__restrict__ rec) {
   constexpr int E = Spline<SF>::ENTRIES;
   constexpr int EY = D > 1 ? E : 1;
-  constexpr int EZ = D > 2 ? E : 1;
   const int n = st.n;
   const int nn = g.num_cells_total;
   // LANES = 1: one lane per particle, the window's y offsets in turn;
@@ -3301,14 +3303,11 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
   float vb[3] = {0.f, 0.f, 0.f}, xb[3] = {0.f, 0.f, 0.f}, G[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f},
                                                                        {0.f, 0.f, 0.f}};
   // one entry's contributions (g2p = 1 adds the G2P weights' position term)
-  // (adj, vel: the node adjoint and velocity records, in global memory or
-  // staged in LDS, indexed by `node`)
-  auto entry = [&](const float *adj, const float *vel, int node, const float *N3, const float *dN3,
-                   const float *d2N3, bool g2p) {
+  auto entry = [&](int node, const float *N3, const float *dN3, const float *d2N3, bool g2p) {
     float wgt, gr[3], H[6];
     entry_derivs(N3, dN3, d2N3, wgt, gr, H);
     float mb, Pb[3] = {0.f, 0.f, 0.f}, fb[3] = {0.f, 0.f, 0.f};
-    load_node_adj<D>(adj, node, mb, Pb, fb);
+    load_node_adj<D>(nbar, node, mb, Pb, fb);
     // gs: the weight's scalar factor; wv = L_bar v_nt - V sigma^T f_bar
     float gs = mb, wv[3] = {0.f, 0.f, 0.f};
 #pragma unroll
@@ -3320,7 +3319,7 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
       for (int a = 0; a < D; ++a) wv[b] -= Sv[a][b] * fb[a];
     if (g2p) {
       float vnt[3] = {0.f, 0.f, 0.f}, dvn[3] = {0.f, 0.f, 0.f};
-      load_node_vel<D, true>(vel, node, vnt, dvn);
+      load_node_vel<D, true>(nodes.vel, node, vnt, dvn);
 #pragma unroll
       for (int b = 0; b < D; ++b) gs += vnt[b] * vpb[b] + dvn[b] * dvb[b];
 #pragma unroll
@@ -3349,7 +3348,7 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
   bool leaves = false;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    const int stride = a == 0 ? 1 : (a == 1 ? g.num_cells[0] : g.num_cells[0] * g.num_cells[1]);
+    const int stride = a == 0 ? 1 : g.num_cells[0];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (a < D && e < E) {
@@ -3390,10 +3389,10 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
       spline_eval<SF>(r, type, g.inv_cell_size, n3[a], d3[a]);
       h3[a] = spline_d2<SF>(r, type, g.inv_cell_size);
     }
-    entry(nbar, nodes.vel, (int)lin, n3, d3, h3, false);
+    entry((int)lin, n3, d3, h3, false);
   };
-  // the window's offsets along y (and z) are picked by selects, so the
-  // in-grid entries stay unrolled without indexing registers at run time
+  // the window's offset along y is picked by selects, so the in-grid entries
+  // stay unrolled without indexing registers at run time
   auto pick = [](const auto *a, int k) { return k == 0 ? a[0] : (k == 1 ? a[1] : (k == 2 ? a[2] : a[3])); };
   {
 #pragma unroll 1
@@ -3401,17 +3400,14 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
       const int oy = pick(off[1], sub);
       const float Ny = pick(N[1], sub), dNy = pick(dN[1], sub), d2Ny = pick(d2N[1], sub);
 #pragma unroll
-      for (int ex = 0; ex < E; ++ex)
-#pragma unroll
-        for (int ez = 0; ez < EZ; ++ez) {
-          const float n3[3] = {N[0][ex], Ny, N[2][ez]}, d3[3] = {dN[0][ex], dNy, dN[2][ez]},
-                      h3[3] = {d2N[0][ex], d2Ny, d2N[2][ez]};
-          entry(nbar, nodes.vel, off[0][ex] + oy + off[2][ez], n3, d3, h3, true);
-        }
+      for (int ex = 0; ex < E; ++ex) {
+        const float n3[3] = {N[0][ex], Ny, 1.f}, d3[3] = {dN[0][ex], dNy, 0.f}, h3[3] = {d2N[0][ex], d2Ny, 0.f};
+        entry(off[0][ex] + oy, n3, d3, h3, true);
+      }
       if (leaves && prm.wrap_quirk) {
 #pragma unroll 1
-        for (int e = 0; e < E * EZ; ++e) {
-          const int e3[3] = {e % E, D > 1 ? sub : 0, D > 2 ? e / E : 0};
+        for (int e = 0; e < E; ++e) {
+          const int e3[3] = {e, D > 1 ? sub : 0, 0};
           wrap_entry(e3);
         }
       }
@@ -3463,8 +3459,9 @@ __global__ __launch_bounds__(256) void p2g_adjoint_kernel(pmpm_params prm, pmpm_
 // Lanes per particle of the adjoint P2G: one once that fills the chip
 // (kAdjointLanesWanted), four below, sixteen while a lane's chain is what counts
 // (3D, windows of 3 and 4; adjoint step, cubic: 1,152 particles 54 us with four
-// and 49 with sixteen, 14,784: 55 and 52, 25,088: 62 and 70). PMPM_ADJOINT_P2G_LANES=1, 4 or 16 in the environment overrides the choice (read at every launch), so the
-// layouts can be checked against each other.
+// and 49 with sixteen, 14,784: 55 and 52, 25,088: 62 and 70).
+// PMPM_ADJOINT_P2G_LANES=1, 4 or 16 in the environment overrides the choice
+// (read at every launch), so the layouts can be checked against each other.
 constexpr int kAdjointLanesWanted = 256 * 4 * 64 * 3;
 constexpr int kAdjointRowLanes = 16384;
 inline int adjoint_p2g_lanes(int n) {
